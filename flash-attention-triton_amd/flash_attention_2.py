@@ -107,7 +107,6 @@ def _assert_forward_inputs(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ma
     assert q.is_cuda and k.is_cuda and v.is_cuda, "All tensors must reside on CUDA device"
     assert q.dtype == k.dtype == v.dtype, "All tensors must be the same type"
     assert q.dtype in _COMPUTE_DTYPES, "Supports only fp16 and bf16"
-    assert q.stride(-1) == k.stride(-1) == v.stride(-1) == 1, "Last dimension must be contiguous"
 
 
 def _flash_attention_forward(
@@ -137,6 +136,7 @@ def _flash_attention_forward(
     _, _, seqlen_k, _ = k.shape
 
     _assert_forward_inputs(q, k, v, max_headdim)
+    assert q.stride(-1) == k.stride(-1) == v.stride(-1) == 1, "Last dimension must be contiguous"
 
     output = torch.empty_like(q)
     softmax_scale = softmax_scale or 1.0 / math.sqrt(headdim)
@@ -396,17 +396,17 @@ def _apply(q, k, v, softmax_scale, kernels_config):  # noqa: ANN001, ANN202
     """Record the attention in the autograd graph: the C++ node when it is built, else the Python class.
 
     With the C++ node the reference's forward wrapper (flash_attention_2.py:283-384) is spelt out
-    here: casts and copies are ordinary differentiable operations in front of the node, the input
-    checks are the launcher's, a negative scale is folded into the sign of q.
+    here: casts are ordinary differentiable operations in front of the node, the input checks are the
+    launcher's, a negative scale is folded into the sign of q.  The node takes strided views and copies
+    only what the kernels cannot read.
     """
     node = _cpp_node()
     if node is None or kernels_config.atomic_dq:  # the C++ node always lets the table choose its backward row
         return FlashAttentionV2Function.apply(q, k, v, softmax_scale, kernels_config)
     initial_dtype = q.dtype
     compute_dtype = _compute_dtype(initial_dtype)
-    if not (q.dtype == k.dtype == v.dtype == compute_dtype
-            and q.is_contiguous() and k.is_contiguous() and v.is_contiguous()):
-        q, k, v = [proj.contiguous().to(compute_dtype) for proj in (q, k, v)]
+    if not q.dtype == k.dtype == v.dtype == compute_dtype:
+        q, k, v = [proj.to(compute_dtype) for proj in (q, k, v)]
     _assert_forward_inputs(q, k, v, kernels_config.max_headdim)
     scale = softmax_scale or 1.0 / math.sqrt(q.shape[-1])
     if scale < 0:

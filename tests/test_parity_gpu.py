@@ -530,6 +530,26 @@ def test_non_contiguous_and_mixed_inputs(fa):
     _assert_close("o (fp64 in)", out64, want[0])
 
 
+@pytest.mark.parametrize("d,pad,offset", [(64, 0, 0), (128, 8, 0), (80, 0, 0), (64, 4, 0), (64, 0, 4), (50, 0, 0), (256, 0, 0)])
+def test_strided_views_equal_contiguous_copies(fa, d, pad, offset):
+    """Transposed slices of one packed projection, with row padding or a storage offset that breaks the
+    16-byte alignment (copied then), and a strided output gradient: the same bits as contiguous copies."""
+    b, h, n = 2, 3, 200
+    gen = torch.Generator().manual_seed(7)
+    packed = torch.randn(offset + b * n * (3 * h * d + pad), generator=gen).to(torch.bfloat16).cuda()
+    rows = packed[offset:].view(b, n, 3 * h * d + pad)[..., : 3 * h * d].view(b, n, 3, h, d)
+    views = [rows[:, :, i].transpose(1, 2).detach().requires_grad_(True) for i in range(3)]
+    copies = [t.detach().contiguous().requires_grad_(True) for t in views]
+    d_o = torch.randn((b, n, h, d), generator=gen).to(torch.bfloat16).cuda().transpose(1, 2)
+    got, want = fa.flash_attention_v2(*views), fa.flash_attention_v2(*copies)
+    assert got.is_contiguous()
+    pairs = [(got, want), *zip(torch.autograd.grad(got, views, d_o), torch.autograd.grad(want, copies, d_o.contiguous()))]
+    with torch.no_grad():
+        pairs.append((fa.flash_attention_v2(*views), fa.flash_attention_v2(*copies)))
+    for x, y in pairs:
+        assert torch.equal(x, y)
+
+
 def test_zero_scale_means_default_and_explicit_scale_is_used(fa):
     """`softmax_scale or default`: 0.0 selects 1/sqrt(D) (flash_attention_2.py:94)."""
     q, k, v, _ = _seeded((1, 2, 96, 64), (1, 2, 96, 64), torch.bfloat16)
