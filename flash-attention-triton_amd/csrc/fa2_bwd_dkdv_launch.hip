@@ -1,7 +1,7 @@
 // Instantiates and launches the dK/dV kernels.
 #include <algorithm>
 
-#include "fa2_bwd_dkdv.hpp"
+#include "fa2_bwd_dkdv_pair.hpp"
 #include "fa2_launch.hpp"
 
 namespace fa2 {
@@ -28,11 +28,26 @@ void launch_atomic(int dp, const BwdParams &p, dim3 grid, dim3 block, hipStream_
   }
 }
 
+template <typename T, bool PAD>
+void launch_pair(int dp, const BwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
+  if (dp == 192)
+    hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 192, PAD>), grid, block, 0, s, p);
+  else
+    hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 256, PAD>), grid, block, 0, s, p);
+}
+
 template <typename T>
 void launch(int dp, const BwdParams &p, dim3 grid, hipStream_t s) {
   const dim3 block(64 * kDkvWaves);
   if (p.dq_accum != nullptr) {  // the caller checked seqpar_atomic_ok
     launch_atomic<T>(dp, p, grid, block, s);
+    return;
+  }
+  if (dkdv_pair_ok(dp, p)) {
+    if (p.headdim == dp)
+      launch_pair<T, false>(dp, p, grid, block, s);
+    else
+      launch_pair<T, true>(dp, p, grid, block, s);
     return;
   }
   if (dkdv_direct_ok(dp, p)) {

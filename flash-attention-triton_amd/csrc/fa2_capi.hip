@@ -282,7 +282,8 @@ int bwd_impl(const fa2_bwd_args &a, void *stream) {
   // The dK/dV kernel keeps the table's group size at every head count: with one or two workgroups
   // per CU its drain is short either way, and measured at 96 heads the single group is 1-2 % slower.
   pk.head_group = kTable[cfg].head_group;
-  pk.n_tiles = (a.seqlen_k + kDkvBlockKV - 1) / kDkvBlockKV;
+  const int block_kv = kTable[cfg].dq_atomic ? kDkvBlockKV : fa2::dkdv_block_kv(dp, pk);
+  pk.n_tiles = (a.seqlen_k + block_kv - 1) / block_kv;
   pq.n_tiles = (a.seqlen_q + kDqBlockQ - 1) / kDqBlockQ;
   const int64_t nwg_k = pk.n_tiles * bh, nwg_q = pq.n_tiles * bh;
   if (nwg_k > 0x7fffffff || nwg_q > 0x7fffffff)

@@ -12,30 +12,38 @@ namespace fa2 {
 // Which kernel a launcher picked (reported to callers that label measurements).
 enum KernelPath { kPathGeneric = 0, kPathDirect = 1 };
 
-// The fast kernels need a head dimension that is a multiple of 8 (whole 16-byte chunks) up to 128
-// (up to 256 in the forward and dQ kernels), 16-byte aligned rows and row offsets inside a tile that
-// fit 32 bits.  A head dimension below the table row's padded one runs the padded variant of the
-// kernel.
+// The fast kernels need a head dimension that is a multiple of 8 (whole 16-byte chunks), 16-byte aligned
+// rows and row offsets inside a tile that fit 32 bits.  A head dimension below the table row's padded one
+// runs the padded variant of the kernel.
 inline bool direct_stride_ok(const Tensor4 &t) { return t.stride_seq < (int64_t(1) << 24); }
 inline bool direct_headdim(int dp, int headdim) {
   return headdim % 8 == 0 && headdim <= dp && (dp == 32 || dp == 64 || dp == 96 || dp == 128);
 }
-// The forward and dQ kernels, which stream K and V, also have fast variants for the rows of 192 and
-// 256 columns (one wave per SIMD, all 160 KiB of LDS).
-inline bool direct_headdim_kv_stream(int dp, int headdim) {
+// The rows of 192 and 256 columns (one wave per SIMD, most or all of the 160 KiB of LDS): forward, dQ and
+// paired dK/dV kernels.
+inline bool direct_headdim_wide(int dp, int headdim) {
   return direct_headdim(dp, headdim) || (headdim % 8 == 0 && headdim <= dp && (dp == 192 || dp == 256));
 }
 inline bool fwd_direct_ok(int dp, const FwdParams &p) {
-  return p.vec && direct_headdim_kv_stream(dp, p.headdim) && direct_stride_ok(p.q) && direct_stride_ok(p.k) &&
+  return p.vec && direct_headdim_wide(dp, p.headdim) && direct_stride_ok(p.q) && direct_stride_ok(p.k) &&
          direct_stride_ok(p.v);
 }
 inline bool dq_direct_ok(int dp, const BwdParams &p) {
-  return p.vec && direct_headdim_kv_stream(dp, p.headdim) && direct_stride_ok(p.k) && direct_stride_ok(p.v);
+  return p.vec && direct_headdim_wide(dp, p.headdim) && direct_stride_ok(p.k) && direct_stride_ok(p.v);
 }
 inline bool dkdv_direct_ok(int dp, const BwdParams &p) {
   return p.vec && direct_headdim(dp, p.headdim) && direct_stride_ok(p.q) && direct_stride_ok(p.d_o) &&
          direct_stride_ok(p.k) && direct_stride_ok(p.v);
 }
+// The paired dK/dV kernel (fa2_bwd_dkdv_pair.hpp) takes the rows of 192 and 256 columns, where a wave
+// cannot hold both accumulators: B=2 H=8 N=4096, 256 columns 275 us against 756 us of the generic kernel,
+// 192 columns 220 us against 337 us.
+inline bool dkdv_pair_ok(int dp, const BwdParams &p) {
+  return dp > 128 && p.vec && direct_headdim_wide(dp, p.headdim) && direct_stride_ok(p.q) &&
+         direct_stride_ok(p.d_o) && direct_stride_ok(p.k) && direct_stride_ok(p.v);
+}
+// Key rows per workgroup of the dK/dV kernel that launch_dkdv picks (p.n_tiles follows from it).
+inline int dkdv_block_kv(int dp, const BwdParams &p) { return dkdv_pair_ok(dp, p) ? kDkvPairBlockKV : kDkvBlockKV; }
 // The sequence-parallel (atomic dQ) kernels: the fast dK/dV kernel's conditions, a head dimension
 // of exactly 32, 64 or 128 and 16-byte aligned dq rows.
 inline bool seqpar_atomic_ok(int dp, const BwdParams &p) {

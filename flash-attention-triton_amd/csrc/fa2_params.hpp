@@ -22,6 +22,7 @@ constexpr int kDqWaves = 4;
 constexpr int kDqBlockQ = 32 * kDqWaves;
 constexpr int kDkvWaves = 4;
 constexpr int kDkvBlockKV = 32 * kDkvWaves;
+constexpr int kDkvPairBlockKV = 64;  // key rows per workgroup of the paired dK/dV kernel (two waves share 32)
 // Rows of the streamed operand per LDS tile.
 constexpr int kFwdBlockKV = 64;
 constexpr int kDqBlockKV = 64;

@@ -73,18 +73,19 @@ typedef struct fa2_config_info {
   int fwd_block_kv;   /* key rows per inner step, forward */
   int fwd_waves;      /* wavefronts (64 lanes) per workgroup, forward */
   int bwd_block_q;    /* query rows per inner step, dK/dV kernel */
-  int bwd_block_kv;   /* key rows per workgroup, dK/dV kernel */
+  int bwd_block_kv;   /* key rows per workgroup, dK/dV kernel (the paired kernel: half of it) */
   int bwd_waves;
   int dq_block_q;     /* query rows per workgroup, dQ kernel */
   int dq_block_kv;
   int dq_waves;
   int lds_direct;     /* the row's LDS-direct kernels (global_load_lds into swizzled tiles): 0 none, 1 forward and
-                         backward, 2 forward and dQ only (one wave per SIMD, all 160 KiB of LDS; generic dK/dV) */
+                         backward, 2 forward and dQ (one wave per SIMD, all 160 KiB of LDS), with dK/dV by the
+                         paired kernel: 64 key rows per workgroup, one pass */
   int fwd_wg_per_cu;  /* workgroups that share a CU (what registers and LDS leave room for) */
   int dq_wg_per_cu;
   int dkdv_wg_per_cu;
   int lds_stages;     /* LDS stages of the streamed operand in the kernels of this row */
-  int dkdv_passes;    /* passes of the dK/dV kernel over the query tiles (2: half the columns each) */
+  int dkdv_passes;    /* passes of the generic dK/dV kernel over the query tiles (2: half the columns each) */
   int head_group;     /* (batch, head) pairs dispatched together; head_group / 8 share one XCD's L2 */
   int dq_atomic;      /* 1: sequence-parallel row - one backward kernel, dQ accumulated with fp32 global atomics
                          in a workspace (never picked by FA2_CONFIG_AUTO; selected by id) */

@@ -550,6 +550,18 @@ def test_strided_views_equal_contiguous_copies(fa, d, pad, offset):
         assert torch.equal(x, y)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("nq,nk,d", [(64, 64, 256), (63, 65, 256), (1, 130, 192), (130, 1, 256), (129, 200, 136),
+                                     (300, 64, 248), (191, 191, 192), (257, 320, 256)])
+def test_paired_dkdv_kernel_edges(fa, nq, nk, d, dtype):
+    """dK/dV with two waves per 32 keys: one to five query tiles (an odd and an even number of LDS stages,
+    a ragged first tile, a lone diagonal tile), key tiles no query sees, padded head dimensions."""
+    q, k, v, d_o = _seeded((1, 2, nq, d), (1, 2, nk, d), dtype)
+    want = oracle.naive_backward(q, k, v, d_o, None, torch.float32)
+    for name, g, w in zip(("o", "dq", "dk", "dv"), _run(fa, q, k, v, d_o, None, True), want):
+        _assert_close(name, g, w)
+
+
 def test_zero_scale_means_default_and_explicit_scale_is_used(fa):
     """`softmax_scale or default`: 0.0 selects 1/sqrt(D) (flash_attention_2.py:94)."""
     q, k, v, _ = _seeded((1, 2, 96, 64), (1, 2, 96, 64), torch.bfloat16)
