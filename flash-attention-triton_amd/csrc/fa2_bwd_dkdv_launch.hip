@@ -1,7 +1,7 @@
 // Instantiates and launches the dK/dV kernels.
 #include <algorithm>
 
-#include "fa2_bwd_dkdv_pair.hpp"
+#include "fa2_bwd_dkdv.hpp"
 #include "fa2_launch.hpp"
 
 namespace fa2 {
@@ -12,7 +12,6 @@ void launch_direct(int dp, const BwdParams &p, dim3 grid, dim3 block, hipStream_
   switch (dp) {
     case 32: hipLaunchKernelGGL((bwd_dkdv_direct_kernel<T, 32, kDkvBlockQ, PAD>), grid, block, 0, s, p); break;
     case 64: hipLaunchKernelGGL((bwd_dkdv_direct_kernel<T, 64, kDkvBlockQ, PAD>), grid, block, 0, s, p); break;
-    case 96: hipLaunchKernelGGL((bwd_dkdv_direct_kernel<T, 96, kDkvBlockQ, PAD>), grid, block, 0, s, p); break;
     default: hipLaunchKernelGGL((bwd_dkdv_direct_kernel<T, 128, kDkvBlockQ, PAD>), grid, block, 0, s, p); break;
   }
 }
@@ -30,10 +29,14 @@ void launch_atomic(int dp, const BwdParams &p, dim3 grid, dim3 block, hipStream_
 
 template <typename T, bool PAD>
 void launch_pair(int dp, const BwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
-  if (dp == 192)
-    hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 192, PAD>), grid, block, 0, s, p);
-  else
-    hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 256, PAD>), grid, block, 0, s, p);
+  switch (dp) {
+    case 32: hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 32, PAD>), grid, block, 0, s, p); break;
+    case 64: hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 64, PAD>), grid, block, 0, s, p); break;
+    case 96: hipLaunchKernelGGL((bwd_dkdv_direct_kernel<T, 96, kDkvBlockQ, PAD>), grid, block, 0, s, p); break;
+    case 128: hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 128, PAD>), grid, block, 0, s, p); break;
+    case 192: hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 192, PAD>), grid, block, 0, s, p); break;
+    default: hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 256, PAD>), grid, block, 0, s, p); break;
+  }
 }
 
 template <typename T>
@@ -43,7 +46,7 @@ void launch(int dp, const BwdParams &p, dim3 grid, hipStream_t s) {
     launch_atomic<T>(dp, p, grid, block, s);
     return;
   }
-  if (dkdv_pair_ok(dp, p)) {
+  if (dkdv_pair_ok(dp, p)) {  // always at 96 columns and above 128
     if (p.headdim == dp)
       launch_pair<T, false>(dp, p, grid, block, s);
     else

@@ -18,6 +18,13 @@
 // dS and exchange have only the wave's own MFMAs to hide under, and at 256 columns some fifty copies per
 // tile between the two halves of the register file.
 //
+// At 128 columns and below one accumulator per wave lets two (three at 64) workgroups share a CU, and
+// workgroups of 64 keys fill the chip from fewer heads: dkdv_pair_ok (fa2_launch.hpp) says where that beats
+// bwd_dkdv_direct_kernel and by how much.  The loop is the faster one per shader cycle (67 % of the matrix
+// pipe's cycles busy against 60 % at 16 x 16384 tokens, D=128), but it moves twice the tile bytes, and on
+// long sequences the board's power limit takes the clock down by what the cycles gained (1.69 GHz against
+// 1.93).
+//
 // The two roles are two instantiations of the loop selected once per wave.  With one loop and selects (or
 // branches) on the role inside it the kernel was 2 to 5 % slower (or spilled).  The barriers of the two
 // instantiations match one to one.
@@ -25,7 +32,7 @@
 
 #include <type_traits>
 
-#include "fa2_bwd_dkdv.hpp"
+#include "fa2_common.hpp"
 
 namespace fa2 {
 
@@ -345,12 +352,17 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem) {
 }
 
 template <typename T, int DP, bool PAD>
-__global__ __launch_bounds__(64 * kDkvWaves, (DkvPairLayout<DP>::WG_PER_CU)) void bwd_dkdv_pair_kernel(const BwdParams p) {
+__device__ __forceinline__ void bwd_dkdv_paired(const BwdParams &p) {
   __shared__ __attribute__((aligned(1024))) short smem[DkvPairLayout<DP>::TOTAL_ELEMS];
   if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 1)
     bwd_dkdv_pair<T, DP, PAD, 1>(p, smem);
   else
     bwd_dkdv_pair<T, DP, PAD, 0>(p, smem);
+}
+
+template <typename T, int DP, bool PAD>
+__global__ __launch_bounds__(64 * kDkvWaves, (DkvPairLayout<DP>::WG_PER_CU)) void bwd_dkdv_pair_kernel(const BwdParams p) {
+  bwd_dkdv_paired<T, DP, PAD>(p);
 }
 
 }  // namespace fa2

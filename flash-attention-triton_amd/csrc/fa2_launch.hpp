@@ -35,12 +35,26 @@ inline bool dkdv_direct_ok(int dp, const BwdParams &p) {
   return p.vec && direct_headdim(dp, p.headdim) && direct_stride_ok(p.q) && direct_stride_ok(p.d_o) &&
          direct_stride_ok(p.k) && direct_stride_ok(p.v);
 }
-// The paired dK/dV kernel (fa2_bwd_dkdv_pair.hpp) takes the rows of 192 and 256 columns, where a wave
-// cannot hold both accumulators: B=2 H=8 N=4096, 256 columns 275 us against 756 us of the generic kernel,
-// 192 columns 220 us against 337 us.
+// Where the paired dK/dV kernel (fa2_bwd_dkdv_pair.hpp) is the better one.  Its workgroups are half as long
+// and start faster; its loop reads every Q and dO tile for 64 keys instead of 128.  Time of the other
+// kernel over its own, bf16, (batch, head) pairs x tokens:
+//   192, 256 columns  2.7 at 256, 1.5 at 192 (16 x 4096): always
+//   96 columns        1.02 (4 x 16384) to 1.6 (4 x 4096), 1.05-1.07 on large grids: always
+//   128 columns       1.59 (1 x 16384), 1.24 (4 x 8192), 1.10 (4 x 12288) below 512 workgroups of 128 keys;
+//                     above, 1.05 (64 x 2048), 1.02 (256 x 4096), 0.99 (16 x 4096), but 0.95 (8 x 8192) and
+//                     0.98 (16 x 16384): there its extra tile loads cost board power, and clock
+//   64 columns        1.56 (4 x 4096), 1.31 (64 x 512), 1.13 (4 x 16384) while the other kernel's workgroups
+//                     are all resident (512); 1.16 (256 x 512), 1.09 (256 x 1024), 1.06 (64 x 2048) while
+//                     they are short or few; 0.97 (256 x 2048), 0.93 (64 x 4096) beyond
+//   32 columns        1.72 (4 x 4096), 1.28 (16 x 4096), 1.03 (1024 x 512); 0.96 (256 x 1024), 0.92 beyond
 inline bool dkdv_pair_ok(int dp, const BwdParams &p) {
-  return dp > 128 && p.vec && direct_headdim_wide(dp, p.headdim) && direct_stride_ok(p.q) &&
-         direct_stride_ok(p.d_o) && direct_stride_ok(p.k) && direct_stride_ok(p.v);
+  if (!(p.vec && direct_headdim_wide(dp, p.headdim) && direct_stride_ok(p.q) && direct_stride_ok(p.d_o) &&
+        direct_stride_ok(p.k) && direct_stride_ok(p.v)))
+    return false;
+  if (dp > 128 || dp == 96) return true;
+  const int64_t wgs = (int64_t)((p.seqlen_k + kDkvBlockKV - 1) / kDkvBlockKV) * p.batch * p.nheads;
+  if (dp == 128) return wgs < 2 * kCUs || p.seqlen_q <= 4096;
+  return wgs <= 2 * kCUs || p.seqlen_q <= 512 || (dp == 64 && wgs * p.seqlen_q <= (1 << 21));
 }
 // Key rows per workgroup of the dK/dV kernel that launch_dkdv picks (p.n_tiles follows from it).
 inline int dkdv_block_kv(int dp, const BwdParams &p) { return dkdv_pair_ok(dp, p) ? kDkvPairBlockKV : kDkvBlockKV; }

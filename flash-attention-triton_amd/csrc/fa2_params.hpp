@@ -8,6 +8,8 @@ namespace fa2 {
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 
+constexpr int kCUs = 256;  // compute units of an MI355X
+
 // One (batch, nheads, seqlen, headdim) tensor: base pointer and strides in elements.
 struct Tensor4 {
   void *ptr;

@@ -552,7 +552,8 @@ def test_strided_views_equal_contiguous_copies(fa, d, pad, offset):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("nq,nk,d", [(64, 64, 256), (63, 65, 256), (1, 130, 192), (130, 1, 256), (129, 200, 136),
-                                     (300, 64, 248), (191, 191, 192), (257, 320, 256)])
+                                     (300, 64, 248), (191, 191, 192), (257, 320, 256), (65, 64, 128), (1, 70, 104),
+                                     (193, 130, 96), (63, 200, 72), (130, 129, 64), (257, 257, 40), (64, 65, 32), (191, 1, 24)])
 def test_paired_dkdv_kernel_edges(fa, nq, nk, d, dtype):
     """dK/dV with two waves per 32 keys: one to five query tiles (an odd and an even number of LDS stages,
     a ragged first tile, a lone diagonal tile), key tiles no query sees, padded head dimensions."""
@@ -560,6 +561,21 @@ def test_paired_dkdv_kernel_edges(fa, nq, nk, d, dtype):
     want = oracle.naive_backward(q, k, v, d_o, None, torch.float32)
     for name, g, w in zip(("o", "dq", "dk", "dv"), _run(fa, q, k, v, d_o, None, True), want):
         _assert_close(name, g, w)
+
+
+@pytest.mark.parametrize("b,h,n,d", [(1, 300, 640, 32), (1, 300, 640, 24), (3, 300, 1030, 64), (3, 300, 1030, 40), (1, 16, 4225, 120)])
+def test_dkdv_kernel_of_large_grids(fa, b, h, n, d):
+    """Grids and lengths beyond the paired dK/dV kernel's range (dkdv_pair_ok): the kernel whose waves hold
+    both accumulators, exact and padded head dimensions, ragged lengths; first and last head checked."""
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    q, k, v, d_o = (torch.randn((b, h, n, d), generator=gen, device="cuda").to(torch.bfloat16) for _ in range(4))
+    qg, kg, vg = (t.clone().requires_grad_(True) for t in (q, k, v))
+    grads = torch.autograd.grad(fa.flash_attention_v2(qg, kg, vg), (qg, kg, vg), d_o)
+    for bi, hi in ((0, 0), (b - 1, h - 1)):
+        one = lambda t: t[bi : bi + 1, hi : hi + 1]  # noqa: E731
+        _, *want = _gpu_fp32_oracle(one(q), one(k), one(v), one(d_o), None)
+        for name, g, w in zip(("dq", "dk", "dv"), grads, want):
+            _assert_close(name, one(g).reshape(w.shape), w)
 
 
 def test_zero_scale_means_default_and_explicit_scale_is_used(fa):
