@@ -54,7 +54,6 @@ struct DkvPairLayout {
   static constexpr int TOTAL_ELEMS = XCHG_BASE + XBUFS * kDkvWaves * XCHG_WAVE;
   static constexpr int PATCH_ELEMS = kDkvWaves * 32 * (DP + 8);
   static_assert(STAT_BASE >= PATCH_ELEMS, "the output patch overlays the stages");
-  static constexpr int WG_PER_CU = DP <= 64 ? 3 : DP <= 128 ? 2 : 1;
 };
 
 template <typename T, int DP, bool PAD, int role>
@@ -75,7 +74,7 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem) {
 
   const int BH = p.batch * p.nheads;
   int bh, kt;  // key tile 0 has the longest query range: rank == key tile
-  map_workgroup(blockIdx.x, BH, p.n_tiles, p.head_group, bh, kt);
+  map_workgroup(p.resident_grid ? balanced_index(blockIdx.x, p.resident_grid) : blockIdx.x, BH, p.n_tiles, p.head_group, bh, kt);
   const int b = bh / p.nheads, hd = bh % p.nheads;
   const int kv0 = kt * L::KEYS;
   const int kv0w = kv0 + 32 * (wave >> 1);
@@ -361,7 +360,7 @@ __device__ __forceinline__ void bwd_dkdv_paired(const BwdParams &p) {
 }
 
 template <typename T, int DP, bool PAD>
-__global__ __launch_bounds__(64 * kDkvWaves, (DkvPairLayout<DP>::WG_PER_CU)) void bwd_dkdv_pair_kernel(const BwdParams p) {
+__global__ __launch_bounds__(64 * kDkvWaves, (dkdv_pair_wg_per_cu(DP))) void bwd_dkdv_pair_kernel(const BwdParams p) {
   bwd_dkdv_paired<T, DP, PAD>(p);
 }
 

@@ -285,7 +285,7 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
 
   const int BH = p.batch * p.nheads;
   int bh, rank;
-  map_workgroup(blockIdx.x, BH, p.n_tiles, p.head_group, bh, rank);
+  map_workgroup(p.resident_grid ? balanced_index(blockIdx.x, p.resident_grid) : blockIdx.x, BH, p.n_tiles, p.head_group, bh, rank);
   const int qt = p.n_tiles - 1 - rank;  // the last query tile sees the most keys
   const int b = bh / p.nheads, hd = bh % p.nheads;
   const int q0 = qt * kDqBlockQ;

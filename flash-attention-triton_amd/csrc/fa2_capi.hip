@@ -76,6 +76,9 @@ constexpr int kTableRows = sizeof(kTable) / sizeof(kTable[0]);
 // the heads there are (fa2::equal_head_groups).
 int head_group(int cfg, int64_t heads) { return fa2::equal_head_groups(kTable[cfg].head_group, heads); }
 
+// Size of a grid that fits the chip at once (0 otherwise), for kernels that share a CU `wg_per_cu` times.
+int resident_grid(int64_t nwg, int wg_per_cu) { return nwg <= (int64_t)fa2::kCUs * wg_per_cu ? (int)nwg : 0; }
+
 // The row FA2_CONFIG_AUTO stands for: the first plain row wide enough for the head dimension.
 int pick_config(int headdim) {
   for (int i = 0; i < kTableRows; i++)
@@ -186,6 +189,7 @@ int fwd_impl(const fa2_fwd_args &a, void *stream) {
 
   const int64_t nwg = (int64_t)p.n_qtiles * a.batch * a.nheads;
   if (nwg > 0x7fffffff) return fail(FA2_ERR_TOO_LARGE, "grid of %lld workgroups too large", (long long)nwg);
+  p.resident_grid = resident_grid(nwg, kTable[cfg].fwd_wg_per_cu);
   fa2::launch_fwd(a.dtype == FA2_DTYPE_BF16, kTable[cfg].headdim_padded, kTable[cfg].fwd_exp_folded != 0, p,
                   dim3((unsigned)nwg), reinterpret_cast<hipStream_t>(stream));
   return launch_status("fa2_fwd launch");
@@ -288,6 +292,10 @@ int bwd_impl(const fa2_bwd_args &a, void *stream) {
   const int64_t nwg_k = pk.n_tiles * bh, nwg_q = pq.n_tiles * bh;
   if (nwg_k > 0x7fffffff || nwg_q > 0x7fffffff)
     return fail(FA2_ERR_TOO_LARGE, "grid of %lld workgroups too large", (long long)std::max(nwg_k, nwg_q));
+
+  const bool pair = block_kv == fa2::kDkvPairBlockKV;
+  pk.resident_grid = resident_grid(nwg_k, pair ? fa2::dkdv_pair_wg_per_cu(dp) : kTable[cfg].dkdv_wg_per_cu);
+  pq.resident_grid = resident_grid(nwg_q, kTable[cfg].dq_wg_per_cu);
 
   auto run_dkdv = [&]() {
     fa2::launch_dkdv(bf16, dp, pk, dim3((unsigned)nwg_k), s);

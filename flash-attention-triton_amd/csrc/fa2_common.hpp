@@ -233,6 +233,20 @@ __host__ __device__ __forceinline__ void map_workgroup(int i, int heads, int til
   rank = r / gsize;
 }
 
+// Order in which a grid that fits the chip at once takes its tiles.  Workgroups i, i + kCUs, i + 2 kCUs ...
+// of such a grid share a CU (they are handed out round-robin, all before the first one ends; read back from
+// the hardware id registers), and with tiles ordered by weight every CU would get the tiles of one weight
+// rank of each round: the first CU the heaviest of all of them.  Every second round is therefore walked
+// backwards, in steps of 8 workgroups, so that a head stays on its XCD.  (bf16, in us: 64 x 1024, D=128:
+// forward 32 -> 28, dQ 40 -> 33; 8 x 4096, D=128: dK/dV 82 -> 76; 16 x 4096, D=128: forward 81 -> 77,
+// dQ 103 -> 97; 8 x 8192, D=64: forward 96 -> 93.)
+__host__ __device__ __forceinline__ int balanced_index(int i, int total) {
+  const int base = i / kCUs * kCUs;
+  if (!((i / kCUs) & 1)) return i;
+  const int steps = min(kCUs, total - base) / 8, r = i - base;
+  return r / 8 < steps ? base + (steps - 1 - r / 8) * 8 + r % 8 : i;
+}
+
 }  // namespace fa2
 
 // ------------------------------------------------------------------------------------------

@@ -319,7 +319,7 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
 
   const int BH = p.batch * p.nheads;
   int bh, rank;
-  map_workgroup(blockIdx.x, BH, p.n_qtiles, p.head_group, bh, rank);
+  map_workgroup(p.resident_grid ? balanced_index(blockIdx.x, p.resident_grid) : blockIdx.x, BH, p.n_qtiles, p.head_group, bh, rank);
   const int qt = p.n_qtiles - 1 - rank;  // the last query tile sees the most keys
   const int b = bh / p.nheads, hd = bh % p.nheads;
   const int q0 = qt * kFwdBlockQ;

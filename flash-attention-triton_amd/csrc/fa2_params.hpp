@@ -25,6 +25,8 @@ constexpr int kDqBlockQ = 32 * kDqWaves;
 constexpr int kDkvWaves = 4;
 constexpr int kDkvBlockKV = 32 * kDkvWaves;
 constexpr int kDkvPairBlockKV = 64;  // key rows per workgroup of the paired dK/dV kernel (two waves share 32)
+// Its workgroups per CU: registers and LDS leave room for three up to 64 columns, two up to 128.
+constexpr int dkdv_pair_wg_per_cu(int dp) { return dp <= 64 ? 3 : dp <= 128 ? 2 : 1; }
 // Rows of the streamed operand per LDS tile.
 constexpr int kFwdBlockKV = 64;
 constexpr int kDqBlockKV = 64;
@@ -36,6 +38,7 @@ struct FwdParams {
   int batch, nheads, seqlen_q, seqlen_k, headdim, seqlen_q_rounded;
   int n_qtiles;
   int head_group;  // (batch, head) pairs whose tiles are dispatched together (multiple of 8)
+  int resident_grid;  // number of workgroups when all of them fit the chip at once, else 0: see balanced_index
   float scale;       // softmax scale (natural units)
   float scale_log2;  // scale * log2(e)
   int vec;           // 16-byte global accesses are legal for every tensor
@@ -55,6 +58,7 @@ struct BwdParams {
   int batch, nheads, seqlen_q, seqlen_k, headdim, seqlen_q_rounded;
   int n_tiles;  // key tiles (dK/dV kernel) or query tiles (dQ kernel)
   int head_group;  // (batch, head) pairs whose tiles are dispatched together (multiple of 8)
+  int resident_grid;  // number of workgroups when all of them fit the chip at once, else 0: see balanced_index
   float scale, scale_log2;
   int vec;
 };

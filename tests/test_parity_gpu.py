@@ -578,6 +578,19 @@ def test_dkdv_kernel_of_large_grids(fa, b, h, n, d):
             _assert_close(name, one(g).reshape(w.shape), w)
 
 
+@pytest.mark.parametrize("b,h,n,d", [(1, 33, 1000, 128), (1, 31, 2000, 128), (1, 85, 1100, 64), (3, 29, 650, 32), (1, 9, 3700, 96)])
+def test_grids_that_fit_the_chip_at_once(fa, b, h, n, d):
+    """Grids of 257 to 1024 workgroups, none a multiple of 256, walk every second round of 256 backwards
+    (balanced_index): every tile of every head exactly once."""
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    q, k, v, d_o = (torch.randn((b, h, n, d), generator=gen, device="cuda").to(torch.bfloat16) for _ in range(4))
+    qg, kg, vg = (t.clone().requires_grad_(True) for t in (q, k, v))
+    out = fa.flash_attention_v2(qg, kg, vg)
+    grads = torch.autograd.grad(out, (qg, kg, vg), d_o)
+    for name, g, w in zip(("o", "dq", "dk", "dv"), (out, *grads), _gpu_fp32_oracle(q, k, v, d_o, None)):
+        _assert_close(name, g.reshape(w.shape), w)
+
+
 def test_zero_scale_means_default_and_explicit_scale_is_used(fa):
     """`softmax_scale or default`: 0.0 selects 1/sqrt(D) (flash_attention_2.py:94)."""
     q, k, v, _ = _seeded((1, 2, 96, 64), (1, 2, 96, 64), torch.bfloat16)
