@@ -268,7 +268,9 @@ struct DqDirectLayout {
 // launched after this one; the separate preprocess launch disappears.
 // PAD: the head dimension is a multiple of 8 below DP; the columns beyond it are zeros in LDS and in
 // the register fragments, and are not stored.
-template <typename T, int DP, int BKV, bool FUSE_DELTA, bool PAD>
+// KG: key groups, as in the forward (fa2_fwd.hpp).  With two the waves' sums over the even and the odd
+// 32-key blocks are added at the end, in that order: B=1 H=8 N=4096 D=128, bf16: 72.5 -> 58.5 us.
+template <typename T, int DP, int BKV, bool FUSE_DELTA, bool PAD, int KG = 1>
 __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_direct_kernel(const BwdParams p) {
   using L = DqDirectLayout<DP, BKV>;
   constexpr int KS = DP / 16, DB = DP / 32, LP = L::LP;
@@ -288,8 +290,10 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
   map_workgroup(p.resident_grid ? balanced_index(blockIdx.x, p.resident_grid) : blockIdx.x, BH, p.n_tiles, p.head_group, bh, rank);
   const int qt = p.n_tiles - 1 - rank;  // the last query tile sees the most keys
   const int b = bh / p.nheads, hd = bh % p.nheads;
-  const int q0 = qt * kDqBlockQ;
-  const int q0w = q0 + 32 * wave;
+  constexpr int BQ = kDqBlockQ / KG;  // query rows of the workgroup
+  const int rg = wave % (kDqWaves / KG), kg = wave / (kDqWaves / KG);  // row group, key group
+  const int q0 = qt * BQ;
+  const int q0w = q0 + 32 * rg;
 
   const short *Q = (const short *)p.q.ptr + b * p.q.stride_batch + hd * p.q.stride_head;
   const short *K = (const short *)p.k.ptr + b * p.k.stride_batch + hd * p.k.stride_head;
@@ -302,9 +306,13 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
   const int seqlen_k = p.seqlen_k;
   const float scale_log2 = p.scale_log2;
 
-  const int kv_end = min(q0 + kDqBlockQ, seqlen_k);
+  const int kv_end = min(q0 + BQ, seqlen_k);
   const int n_tiles = (kv_end + BKV - 1) / BKV;
-  const int n_mine = min((kv_end + BLK - 1) / BLK, q0w / BLK + 1);  // 32-key blocks of this wave
+  // 32-key blocks of this wave: with two key groups those in its group's half of the tiles.  The wave's
+  // i-th block is key block block_at(i) of the sequence.
+  const int n_below = min((kv_end + BLK - 1) / BLK, q0w / BLK + 1);
+  const int n_mine = KG == 1 ? n_below : (n_below - kg + 1) / 2;
+  auto block_at = [&](int i) { return KG == 1 ? i : 2 * i + kg; };
   const int n_full = min(q0w + 1, seqlen_k) / BLK;                   // leading blocks without mask
   const int n_inside = seqlen_k / BKV;
 
@@ -352,7 +360,7 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
       }
       delta = sum_over_halves(part);  // 0 for rows beyond the sequence (loads return zeros)
       float *dout = p.delta_out + (int64_t)bh * p.seqlen_q_rounded;
-      if (h == 0 && ok) dout[row] = delta;
+      if (h == 0 && kg == 0 && ok) dout[row] = delta;
       if (qt == p.n_tiles - 1)  // rows [seqlen_q, seqlen_q_rounded) are defined to be zero
         for (int r = p.seqlen_q + tid; r < p.seqlen_q_rounded; r += 64 * kDqWaves) dout[r] = 0.f;
     } else if (ok) {
@@ -362,7 +370,7 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
 
   // Swizzled fragment addresses (32-bit LDS pointers).  knext: K rows of the tile the next block
   // lies in; vrow: V rows of the current tile; klo/khi: transposed K fragments of the current tile.
-  const lds_cptr lds0 = to_lds(smem);
+  const lds_cptr lds0 = to_lds(smem) + kg * BLK * LP;  // the key group's half of every tile
   lds_cptr knext[KS], vrow[KS], klo[DB], khi[DB];
 #pragma unroll
   for (int ks = 0; ks < KS; ks++) {
@@ -416,7 +424,7 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
     constexpr int HALF = decltype(half_tag)::value;
     constexpr bool SPREAD = decltype(spread_tag)::value;
     constexpr bool INNER = decltype(inner_tag)::value;
-    const int kt = j / 2 + 2, vt = j / 2 + 1;  // tiles loaded during this block (SPREAD)
+    const int kt = j / (2 / KG) + 2, vt = j / (2 / KG) + 1;  // tiles loaded during this block (SPREAD)
     if (!INNER && j >= n_mine) {
       if (SPREAD) {  // not reached: skipped blocks lie in the last two tiles, which load nothing
         issue_k(kt);
@@ -435,12 +443,12 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
       ring[ks] = lds_read_128(vrow[ks] + HOFF);
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (!INNER && j >= n_full) {
+    if (!INNER && block_at(j) >= n_full) {
       // Diagonal and ragged blocks: masked scores become -inf, their probabilities 0.  The empty asm
       // statement keeps this a branch that interior blocks skip (the test is cheap enough that the
       // optimiser would otherwise run it for every block).
       asm volatile("");
-      const int lim = key_limit - j * BLK;
+      const int lim = key_limit - block_at(j) * BLK;
 #pragma unroll
       for (int i = 0; i < 16; i++)
         if (8 * (i >> 2) + (i & 3) > lim) s[i] = -INFINITY;
@@ -472,7 +480,7 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
       constexpr int HALF_SLOTS = KS / 2;
       const int ks2 = slot / DB, db = slot % DB;
       dqacc[db] = Elem<T>::mfma(ring[slot], dsf[ks2], dqacc[db]);
-      ring[slot] = lds_read_128(knext[slot] + (HALF == 0 ? BLK * LP : 0));
+      ring[slot] = lds_read_128(knext[slot] + (HALF == 0 && KG == 1 ? BLK * LP : 0));
       if (slot < HALF_SLOTS) {
 #pragma unroll
         for (int i = part(8, HALF_SLOTS, slot); i < part(8, HALF_SLOTS, slot + 1); i++)
@@ -501,12 +509,13 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
     }
   };
   auto tile = [&](int t, auto spread_tag) __attribute__((always_inline)) {
-    block(2 * t, std::integral_constant<int, 0>{}, spread_tag, spread_tag);
-    // knext -> K tile t+1 before the second block prefetches from it.
+    if constexpr (KG == 1) block(2 * t, std::integral_constant<int, 0>{}, spread_tag, spread_tag);
+    // knext -> K tile t+1 before the tile's last block prefetches from it.
     const int dk = k_step(t);
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) knext[ks] += dk;
-    block(2 * t + 1, std::integral_constant<int, 1>{}, std::false_type{}, spread_tag);
+    if constexpr (KG == 1) block(2 * t + 1, std::integral_constant<int, 1>{}, std::false_type{}, spread_tag);
+    else block(t, std::integral_constant<int, 0>{}, spread_tag, spread_tag);
     end_tile(t);
   };
   int t = 0;
@@ -518,7 +527,34 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
     tile(t, std::false_type{});
   }
 
-  short *patch = smem + wave * 32 * (DP + 8);
+  // Two key groups: the second hands its accumulator to the first, which adds and stores.  The areas
+  // overlay the stages: the loop's last barrier ordered them after all reads.
+  constexpr int MERGE_FLOATS = KG == 1 ? 0 : DB * 16 * 64;  // per row group
+  static_assert(KG == 1 || 2 * MERGE_FLOATS * 2 + 2 * 32 * (DP + 8) <= L::TOTAL_ELEMS, "merge area and patch overlay the stages");
+  if constexpr (KG > 1) {
+    // (The lane number is formed anew: kept across the loop, it was the one register too many.)
+    const int here = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    float *area = reinterpret_cast<float *>(smem) + rg * MERGE_FLOATS + 4 * here;
+    if (kg == 1) {
+#pragma unroll
+      for (int db = 0; db < DB; db++)
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+          *reinterpret_cast<f32x4 *>(area + (db * 4 + g) * 256) =
+              f32x4{dqacc[db][4 * g], dqacc[db][4 * g + 1], dqacc[db][4 * g + 2], dqacc[db][4 * g + 3]};
+    }
+    __syncthreads();
+    if (kg == 1) return;
+#pragma unroll
+    for (int db = 0; db < DB; db++)
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        const f32x4 x = *reinterpret_cast<const f32x4 *>(area + (db * 4 + g) * 256);
+#pragma unroll
+        for (int e = 0; e < 4; e++) dqacc[db][4 * g + e] += x[e];
+      }
+  }
+  short *patch = smem + KG * MERGE_FLOATS * 2 + wave * 32 * (DP + 8);
   store_transposed_acc<T, DP>(dqacc, p.scale, patch, DQ + (int64_t)q0w * p.dq.stride_seq,
                               p.dq.stride_seq, p.seqlen_q - q0w, hdim, true);
 }

@@ -181,11 +181,12 @@ int fwd_impl(const fa2_fwd_args &a, void *stream) {
   p.seqlen_k = a.seqlen_k;
   p.headdim = a.headdim;
   p.seqlen_q_rounded = a.seqlen_q_rounded;
-  p.n_qtiles = (a.seqlen_q + kFwdBlockQ - 1) / kFwdBlockQ;
   p.head_group = head_group(cfg, (int64_t)a.batch * a.nheads);
   p.scale = a.softmax_scale;
   p.scale_log2 = a.softmax_scale * fa2::kLog2e;
   p.vec = vec_ok(p.q, a.headdim) && vec_ok(p.k, a.headdim) && vec_ok(p.v, a.headdim) && vec_ok(p.o, a.headdim);
+  const int block_q = kFwdBlockQ / fa2::fwd_key_groups(kTable[cfg].headdim_padded, p);
+  p.n_qtiles = (a.seqlen_q + block_q - 1) / block_q;
 
   const int64_t nwg = (int64_t)p.n_qtiles * a.batch * a.nheads;
   if (nwg > 0x7fffffff) return fail(FA2_ERR_TOO_LARGE, "grid of %lld workgroups too large", (long long)nwg);
@@ -288,7 +289,8 @@ int bwd_impl(const fa2_bwd_args &a, void *stream) {
   pk.head_group = kTable[cfg].head_group;
   const int block_kv = kTable[cfg].dq_atomic ? kDkvBlockKV : fa2::dkdv_block_kv(dp, pk);
   pk.n_tiles = (a.seqlen_k + block_kv - 1) / block_kv;
-  pq.n_tiles = (a.seqlen_q + kDqBlockQ - 1) / kDqBlockQ;
+  const int block_q = kDqBlockQ / fa2::dq_key_groups(dp, pq);
+  pq.n_tiles = (a.seqlen_q + block_q - 1) / block_q;
   const int64_t nwg_k = pk.n_tiles * bh, nwg_q = pq.n_tiles * bh;
   if (nwg_k > 0x7fffffff || nwg_q > 0x7fffffff)
     return fail(FA2_ERR_TOO_LARGE, "grid of %lld workgroups too large", (long long)std::max(nwg_k, nwg_q));

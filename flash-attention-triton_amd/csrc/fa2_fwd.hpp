@@ -284,8 +284,6 @@ struct FwdDirectLayout {
   static constexpr int TOTAL_ELEMS = (STAGE_ELEMS > PATCH_ELEMS) ? STAGE_ELEMS : PATCH_ELEMS;
 };
 
-
-
 // Which half of a 64-row tile a step works on, and whether the step is known to lie well inside
 // the wave's key range (no block-count tests needed).
 template <int HALF, bool INNER>
@@ -296,11 +294,17 @@ struct HalfTag {
 
 // PAD: the head dimension is a multiple of 8 below DP; the columns beyond it are zeros in LDS and in
 // the register fragments, and are not stored.
+// KG: key groups.  With one, a wave multiplies both 32-key blocks of every tile by its 32 query rows.  With
+// two, waves 0, 1 take the first and waves 2, 3 the second block of every tile, for the same 64 rows, and the
+// results are merged at the end: half the blocks per wave, for grids that do not fill the chip (key_groups
+// in fa2_launch.hpp has the rule).  B=1 H=8 N=4096 D=128, bf16: 62.6 -> 48.0 us; B=2 H=4 N=512 D=64, fp16:
+// 9.9 -> 7.1 us.  There a wave's own chain is what takes the time: QK^T, softmax and PV of one block after
+// the other at 0.5 us each, with at most one other wave on its SIMD.
 // PRE: the Q fragments are multiplied by scale * log2(e) and rounded to half precision once, and
 // every score chain starts from minus the maximum in use (the MFMA's C operand), so that the score
 // MFMAs deliver the base-2 exponents themselves and no multiply-add is left in front of the
 // exponentials.
-template <typename T, int DP, int BKV, bool PAD, bool PRE>
+template <typename T, int DP, int BKV, bool PAD, bool PRE, int KG = 1>
 __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direct_kernel(const FwdParams p) {
   using L = FwdDirectLayout<DP, BKV>;
   constexpr int KS = DP / 16, DB = DP / 32, LP = L::LP;
@@ -322,8 +326,10 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
   map_workgroup(p.resident_grid ? balanced_index(blockIdx.x, p.resident_grid) : blockIdx.x, BH, p.n_qtiles, p.head_group, bh, rank);
   const int qt = p.n_qtiles - 1 - rank;  // the last query tile sees the most keys
   const int b = bh / p.nheads, hd = bh % p.nheads;
-  const int q0 = qt * kFwdBlockQ;
-  const int q0w = q0 + 32 * wave;
+  constexpr int BQ = kFwdBlockQ / KG;  // query rows of the workgroup
+  const int rg = wave % (kFwdWaves / KG), kg = wave / (kFwdWaves / KG);  // row group, key group
+  const int q0 = qt * BQ;
+  const int q0w = q0 + 32 * rg;
 
   const short *Q = (const short *)p.q.ptr + b * p.q.stride_batch + hd * p.q.stride_head;
   const short *K = (const short *)p.k.ptr + b * p.k.stride_batch + hd * p.k.stride_head;
@@ -336,10 +342,14 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
   const int seqlen_k = p.seqlen_k;
   const float scale_log2 = p.scale_log2;
 
-  const int kv_end = min(q0 + kFwdBlockQ, seqlen_k);
+  const int kv_end = min(q0 + BQ, seqlen_k);
   const int n_tiles = (kv_end + BKV - 1) / BKV;
-  // Blocks this wave multiplies: those that exist and start at or before its last query row.
-  const int n_mine = min((kv_end + BLK - 1) / BLK, q0w / BLK + 1);
+  // Blocks this wave multiplies: those that exist, start at or before its last query row and (with two key
+  // groups) lie in the half of the tiles that is its group's.  The wave's i-th block is key block
+  // block_at(i) of the sequence.
+  const int n_below = min((kv_end + BLK - 1) / BLK, q0w / BLK + 1);
+  const int n_mine = KG == 1 ? n_below : (n_below - kg + 1) / 2;
+  auto block_at = [&](int i) { return KG == 1 ? i : 2 * i + kg; };
   // Leading blocks that need no mask (entirely at or below the wave's first row, inside the keys).
   const int n_full = min(q0w + 1, seqlen_k) / BLK;
   const int n_inside = seqlen_k / BKV;  // tiles whose every row exists
@@ -364,31 +374,38 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
   // fragments.  Loaded straight into registers, a wave's fragment loads touch 32 different rows
   // each, eight times over, and keep the CU's address path busy for a microsecond per workgroup.
   // Rows beyond the sequence are read from its last row: finite values whose results are never stored.
-  constexpr unsigned Q_LO = 2u * (unsigned)(L::K_BASE + 2 * L::TILE_ELEMS);
+  // With two key groups, whose waves take one block per tile, tile t brings in K_{t+3}, K_2 is loaded here
+  // as well and the 64 query rows go through the second V stage.
   constexpr unsigned Q_HI = 2u * (unsigned)(L::V_BASE + 1 * L::TILE_ELEMS);
+  constexpr unsigned Q_LO = KG == 1 ? 2u * (unsigned)(L::K_BASE + 2 * L::TILE_ELEMS) : Q_HI;
+  constexpr int K_AHEAD = KG == 1 ? 2 : 3;  // tile t loads K tile t + K_AHEAD
   const TileLoader<DP, BKV, kFwdWaves, PAD> qload(Q + (int64_t)q0 * p.q.stride_seq, p.q.stride_seq, hdim / 8);
   const int q_rows = p.seqlen_q - q0;  // rows of this query tile that exist (>= 1)
   issue_k(0);
   if (q_rows >= BKV) qload.issue(0, lds_base + Q_LO); else qload.issue_clamped(0, q_rows, lds_base + Q_LO);
-  if (q_rows >= 2 * BKV) qload.issue(BKV, lds_base + Q_HI); else qload.issue_clamped(BKV, q_rows, lds_base + Q_HI);
+  if (KG == 1) {
+    if (q_rows >= 2 * BKV) qload.issue(BKV, lds_base + Q_HI); else qload.issue_clamped(BKV, q_rows, lds_base + Q_HI);
+  }
   issue_v(0);
   if (n_tiles > 1) issue_k(1);
+  if (KG > 1 && n_tiles > 2) issue_k(2);
 
   // Fragment addresses (swizzled, 32-bit LDS pointers).  kcur points into the stage of the K tile
   // after the current one, vcur into the stage of the current V tile; both advance by a uniform
   // amount per tile, and half-tile offsets are immediates.
   lds_cptr kcur[KS], vlo[DB], vhi[DB];
   const lds_cptr lds0 = to_lds(smem);
+  const lds_cptr half0 = lds0 + kg * BLK * LP;  // the key group's half of every tile
 #pragma unroll
-  for (int ks = 0; ks < KS; ks++) kcur[ks] = lds0 + L::K_BASE + swz_off<LP>(c, 2 * ks + h);
+  for (int ks = 0; ks < KS; ks++) kcur[ks] = half0 + L::K_BASE + swz_off<LP>(c, 2 * ks + h);
   {
     const int rowlo = 4 * h + (i16 >> 2);
     const int sub = (i16 & 1) * 4;
 #pragma unroll
     for (int db = 0; db < DB; db++) {
       const int chunk = 4 * db + 2 * g2 + ((i16 & 3) >> 1);
-      vlo[db] = lds0 + L::V_BASE + swz_off<LP>(rowlo, chunk) + sub;
-      vhi[db] = lds0 + L::V_BASE + swz_off<LP>(rowlo + 8, chunk) + sub;
+      vlo[db] = half0 + L::V_BASE + swz_off<LP>(rowlo, chunk) + sub;
+      vhi[db] = half0 + L::V_BASE + swz_off<LP>(rowlo + 8, chunk) + sub;
     }
   }
   // K fragment ks of the half-tile `half` of the tile kcur points at.
@@ -426,15 +443,16 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
   // K_0 and Q have landed once at most the loads of V_0 (and K_1) are outstanding: loads complete
   // in the order they were issued.
   constexpr int LOADS_PER_TILE = TileLoader<DP, BKV, kFwdWaves, PAD>::LOADS;
-  static_assert(2 * LOADS_PER_TILE < 64, "vmcnt field");
-  if (n_tiles > 1) wait_vmem<2 * LOADS_PER_TILE>(); else wait_vmem<LOADS_PER_TILE>();
+  static_assert(3 * LOADS_PER_TILE < 64, "vmcnt field");
+  if (KG > 1 && n_tiles > 2) wait_vmem<3 * LOADS_PER_TILE>();
+  else if (n_tiles > 1) wait_vmem<2 * LOADS_PER_TILE>(); else wait_vmem<LOADS_PER_TILE>();
   __syncthreads();
 
   // Q^T fragments (B operand of S^T = K Q^T): lane (c, h) holds Q[q0w + c][16 ks + 8 h + j].
   s16x8 qf[KS];
   {
-    const lds_cptr qrows = lds0 + ((wave >> 1) ? (int)(Q_HI / 2) : (int)(Q_LO / 2));
-    const int r = 32 * (wave & 1) + c;
+    const lds_cptr qrows = lds0 + ((rg >> 1) ? (int)(Q_HI / 2) : (int)(Q_LO / 2));
+    const int r = 32 * (rg & 1) + c;
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) qf[ks] = lds_read_128(qrows + swz_off<LP>(r, 2 * ks + h));
     if (PRE) {
@@ -454,16 +472,20 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
     sc = zero;
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) sc = Elem<T>::mfma(ring[ks], qf[ks], sc);
-    if (0 >= n_full) apply_mask(sc, 0);
+    if (block_at(0) >= n_full) apply_mask(sc, block_at(0) * BLK);
     m_ref = row_max(sc);  // finite: every query row sees key 0
+    // (the second key group's rows see its first key unless that block is not the wave's: no probabilities)
+    if (KG > 1 && n_mine <= 0) m_ref = 0.f;
     const float mc = m_ref * scale_log2;
 #pragma unroll
     for (int i = 0; i < 16; i++) {
       e[i] = PRE ? fast_exp2(sc[i] - m_ref) : fast_exp2(sc[i] * scale_log2 - mc);
       l_run += e[i];
     }
+    if (KG == 1) {
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) ring[ks] = k_frag(1, ks);
+      for (int ks = 0; ks < KS; ks++) ring[ks] = k_frag(1, ks);
+    }
     // From here on kcur addresses K tile 1 (the tile after the current one).
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) kcur[ks] += L::TILE_ELEMS;
@@ -472,6 +494,13 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
   // the first tile's loads (K_2, V_1) are about to overwrite.
   wait_vmem_all();
   __syncthreads();
+  if (KG > 1) {  // the next block is the group's half of tile 1; kcur moves on to tile 2
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+      ring[ks] = k_frag(0, ks);
+      kcur[ks] += L::TILE_ELEMS;
+    }
+  }
 
   // PRE: the C operand every later score chain starts from.
   f32x16 negm = zero;
@@ -510,12 +539,12 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
     constexpr bool INNER = decltype(spread_tag)::value || decltype(half_tag)::inner;
     if (!INNER && j >= n_mine) {
       if (SPREAD) {  // not reached: the skipped blocks lie in the last two tiles, which load nothing
-        issue_k(j / 2 + 2);
-        issue_v(j / 2 + 1);
+        issue_k(j / (2 / KG) + K_AHEAD);
+        issue_v(j / (2 / KG) + 1);
       }
       return;
     }
-    const int kt = j / 2 + 2, vt = j / 2 + 1;  // tiles loaded during this step (SPREAD)
+    const int kt = j / (2 / KG) + K_AHEAD, vt = j / (2 / KG) + 1;  // tiles loaded during this step (SPREAD)
     const unsigned kdst = lds_base + 2u * (unsigned)(L::K_BASE + (kt % L::K_STAGES) * L::TILE_ELEMS);
     const unsigned vdst = lds_base + 2u * (unsigned)(L::V_BASE + (vt % L::V_STAGES) * L::TILE_ELEMS);
     typedef unsigned u32x4v __attribute__((ext_vector_type(4)));
@@ -537,7 +566,7 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
     }
     // S_{j+1} of a SPREAD step is the second half of a tile that ends before the workgroup's first
     // query row: never masked.  (The step after it may produce the first block of the diagonal.)
-    if (!SPREAD && j + 1 >= n_full) apply_mask(sc, (j + 1) * BLK);
+    if (!SPREAD && block_at(j + 1) >= n_full) apply_mask(sc, block_at(j + 1) * BLK);
     const s16x8 pf[2] = {__builtin_bit_cast(s16x8, w[0]), __builtin_bit_cast(s16x8, w[1])};
     const float mc = m_ref * scale_log2;
     float lsum[2] = {0.f, 0.f};  // this lane's sum of the new probabilities, in two chains
@@ -595,7 +624,7 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
   auto end_tile = [&](int t) {
     wait_vmem_all();
     tile_barrier();
-    const int dk = ((t + 2) % L::K_STAGES == 0) ? -(L::K_STAGES - 1) * L::TILE_ELEMS : L::TILE_ELEMS;
+    const int dk = ((t + K_AHEAD) % L::K_STAGES == 0) ? -(L::K_STAGES - 1) * L::TILE_ELEMS : L::TILE_ELEMS;
     const int dv = ((t + 1) % L::V_STAGES == 0) ? -(L::V_STAGES - 1) * L::TILE_ELEMS : L::TILE_ELEMS;
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) kcur[ks] += dk;
@@ -607,28 +636,69 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
   };
   int t = 0;
   // Tiles whose loads are whole tiles inside the keys: spread over the first step.
-  const int n_spread = min(n_tiles, n_inside) - 2;
+  const int n_spread = min(n_tiles, n_inside) - K_AHEAD;
   for (; t < n_spread; t++) {
-    step(2 * t, HalfTag<0, true>{}, std::true_type{});
-    step(2 * t + 1, HalfTag<1, true>{}, std::false_type{});
+    if constexpr (KG == 1) {
+      step(2 * t, HalfTag<0, true>{}, std::true_type{});
+      step(2 * t + 1, HalfTag<1, true>{}, std::false_type{});
+    } else {
+      step(t, HalfTag<0, true>{}, std::true_type{});
+    }
     end_tile(t);
   }
   // The last tiles: whatever is left to load (possibly a ragged tile) is issued at once.
   for (; t < n_tiles; t++) {
-    if (t + 2 < n_tiles) issue_k(t + 2);
+    if (t + K_AHEAD < n_tiles) issue_k(t + K_AHEAD);
     if (t + 1 < n_tiles) issue_v(t + 1);
-    step(2 * t, HalfTag<0, false>{}, std::false_type{});
-    step(2 * t + 1, HalfTag<1, false>{}, std::false_type{});
+    if constexpr (KG == 1) {
+      step(2 * t, HalfTag<0, false>{}, std::false_type{});
+      step(2 * t + 1, HalfTag<1, false>{}, std::false_type{});
+    } else {
+      step(t, HalfTag<0, false>{}, std::false_type{});
+    }
     end_tile(t);
   }
-  const float l_tot = sum_over_halves(l_run);
+  float l_tot = sum_over_halves(l_run);
+  // Two key groups: the second hands its maximum, sum and accumulator to the first, which merges them with
+  // the rescale of an online-softmax step and stores.  The areas overlay the stages: the loop's last
+  // barrier ordered them after all reads.
+  constexpr int MERGE_FLOATS = KG == 1 ? 0 : (DB * 16 + 2) * 64;  // per row group
+  static_assert(KG == 1 || 2 * MERGE_FLOATS * 2 + 2 * 32 * (DP + 8) <= L::TOTAL_ELEMS, "merge area and patch overlay the stages");
+  if constexpr (KG > 1) {
+    float *area = reinterpret_cast<float *>(smem) + rg * MERGE_FLOATS + 4 * lane;
+    if (kg == 1) {
+#pragma unroll
+      for (int db = 0; db < DB; db++)
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+          *reinterpret_cast<f32x4 *>(area + (db * 4 + g) * 256) =
+              f32x4{oacc[db][4 * g], oacc[db][4 * g + 1], oacc[db][4 * g + 2], oacc[db][4 * g + 3]};
+      area[DB * 1024 - 3 * lane] = n_mine > 0 ? m_ref : -INFINITY;
+      area[DB * 1024 - 3 * lane + 64] = l_tot;
+    }
+    __syncthreads();
+    if (kg == 1) return;
+    const float m1 = area[DB * 1024 - 3 * lane], l1 = area[DB * 1024 - 3 * lane + 64];
+    const float m_new = fmaxf(m_ref, m1), unit = PRE ? 1.f : scale_log2;
+    const float a0 = fast_exp2((m_ref - m_new) * unit), a1 = fast_exp2((m1 - m_new) * unit);
+    m_ref = m_new;
+    l_tot = l_tot * a0 + l1 * a1;
+#pragma unroll
+    for (int db = 0; db < DB; db++)
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        const f32x4 x = *reinterpret_cast<const f32x4 *>(area + (db * 4 + g) * 256);
+#pragma unroll
+        for (int e2 = 0; e2 < 4; e2++) oacc[db][4 * g + e2] = oacc[db][4 * g + e2] * a0 + x[e2] * a1;
+      }
+  }
   const float inv_l = 1.f / l_tot;
   if (h == 0 && q0w + c < p.seqlen_q) LSE[q0w + c] = m_ref * (PRE ? kLn2 : p.scale) + __logf(l_tot);
   if (qt == p.n_qtiles - 1) {
-    for (int r = p.seqlen_q + tid; r < p.seqlen_q_rounded; r += NTHREADS) LSE[r] = 0.f;
+    for (int r = p.seqlen_q + tid; r < p.seqlen_q_rounded; r += NTHREADS / KG) LSE[r] = 0.f;
   }
   // The patch overlays the stages; the loop's last barrier already ordered it after all reads.
-  short *patch = smem + wave * 32 * (DP + 8);
+  short *patch = smem + KG * MERGE_FLOATS * 2 + wave * 32 * (DP + 8);
   store_transposed_acc<T, DP>(oacc, inv_l, patch, O + (int64_t)q0w * p.o.stride_seq,
                               p.o.stride_seq, p.seqlen_q - q0w, hdim, true);
 }

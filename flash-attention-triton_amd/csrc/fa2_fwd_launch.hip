@@ -22,14 +22,24 @@ void launch_generic(int dp, const FwdParams &p, dim3 grid, dim3 block, hipStream
 // kernels live in a translation unit of their own (fa2_fwd_launch_wide.hip): compiled beside the
 // narrower instantiations the 256-column kernel, which uses all 512 registers, came out with 40-60
 // spilled registers and reloads inside its tile loop; alone it spills two, outside the loop.
-template <typename T, bool PAD, bool PRE>
+template <typename T, bool PAD, bool PRE, int KG>
 void launch_direct(int dp, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
   switch (dp) {
-    case 32: hipLaunchKernelGGL((fwd_direct_kernel<T, 32, kFwdBlockKV, PAD, PRE>), grid, block, 0, s, p); break;
-    case 64: hipLaunchKernelGGL((fwd_direct_kernel<T, 64, kFwdBlockKV, PAD, PRE>), grid, block, 0, s, p); break;
-    case 96: hipLaunchKernelGGL((fwd_direct_kernel<T, 96, kFwdBlockKV, PAD, PRE>), grid, block, 0, s, p); break;
-    case 128: hipLaunchKernelGGL((fwd_direct_kernel<T, 128, kFwdBlockKV, PAD, PRE>), grid, block, 0, s, p); break;
-    default: launch_fwd_direct_wide(std::is_same<T, __bf16>::value, dp, PAD, p, grid, block, s); break;
+    case 32: hipLaunchKernelGGL((fwd_direct_kernel<T, 32, kFwdBlockKV, PAD, PRE, KG>), grid, block, 0, s, p); break;
+    case 64: hipLaunchKernelGGL((fwd_direct_kernel<T, 64, kFwdBlockKV, PAD, PRE, KG>), grid, block, 0, s, p); break;
+    case 96: hipLaunchKernelGGL((fwd_direct_kernel<T, 96, kFwdBlockKV, PAD, PRE, KG>), grid, block, 0, s, p); break;
+    case 128: hipLaunchKernelGGL((fwd_direct_kernel<T, 128, kFwdBlockKV, PAD, PRE, KG>), grid, block, 0, s, p); break;
+    default: launch_fwd_direct_wide(std::is_same<T, __bf16>::value, dp, PAD, KG, p, grid, block, s); break;
+  }
+}
+
+template <typename T, int KG>
+void launch_groups(int dp, bool folded, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
+  const bool pad = p.headdim != dp;
+  if (folded) {
+    if (pad) launch_direct<T, true, true, KG>(dp, p, grid, block, s); else launch_direct<T, false, true, KG>(dp, p, grid, block, s);
+  } else {
+    if (pad) launch_direct<T, true, false, KG>(dp, p, grid, block, s); else launch_direct<T, false, false, KG>(dp, p, grid, block, s);
   }
 }
 
@@ -37,12 +47,10 @@ template <typename T>
 void launch(int dp, bool folded, const FwdParams &p, dim3 grid, hipStream_t s) {
   const dim3 block(64 * kFwdWaves);
   if (fwd_direct_ok(dp, p)) {
-    const bool pad = p.headdim != dp;
-    if (folded) {
-      if (pad) launch_direct<T, true, true>(dp, p, grid, block, s); else launch_direct<T, false, true>(dp, p, grid, block, s);
-    } else {
-      if (pad) launch_direct<T, true, false>(dp, p, grid, block, s); else launch_direct<T, false, false>(dp, p, grid, block, s);
-    }
+    if (fwd_key_groups(dp, p) == 2)
+      launch_groups<T, 2>(dp, folded, p, grid, block, s);
+    else
+      launch_groups<T, 1>(dp, folded, p, grid, block, s);
     return;
   }
   if (p.vec)

@@ -10,22 +10,30 @@ namespace {
 // (it then switches no lane off): with the number of columns a run-time value the compiler keeps the
 // kernel within its 512 registers, with a constant 256 it spills about forty of them, with reloads
 // inside the tile loop, where they queue behind the tile loads (same counter).
-template <typename T, bool PAD>
+template <typename T, bool PAD, int KG>
 void launch_wide(int dp, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
   if (dp == 192)
-    hipLaunchKernelGGL((fwd_direct_kernel<T, 192, kFwdBlockKV, PAD, false>), grid, block, 0, s, p);
+    hipLaunchKernelGGL((fwd_direct_kernel<T, 192, kFwdBlockKV, PAD, false, KG>), grid, block, 0, s, p);
   else
-    hipLaunchKernelGGL((fwd_direct_kernel<T, 256, kFwdBlockKV, true, false>), grid, block, 0, s, p);
+    hipLaunchKernelGGL((fwd_direct_kernel<T, 256, kFwdBlockKV, true, false, KG>), grid, block, 0, s, p);
+}
+
+template <typename T>
+void launch_groups(int dp, bool pad, int key_groups, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
+  if (key_groups == 2) {
+    if (pad) launch_wide<T, true, 2>(dp, p, grid, block, s); else launch_wide<T, false, 2>(dp, p, grid, block, s);
+  } else {
+    if (pad) launch_wide<T, true, 1>(dp, p, grid, block, s); else launch_wide<T, false, 1>(dp, p, grid, block, s);
+  }
 }
 
 }  // namespace
 
-void launch_fwd_direct_wide(bool bf16, int dp, bool pad, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
-  if (bf16) {
-    if (pad) launch_wide<__bf16, true>(dp, p, grid, block, s); else launch_wide<__bf16, false>(dp, p, grid, block, s);
-  } else {
-    if (pad) launch_wide<_Float16, true>(dp, p, grid, block, s); else launch_wide<_Float16, false>(dp, p, grid, block, s);
-  }
+void launch_fwd_direct_wide(bool bf16, int dp, bool pad, int key_groups, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
+  if (bf16)
+    launch_groups<__bf16>(dp, pad, key_groups, p, grid, block, s);
+  else
+    launch_groups<_Float16>(dp, pad, key_groups, p, grid, block, s);
 }
 
 }  // namespace fa2

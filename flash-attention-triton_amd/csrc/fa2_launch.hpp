@@ -24,12 +24,43 @@ inline bool direct_headdim(int dp, int headdim) {
 inline bool direct_headdim_wide(int dp, int headdim) {
   return direct_headdim(dp, headdim) || (headdim % 8 == 0 && headdim <= dp && (dp == 192 || dp == 256));
 }
+// Key groups of the forward and dQ kernels.  With two, a workgroup owns 64 query rows instead of 128 and two
+// waves share 32 of them, one taking the even and the other the odd 32-key blocks; they merge their results
+// through LDS at the end.  Every wave's chain of blocks is half as long and the grid has twice the
+// workgroups, but every K and V tile is loaded for half the rows and every block ends at a barrier.  So two
+// groups win while the grid leaves CUs idle.  Time of one group over two, bf16, (batch, head) pairs x
+// tokens, forward / dQ, by workgroups of 128 rows:
+//   to 128      1.06-1.2 / 1.03-1.15 (128, 256 tokens), 1.3-1.7 / 1.25-1.65 beyond, any head dimension
+//   to 256      128 columns 1.14 / 1.04 (64 x 512), 1.30 / 1.24 (8 x 4096); 64 columns 1.23 / 1.09, 1.46 / 1.35;
+//               but 0.96 / 0.84 (200 x 128, 128 columns).  192 and 256 columns (one workgroup per CU either
+//               way): 1.09 / 1.04 (32 x 1024), 0.95 / 0.91 (64 x 512)
+//   to 384      64 columns 1.17 / 1.09 (96 x 512); 96 columns 1.10 / 1.08 (24 x 2048); 128 columns
+//               1.11 / 1.04 (12 x 4096), 1.07 / 0.94 (24 x 2048)
+//   to 512      32 columns 1.11 / 1.06 (64 x 1024), 1.23 / 1.10 (16 x 4096); 64 columns 1.07 / 1.01 (16 x 4096),
+//               0.94 / 0.86 (64 x 1024); 128 columns 0.98 / 0.94 (16 x 4096)
+//   beyond      0.75-0.98
+inline int key_groups(int dp, int64_t heads, int seqlen_q) {
+  const int64_t wgs = heads * ((seqlen_q + kFwdBlockQ - 1) / kFwdBlockQ);
+  static_assert(kFwdBlockQ == kDqBlockQ, "one rule for both kernels");
+  const bool two = wgs <= kCUs / 2       ? true
+                   : wgs <= kCUs         ? seqlen_q >= (dp > 128 ? 1024 : 256)
+                   : wgs <= 3 * kCUs / 2 ? dp <= 128 && seqlen_q >= (dp == 128 ? 4096 : dp == 96 ? 2048 : 512)
+                   : wgs <= 2 * kCUs     ? dp <= 64 && seqlen_q >= (dp == 64 ? 4096 : 1024)
+                                         : false;
+  return two ? 2 : 1;
+}
 inline bool fwd_direct_ok(int dp, const FwdParams &p) {
   return p.vec && direct_headdim_wide(dp, p.headdim) && direct_stride_ok(p.q) && direct_stride_ok(p.k) &&
          direct_stride_ok(p.v);
 }
+inline int fwd_key_groups(int dp, const FwdParams &p) {
+  return fwd_direct_ok(dp, p) ? key_groups(dp, (int64_t)p.batch * p.nheads, p.seqlen_q) : 1;
+}
 inline bool dq_direct_ok(int dp, const BwdParams &p) {
   return p.vec && direct_headdim_wide(dp, p.headdim) && direct_stride_ok(p.k) && direct_stride_ok(p.v);
+}
+inline int dq_key_groups(int dp, const BwdParams &p) {
+  return dq_direct_ok(dp, p) ? key_groups(dp, (int64_t)p.batch * p.nheads, p.seqlen_q) : 1;
 }
 inline bool dkdv_direct_ok(int dp, const BwdParams &p) {
   return p.vec && direct_headdim(dp, p.headdim) && direct_stride_ok(p.q) && direct_stride_ok(p.d_o) &&
@@ -81,7 +112,7 @@ inline int equal_head_groups(int group, int64_t heads) {
 // multiplied by scale * log2(e) and rounded once); the generic forward ignores it.
 void launch_fwd(bool bf16, int dp, bool folded, const FwdParams &p, dim3 grid, hipStream_t s);
 // The 192- and 256-column LDS-direct forward kernels (dp is 192 or 256), instantiated apart from the others.
-void launch_fwd_direct_wide(bool bf16, int dp, bool pad, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s);
+void launch_fwd_direct_wide(bool bf16, int dp, bool pad, int key_groups, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s);
 void launch_preprocess(bool bf16, const PreParams &p, dim3 grid, hipStream_t s);
 // fuse_delta: the fast dQ kernel also forms delta from O and dO (dq_direct_ok must hold).
 void launch_dq(bool bf16, int dp, const BwdParams &p, dim3 grid, bool fuse_delta, hipStream_t s);

@@ -591,6 +591,25 @@ def test_grids_that_fit_the_chip_at_once(fa, b, h, n, d):
         _assert_close(name, g.reshape(w.shape), w)
 
 
+@pytest.mark.parametrize("heads", [2, 400], ids=["two_groups", "one_group"])
+@pytest.mark.parametrize("nq,nk,d", [(1, 1, 64), (32, 32, 128), (33, 31, 128), (64, 200, 96), (65, 65, 32), (129, 20, 128),
+                                     (192, 193, 64), (257, 256, 72), (191, 300, 256), (97, 33, 200)])
+def test_key_groups_edges(fa, nq, nk, d, heads):
+    """Forward (with and without a backward to follow) and dQ with the 32-key blocks of a tile split between
+    two waves, and the same sizes on a grid that takes one group: waves without any block, one to five
+    tiles, ragged query and key ends."""
+    q, k, v, d_o = (t.cuda() for t in _seeded((1, heads, nq, d), (1, heads, nk, d), torch.bfloat16, 1.5))
+    qg = q.clone().requires_grad_(True)
+    out = fa.flash_attention_v2(qg, k, v)
+    (dq,) = torch.autograd.grad(out, (qg,), d_o)
+    with torch.no_grad():
+        only = fa.flash_attention_v2(q, k, v)
+    one = lambda t: t[:, heads - 1 : heads]  # noqa: E731
+    o, want, _, _ = _gpu_fp32_oracle(one(q), one(k), one(v), one(d_o), None)
+    for name, g, w in (("o", out, o), ("dq", dq, want), ("o (forward only)", only, o)):
+        _assert_close(name, one(g).reshape(w.shape), w)
+
+
 def test_zero_scale_means_default_and_explicit_scale_is_used(fa):
     """`softmax_scale or default`: 0.0 selects 1/sqrt(D) (flash_attention_2.py:94)."""
     q, k, v, _ = _seeded((1, 2, 96, 64), (1, 2, 96, 64), torch.bfloat16)
