@@ -474,8 +474,19 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
     for (int ks = 0; ks < KS; ks++) sc = Elem<T>::mfma(ring[ks], qf[ks], sc);
     if (block_at(0) >= n_full) apply_mask(sc, block_at(0) * BLK);
     m_ref = row_max(sc);  // finite: every query row sees key 0
-    // (the second key group's rows see its first key unless that block is not the wave's: no probabilities)
-    if (KG > 1 && n_mine <= 0) m_ref = 0.f;
+    // The second key group's first block is block 1: no probabilities where it is not the wave's.  Where it
+    // holds keys whose scores are all -inf (a bias column that hides keys) the row starts from block 0's
+    // maximum, as with one group.
+    if (KG > 1 && n_mine <= 0) {
+      m_ref = 0.f;
+    } else if (KG > 1 && kg == 1 && __builtin_amdgcn_ballot_w64(m_ref == -INFINITY) != 0) {
+      f32x16 s0 = zero;
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) s0 = Elem<T>::mfma(lds_read_128(kcur[ks] - BLK * LP), qf[ks], s0);
+      if (n_full < 1) apply_mask(s0, 0);
+      const float m0 = row_max(s0);
+      if (m_ref == -INFINITY) m_ref = m0;
+    }
     const float mc = m_ref * scale_log2;
 #pragma unroll
     for (int i = 0; i < 16; i++) {

@@ -610,6 +610,27 @@ def test_key_groups_edges(fa, nq, nk, d, heads):
         _assert_close(name, one(g).reshape(w.shape), w)
 
 
+@pytest.mark.parametrize("heads", [2, 400], ids=["two_groups", "one_group"])
+@pytest.mark.parametrize("first,last", [(32, 64), (32, 300), (96, 128), (1, 64)])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_keys_hidden_by_a_bias_column(fa, d, first, last, heads):
+    """q carries a column of ones and k a column that is -inf for keys first .. last - 1: their scores are
+    -inf and the other keys share the row, also where the hidden keys are a key group's whole first block."""
+    q, k, v, _ = (t.cuda() for t in _seeded((1, heads, 300, d), (1, heads, 300, d), torch.bfloat16))
+    q[..., -1] = 1.0
+    k[..., -1] = 0.0
+    k[:, :, first:last, -1] = float("-inf")
+    one = lambda t: t[:, heads - 1 :].float()  # noqa: E731
+    s = one(q) @ one(k).transpose(-1, -2).contiguous() / math.sqrt(d)
+    s = s.masked_fill(~torch.ones(300, 300, dtype=torch.bool, device="cuda").tril(), float("-inf"))
+    want = torch.softmax(s, -1) @ one(v)
+    outs = {"o": fa.flash_attention_v2(q.clone().requires_grad_(True), k, v).detach()}
+    with torch.no_grad():
+        outs["o (forward only)"] = fa.flash_attention_v2(q, k, v)
+    for name, out in outs.items():
+        _assert_close(name, one(out), want)
+
+
 def test_zero_scale_means_default_and_explicit_scale_is_used(fa):
     """`softmax_scale or default`: 0.0 selects 1/sqrt(D) (flash_attention_2.py:94)."""
     q, k, v, _ = _seeded((1, 2, 96, 64), (1, 2, 96, 64), torch.bfloat16)
