@@ -61,8 +61,6 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem) {
   using L = DkvPairLayout<DP>;
   constexpr int BQ = L::BQ, KS = DP / 16, DB = DP / 32, LP = L::LP;
   constexpr int NTHREADS = 64 * kDkvWaves;
-  // With one wave per SIMD the S and dP chains are written out with vector-register accumulators
-  // (VgprMfma); with two the compiler has no accumulation registers to place them in.
   using Loader = TileLoader<DP, BQ, kDkvWaves, PAD>;
   constexpr int LOADS = Loader::LOADS;
 

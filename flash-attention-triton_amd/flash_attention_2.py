@@ -10,7 +10,8 @@ Differences from the reference, all deliberate:
 * bf16 inputs are computed with bf16 MFMA; the reference down-casts everything to fp16
   (flash_attention_2.py:316).  fp16 inputs use fp16 MFMA; any other dtype is down-cast to fp16
   and the output cast back, as in the reference.
-* fp16/bf16 contiguous inputs are used as they are: no cast or copy kernels run.
+* fp16/bf16 inputs, contiguous or views with aligned rows, are used as they are: no cast or copy
+  kernels run.
 * A forward that nothing will differentiate (under ``torch.no_grad()``, or with no input that
   requires a gradient) on bf16 inputs up to head dimension 128 multiplies Q by
   softmax_scale * log2(e) and rounds it to bf16 once, so that the score MFMAs deliver base-2
