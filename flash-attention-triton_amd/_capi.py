@@ -83,6 +83,7 @@ SIGNATURES = {
     "fa2_bwd_fused_noalloc": (_i, [_p] * 9 + [_i] * 6 + [_i64] * 24 + [_f, _i, _i, _i, _p]),
     "fa2_fwd_packed": (_i, [ctypes.POINTER(FwdArgs), _p]),
     "fa2_bwd_packed": (_i, [ctypes.POINTER(BwdArgs), _p]),
+    "fa2_bwd_packed_f32_grads": (_i, [ctypes.POINTER(BwdArgs), _p]),
 }
 
 _lib = None

@@ -60,8 +60,6 @@ __global__ __launch_bounds__(64 * kDkvWaves, 1) void bwd_dkdv_kernel(const BwdPa
   const short *K = (const short *)p.k.ptr + b * p.k.stride_batch + hd * p.k.stride_head;
   const short *V = (const short *)p.v.ptr + b * p.v.stride_batch + hd * p.v.stride_head;
   const short *DO = (const short *)p.d_o.ptr + b * p.d_o.stride_batch + hd * p.d_o.stride_head;
-  short *DK = (short *)p.dk.ptr + b * p.dk.stride_batch + hd * p.dk.stride_head;
-  short *DV = (short *)p.dv.ptr + b * p.dv.stride_batch + hd * p.dv.stride_head;
   const float *LSE = p.lse + (int64_t)bh * p.seqlen_q_rounded;
   const float *DELTA = p.delta + (int64_t)bh * p.seqlen_q_rounded;
 
@@ -221,13 +219,13 @@ __global__ __launch_bounds__(64 * kDkvWaves, 1) void bwd_dkdv_kernel(const BwdPa
   // stages: the loop's last barrier ordered it after all reads, and the barrier below orders the
   // next pass's tile stores after it.
   short *patch = smem + wave * 32 * (DP + 8);
-  store_transposed_acc<T, 32 * DBP>(dvacc, 1.0f, patch, DV + (int64_t)kv0w * p.dv.stride_seq + col0,
-                                    p.dv.stride_seq, p.seqlen_k - kv0w, p.headdim - col0, vec);
+  store_transposed_acc<T, 32 * DBP>(dvacc, 1.0f, patch, grad_rows(p, p.dv, b, hd, kv0w, col0),
+                                     p.dv.stride_seq, p.seqlen_k - kv0w, p.headdim - col0, vec, p.grads_f32);
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  store_transposed_acc<T, 32 * DBP>(dkacc, p.scale, patch, DK + (int64_t)kv0w * p.dk.stride_seq + col0,
-                                    p.dk.stride_seq, p.seqlen_k - kv0w, p.headdim - col0, vec);
+  store_transposed_acc<T, 32 * DBP>(dkacc, p.scale, patch, grad_rows(p, p.dk, b, hd, kv0w, col0),
+                                     p.dk.stride_seq, p.seqlen_k - kv0w, p.headdim - col0, vec, p.grads_f32);
   if (pass + 1 < NPASS) __syncthreads();
   }
 }
@@ -336,8 +334,6 @@ __global__ __launch_bounds__(64 * kDkvWaves, (DP <= 96 && !ATOMIC_DQ ? 2 : 1)) v
   const short *K = (const short *)p.k.ptr + b * p.k.stride_batch + hd * p.k.stride_head;
   const short *V = (const short *)p.v.ptr + b * p.v.stride_batch + hd * p.v.stride_head;
   const short *DO = (const short *)p.d_o.ptr + b * p.d_o.stride_batch + hd * p.d_o.stride_head;
-  short *DK = (short *)p.dk.ptr + b * p.dk.stride_batch + hd * p.dk.stride_head;
-  short *DV = (short *)p.dv.ptr + b * p.dv.stride_batch + hd * p.dv.stride_head;
   const float *LSE = p.lse + (int64_t)bh * p.seqlen_q_rounded;
   const float *DELTA = p.delta + (int64_t)bh * p.seqlen_q_rounded;
 
@@ -683,13 +679,13 @@ __global__ __launch_bounds__(64 * kDkvWaves, (DP <= 96 && !ATOMIC_DQ ? 2 : 1)) v
   for (; t < n_tiles; t++) tile(t, std::true_type{}, std::false_type{});
 
   short *patch = smem + wave * 32 * (DP + 8);
-  store_transposed_acc<T, DP>(dvacc, 1.0f, patch, DV + (int64_t)kv0w * p.dv.stride_seq,
-                              p.dv.stride_seq, p.seqlen_k - kv0w, hdim, true);
+  store_transposed_acc<T, DP>(dvacc, 1.0f, patch, grad_rows(p, p.dv, b, hd, kv0w),
+                              p.dv.stride_seq, p.seqlen_k - kv0w, hdim, true, p.grads_f32);
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  store_transposed_acc<T, DP>(dkacc, p.scale, patch, DK + (int64_t)kv0w * p.dk.stride_seq,
-                              p.dk.stride_seq, p.seqlen_k - kv0w, hdim, true);
+  store_transposed_acc<T, DP>(dkacc, p.scale, patch, grad_rows(p, p.dk, b, hd, kv0w),
+                              p.dk.stride_seq, p.seqlen_k - kv0w, hdim, true, p.grads_f32);
 }
 
 // ---- fp32 dQ accumulator of the sequence-parallel mode ------------------------------------------

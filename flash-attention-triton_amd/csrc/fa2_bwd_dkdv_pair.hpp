@@ -341,11 +341,10 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem) {
 
   // The patch overlays the stages; reads of them that are still in flight fetch values nobody uses.
   const Tensor4 &out = role ? p.dk : p.dv;
-  short *OUT = (short *)out.ptr + b * out.stride_batch + hd * out.stride_head;
   __syncthreads();
   short *patch = smem + wave * 32 * (DP + 8);
-  store_transposed_acc<T, DP>(acc, role ? p.scale : 1.0f, patch, OUT + (int64_t)kv0w * out.stride_seq, out.stride_seq,
-                              p.seqlen_k - kv0w, hdim, true);
+  store_transposed_acc<T, DP>(acc, role ? p.scale : 1.0f, patch, grad_rows(p, out, b, hd, kv0w), out.stride_seq,
+                              p.seqlen_k - kv0w, hdim, true, p.grads_f32);
 }
 
 template <typename T, int DP, bool PAD>

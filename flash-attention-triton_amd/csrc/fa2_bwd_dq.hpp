@@ -104,7 +104,6 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 96 ? 2 : 1)) void bwd_dq_kern
   const short *K = (const short *)p.k.ptr + b * p.k.stride_batch + hd * p.k.stride_head;
   const short *V = (const short *)p.v.ptr + b * p.v.stride_batch + hd * p.v.stride_head;
   const short *DO = (const short *)p.d_o.ptr + b * p.d_o.stride_batch + hd * p.d_o.stride_head;
-  short *DQ = (short *)p.dq.ptr + b * p.dq.stride_batch + hd * p.dq.stride_head;
 
   // B operands: lane (c, h) holds row q0w + c of Q and of dO, columns 16 ks + 8 h + j.
   s16x8 qf[KS], gf[KS];
@@ -239,8 +238,8 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 96 ? 2 : 1)) void bwd_dq_kern
   }
 
   short *patch = smem + wave * 32 * (DP + 8);
-  store_transposed_acc<T, DP>(dqacc, p.scale, patch, DQ + (int64_t)q0w * p.dq.stride_seq,
-                              p.dq.stride_seq, p.seqlen_q - q0w, p.headdim, vec);
+  store_transposed_acc<T, DP>(dqacc, p.scale, patch, grad_rows(p, p.dq, b, hd, q0w),
+                              p.dq.stride_seq, p.seqlen_q - q0w, p.headdim, vec, p.grads_f32);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -299,7 +298,6 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
   const short *K = (const short *)p.k.ptr + b * p.k.stride_batch + hd * p.k.stride_head;
   const short *V = (const short *)p.v.ptr + b * p.v.stride_batch + hd * p.v.stride_head;
   const short *DO = (const short *)p.d_o.ptr + b * p.d_o.stride_batch + hd * p.d_o.stride_head;
-  short *DQ = (short *)p.dq.ptr + b * p.dq.stride_batch + hd * p.dq.stride_head;
 
   const int hdim = PAD ? p.headdim : DP;
   const TileLoader<DP, BKV, kDqWaves, PAD> kload(K, p.k.stride_seq, hdim / 8), vload(V, p.v.stride_seq, hdim / 8);
@@ -555,8 +553,8 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
       }
   }
   short *patch = smem + KG * MERGE_FLOATS * 2 + wave * 32 * (DP + 8);
-  store_transposed_acc<T, DP>(dqacc, p.scale, patch, DQ + (int64_t)q0w * p.dq.stride_seq,
-                              p.dq.stride_seq, p.seqlen_q - q0w, hdim, true);
+  store_transposed_acc<T, DP>(dqacc, p.scale, patch, grad_rows(p, p.dq, b, hd, q0w),
+                              p.dq.stride_seq, p.seqlen_q - q0w, hdim, true, p.grads_f32);
 }
 
 

@@ -223,7 +223,7 @@ int preprocess_impl(const fa2_tensor &o, const fa2_tensor &d_o, float *delta, in
 // runs second), otherwise by the preprocess kernel launched from here.  With the rows the table
 // picks by itself `deterministic` and `workspace` are accepted and not needed: dQ is written once,
 // in a fixed order, in both modes.  The sequence-parallel rows (dq_atomic) take the workspace.
-int bwd_impl(const fa2_bwd_args &a, void *stream) {
+int bwd_impl(const fa2_bwd_args &a, void *stream, bool grads_f32 = false) {
   int rc = check_common(a.batch, a.nheads, a.seqlen_q, a.seqlen_k, a.headdim, a.seqlen_q_rounded, a.dtype);
   if (rc) return rc;
   const bool fused = a.o.ptr != nullptr;
@@ -280,6 +280,7 @@ int bwd_impl(const fa2_bwd_args &a, void *stream) {
   const bool bf16 = a.dtype == FA2_DTYPE_BF16;
   const int dp = kTable[cfg].headdim_padded;
   const int64_t bh = (int64_t)a.batch * a.nheads;
+  p.grads_f32 = grads_f32;
   p.dq_accum = nullptr;
   p.dq_accum_rows = 0;
 
@@ -307,6 +308,7 @@ int bwd_impl(const fa2_bwd_args &a, void *stream) {
   if (kTable[cfg].dq_atomic) {
     // Sequence-parallel mode: clear the accumulator, (form delta), one key-tile-parallel kernel for
     // dK, dV and the atomic dQ contributions, then dq = scale * accumulator.
+    if (grads_f32) return fail(FA2_ERR_BAD_CONFIG, "config %d writes dQ in the inputs' type only", cfg);
     if (a.deterministic)
       return fail(FA2_ERR_BAD_CONFIG, "config %d accumulates dQ with atomics: not available with deterministic=1", cfg);
     if (!(want_dq && want_dkdv))
@@ -444,6 +446,11 @@ int fa2_fwd_packed(const fa2_fwd_args *args, void *stream) {
 int fa2_bwd_packed(const fa2_bwd_args *args, void *stream) {
   if (args == nullptr) return fail(FA2_ERR_NULL_POINTER, "args is NULL");
   return bwd_impl(*args, stream);
+}
+
+int fa2_bwd_packed_f32_grads(const fa2_bwd_args *args, void *stream) {
+  if (args == nullptr) return fail(FA2_ERR_NULL_POINTER, "args is NULL");
+  return bwd_impl(*args, stream, true);
 }
 
 int fa2_fwd(const void *q, const void *k, const void *v, void *o, float *lse, int batch, int nheads,

@@ -179,15 +179,38 @@ __device__ __forceinline__ void store_chunk(short *row, int d0, int headdim, boo
   }
 }
 
+// The same into an fp32 row: the half-precision values widened.
+template <typename T>
+__device__ __forceinline__ void store_chunk_widened(float *row, int d0, int headdim, bool row_ok, bool vec, s16x8 v) {
+  if (!row_ok) return;
+  float x[8];
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    const short e = v[j];
+    x[j] = (float)__builtin_bit_cast(T, e);
+  }
+  if (vec) {
+    if (d0 < headdim) {
+      *reinterpret_cast<f32x4 *>(row + d0) = f32x4{x[0], x[1], x[2], x[3]};
+      *reinterpret_cast<f32x4 *>(row + d0 + 4) = f32x4{x[4], x[5], x[6], x[7]};
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+      if (d0 + j < headdim) row[d0 + j] = x[j];
+  }
+}
+
 // Write a wave's transposed accumulator (DB blocks of 32 headdim rows x 32 sequence columns,
 // lane (c, h) holding sequence position c) to a (seqlen, headdim) tensor.  The values go through
 // a wave-private LDS patch of 32 x (DP + 8) elements so that global stores are 16-byte and
-// row-contiguous.  The caller guarantees the patch is not in use by anyone else.
+// row-contiguous.  The caller guarantees the patch is not in use by anyone else.  With `f32` (uniform)
+// the rows are fp32 and receive the rounded values widened.
 template <typename T, int DP>
 __device__ __forceinline__ void store_transposed_acc(const f32x16 (&acc)[DP / 32], float mult,
-                                                     short *patch, short *dst_rows,
+                                                     short *patch, void *dst_rows,
                                                      int64_t stride_seq, int rows_valid,
-                                                     int headdim, bool vec) {
+                                                     int headdim, bool vec, bool f32 = false) {
   constexpr int LD = DP + 8;
   constexpr int CPR = DP / 8;
   const int lane = threadIdx.x & 63;
@@ -204,13 +227,28 @@ __device__ __forceinline__ void store_transposed_acc(const f32x16 (&acc)[DP / 32
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  if (f32) {  // (not unrolled: unrolled, its addresses cost the 256-column dQ kernel two spilled registers)
+#pragma unroll 1
+    for (int id = lane; id < 32 * CPR; id += 64) {
+      const int r = id / CPR, cc = id % CPR;
+      const s16x8 v = *reinterpret_cast<const s16x8 *>(patch + r * LD + cc * 8);
+      store_chunk_widened<T>((float *)dst_rows + (int64_t)r * stride_seq, cc * 8, headdim, r < rows_valid, vec, v);
+    }
+    return;
+  }
 #pragma unroll
   for (int it = 0; it < (32 * CPR) / 64; it++) {
     int id = lane + 64 * it;
     int r = id / CPR, cc = id % CPR;
     s16x8 v = *reinterpret_cast<const s16x8 *>(patch + r * LD + cc * 8);
-    store_chunk(dst_rows + (int64_t)r * stride_seq, cc * 8, headdim, r < rows_valid, vec, v);
+    store_chunk((short *)dst_rows + (int64_t)r * stride_seq, cc * 8, headdim, r < rows_valid, vec, v);
   }
+}
+
+// Address of element (b, hd, row, col) of a gradient.
+__device__ __forceinline__ void *grad_rows(const BwdParams &p, const Tensor4 &t, int b, int hd, int row, int col = 0) {
+  const int64_t at = b * t.stride_batch + hd * t.stride_head + row * t.stride_seq + col;
+  return (char *)t.ptr + (at << (p.grads_f32 ? 2 : 1));
 }
 
 // Workgroup index -> (batch*head, tile rank); rank 0 is the heaviest tile of a head.

@@ -61,6 +61,7 @@ struct BwdParams {
   int resident_grid;  // number of workgroups when all of them fit the chip at once, else 0: see balanced_index
   float scale, scale_log2;
   int vec;
+  bool grads_f32;  // dq, dk and dv are fp32 tensors (strides in fp32 elements)
 };
 
 struct PreParams {

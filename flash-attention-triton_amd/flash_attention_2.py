@@ -98,8 +98,10 @@ def _device_guard(device: torch.device):
     return torch.cuda.device(device)
 
 
-def _assert_forward_inputs(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, max_headdim: int) -> None:
-    """The forward launcher's input checks (reference: flash_attention_2.py:85-90)."""
+def _assert_forward_inputs(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, max_headdim: int,
+                           compute_dtype: torch.dtype | None = None) -> None:
+    """The forward launcher's input checks (reference: flash_attention_2.py:85-90).  ``compute_dtype``: the type
+    the node casts q, k and v to (default: it does not cast)."""
     batch, nheads, _, headdim = q.shape
     _, _, seqlen_k, _ = k.shape
     assert k.shape == (batch, nheads, seqlen_k, headdim)
@@ -107,7 +109,7 @@ def _assert_forward_inputs(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ma
     assert headdim <= max_headdim, f"Supports head dimensions only up to {max_headdim}"
     assert q.is_cuda and k.is_cuda and v.is_cuda, "All tensors must reside on CUDA device"
     assert q.dtype == k.dtype == v.dtype, "All tensors must be the same type"
-    assert q.dtype in _COMPUTE_DTYPES, "Supports only fp16 and bf16"
+    assert (compute_dtype or q.dtype) in _COMPUTE_DTYPES, "Supports only fp16 and bf16"
 
 
 def _flash_attention_forward(
@@ -397,18 +399,19 @@ def _apply(q, k, v, softmax_scale, kernels_config):  # noqa: ANN001, ANN202
     """Record the attention in the autograd graph: the C++ node when it is built, else the Python class.
 
     With the C++ node the reference's forward wrapper (flash_attention_2.py:283-384) is spelt out
-    here: casts are ordinary differentiable operations in front of the node, the input checks are the
-    launcher's, a negative scale is folded into the sign of q.  The node takes strided views and copies
-    only what the kernels cannot read.
+    here: casts are the node's for fp32 and ordinary differentiable operations in front of it for other
+    types, the input checks are the launcher's, a negative scale is folded into the sign of q.  The node
+    takes strided views and copies only what the kernels cannot read.
     """
     node = _cpp_node()
     if node is None or kernels_config.atomic_dq:  # the C++ node always lets the table choose its backward row
         return FlashAttentionV2Function.apply(q, k, v, softmax_scale, kernels_config)
     initial_dtype = q.dtype
     compute_dtype = _compute_dtype(initial_dtype)
-    if not q.dtype == k.dtype == v.dtype == compute_dtype:
+    in_node = q.dtype == k.dtype == v.dtype == torch.float32  # the node casts these itself
+    if not in_node and not q.dtype == k.dtype == v.dtype == compute_dtype:
         q, k, v = [proj.to(compute_dtype) for proj in (q, k, v)]
-    _assert_forward_inputs(q, k, v, kernels_config.max_headdim)
+    _assert_forward_inputs(q, k, v, kernels_config.max_headdim, compute_dtype)
     scale = softmax_scale or 1.0 / math.sqrt(q.shape[-1])
     if scale < 0:
         q, scale = -q, -scale
@@ -417,7 +420,7 @@ def _apply(q, k, v, softmax_scale, kernels_config):  # noqa: ANN001, ANN202
                     and not getattr(kernels_config, "exact_scale", False) and not _EXACT_SCALE_ONLY)
     output = node.flash_attention_v2(q, k, v, scale, bool(kernels_config.deterministic), kernels_config.max_headdim,
                                      forward_only)
-    return output if initial_dtype == compute_dtype else output.to(initial_dtype)
+    return output if output.dtype == initial_dtype else output.to(initial_dtype)
 
 
 # ============================ gfx950 DEFAULT CONFIGURATIONS ============================

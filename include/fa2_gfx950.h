@@ -306,6 +306,13 @@ int fa2_bwd_fused_noalloc(const void *q, const void *k, const void *v, const voi
  */
 int fa2_bwd_packed(const fa2_bwd_args *args, void *stream);
 
+/*
+ * fa2_bwd_packed with dq, dk and dv as fp32 tensors (strides in fp32 elements): the same values, rounded to
+ * the inputs' type and widened, without the pass over each that a caller with fp32 tensors would run to
+ * widen them (flash_attention_2.py:316, 384).  Not for the rows with dq_atomic = 1.
+ */
+int fa2_bwd_packed_f32_grads(const fa2_bwd_args *args, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -631,6 +631,28 @@ def test_keys_hidden_by_a_bias_column(fa, d, first, last, heads):
         _assert_close(name, one(out), want)
 
 
+@pytest.mark.parametrize("b,h,n,d,transposed", [(1, 2, 1, 64, False), (2, 3, 200, 64, True), (1, 2, 130, 50, False), (1, 2, 130, 50, True),
+                                                (1, 2, 97, 80, True), (1, 300, 640, 32, False), (1, 16, 4225, 128, False),
+                                                (1, 2, 257, 96, True), (1, 2, 200, 256, False), (1, 400, 65, 200, False)])
+def test_fp32_gradients_are_the_fp16_ones_widened(fa, b, h, n, d, transposed):
+    """fp32 tensors are computed in fp16 and the kernels store their gradients widened: the bits of the same
+    call on fp16 tensors, for the kernels of small and large grids, padded columns and scalar rows."""
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    shape = (b, n, h, d) if transposed else (b, h, n, d)
+    q, k, v, d_o = (torch.randn(shape, generator=gen, device="cuda") for _ in range(4))
+    view = (lambda t: t.transpose(1, 2)) if transposed else (lambda t: t)
+    results = []
+    for dtype in (torch.float32, torch.float16):
+        leaves = [t.to(dtype).requires_grad_(True) for t in (q, k, v)]
+        out = fa.flash_attention_v2(*map(view, leaves))
+        results.append([out, *torch.autograd.grad(out, leaves, view(d_o).to(dtype))])
+        with torch.no_grad():
+            results[-1].append(fa.flash_attention_v2(*map(view, leaves)))
+    for wide, half in zip(*results):
+        assert wide.dtype == torch.float32 and half.dtype == torch.float16
+        assert torch.equal(wide, half.float())
+
+
 def test_zero_scale_means_default_and_explicit_scale_is_used(fa):
     """`softmax_scale or default`: 0.0 selects 1/sqrt(D) (flash_attention_2.py:94)."""
     q, k, v, _ = _seeded((1, 2, 96, 64), (1, 2, 96, 64), torch.bfloat16)
