@@ -343,7 +343,7 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem) {
   const Tensor4 &out = role ? p.dk : p.dv;
   __syncthreads();
   short *patch = smem + wave * 32 * (DP + 8);
-  store_transposed_acc<T, DP>(acc, role ? p.scale : 1.0f, patch, grad_rows(p, out, b, hd, kv0w), out.stride_seq,
+  store_transposed_acc<T, DP, true>(acc, role ? p.scale : 1.0f, patch, grad_rows(p, out, b, hd, kv0w), out.stride_seq,
                               p.seqlen_k - kv0w, hdim, true, p.grads_f32);
 }
 

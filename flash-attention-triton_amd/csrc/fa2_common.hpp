@@ -206,7 +206,7 @@ __device__ __forceinline__ void store_chunk_widened(float *row, int d0, int head
 // a wave-private LDS patch of 32 x (DP + 8) elements so that global stores are 16-byte and
 // row-contiguous.  The caller guarantees the patch is not in use by anyone else.  With `f32` (uniform)
 // the rows are fp32 and receive the rounded values widened.
-template <typename T, int DP>
+template <typename T, int DP, bool UNROLL_F32 = false>
 __device__ __forceinline__ void store_transposed_acc(const f32x16 (&acc)[DP / 32], float mult,
                                                      short *patch, void *dst_rows,
                                                      int64_t stride_seq, int rows_valid,
@@ -227,9 +227,13 @@ __device__ __forceinline__ void store_transposed_acc(const f32x16 (&acc)[DP / 32
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  if (f32) {  // (not unrolled: unrolled, its addresses cost the 256-column dQ kernel two spilled registers)
-#pragma unroll 1
-    for (int id = lane; id < 32 * CPR; id += 64) {
+  if (f32) {
+    // At 256 columns registers decide: unrolled, the addresses cost the dQ kernel two spills to scratch; rolled,
+    // the loop costs the paired dK/dV kernel five.
+    constexpr int U = UNROLL_F32 ? (32 * CPR) / 64 : 1;
+#pragma unroll U
+    for (int it = 0; it < (32 * CPR) / 64; it++) {
+      const int id = lane + 64 * it;
       const int r = id / CPR, cc = id % CPR;
       const s16x8 v = *reinterpret_cast<const s16x8 *>(patch + r * LD + cc * 8);
       store_chunk_widened<T>((float *)dst_rows + (int64_t)r * stride_seq, cc * 8, headdim, r < rows_valid, vec, v);
