@@ -473,25 +473,35 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) sc = Elem<T>::mfma(ring[ks], qf[ks], sc);
     if (block_at(0) >= n_full) apply_mask(sc, block_at(0) * BLK);
-    m_ref = row_max(sc);  // finite: every query row sees key 0
-    // The second key group's first block is block 1: no probabilities where it is not the wave's.  Where it
-    // holds keys whose scores are all -inf (a bias column that hides keys) the row starts from block 0's
-    // maximum, as with one group.
-    if (KG > 1 && n_mine <= 0) {
-      m_ref = 0.f;
-    } else if (KG > 1 && kg == 1 && __builtin_amdgcn_ballot_w64(m_ref == -INFINITY) != 0) {
+    if (KG > 1 && kg == 1) {
+      // The second key group's first block is block 1, which may hold nothing but keys above the diagonal or
+      // keys that a bias hides (-inf, or the type's lowest value).  Its rows start from block 0's maximum, as
+      // the first group's and those of a launch with one group do: the same probabilities, rounded to half
+      // precision at the same scale, whatever the grid.  One score chain more in this prologue costs less
+      // than the timing's noise (B=1 H=16 N=333 D=128, bf16: 9.20 us with the group's own maximum, 9.17 us so;
+      // B=1 H=8 N=4096 D=128, forward and backward: 186.1 and 186.2 us).
       f32x16 s0 = zero;
 #pragma unroll
       for (int ks = 0; ks < KS; ks++) s0 = Elem<T>::mfma(lds_read_128(kcur[ks] - BLK * LP), qf[ks], s0);
       if (n_full < 1) apply_mask(s0, 0);
-      const float m0 = row_max(s0);
-      if (m_ref == -INFINITY) m_ref = m0;
+      m_ref = row_max(s0);
+    } else {
+      m_ref = row_max(sc);  // finite: every query row sees key 0
     }
-    const float mc = m_ref * scale_log2;
+    auto exponentials = [&]() {
+      const float mc = m_ref * scale_log2;
+      l_run = 0.f;
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-      e[i] = PRE ? fast_exp2(sc[i] - m_ref) : fast_exp2(sc[i] * scale_log2 - mc);
-      l_run += e[i];
+      for (int i = 0; i < 16; i++) {
+        e[i] = PRE ? fast_exp2(sc[i] - m_ref) : fast_exp2(sc[i] * scale_log2 - mc);
+        l_run += e[i];
+      }
+    };
+    exponentials();
+    // Block 1 far above block 0's maximum: what a step does then (below), with nothing accumulated yet.
+    if (KG > 1 && kg == 1 && __builtin_amdgcn_ballot_w64(!(l_run <= kSumTrigger)) != 0) {
+      m_ref = fmaxf(m_ref, row_max(sc));
+      exponentials();
     }
     if (KG == 1) {
 #pragma unroll

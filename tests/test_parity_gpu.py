@@ -631,6 +631,46 @@ def test_keys_hidden_by_a_bias_column(fa, d, first, last, heads):
         _assert_close(name, one(out), want)
 
 
+@pytest.mark.parametrize("heads", [2, 400], ids=["two_groups", "one_group"])
+@pytest.mark.parametrize("bias", [-1e30, -3e38])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_second_block_hidden_by_a_finite_bias(fa, d, bias, heads):
+    """Keys 32..63 pushed down by a large finite number instead of -inf (the way masks of the type's lowest
+    value do): the second key group, whose first block holds nothing else, must not start from their scores."""
+    q, k, v, _ = (t.cuda() for t in _seeded((1, heads, 300, d), (1, heads, 300, d), torch.bfloat16))
+    q[..., -1] = 1.0
+    k[..., -1] = 0.0
+    k[:, :, 32:64, -1] = bias
+    one = lambda t: t[:, heads - 1 :].float()  # noqa: E731
+    s = one(q) @ one(k).transpose(-1, -2).contiguous() / math.sqrt(d)
+    s = s.masked_fill(~torch.ones(300, 300, dtype=torch.bool, device="cuda").tril(), float("-inf"))
+    want = torch.softmax(s, -1) @ one(v)
+    _assert_close("o", one(fa.flash_attention_v2(q.clone().requires_grad_(True), k, v).detach()), want)
+    with torch.no_grad():
+        _assert_close("o (forward only)", one(fa.flash_attention_v2(q, k, v)), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("n,d", [(333, 128), (512, 64), (1000, 96), (700, 256)])
+def test_key_groups_round_the_same_probabilities(fa, n, d, dtype):
+    """A head alone (two key groups) and the same head in a grid of one group: the probabilities are rounded to
+    half precision at the same scale, so only the order of the fp32 sums differs.  Its error is about 3e-7 of
+    a value; one output in 3e-7 / 2^-9 (bf16; 2^-12 in fp16) = 1.5e-4 (1.2e-3) then lands on the other side of
+    a rounding boundary and moves by up to 2^-7 (2^-10) of itself: sqrt(1.5e-4) * 2^-7 = 1e-4 of the norm at
+    most (4e-5 in fp16)."""
+    q, k, v, _ = (t.cuda() for t in _seeded((1, 1, n, d), (1, 1, n, d), dtype))
+    many = [t.expand(1, 400, n, d).contiguous() for t in (q, k, v)]
+    bound = 1e-4 if dtype == torch.bfloat16 else 4e-5
+    leaf = [t.clone().requires_grad_(True) for t in (q, k, v)]
+    pairs = [("o", fa.flash_attention_v2(*leaf), fa.flash_attention_v2(many[0].requires_grad_(True), *many[1:]))]
+    with torch.no_grad():
+        pairs.append(("o (forward only)", fa.flash_attention_v2(q, k, v), fa.flash_attention_v2(*many)))
+    for name, got, want in pairs:
+        got, want = got.detach().double(), want.detach()[:, -1:].double()
+        rel = ((got - want).norm() / want.norm()).item()
+        assert rel <= bound, f"{name}: relative difference {rel:.2e} > {bound:.0e}"
+
+
 @pytest.mark.parametrize("b,h,n,d,transposed", [(1, 2, 1, 64, False), (2, 3, 200, 64, True), (1, 2, 130, 50, False), (1, 2, 130, 50, True),
                                                 (1, 2, 97, 80, True), (1, 300, 640, 32, False), (1, 16, 4225, 128, False),
                                                 (1, 2, 257, 96, True), (1, 2, 200, 256, False), (1, 400, 65, 200, False)])
