@@ -149,8 +149,15 @@ struct FlashAttentionV2 : public torch::autograd::Function<FlashAttentionV2> {
   }
 };
 
+// A tensor the node may save.  Autograd refuses to save a tensor made in inference mode; a strided view of
+// one goes in as a copy, which is an ordinary tensor.
+at::Tensor savable(const at::Tensor &t) { return t.is_inference() && !t.is_contiguous() ? t.contiguous() : t; }
+
 at::Tensor flash_attention_v2(const at::Tensor &q, const at::Tensor &k, const at::Tensor &v,
                               double softmax_scale, bool deterministic, int64_t max_headdim, bool forward_only) {
+  if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad()))
+    return FlashAttentionV2::apply(savable(q), savable(k), savable(v), softmax_scale, deterministic, max_headdim,
+                                   forward_only);
   return FlashAttentionV2::apply(q, k, v, softmax_scale, deterministic, max_headdim, forward_only);
 }
 

@@ -550,6 +550,22 @@ def test_strided_views_equal_contiguous_copies(fa, d, pad, offset):
         assert torch.equal(x, y)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+def test_strided_views_made_in_inference_mode(fa, dtype):
+    """k and v as transposed views of tensors made under torch.inference_mode, which autograd cannot save, beside
+    a q that wants its gradient: the bits of ordinary contiguous tensors."""
+    q, kv, _, d_o = (t.cuda() for t in _seeded((2, 3, 200, 64), (2, 200, 3, 64), dtype))
+    with torch.inference_mode():
+        made = kv.clone()
+    results = []
+    for keys in (made.transpose(1, 2), kv.transpose(1, 2).contiguous()):
+        leaf = q.clone().requires_grad_(True)
+        out = fa.flash_attention_v2(leaf, keys, keys)
+        results.append((out, *torch.autograd.grad(out, leaf, d_o)))
+    for got, want in zip(*results):
+        assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("nq,nk,d", [(64, 64, 256), (63, 65, 256), (1, 130, 192), (130, 1, 256), (129, 200, 136),
                                      (300, 64, 248), (191, 191, 192), (257, 320, 256), (65, 64, 128), (1, 70, 104),
