@@ -35,29 +35,32 @@ template <typename T>
 __global__ __launch_bounds__(256) void bwd_preprocess_kernel(const PreParams p) {
   const int tid = threadIdx.x;
   const int sub = tid & 15;
-  // One-dimensional grid: row tiles of one (batch, head) pair are consecutive workgroups.
+  // Row tiles of one (batch, head) pair are consecutive.  (More than one tile per workgroup only where a grid of
+  // all of them could not be launched: past a million heads.)
   const int tiles = (p.seqlen_q_rounded + 15) / 16;
-  const int bh = blockIdx.x / tiles;
-  const int row = (blockIdx.x - bh * tiles) * 16 + (tid >> 4);
-  const int b = bh / p.nheads, hd = bh % p.nheads;
   const bool vec = p.vec != 0;
-  float acc = 0.f;
-  if (row < p.seqlen_q) {
-    const short *orow = (const short *)p.o.ptr + b * p.o.stride_batch + hd * p.o.stride_head +
-                        (int64_t)row * p.o.stride_seq;
-    const short *grow = (const short *)p.d_o.ptr + b * p.d_o.stride_batch +
-                        hd * p.d_o.stride_head + (int64_t)row * p.d_o.stride_seq;
-    for (int d0 = sub * 8; d0 < p.headdim; d0 += 128) {
-      s16x8 a = load_chunk(orow, d0, p.headdim, true, vec);
-      s16x8 g = load_chunk(grow, d0, p.headdim, true, vec);
+  for (unsigned t = blockIdx.x; t < p.n_tiles; t += gridDim.x) {
+    const int bh = t / tiles;
+    const int row = (t - bh * tiles) * 16 + (tid >> 4);
+    const int b = bh / p.nheads, hd = bh % p.nheads;
+    float acc = 0.f;
+    if (row < p.seqlen_q) {
+      const short *orow = (const short *)p.o.ptr + b * p.o.stride_batch + hd * p.o.stride_head +
+                          (int64_t)row * p.o.stride_seq;
+      const short *grow = (const short *)p.d_o.ptr + b * p.d_o.stride_batch +
+                          hd * p.d_o.stride_head + (int64_t)row * p.d_o.stride_seq;
+      for (int d0 = sub * 8; d0 < p.headdim; d0 += 128) {
+        s16x8 a = load_chunk(orow, d0, p.headdim, true, vec);
+        s16x8 g = load_chunk(grow, d0, p.headdim, true, vec);
 #pragma unroll
-      for (int j = 0; j < 8; j++) acc += Elem<T>::to_float(a[j]) * Elem<T>::to_float(g[j]);
+        for (int j = 0; j < 8; j++) acc += Elem<T>::to_float(a[j]) * Elem<T>::to_float(g[j]);
+      }
     }
-  }
 #pragma unroll
-  for (int off = 8; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, 16);
-  if (sub == 0 && row < p.seqlen_q_rounded)
-    p.delta[(int64_t)bh * p.seqlen_q_rounded + row] = acc;
+    for (int off = 8; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, 16);
+    if (sub == 0 && row < p.seqlen_q_rounded)
+      p.delta[(int64_t)bh * p.seqlen_q_rounded + row] = acc;
+  }
 }
 
 // ------------------------------------------------------------------------------------------

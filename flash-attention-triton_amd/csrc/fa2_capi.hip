@@ -189,7 +189,8 @@ int fwd_impl(const fa2_fwd_args &a, void *stream) {
   p.n_qtiles = (a.seqlen_q + block_q - 1) / block_q;
 
   const int64_t nwg = (int64_t)p.n_qtiles * a.batch * a.nheads;
-  if (nwg > 0x7fffffff) return fail(FA2_ERR_TOO_LARGE, "grid of %lld workgroups too large", (long long)nwg);
+  if (nwg > fa2::kMaxWorkgroups)
+    return fail(FA2_ERR_TOO_LARGE, "grid of %lld workgroups too large", (long long)nwg);
   p.resident_grid = resident_grid(nwg, kTable[cfg].fwd_wg_per_cu);
   fa2::launch_fwd(a.dtype == FA2_DTYPE_BF16, kTable[cfg].headdim_padded, kTable[cfg].fwd_exp_folded != 0, p,
                   dim3((unsigned)nwg), reinterpret_cast<hipStream_t>(stream));
@@ -214,7 +215,9 @@ int preprocess_impl(const fa2_tensor &o, const fa2_tensor &d_o, float *delta, in
   p.vec = vec_ok(p.o, headdim) && vec_ok(p.d_o, headdim);
   const int64_t nwg = (int64_t)((seqlen_q_rounded + 15) / 16) * batch * nheads;
   if (nwg > 0x7fffffff) return fail(FA2_ERR_TOO_LARGE, "grid of %lld workgroups too large", (long long)nwg);
-  fa2::launch_preprocess(dtype == FA2_DTYPE_BF16, p, dim3((unsigned)nwg), reinterpret_cast<hipStream_t>(stream));
+  p.n_tiles = (unsigned)nwg;
+  fa2::launch_preprocess(dtype == FA2_DTYPE_BF16, p, dim3((unsigned)std::min<int64_t>(nwg, fa2::kMaxWorkgroups)),
+                         reinterpret_cast<hipStream_t>(stream));
   return launch_status("fa2_bwd_preprocess launch");
 }
 
@@ -293,7 +296,7 @@ int bwd_impl(const fa2_bwd_args &a, void *stream, bool grads_f32 = false) {
   const int block_q = kDqBlockQ / fa2::dq_key_groups(dp, pq);
   pq.n_tiles = (a.seqlen_q + block_q - 1) / block_q;
   const int64_t nwg_k = pk.n_tiles * bh, nwg_q = pq.n_tiles * bh;
-  if (nwg_k > 0x7fffffff || nwg_q > 0x7fffffff)
+  if (nwg_k > fa2::kMaxWorkgroups || nwg_q > fa2::kMaxWorkgroups)
     return fail(FA2_ERR_TOO_LARGE, "grid of %lld workgroups too large", (long long)std::max(nwg_k, nwg_q));
 
   const bool pair = block_kv == fa2::kDkvPairBlockKV;

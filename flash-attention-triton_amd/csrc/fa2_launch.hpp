@@ -63,14 +63,14 @@ inline int dq_key_groups(int dp, const BwdParams &p) {
   return dq_direct_ok(dp, p) ? key_groups(dp, (int64_t)p.batch * p.nheads, p.seqlen_q) : 1;
 }
 inline bool dkdv_direct_ok(int dp, const BwdParams &p) {
-  return p.vec && direct_headdim(dp, p.headdim) && direct_stride_ok(p.q) && direct_stride_ok(p.d_o) &&
+  return p.vec && direct_headdim(dp, p.headdim) && dp != 96 && direct_stride_ok(p.q) && direct_stride_ok(p.d_o) &&
          direct_stride_ok(p.k) && direct_stride_ok(p.v);
 }
 // Where the paired dK/dV kernel (fa2_bwd_dkdv_pair.hpp) is the better one.  Its workgroups are half as long
 // and start faster; its loop reads every Q and dO tile for 64 keys instead of 128.  Time of the other
 // kernel over its own, bf16, (batch, head) pairs x tokens:
-//   192, 256 columns  2.7 at 256, 1.5 at 192 (16 x 4096): always
-//   96 columns        1.02 (4 x 16384) to 1.6 (4 x 4096), 1.05-1.07 on large grids: always
+//   192, 256 columns  2.7 at 256, 1.5 at 192 (16 x 4096): always (the other one is the generic kernel)
+//   96 columns        1.02 (4 x 16384) to 1.6 (4 x 4096), 1.05-1.07 on large grids: always (likewise)
 //   128 columns       1.59 (1 x 16384), 1.24 (4 x 8192), 1.10 (4 x 12288) below 512 workgroups of 128 keys;
 //                     above, 1.05 (64 x 2048), 1.02 (256 x 4096), 0.99 (16 x 4096), but 0.95 (8 x 8192) and
 //                     0.98 (16 x 16384): there its extra tile loads cost board power, and clock
@@ -82,6 +82,9 @@ inline bool dkdv_pair_ok(int dp, const BwdParams &p) {
   if (!(p.vec && direct_headdim_wide(dp, p.headdim) && direct_stride_ok(p.q) && direct_stride_ok(p.d_o) &&
         direct_stride_ok(p.k) && direct_stride_ok(p.v)))
     return false;
+  // Twice the workgroups: not where only tiles of 128 keys make a grid that can be launched (more than 8.4
+  // million heads).
+  if ((int64_t)((p.seqlen_k + kDkvPairBlockKV - 1) / kDkvPairBlockKV) * p.batch * p.nheads > kMaxWorkgroups) return false;
   if (dp > 128 || dp == 96) return true;
   const int64_t wgs = (int64_t)((p.seqlen_k + kDkvBlockKV - 1) / kDkvBlockKV) * p.batch * p.nheads;
   if (dp == 128) return wgs < 2 * kCUs || p.seqlen_q <= 4096;

@@ -9,6 +9,9 @@ constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 
 constexpr int kCUs = 256;  // compute units of an MI355X
+// Workgroups of 256 threads a launch may have: the hardware is handed the grid in threads, as a 32-bit number, and
+// of a larger grid only what is left modulo 2^32 runs, without an error.
+constexpr long long kMaxWorkgroups = 0xffffffffll / 256;
 
 // One (batch, nheads, seqlen, headdim) tensor: base pointer and strides in elements.
 struct Tensor4 {
@@ -68,6 +71,7 @@ struct PreParams {
   Tensor4 o, d_o;
   float *delta;
   int batch, nheads, seqlen_q, headdim, seqlen_q_rounded;
+  unsigned n_tiles;  // tiles of 16 rows over all (batch, head) pairs
   int vec;
 };
 

@@ -95,8 +95,32 @@ int check_mapping() {
   return bad;
 }
 
+// The paired dK/dV kernel has twice the workgroups of the others: it is not picked where only they make a grid
+// that can be launched.
+int check_launchable_grids() {
+  int bad = 0, cases = 0;
+  for (int dp : {32, 64, 96, 128, 192, 256})
+    for (int seqlen : {1, 64, 65, 128, 129, 4096, 100000})
+      for (int64_t wgs : {int64_t(512), int64_t(fa2::kMaxWorkgroups) / 2, int64_t(fa2::kMaxWorkgroups) / 2 + 1, int64_t(fa2::kMaxWorkgroups)}) {
+        fa2::BwdParams p{};
+        p.headdim = dp;
+        p.vec = 1;
+        p.batch = (int)(wgs / ((seqlen + fa2::kDkvBlockKV - 1) / fa2::kDkvBlockKV));
+        p.nheads = 1;
+        p.seqlen_q = p.seqlen_k = seqlen;
+        if (p.batch == 0) continue;
+        const int keys = fa2::dkdv_block_kv(dp, p);
+        if ((int64_t)((seqlen + keys - 1) / keys) * p.batch > fa2::kMaxWorkgroups) bad++;
+        if (dp == 96 && fa2::dkdv_direct_ok(dp, p)) bad++;  // there is no such kernel
+        cases++;
+      }
+  printf("launchable grids, %d cases: %s\n", cases, bad ? "FAILED" : "ok");
+  return bad;
+}
+
 int main() {
   int bad = check_mapping();
+  bad += check_launchable_grids();
   bad += check<32>();
   bad += check<64>();
   bad += check<96>();

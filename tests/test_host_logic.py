@@ -289,6 +289,21 @@ def test_cpp_autograd_node_is_built_and_matches_the_library(capi, fa2_module):
         fa2_module._apply(q, q, q, None, fa2_module.GFX950_KERNEL_CONFIG_DETERMINISTIC)
 
 
+def test_grids_beyond_a_launch_are_refused(capi):
+    """Of a grid of 2^32 threads and more only the remainder modulo 2^32 would run, silently: the entry points
+    refuse it before anything touches a device."""
+    lib = capi.load()
+    heads = 2**24  # 256 threads each
+    t = capi.Tensor(16, 0, 0, 0)
+    fwd = capi.FwdArgs(q=t, k=t, v=t, o=t, lse=16, batch=heads, nheads=1, seqlen_q=1, seqlen_k=1, headdim=8,
+                       seqlen_q_rounded=1, softmax_scale=1.0, dtype=capi.FA2_DTYPE_F16, config_id=capi.FA2_CONFIG_AUTO)
+    assert lib.fa2_status_string(lib.fa2_fwd_packed(fwd, None)) == b"FA2_ERR_TOO_LARGE"
+    bwd = capi.BwdArgs(q=t, k=t, v=t, o=t, d_o=t, dq=t, dk=t, dv=t, lse=16, delta=16, batch=heads, nheads=1, seqlen_q=1,
+                       seqlen_k=1, headdim=8, seqlen_q_rounded=1, softmax_scale=1.0, dtype=capi.FA2_DTYPE_F16,
+                       config_id=capi.FA2_CONFIG_AUTO)
+    assert lib.fa2_status_string(lib.fa2_bwd_packed(bwd, None)) == b"FA2_ERR_TOO_LARGE"
+
+
 def test_noalloc_entry_point_refuses_sizes_beyond_its_scratch(capi):
     """The size check of fa2_bwd_fused_noalloc comes before anything touches a device."""
     lib = capi.load()

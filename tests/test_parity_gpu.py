@@ -594,6 +594,21 @@ def test_dkdv_kernel_of_large_grids(fa, b, h, n, d):
             _assert_close(name, one(g).reshape(w.shape), w)
 
 
+def test_delta_of_more_tiles_than_a_launch_has_workgroups(fa):
+    """delta is formed in tiles of 16 rows (four columns: no 16-byte rows, so by a kernel of its own): sixteen tiles
+    for each of 1.1 million heads are more than one launch takes."""
+    b, n, d = 1_100_000, 2, 4
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    q, k, v, d_o = (torch.randn((b, 1, n, d), generator=gen, device="cuda").to(torch.bfloat16) for _ in range(4))
+    qg, kg, vg = (t.clone().requires_grad_(True) for t in (q, k, v))
+    grads = torch.autograd.grad(fa.flash_attention_v2(qg, kg, vg), (qg, kg, vg), d_o)
+    for i in (0, 60_000, 1_048_575, b - 1):
+        one = [t[i : i + 1] for t in (q, k, v, d_o)]
+        _, *want = _gpu_fp32_oracle(*one, None)
+        for name, g, w in zip(("dq", "dk", "dv"), grads, want):
+            _assert_close(name, g[i : i + 1].reshape(w.shape), w)
+
+
 @pytest.mark.parametrize("b,h,n,d", [(1, 33, 1000, 128), (1, 31, 2000, 128), (1, 85, 1100, 64), (3, 29, 650, 32), (1, 9, 3700, 96)])
 def test_grids_that_fit_the_chip_at_once(fa, b, h, n, d):
     """Grids of 257 to 1024 workgroups, none a multiple of 256, walk every second round of 256 backwards
