@@ -16,7 +16,8 @@
 // 756 -> 275 us (1000 TFLOP/s over the four products, 72 % of a large library matmul's rate on the same
 // card); D=192 (in one pass) 337 -> 220 us.  What bounds it now: one wave per SIMD, whose exponentials,
 // dS and exchange have only the wave's own MFMAs to hide under, and at 256 columns some fifty copies per
-// tile between the two halves of the register file.
+// tile between the two halves of the register file (40 values live in accumulation registers that the
+// vector instructions cannot reach, 48 in the padded kernel; none in scratch memory).
 //
 // At 128 columns and below one accumulator per wave lets two (three at 64) workgroups share a CU, and
 // workgroups of 64 keys fill the chip from fewer heads: dkdv_pair_ok (fa2_launch.hpp) says where that beats
@@ -167,8 +168,10 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem) {
   typedef const __attribute__((address_space(3))) float *stat_ptr;
   typedef const __attribute__((address_space(3))) f32x4 *stat4_ptr;
   stat_ptr stat = reinterpret_cast<stat_ptr>(lds0 + L::STAT_BASE) + 32 * role + 4 * h;
-  short *xput = smem + L::XCHG_BASE + wave * L::XCHG_WAVE + 8 * lane;
-  const short *xget = smem + L::XCHG_BASE + (wave ^ 1) * L::XCHG_WAVE + 8 * lane;
+  // Exchange areas of the pair, role 0's and then role 1's, both at constant offsets from one address.  (With an
+  // address for each the padded kernel at 256 columns was one register short: 20 bytes of scratch per lane.)
+  short *xchg = smem + L::XCHG_BASE + (wave & ~1) * L::XCHG_WAVE + 8 * lane;
+  constexpr int XPUT = role * L::XCHG_WAVE, XGET = (1 - role) * L::XCHG_WAVE;
 
   f32x16 acc[DB];
 #pragma unroll
@@ -270,8 +273,8 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem) {
     // The partner has taken what it was given for the tile before.
     if (L::XBUFS == 1) tile_barrier();
     auto give = [&](const s16x8 (&x)[2]) {
-      *reinterpret_cast<s16x8 *>(xput + xoff) = x[0];
-      *reinterpret_cast<s16x8 *>(xput + xoff + 64 * 8) = x[1];
+      *reinterpret_cast<s16x8 *>(xchg + xoff + XPUT) = x[0];
+      *reinterpret_cast<s16x8 *>(xchg + xoff + XPUT + 64 * 8) = x[1];
     };
     s16x8 df[2];
     auto pack_ds = [&]() {
@@ -303,8 +306,8 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem) {
     if (t >= 1 && t + 1 < n_tiles) store_stats(t + 1);
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     tile_barrier();
-    const s16x8 got[2] = {*reinterpret_cast<const s16x8 *>(xget + xoff),
-                          *reinterpret_cast<const s16x8 *>(xget + xoff + 64 * 8)};
+    const s16x8 got[2] = {*reinterpret_cast<const s16x8 *>(xchg + xoff + XGET),
+                          *reinterpret_cast<const s16x8 *>(xchg + xoff + XGET + 64 * 8)};
     if (t + 2 < n_tiles) {
       load_stats(t + 2);
       if (!SPREAD) issue_tile(t + 2);

@@ -228,8 +228,8 @@ __device__ __forceinline__ void store_transposed_acc(const f32x16 (&acc)[DP / 32
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   if (f32) {
-    // At 256 columns registers decide: unrolled, the addresses cost the dQ kernel two spills to scratch; rolled,
-    // the loop costs the paired dK/dV kernel five.
+    // At 256 columns registers decide: unrolled, the addresses cost the dQ kernel 12 bytes of scratch per lane;
+    // rolled, the loop costs the paired dK/dV kernel 20.  So chosen, neither uses any, padded or not.
     constexpr int U = UNROLL_F32 ? (32 * CPR) / 64 : 1;
 #pragma unroll U
     for (int it = 0; it < (32 * CPR) / 64; it++) {

@@ -1,7 +1,7 @@
 """What the compiler made of the kernels, read from the metadata of the code objects inside
 libfa2_gfx950.so (no GPU needed): register and LDS use per kernel must leave room for the workgroups
-per CU the gfx950 table states, and the LDS-direct kernels must not spill vector registers (a spill
-inside a tile loop shares the vmcnt counter with the tile loads and stalls on them)."""
+per CU the gfx950 table states, and the LDS-direct kernels must not spill vector registers to memory
+(a spill inside a tile loop shares the vmcnt counter with the tile loads and stalls on them)."""
 
 from __future__ import annotations
 
@@ -17,9 +17,12 @@ TOOLS = [LLVM / "llvm-objcopy", LLVM / "clang-offload-bundler", LLVM / "llvm-rea
 LDS_PER_CU = 160 * 1024
 REGS_PER_LANE = 512  # VGPRs + accumulation registers per SIMD lane, shared by the waves on the SIMD
 
-# No LDS-direct kernel may spill.  (The forward at 256 columns is instantiated in its padded form only:
-# with the column count a compile-time 256 the compiler spilled about forty registers.)
-KNOWN_SPILLS: dict = {}
+# No LDS-direct kernel may spill to scratch memory.  (The forward at 256 columns is instantiated in its padded form
+# only: with the column count a compile-time 256 the compiler spilled about forty registers.)  Spills into
+# accumulation registers, which cost a copy each way but no memory access: (kernel, columns, padded) -> how many.
+KNOWN_SPILLS: dict = {("bwd_dkdv_pair_kernel", 256, False): 40, ("bwd_dkdv_pair_kernel", 256, True): 48}
+# Workgroups per CU of the paired dK/dV kernel (dkdv_pair_wg_per_cu in fa2_params.hpp).
+PAIR_WG_PER_CU = {32: 3, 64: 3, 128: 2, 192: 1, 256: 1}
 
 
 def _kernel_records(library: pathlib.Path, tmp: pathlib.Path) -> list[dict]:
@@ -58,9 +61,10 @@ def _parse(name: str):
         return None
     kernel, dp, rest = m.group(1), int(m.group(2)), m.group(3)
     flags = re.findall(r"Lb([01])E", rest)
-    # fwd_direct<T, DP, BKV, PAD>; bwd_dq_direct<T, DP, BKV, FUSE_DELTA, PAD>; bwd_dkdv_direct<T, DP, BQ, PAD, ATOMIC>
+    # fwd_direct<T, DP, BKV, PAD>; bwd_dq_direct<T, DP, BKV, FUSE_DELTA, PAD>; bwd_dkdv_direct<T, DP, BQ, PAD, ATOMIC>;
+    # bwd_dkdv_pair<T, DP, PAD>
     pad = {"fwd_direct_kernel": lambda f: f[0], "bwd_dq_direct_kernel": lambda f: f[1],
-           "bwd_dkdv_direct_kernel": lambda f: f[0]}.get(kernel, lambda f: "0")(flags) == "1" if flags else False
+           "bwd_dkdv_direct_kernel": lambda f: f[0], "bwd_dkdv_pair_kernel": lambda f: f[0]}.get(kernel, lambda f: "0")(flags) == "1" if flags else False
     atomic = kernel == "bwd_dkdv_direct_kernel" and len(flags) > 1 and flags[1] == "1"
     return kernel, dp, pad, atomic
 
@@ -89,16 +93,19 @@ def test_lds_direct_kernels_do_not_spill(records):
     seen = set()
     for r in records:
         parsed = _parse(r["name"])
-        if not parsed or not parsed[0].endswith("_direct_kernel"):
+        if not parsed or not parsed[0].endswith(("_direct_kernel", "_pair_kernel")):
             continue
         kernel, dp, pad, _ = parsed
         seen.add((kernel, dp))
+        scratch = int(r["private_segment_fixed_size"])
+        assert scratch == 0, f"{r['name']}: {scratch} bytes of scratch per lane"
         allowed = KNOWN_SPILLS.get((kernel, dp, pad), 0)
         assert int(r["vgpr_spill_count"]) <= allowed, f"{r['name']}: {r['vgpr_spill_count']} vector registers spilled"
     for dp in (32, 64, 96, 128):
         assert {("fwd_direct_kernel", dp), ("bwd_dq_direct_kernel", dp), ("bwd_dkdv_direct_kernel", dp)} <= seen
     for dp in (192, 256):
         assert {("fwd_direct_kernel", dp), ("bwd_dq_direct_kernel", dp)} <= seen
+    assert {("bwd_dkdv_pair_kernel", dp) for dp in PAIR_WG_PER_CU} <= seen
 
 
 def test_registers_and_lds_leave_room_for_the_tables_workgroups(records):
@@ -111,7 +118,7 @@ def test_registers_and_lds_leave_room_for_the_tables_workgroups(records):
     checked = 0
     for r in records:
         parsed = _parse(r["name"])
-        if not parsed or parsed[0] not in column or parsed[3]:
+        if not parsed or parsed[0] not in (*column, "bwd_dkdv_pair_kernel") or parsed[3]:
             continue
         kernel, dp, _, _ = parsed
         if kernel == "bwd_dkdv_direct_kernel" and dp > 128:
@@ -119,10 +126,10 @@ def test_registers_and_lds_leave_room_for_the_tables_workgroups(records):
         regs = (int(r["vgpr_count"]) + 7) // 8 * 8  # the count includes the accumulation registers
         by_registers = min(8, REGS_PER_LANE // regs)  # waves per SIMD = workgroups per CU (4 waves, one per SIMD)
         by_lds = LDS_PER_CU // int(r["group_segment_fixed_size"])
-        want = rows[dp][column[kernel]]
+        want = PAIR_WG_PER_CU[dp] if kernel == "bwd_dkdv_pair_kernel" else rows[dp][column[kernel]]
         assert min(by_registers, by_lds) >= want, (r["name"], by_registers, by_lds, want)
         checked += 1
-    assert checked >= 3 * 4 * 2
+    assert checked >= 3 * 4 * 2 + 2 * 2 * len(PAIR_WG_PER_CU)
 
 
 # Two places in the kernels rest on facts about the compiler that no language rule guarantees: the
