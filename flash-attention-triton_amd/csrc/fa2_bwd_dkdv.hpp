@@ -4,7 +4,7 @@
 
 #include <type_traits>
 
-#include "fa2_bwd_dkdv_pair.hpp"
+#include "fa2_common.hpp"
 
 namespace fa2 {
 
@@ -294,11 +294,7 @@ struct DkvDirectLayout {
 // (at DB = 4: 32 of the 128 columns each, all 128 keys).  The result leaves the MFMA with the head
 // dimension across lanes, so every atomic instruction covers two 128-byte row segments.
 template <typename T, int DP, int BQ, bool PAD, bool ATOMIC_DQ = false>
-__global__ __launch_bounds__(64 * kDkvWaves, (DP <= 96 && !ATOMIC_DQ ? 2 : 1)) void bwd_dkdv_direct_kernel(const BwdParams p) {
-  if constexpr (DP == 96) {  // the paired form, at every size (dkdv_pair_ok)
-    bwd_dkdv_paired<T, DP, PAD>(p);
-    return;
-  }
+__global__ __launch_bounds__(64 * kDkvWaves, (DP <= 64 && !ATOMIC_DQ ? 2 : 1)) void bwd_dkdv_direct_kernel(const BwdParams p) {
   using L = DkvDirectLayout<DP, BQ>;
   constexpr int KS = DP / 16, DB = DP / 32, LP = L::LP;
   constexpr int NTHREADS = 64 * kDkvWaves;

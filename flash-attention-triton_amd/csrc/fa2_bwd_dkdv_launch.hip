@@ -2,6 +2,7 @@
 #include <algorithm>
 
 #include "fa2_bwd_dkdv.hpp"
+#include "fa2_bwd_dkdv_pair.hpp"
 #include "fa2_launch.hpp"
 
 namespace fa2 {
@@ -32,7 +33,7 @@ void launch_pair(int dp, const BwdParams &p, dim3 grid, dim3 block, hipStream_t 
   switch (dp) {
     case 32: hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 32, PAD>), grid, block, 0, s, p); break;
     case 64: hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 64, PAD>), grid, block, 0, s, p); break;
-    case 96: hipLaunchKernelGGL((bwd_dkdv_direct_kernel<T, 96, kDkvBlockQ, PAD>), grid, block, 0, s, p); break;
+    case 96: hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 96, PAD>), grid, block, 0, s, p); break;
     case 128: hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 128, PAD>), grid, block, 0, s, p); break;
     case 192: hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 192, PAD>), grid, block, 0, s, p); break;
     default: hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 256, PAD>), grid, block, 0, s, p); break;

@@ -351,17 +351,12 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem) {
 }
 
 template <typename T, int DP, bool PAD>
-__device__ __forceinline__ void bwd_dkdv_paired(const BwdParams &p) {
+__global__ __launch_bounds__(64 * kDkvWaves, (dkdv_pair_wg_per_cu(DP))) void bwd_dkdv_pair_kernel(const BwdParams p) {
   __shared__ __attribute__((aligned(1024))) short smem[DkvPairLayout<DP>::TOTAL_ELEMS];
   if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 1)
     bwd_dkdv_pair<T, DP, PAD, 1>(p, smem);
   else
     bwd_dkdv_pair<T, DP, PAD, 0>(p, smem);
-}
-
-template <typename T, int DP, bool PAD>
-__global__ __launch_bounds__(64 * kDkvWaves, (dkdv_pair_wg_per_cu(DP))) void bwd_dkdv_pair_kernel(const BwdParams p) {
-  bwd_dkdv_paired<T, DP, PAD>(p);
 }
 
 }  // namespace fa2

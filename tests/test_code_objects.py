@@ -22,7 +22,7 @@ REGS_PER_LANE = 512  # VGPRs + accumulation registers per SIMD lane, shared by t
 # accumulation registers, which cost a copy each way but no memory access: (kernel, columns, padded) -> how many.
 KNOWN_SPILLS: dict = {("bwd_dkdv_pair_kernel", 256, False): 40, ("bwd_dkdv_pair_kernel", 256, True): 48}
 # Workgroups per CU of the paired dK/dV kernel (dkdv_pair_wg_per_cu in fa2_params.hpp).
-PAIR_WG_PER_CU = {32: 3, 64: 3, 128: 2, 192: 1, 256: 1}
+PAIR_WG_PER_CU = {32: 3, 64: 3, 96: 2, 128: 2, 192: 1, 256: 1}
 
 
 def _kernel_records(library: pathlib.Path, tmp: pathlib.Path) -> list[dict]:
@@ -101,10 +101,9 @@ def test_lds_direct_kernels_do_not_spill(records):
         assert scratch == 0, f"{r['name']}: {scratch} bytes of scratch per lane"
         allowed = KNOWN_SPILLS.get((kernel, dp, pad), 0)
         assert int(r["vgpr_spill_count"]) <= allowed, f"{r['name']}: {r['vgpr_spill_count']} vector registers spilled"
-    for dp in (32, 64, 96, 128):
-        assert {("fwd_direct_kernel", dp), ("bwd_dq_direct_kernel", dp), ("bwd_dkdv_direct_kernel", dp)} <= seen
-    for dp in (192, 256):
+    for dp in (32, 64, 96, 128, 192, 256):
         assert {("fwd_direct_kernel", dp), ("bwd_dq_direct_kernel", dp)} <= seen
+    assert {dp for kernel, dp in seen if kernel == "bwd_dkdv_direct_kernel"} == {32, 64, 128}
     assert {("bwd_dkdv_pair_kernel", dp) for dp in PAIR_WG_PER_CU} <= seen
 
 
@@ -129,7 +128,7 @@ def test_registers_and_lds_leave_room_for_the_tables_workgroups(records):
         want = PAIR_WG_PER_CU[dp] if kernel == "bwd_dkdv_pair_kernel" else rows[dp][column[kernel]]
         assert min(by_registers, by_lds) >= want, (r["name"], by_registers, by_lds, want)
         checked += 1
-    assert checked >= 3 * 4 * 2 + 2 * 2 * len(PAIR_WG_PER_CU)
+    assert checked >= (3 * 4 - 1) * 2 + 2 * 2 * len(PAIR_WG_PER_CU)
 
 
 # Two places in the kernels rest on facts about the compiler that no language rule guarantees: the
