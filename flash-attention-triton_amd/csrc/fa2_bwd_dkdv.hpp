@@ -321,7 +321,10 @@ __global__ __launch_bounds__(64 * kDkvWaves, (DP <= 64 && !ATOMIC_DQ ? 2 : 1)) v
   // Key tile 0 has the longest query range: issue tiles in ascending order (heaviest first).
   const int BH = p.batch * p.nheads;
   int bh, kt;  // key tile 0 has the longest query range: rank == key tile
-  map_workgroup(p.resident_grid ? balanced_index(blockIdx.x, p.resident_grid) : blockIdx.x, BH, p.n_tiles, p.head_group, bh, kt);
+  // (Grids that fit the chip at once reach this kernel at 32 columns only: dkdv_pair_ok gives the paired kernel the
+  // others, and the atomic rows have one workgroup per CU.)
+  const int index = DP == 32 && !ATOMIC_DQ && p.resident_grid ? balanced_index(blockIdx.x, p.resident_grid) : blockIdx.x;
+  map_workgroup(index, BH, p.n_tiles, p.head_group, bh, kt);
   const int b = bh / p.nheads, hd = bh % p.nheads;
   const int kv0 = kt * kDkvBlockKV;
   const int kv0w = kv0 + 32 * wave;

@@ -95,6 +95,27 @@ int check_mapping() {
   return bad;
 }
 
+// balanced_index on every grid of up to four rounds: a permutation of the grid that keeps a workgroup's index modulo 8
+// (the XCD a head stays on) and its round, and walks the second and fourth round backwards.
+int check_balanced_index() {
+  int bad = 0;
+  for (int total = 1; total <= 4 * fa2::kCUs; total++) {
+    std::vector<int> seen(total, 0);
+    for (int i = 0; i < total; i++) {
+      const int j = fa2::balanced_index(i, total);
+      if (j < 0 || j >= total) { bad++; continue; }
+      seen[j]++;
+      bad += j % 8 != i % 8 || j / fa2::kCUs != i / fa2::kCUs;
+      if (!(i / fa2::kCUs & 1)) bad += j != i;
+    }
+    for (int v : seen) bad += v != 1;
+    for (int base = fa2::kCUs; base + 16 <= total; base += 2 * fa2::kCUs)  // its first steps take its last tiles
+      bad += fa2::balanced_index(base, total) <= fa2::balanced_index(base + 8, total);
+  }
+  printf("balanced index, %d grids: %s\n", 4 * fa2::kCUs, bad ? "FAILED" : "ok");
+  return bad;
+}
+
 // The paired dK/dV kernel has twice the workgroups of the others: it is not picked where only they make a grid
 // that can be launched.
 int check_launchable_grids() {
@@ -120,6 +141,7 @@ int check_launchable_grids() {
 
 int main() {
   int bad = check_mapping();
+  bad += check_balanced_index();
   bad += check_launchable_grids();
   bad += check<32>();
   bad += check<64>();
