@@ -15,7 +15,7 @@ import threading
 # The in-tree build; FA2_GFX950_LIBRARY names another build of the same ABI (e.g. one under test).
 LIBRARY_PATH = pathlib.Path(os.environ.get("FA2_GFX950_LIBRARY") or
                             pathlib.Path(__file__).resolve().parent / "csrc" / "libfa2_gfx950.so")
-ABI_VERSION = 5
+ABI_VERSION = 6
 
 FA2_DTYPE_F16 = 0
 FA2_DTYPE_BF16 = 1
@@ -104,13 +104,14 @@ def load() -> ctypes.CDLL:
                     "(hipcc --offload-arch=gfx950); there is no fallback path."
                 )
             lib = ctypes.CDLL(str(LIBRARY_PATH))
+            lib.fa2_abi_version.restype = _i
+            got = lib.fa2_abi_version()  # before the other symbols: a library of another version may lack some
+            if got != ABI_VERSION:
+                raise RuntimeError(f"libfa2_gfx950.so has ABI version {got}, binding expects {ABI_VERSION}")
             for name, (restype, argtypes) in SIGNATURES.items():
                 fn = getattr(lib, name)
                 fn.restype = restype
                 fn.argtypes = argtypes
-            got = lib.fa2_abi_version()
-            if got != ABI_VERSION:
-                raise RuntimeError(f"libfa2_gfx950.so has ABI version {got}, binding expects {ABI_VERSION}")
             _lib = lib
     return _lib
 

@@ -169,5 +169,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "q, k, v: CUDA fp16/bf16/fp32 (B, H, N, D), any strides; softmax_scale > 0; returns o in their type",
         py::arg("q"), py::arg("k"), py::arg("v"), py::arg("softmax_scale"), py::arg("deterministic"),
         py::arg("max_headdim"), py::arg("forward_only") = false);
-  m.def("abi_version", []() { return fa2_abi_version(); });
+  m.def("abi_version", []() { return FA2_ABI_VERSION; });  // of the header this node was compiled with
 }

@@ -33,7 +33,9 @@
 extern "C" {
 #endif
 
-#define FA2_ABI_VERSION 5
+/* Raised with every entry point added or changed and every change of what a field means: 6 brought
+ * fa2_bwd_packed_f32_grads and the paired dK/dV kernel (bwd_block_kv, lds_direct and dkdv_passes below). */
+#define FA2_ABI_VERSION 6
 
 /* Largest head dimension the kernels accept (the table's `max_headdim`). */
 #define FA2_MAX_HEADDIM 256

@@ -5,8 +5,10 @@ from __future__ import annotations
 
 import ctypes
 import dataclasses
+import hashlib
 import pathlib
 import re
+import subprocess
 
 import pytest
 import torch
@@ -41,6 +43,30 @@ def test_library_exports_every_declared_symbol(capi):
     for name in names:
         assert hasattr(lib, name), f"libfa2_gfx950.so does not export {name}"
     assert sorted(capi.SIGNATURES) == names, "ctypes binding and header disagree on the entry points"
+
+
+# sha256 (first 16 digits) of include/fa2_gfx950.h without comments, white space and the version itself, per ABI
+# version.  A change of the interface needs a new version and a line here.
+INTERFACES = {6: "94837833e0c9a376"}
+
+
+def test_abi_version_follows_the_interface(capi):
+    text = re.sub(r"/\*.*?\*/", " ", (ROOT / "include" / "fa2_gfx950.h").read_text(), flags=re.S)
+    version = int(re.search(r"#define FA2_ABI_VERSION (\d+)", text).group(1))
+    text = " ".join(re.sub(r"#define FA2_ABI_VERSION \d+", "", text).split())
+    assert version == capi.ABI_VERSION == max(INTERFACES)
+    assert hashlib.sha256(text.encode()).hexdigest()[:16] == INTERFACES[version]
+
+
+def test_library_of_another_version_is_refused_by_name(capi, tmp_path, monkeypatch):
+    """Also one that lacks entry points of this version: the error says which version it has, not which symbol."""
+    (tmp_path / "old.c").write_text("int fa2_abi_version(void) { return 5; }\n")
+    old = tmp_path / "libfa2_gfx950.so"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(old), str(tmp_path / "old.c")], check=True)
+    monkeypatch.setattr(capi, "LIBRARY_PATH", old)
+    monkeypatch.setattr(capi, "_lib", None)
+    with pytest.raises(RuntimeError, match="ABI version 5, binding expects"):
+        capi.load()
 
 
 def test_abi_version_and_table(capi):
