@@ -78,6 +78,12 @@ def _measured_traffic(workload: str) -> tuple[dict, str]:
     return rows, "profiles/" + TRAFFIC_PROFILE.name
 
 
+def kernel_name(launch: dict, part: str) -> str:
+    """Name of the kernel a part of a call runs, from the library's own account of it (capi.launch_info)."""
+    suffix = {"generic": "kernel", "direct": "direct_kernel", "paired": "pair_kernel"}[launch[part]["form"]]
+    return {"fwd": "fwd_", "dq": "bwd_dq_", "dkdv": "bwd_dkdv_"}[part] + suffix
+
+
 class ClockSampler:
     """Samples the shader clock the driver reports (sysfs pp_dpm_sclk, the level marked '*') from
     a background thread while a timed region runs."""
@@ -490,20 +496,20 @@ def main() -> int:
     # FLOPs per launch, counted in causal GEMMs of fwd_flops / 2 each: the forward kernel owns 2
     # (S, PV), the dK/dV kernel 4 (S, dP, dV, dK), the dQ kernel 3 (S, dP, dQ).  The whole backward
     # is priced at the conventional 5 (2.5 x forward) although the two kernels execute 7.
-    # The LDS-direct kernels run when the table row has them and the head dimension needs no
-    # padding (the bench tensors are contiguous and 16-byte aligned); otherwise the generic ones.
+    # The library says which form of each kernel these sizes take (the bench tensors are contiguous and aligned).
     fa2 = importlib.import_module("flash-attention-triton_amd.flash_attention_2")
     row_id = capi.load().fa2_pick_config(fa2._COMPUTE_DTYPES[w.dtype], w.headdim, w.seqlen, w.seqlen, int(det))
     row = capi.config_table()[row_id]
-    kind = "direct_kernel" if row["lds_direct"] and row["headdim_padded"] == w.headdim else "kernel"
     only_row = capi.config_table()[capi.load().fa2_pick_config_forward_only(fa2._COMPUTE_DTYPES[w.dtype], w.headdim,
                                                                            w.seqlen, w.seqlen)]
+    launch = capi.launch_info(w.batch, w.nheads, w.seqlen, w.seqlen, w.headdim, row_id)
+    launch_only = capi.launch_info(w.batch, w.nheads, w.seqlen, w.seqlen, w.headdim, only_row["id"])
     kernels = {
-        "fwd": (f"fwd_{kind} (fa2_fwd, table row {row['id']}: the forward a backward follows)", 1.0 * w.fwd_flops),
-        "fwd_forward_only": (f"fwd_{kind} (fa2_fwd, table row {only_row['id']}: the forward nothing differentiates, "
+        "fwd": (f"{kernel_name(launch, 'fwd')} (fa2_fwd, table row {row['id']}: the forward a backward follows)", 1.0 * w.fwd_flops),
+        "fwd_forward_only": (f"{kernel_name(launch_only, 'fwd')} (fa2_fwd, table row {only_row['id']}: the forward nothing differentiates, "
                              "timed as fwd_ms)", 1.0 * w.fwd_flops),
-        "bwd_dkdv": (f"bwd_dkdv_{kind} (fa2_bwd, dK/dV half)", 2.0 * w.fwd_flops),
-        "bwd_dq": (f"bwd_dq_{kind} (fa2_bwd, dQ half)", 1.5 * w.fwd_flops),
+        "bwd_dkdv": (f"{kernel_name(launch, 'dkdv')} (fa2_bwd, dK/dV half)", 2.0 * w.fwd_flops),
+        "bwd_dq": (f"{kernel_name(launch, 'dq')} (fa2_bwd, dQ half)", 1.5 * w.fwd_flops),
     }
     dominant = max((name for name in kernels if name != "fwd_forward_only"), key=lambda name: leg_ms[name])
     traffic, traffic_source = _measured_traffic(w.name)
@@ -578,6 +584,8 @@ def main() -> int:
         "kernel_ms": leg_ms,
         "table_row": row,
         "table_row_forward_only": only_row,
+        "launch": launch,
+        "launch_forward_only": launch_only["fwd"],
     }
     if args.traffic_calibration:
         src = torch.ones(CALIBRATION_BYTES // 4, device=dev, dtype=torch.float32)

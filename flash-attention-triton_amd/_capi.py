@@ -15,7 +15,7 @@ import threading
 # The in-tree build; FA2_GFX950_LIBRARY names another build of the same ABI (e.g. one under test).
 LIBRARY_PATH = pathlib.Path(os.environ.get("FA2_GFX950_LIBRARY") or
                             pathlib.Path(__file__).resolve().parent / "csrc" / "libfa2_gfx950.so")
-ABI_VERSION = 6
+ABI_VERSION = 7
 
 FA2_DTYPE_F16 = 0
 FA2_DTYPE_BF16 = 1
@@ -39,6 +39,19 @@ class ConfigInfo(ctypes.Structure):
 
     def as_dict(self) -> dict:
         return {name: getattr(self, name) for name, _ in self._fields_}
+
+
+class LaunchPart(ctypes.Structure):
+    """Mirror of ``fa2_launch_part``: form, tile and grid of one kernel of a call."""
+
+    _fields_ = [*((name, _i) for name in ("form", "block_rows", "key_groups", "wg_per_cu", "resident")),
+                ("workgroups", _i64)]
+
+
+class LaunchInfo(ctypes.Structure):
+    """Mirror of ``fa2_launch_info``."""
+
+    _fields_ = [("config_id", _i), ("fwd", LaunchPart), ("dq", LaunchPart), ("dkdv", LaunchPart)]
 
 
 class Tensor(ctypes.Structure):
@@ -81,6 +94,7 @@ SIGNATURES = {
     "fa2_bwd": (_i, [_p] * 10 + [_i] * 6 + [_i64] * 21 + [_f, _i, _i, _i, _p]),
     "fa2_bwd_fused": (_i, [_p] * 11 + [_i] * 6 + [_i64] * 24 + [_f, _i, _i, _i, _p]),
     "fa2_bwd_fused_noalloc": (_i, [_p] * 9 + [_i] * 6 + [_i64] * 24 + [_f, _i, _i, _i, _p]),
+    "fa2_launch_info_get": (_i, [_i] * 6 + [ctypes.POINTER(LaunchInfo)]),
     "fa2_fwd_packed": (_i, [ctypes.POINTER(FwdArgs), _p]),
     "fa2_bwd_packed": (_i, [ctypes.POINTER(BwdArgs), _p]),
     "fa2_bwd_packed_f32_grads": (_i, [ctypes.POINTER(BwdArgs), _p]),
@@ -133,3 +147,19 @@ def config_table() -> list[dict]:
         check(lib.fa2_config_get(i, ctypes.byref(info)), "fa2_config_get")
         rows.append(info.as_dict())
     return rows
+
+
+FORMS = ("generic", "direct", "paired")
+
+
+def launch_info(batch: int, nheads: int, seqlen_q: int, seqlen_k: int, headdim: int,
+                config_id: int = FA2_CONFIG_AUTO) -> dict:
+    """What a forward and a backward on contiguous tensors of these sizes launch (fa2_launch_info_get)."""
+    info = LaunchInfo()
+    check(load().fa2_launch_info_get(batch, nheads, seqlen_q, seqlen_k, headdim, config_id, ctypes.byref(info)),
+          "fa2_launch_info_get")
+    out = {"config_id": info.config_id}
+    for part in ("fwd", "dq", "dkdv"):
+        out[part] = {name: getattr(getattr(info, part), name) for name, *_ in LaunchPart._fields_}
+        out[part]["form"] = FORMS[out[part]["form"]]
+    return out

@@ -157,6 +157,41 @@ int launch_status(const char *what) {
 
 bool good_scale(float s) { return s > 0.f && std::isfinite(s); }
 
+// Kernel form, tiles and grid of a forward: completes `p` and returns the number of workgroups.
+int64_t plan_fwd(int cfg, fa2::FwdParams &p) {
+  const int64_t bh = (int64_t)p.batch * p.nheads;
+  const int block_q = kFwdBlockQ / fa2::fwd_key_groups(kTable[cfg].headdim_padded, p);
+  p.head_group = head_group(cfg, bh);
+  p.n_qtiles = (p.seqlen_q + block_q - 1) / block_q;
+  const int64_t nwg = p.n_qtiles * bh;
+  p.resident_grid = resident_grid(nwg, kTable[cfg].fwd_wg_per_cu);
+  return nwg;
+}
+
+// The same for the two kernels of a backward.
+int64_t plan_dkdv(int cfg, fa2::BwdParams &p) {
+  const int dp = kTable[cfg].headdim_padded;
+  // The dK/dV kernel keeps the table's group size at every head count: with one or two workgroups
+  // per CU its drain is short either way, and measured at 96 heads the single group is 1-2 % slower.
+  p.head_group = kTable[cfg].head_group;
+  const int block_kv = kTable[cfg].dq_atomic ? kDkvBlockKV : fa2::dkdv_block_kv(dp, p);
+  p.n_tiles = (p.seqlen_k + block_kv - 1) / block_kv;
+  const int64_t nwg = p.n_tiles * ((int64_t)p.batch * p.nheads);
+  const bool pair = block_kv == fa2::kDkvPairBlockKV;
+  p.resident_grid = resident_grid(nwg, pair ? fa2::dkdv_pair_wg_per_cu(dp) : kTable[cfg].dkdv_wg_per_cu);
+  return nwg;
+}
+
+int64_t plan_dq(int cfg, fa2::BwdParams &p) {
+  const int64_t bh = (int64_t)p.batch * p.nheads;
+  const int block_q = kDqBlockQ / fa2::dq_key_groups(kTable[cfg].headdim_padded, p);
+  p.head_group = head_group(cfg, bh);
+  p.n_tiles = (p.seqlen_q + block_q - 1) / block_q;
+  const int64_t nwg = p.n_tiles * bh;
+  p.resident_grid = resident_grid(nwg, kTable[cfg].dq_wg_per_cu);
+  return nwg;
+}
+
 int fwd_impl(const fa2_fwd_args &a, void *stream) {
   int rc = check_common(a.batch, a.nheads, a.seqlen_q, a.seqlen_k, a.headdim, a.seqlen_q_rounded, a.dtype);
   if (rc) return rc;
@@ -181,17 +216,13 @@ int fwd_impl(const fa2_fwd_args &a, void *stream) {
   p.seqlen_k = a.seqlen_k;
   p.headdim = a.headdim;
   p.seqlen_q_rounded = a.seqlen_q_rounded;
-  p.head_group = head_group(cfg, (int64_t)a.batch * a.nheads);
   p.scale = a.softmax_scale;
   p.scale_log2 = a.softmax_scale * fa2::kLog2e;
   p.vec = vec_ok(p.q, a.headdim) && vec_ok(p.k, a.headdim) && vec_ok(p.v, a.headdim) && vec_ok(p.o, a.headdim);
-  const int block_q = kFwdBlockQ / fa2::fwd_key_groups(kTable[cfg].headdim_padded, p);
-  p.n_qtiles = (a.seqlen_q + block_q - 1) / block_q;
 
-  const int64_t nwg = (int64_t)p.n_qtiles * a.batch * a.nheads;
+  const int64_t nwg = plan_fwd(cfg, p);
   if (nwg > fa2::kMaxWorkgroups)
     return fail(FA2_ERR_TOO_LARGE, "grid of %lld workgroups too large", (long long)nwg);
-  p.resident_grid = resident_grid(nwg, kTable[cfg].fwd_wg_per_cu);
   fa2::launch_fwd(a.dtype == FA2_DTYPE_BF16, kTable[cfg].headdim_padded, kTable[cfg].fwd_exp_folded != 0, p,
                   dim3((unsigned)nwg), reinterpret_cast<hipStream_t>(stream));
   return launch_status("fa2_fwd launch");
@@ -272,7 +303,6 @@ int bwd_impl(const fa2_bwd_args &a, void *stream, bool grads_f32 = false) {
   p.seqlen_k = a.seqlen_k;
   p.headdim = a.headdim;
   p.seqlen_q_rounded = a.seqlen_q_rounded;
-  p.head_group = head_group(cfg, (int64_t)a.batch * a.nheads);
   p.scale = a.softmax_scale;
   p.scale_log2 = a.softmax_scale * fa2::kLog2e;
   p.vec = vec_ok(p.q, a.headdim) && vec_ok(p.k, a.headdim) && vec_ok(p.v, a.headdim) &&
@@ -288,20 +318,9 @@ int bwd_impl(const fa2_bwd_args &a, void *stream, bool grads_f32 = false) {
   p.dq_accum_rows = 0;
 
   fa2::BwdParams pk = p, pq = p;
-  // The dK/dV kernel keeps the table's group size at every head count: with one or two workgroups
-  // per CU its drain is short either way, and measured at 96 heads the single group is 1-2 % slower.
-  pk.head_group = kTable[cfg].head_group;
-  const int block_kv = kTable[cfg].dq_atomic ? kDkvBlockKV : fa2::dkdv_block_kv(dp, pk);
-  pk.n_tiles = (a.seqlen_k + block_kv - 1) / block_kv;
-  const int block_q = kDqBlockQ / fa2::dq_key_groups(dp, pq);
-  pq.n_tiles = (a.seqlen_q + block_q - 1) / block_q;
-  const int64_t nwg_k = pk.n_tiles * bh, nwg_q = pq.n_tiles * bh;
+  const int64_t nwg_k = plan_dkdv(cfg, pk), nwg_q = plan_dq(cfg, pq);
   if (nwg_k > fa2::kMaxWorkgroups || nwg_q > fa2::kMaxWorkgroups)
     return fail(FA2_ERR_TOO_LARGE, "grid of %lld workgroups too large", (long long)std::max(nwg_k, nwg_q));
-
-  const bool pair = block_kv == fa2::kDkvPairBlockKV;
-  pk.resident_grid = resident_grid(nwg_k, pair ? fa2::dkdv_pair_wg_per_cu(dp) : kTable[cfg].dkdv_wg_per_cu);
-  pq.resident_grid = resident_grid(nwg_q, kTable[cfg].dq_wg_per_cu);
 
   auto run_dkdv = [&]() {
     fa2::launch_dkdv(bf16, dp, pk, dim3((unsigned)nwg_k), s);
@@ -439,6 +458,54 @@ int fa2_pick_config(int dtype, int headdim, int seqlen_q, int seqlen_k, int dete
 int fa2_pick_config_forward_only(int dtype, int headdim, int seqlen_q, int seqlen_k) {
   const int id = fa2_pick_config(dtype, headdim, seqlen_q, seqlen_k, 0);  // validates
   return id < 0 ? id : pick_config_forward_only(dtype, headdim);
+}
+
+int fa2_launch_info_get(int batch, int nheads, int seqlen_q, int seqlen_k, int headdim, int config_id,
+                        fa2_launch_info *out) {
+  if (out == nullptr) return fail(FA2_ERR_NULL_POINTER, "out is NULL");
+  int rc = check_common(batch, nheads, seqlen_q, seqlen_k, headdim, seqlen_q, FA2_DTYPE_F16);
+  int cfg;
+  if (rc || (rc = resolve_config(config_id, headdim, &cfg))) return rc;
+  const fa2_config_info &row = kTable[cfg];
+  const int dp = row.headdim_padded;
+  auto contiguous = [&](int seqlen) {
+    return fa2::Tensor4{nullptr, (int64_t)nheads * seqlen * headdim, (int64_t)seqlen * headdim, headdim};
+  };
+  const fa2::Tensor4 tq = contiguous(seqlen_q), tk = contiguous(seqlen_k);
+  fa2::FwdParams f = {};
+  fa2::BwdParams k = {};
+  f.q = f.o = k.q = k.o = k.d_o = k.dq = tq;
+  f.k = f.v = k.k = k.v = k.dk = k.dv = tk;
+  f.batch = k.batch = batch;
+  f.nheads = k.nheads = nheads;
+  f.seqlen_q = k.seqlen_q = seqlen_q;
+  f.seqlen_k = k.seqlen_k = seqlen_k;
+  f.headdim = k.headdim = headdim;
+  f.vec = k.vec = headdim % 8 == 0;
+  fa2::BwdParams q = k;
+  auto part = [](int form, int block_rows, int key_groups, int wg_per_cu, int resident, int64_t nwg) {
+    const bool fast = form != FA2_FORM_GENERIC;
+    return fa2_launch_part{form, block_rows, key_groups, fast ? wg_per_cu : 0, fast && resident != 0, nwg};
+  };
+
+  *out = fa2_launch_info{};
+  out->config_id = cfg;
+  int64_t nwg = plan_fwd(cfg, f);
+  int groups = fa2::fwd_key_groups(dp, f);
+  out->fwd = part(fa2::fwd_direct_ok(dp, f) ? FA2_FORM_DIRECT : FA2_FORM_GENERIC, kFwdBlockQ / groups, groups,
+                  row.fwd_wg_per_cu, f.resident_grid, nwg);
+  if (row.fwd_exp_folded) return FA2_OK;
+  nwg = plan_dkdv(cfg, k);
+  const bool pair = !row.dq_atomic && fa2::dkdv_pair_ok(dp, k);
+  out->dkdv = part(pair ? FA2_FORM_PAIRED : fa2::dkdv_direct_ok(dp, k) ? FA2_FORM_DIRECT : FA2_FORM_GENERIC,
+                   pair ? fa2::kDkvPairBlockKV : kDkvBlockKV, 1, pair ? fa2::dkdv_pair_wg_per_cu(dp) : row.dkdv_wg_per_cu,
+                   k.resident_grid, nwg);
+  if (row.dq_atomic) return FA2_OK;
+  nwg = plan_dq(cfg, q);
+  groups = fa2::dq_key_groups(dp, q);
+  out->dq = part(fa2::dq_direct_ok(dp, q) ? FA2_FORM_DIRECT : FA2_FORM_GENERIC, kDqBlockQ / groups, groups,
+                 row.dq_wg_per_cu, q.resident_grid, nwg);
+  return FA2_OK;
 }
 
 int fa2_fwd_packed(const fa2_fwd_args *args, void *stream) {

@@ -9,9 +9,6 @@
 
 namespace fa2 {
 
-// Which kernel a launcher picked (reported to callers that label measurements).
-enum KernelPath { kPathGeneric = 0, kPathDirect = 1 };
-
 // The fast kernels need a head dimension that is a multiple of 8 (whole 16-byte chunks), 16-byte aligned
 // rows and row offsets inside a tile that fit 32 bits.  A head dimension below the table row's padded one
 // runs the padded variant of the kernel.

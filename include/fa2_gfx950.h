@@ -34,8 +34,9 @@ extern "C" {
 #endif
 
 /* Raised with every entry point added or changed and every change of what a field means: 6 brought
- * fa2_bwd_packed_f32_grads and the paired dK/dV kernel (bwd_block_kv, lds_direct and dkdv_passes below). */
-#define FA2_ABI_VERSION 6
+ * fa2_bwd_packed_f32_grads and the paired dK/dV kernel (bwd_block_kv, lds_direct and dkdv_passes below), 7
+ * fa2_launch_info_get. */
+#define FA2_ABI_VERSION 7
 
 /* Largest head dimension the kernels accept (the table's `max_headdim`). */
 #define FA2_MAX_HEADDIM 256
@@ -100,6 +101,31 @@ typedef struct fa2_config_info {
                          which recompute the probabilities from Q itself; see fa2_pick_config_forward_only */
 } fa2_config_info;
 
+/* Kernel forms.  FA2_FORM_GENERIC is the fallback for operands the LDS-direct kernels cannot read. */
+typedef enum fa2_form {
+  FA2_FORM_GENERIC = 0, /* fwd_kernel, bwd_dq_kernel, bwd_dkdv_kernel */
+  FA2_FORM_DIRECT = 1,  /* fwd_direct_kernel, bwd_dq_direct_kernel, bwd_dkdv_direct_kernel */
+  FA2_FORM_PAIRED = 2   /* bwd_dkdv_pair_kernel */
+} fa2_form;
+
+/*
+ * What a call launches.  A table row leaves some of it open: the rules in csrc/fa2_launch.hpp choose by
+ * grid, length and alignment, and this record says what they chose.  `resident` is 1 where all workgroups
+ * fit the chip at once (their order is then balanced over the CUs).
+ */
+typedef struct fa2_launch_part {
+  int form;         /* fa2_form */
+  int block_rows;   /* query rows (forward, dQ) or key rows (dK/dV) per workgroup */
+  int key_groups;   /* forward and dQ: 2 when two waves share 32 query rows and split the keys, else 1 */
+  int wg_per_cu;    /* workgroups that share a CU (0: not stated, for the generic kernels) */
+  int resident;
+  int64_t workgroups;
+} fa2_launch_part;
+typedef struct fa2_launch_info {
+  int config_id;    /* the table row */
+  fa2_launch_part fwd, dq, dkdv; /* dq of a dq_atomic row: all zero (its dK/dV kernel forms dQ) */
+} fa2_launch_info;
+
 /* One (batch, nheads, seqlen, headdim) tensor: device pointer and strides in elements. */
 typedef struct fa2_tensor {
   const void *ptr;
@@ -156,11 +182,19 @@ int fa2_config_get(int config_id, fa2_config_info *out);
  * Table lookup: replaces _select_optimal_gpu_architecture (flash_attention_2.py:617-642).
  * Returns the row id (>= 0) that FA2_CONFIG_AUTO stands for, or a negative fa2_status on error.
  * The row depends on the head dimension (the padded dimension the kernels are instantiated for).
- * dtype, seqlen_q, seqlen_k and deterministic are validated and do not change the row: every row
- * runs 128-row workgroups over 64-row streamed tiles in both types, and both backward modes run
- * the same atomic-free kernels.
+ * dtype, seqlen_q, seqlen_k and deterministic are validated and do not change the row: a row's
+ * kernels come in both types, both backward modes run the same atomic-free ones, and which form of
+ * them a call takes is decided by its sizes (fa2_launch_info_get).
  */
 int fa2_pick_config(int dtype, int headdim, int seqlen_q, int seqlen_k, int deterministic);
+
+/*
+ * The kernels a forward and a backward of these sizes launch, for 16-byte aligned contiguous tensors.
+ * Touches no device.  No counterpart in the reference.  A forward-only row (fwd_exp_folded) has no
+ * backward: dq and dkdv come back all zero.
+ */
+int fa2_launch_info_get(int batch, int nheads, int seqlen_q, int seqlen_k, int headdim, int config_id,
+                        fa2_launch_info *out);
 
 /*
  * The row for a forward whose log-sum-exp no backward will read (inference, evaluation under

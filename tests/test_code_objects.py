@@ -21,8 +21,8 @@ REGS_PER_LANE = 512  # VGPRs + accumulation registers per SIMD lane, shared by t
 # only: with the column count a compile-time 256 the compiler spilled about forty registers.)  Spills into
 # accumulation registers, which cost a copy each way but no memory access: (kernel, columns, padded) -> how many.
 KNOWN_SPILLS: dict = {("bwd_dkdv_pair_kernel", 256, False): 40, ("bwd_dkdv_pair_kernel", 256, True): 48}
-# Workgroups per CU of the paired dK/dV kernel (dkdv_pair_wg_per_cu in fa2_params.hpp).
-PAIR_WG_PER_CU = {32: 3, 64: 3, 96: 2, 128: 2, 192: 1, 256: 1}
+# Columns the paired dK/dV kernel exists at.
+PAIR_COLUMNS = (32, 64, 96, 128, 192, 256)
 
 
 def _kernel_records(library: pathlib.Path, tmp: pathlib.Path) -> list[dict]:
@@ -104,7 +104,7 @@ def test_lds_direct_kernels_do_not_spill(records):
     for dp in (32, 64, 96, 128, 192, 256):
         assert {("fwd_direct_kernel", dp), ("bwd_dq_direct_kernel", dp)} <= seen
     assert {dp for kernel, dp in seen if kernel == "bwd_dkdv_direct_kernel"} == {32, 64, 128}
-    assert {("bwd_dkdv_pair_kernel", dp) for dp in PAIR_WG_PER_CU} <= seen
+    assert {("bwd_dkdv_pair_kernel", dp) for dp in PAIR_COLUMNS} <= seen
 
 
 def test_registers_and_lds_leave_room_for_the_tables_workgroups(records):
@@ -114,6 +114,9 @@ def test_registers_and_lds_leave_room_for_the_tables_workgroups(records):
     rows = {r["headdim_padded"]: r for r in capi.config_table() if not r["dq_atomic"] and not r["fwd_exp_folded"]}
     column = {"fwd_direct_kernel": "fwd_wg_per_cu", "bwd_dq_direct_kernel": "dq_wg_per_cu",
               "bwd_dkdv_direct_kernel": "dkdv_wg_per_cu"}
+    paired = {dp: capi.launch_info(1, 1, 64, 64, dp)["dkdv"] for dp in PAIR_COLUMNS}
+    assert all(p["form"] == "paired" for p in paired.values())
+    pair_wg_per_cu = {dp: p["wg_per_cu"] for dp, p in paired.items()}
     checked = 0
     for r in records:
         parsed = _parse(r["name"])
@@ -125,10 +128,10 @@ def test_registers_and_lds_leave_room_for_the_tables_workgroups(records):
         regs = (int(r["vgpr_count"]) + 7) // 8 * 8  # the count includes the accumulation registers
         by_registers = min(8, REGS_PER_LANE // regs)  # waves per SIMD = workgroups per CU (4 waves, one per SIMD)
         by_lds = LDS_PER_CU // int(r["group_segment_fixed_size"])
-        want = PAIR_WG_PER_CU[dp] if kernel == "bwd_dkdv_pair_kernel" else rows[dp][column[kernel]]
+        want = pair_wg_per_cu[dp] if kernel == "bwd_dkdv_pair_kernel" else rows[dp][column[kernel]]
         assert min(by_registers, by_lds) >= want, (r["name"], by_registers, by_lds, want)
         checked += 1
-    assert checked >= (3 * 4 - 1) * 2 + 2 * 2 * len(PAIR_WG_PER_CU)
+    assert checked >= (3 * 4 - 1) * 2 + 2 * 2 * len(PAIR_COLUMNS)
 
 
 # Two places in the kernels rest on facts about the compiler that no language rule guarantees: the

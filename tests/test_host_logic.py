@@ -47,7 +47,7 @@ def test_library_exports_every_declared_symbol(capi):
 
 # sha256 (first 16 digits) of include/fa2_gfx950.h without comments, white space and the version itself, per ABI
 # version.  A change of the interface needs a new version and a line here.
-INTERFACES = {6: "94837833e0c9a376"}
+INTERFACES = {6: "94837833e0c9a376", 7: "f98a87f9170d5460"}
 
 
 def test_abi_version_follows_the_interface(capi):
@@ -373,6 +373,46 @@ def test_workload_table_matches_baseline(workloads):
     q2, *_ = workloads.make_inputs(w["C1"], heads=3)
     assert q.dtype == torch.float16 and q.shape == (2, 4, 512, 64)
     torch.testing.assert_close(q2[:, 0], q.reshape(8, 512, 64)[:3], atol=0, rtol=0)
+
+
+def test_launch_info_says_what_a_call_launches(capi, workloads):
+    """fa2_launch_info_get against tiles and grids written out here, and the kernel names the bench derives from it."""
+    import importlib
+
+    bench = importlib.import_module("bench")
+    rows = capi.config_table()
+
+    def part(form, block_rows, key_groups, wg_per_cu, resident, workgroups):
+        return dict(form=form, block_rows=block_rows, key_groups=key_groups, wg_per_cu=wg_per_cu, resident=resident,
+                    workgroups=workgroups)
+
+    info = capi.launch_info(2, 32, 4096, 4096, 128)
+    assert info == {"config_id": 3, "fwd": part("direct", 128, 1, 2, 0, 2048), "dq": part("direct", 128, 1, 2, 0, 2048),
+                    "dkdv": part("paired", 64, 1, 2, 0, 4096)}
+    assert [bench.kernel_name(info, p) for p in ("fwd", "dq", "dkdv")] == [
+        "fwd_direct_kernel", "bwd_dq_direct_kernel", "bwd_dkdv_pair_kernel"]
+    info = capi.launch_info(1, 16, 16384, 16384, 128)  # longer than the paired kernel pays
+    assert info["dkdv"] == part("direct", 128, 1, 1, 0, 2048)
+    assert bench.kernel_name(info, "dkdv") == "bwd_dkdv_direct_kernel"
+    info = capi.launch_info(2, 4, 512, 512, 64)  # 32 workgroups of 128 rows for 256 CUs: two key groups
+    assert info["fwd"] == info["dq"] == part("direct", 64, 2, 3, 1, 64)
+    assert info["dkdv"] == part("paired", 64, 1, 3, 1, 64)
+    assert capi.launch_info(32, 20, 1024, 1024, 96)["dkdv"] == part("paired", 64, 1, 2, 0, 10240)
+    info = capi.launch_info(2, 8, 100, 200, 50)  # 50 columns: no 16-byte rows
+    assert info["fwd"] == info["dq"] == part("generic", 128, 1, 0, 0, 16)
+    assert info["dkdv"] == part("generic", 128, 1, 0, 0, 32)
+    assert [bench.kernel_name(info, p) for p in ("fwd", "dq", "dkdv")] == ["fwd_kernel", "bwd_dq_kernel", "bwd_dkdv_kernel"]
+    atomic = next(r for r in rows if r["dq_atomic"] and r["headdim_padded"] == 128)
+    info = capi.launch_info(2, 32, 4096, 4096, 128, atomic["id"])
+    assert info["dkdv"] == part("direct", 128, 1, atomic["dkdv_wg_per_cu"], 0, 2048) and not any(
+        v for k, v in info["dq"].items() if k != "form")
+    folded = next(r for r in rows if r["fwd_exp_folded"] and r["headdim_padded"] == 128)
+    info = capi.launch_info(2, 32, 4096, 4096, 128, folded["id"])
+    assert info["fwd"]["form"] == "direct" and info["dkdv"]["workgroups"] == info["dq"]["workgroups"] == 0
+    with pytest.raises(RuntimeError, match="FA2_ERR_BAD_SHAPE"):
+        capi.launch_info(0, 1, 1, 1, 64)
+    with pytest.raises(RuntimeError, match="FA2_ERR_BAD_CONFIG"):
+        capi.launch_info(1, 1, 1, 1, 64, 99)
 
 
 def test_traffic_stamp_ignores_comments_and_follows_code(tmp_path, monkeypatch):
