@@ -43,9 +43,12 @@ int dtype_code(const at::Tensor &t) { return t.scalar_type() == at::kBFloat16 ? 
 // The tensor as the kernels can read it.  They take any batch, head and row stride, so a view such as
 // (batch, token, head, column) memory transposed to (batch, head, token, column) goes in as it is,
 // provided it meets what the LDS-direct kernels ask of their operands: whole 16-byte chunks, aligned
-// rows and a row stride below 2^24 elements (fa2_launch.hpp).  Anything else is copied, because a copy is
-// cheaper than the generic kernels.  B=256 H=16 N=512 D=64, bf16 views, forward + backward: 1661 us with
-// the four copies (568 us of them), 1205 us without.
+// rows and a row stride below 2^24 elements (fa2_launch.hpp).  Any other strided view is copied: one with
+// whole chunks but odd alignment because a copy is cheaper than the generic kernels, one without (head
+// dimension not a multiple of 8) so that those kernels, which run either way, read rows that lie together.
+// A contiguous tensor goes in as it is; the generic kernels run where its base is not 16-byte aligned.
+// B=256 H=16 N=512 D=64, bf16 views, forward + backward: 1661 us with the four copies (568 us of them),
+// 1205 us without.
 at::Tensor readable(const at::Tensor &t) {
   if (t.is_contiguous()) return t;
   const bool direct = t.stride(3) == 1 && t.size(3) % 8 == 0 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 &&

@@ -550,6 +550,92 @@ def test_strided_views_equal_contiguous_copies(fa, d, pad, offset):
         assert torch.equal(x, y)
 
 
+def _kv_expanded(x, b, h, n, d):
+    """One head's rows expanded over the heads (stride 0)."""
+    return x[: b * n * d].view(b, 1, n, d).expand(b, h, n, d)
+
+
+def _batch_expanded(x, b, h, n, d):
+    return x[: h * n * d].view(1, h, n, d).expand(b, h, n, d)
+
+
+def _cache_slice(x, b, h, n, d):
+    """The filled part of a cache with room for more tokens: (batch, head) strides longer than n rows."""
+    return x[: b * h * (n + 24) * d].view(b, h, n + 24, d)[:, :, 8 : 8 + n]
+
+
+def _every_other_row(x, b, h, n, d):
+    return x[: b * h * 2 * n * d].view(b, h, 2 * n, d)[:, :, ::2]
+
+
+def _tokens_first(x, b, h, n, d):
+    return x[: b * h * n * d].view(n, b, h, d).permute(1, 2, 0, 3)
+
+
+def _columns_first(x, b, h, n, d):
+    """Columns are not contiguous: copied."""
+    return x[: b * h * n * d].view(b, h, d, n).transpose(2, 3)
+
+
+def _heads_first(x, b, h, n, d):
+    return x[: b * h * n * d].view(h, b, n, d).transpose(0, 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+@pytest.mark.parametrize("d", [64, 96, 192, 50])
+@pytest.mark.parametrize("layouts", [(_tokens_first, _kv_expanded, _kv_expanded, _heads_first),
+                                     (_heads_first, _cache_slice, _tokens_first, _every_other_row),
+                                     (_every_other_row, _batch_expanded, _columns_first, _batch_expanded),
+                                     (_columns_first, _tokens_first, _cache_slice, _kv_expanded)],
+                         ids=lambda f: "-".join(x.__name__[1:] for x in f))
+def test_strides_differ_from_tensor_to_tensor(fa, layouts, d, dtype):
+    """q, k, v and the output's gradient each in a layout of its own (expanded over heads or batches, slices of a
+    longer buffer, token or head first, columns not contiguous): the bits of contiguous copies, and gradients of
+    expanded tensors that add up."""
+    b, h, n = 2, 3, 200
+    gen = torch.Generator().manual_seed(12)
+    views = [f(torch.randn(b * h * 2 * n * d, generator=gen).to(dtype).cuda(), b, h, n, d) for f in layouts]
+    assert all(t.shape == (b, h, n, d) for t in views)
+    copies = [t.contiguous() for t in views]
+    results = []
+    for q, k, v, d_o in (views, copies):
+        leaves = [t.detach().requires_grad_(True) for t in (q, k, v)]
+        out = fa.flash_attention_v2(*leaves)
+        results.append([out, *torch.autograd.grad(out, leaves, d_o)])
+        with torch.no_grad():
+            results[-1].append(fa.flash_attention_v2(*leaves))
+    for got, want in zip(*results):
+        assert got.shape == want.shape and torch.equal(got, want)
+    # Through the expansion itself: the gradient of the one stored row is the sum over what shares it.
+    if layouts[1] is _kv_expanded:
+        base = views[1][:, :1].detach().clone().requires_grad_(True)
+        q, _, v, d_o = views
+        out = fa.flash_attention_v2(q, base.expand(b, h, n, d), v)
+        (got,) = torch.autograd.grad(out, base, d_o)
+        want = results[1][2].sum(1, keepdim=True)
+        assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("rows_apart", [(1 << 24) - 8, 1 << 24])
+def test_rows_far_apart(fa, rows_apart):
+    """Row strides at the limit of what the LDS-direct kernels index inside a tile (2^24 elements) and beyond it, where
+    the view is copied."""
+    n, d = 70, 64
+    buffer = torch.empty((n - 1) * rows_apart + 3 * d, dtype=torch.bfloat16, device="cuda")
+    views = [buffer[i * d :].as_strided((1, 1, n, d), (d, d, rows_apart, 1)) for i in range(3)]
+    gen = torch.Generator(device="cuda").manual_seed(13)
+    for t in views:
+        t.copy_(torch.randn(t.shape, generator=gen, device="cuda"))
+    d_o = torch.randn(1, 1, n, d, generator=gen, device="cuda").bfloat16()
+    results = []
+    for q, k, v in (views, [t.contiguous() for t in views]):
+        leaves = [t.detach().requires_grad_(True) for t in (q, k, v)]
+        out = fa.flash_attention_v2(*leaves)
+        results.append([out, *torch.autograd.grad(out, leaves, d_o)])
+    for got, want in zip(*results):
+        assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
 def test_strided_views_made_in_inference_mode(fa, dtype):
     """k and v as transposed views of tensors made under torch.inference_mode, which autograd cannot save, beside
