@@ -21,7 +21,7 @@ void launch_generic(int dp, const FwdParams &p, dim3 grid, dim3 block, hipStream
 // of the chain's start value are more than the 256-column kernel has left.  The 192- and 256-column
 // kernels live in a translation unit of their own (fa2_fwd_launch_wide.hip): compiled beside the
 // narrower instantiations the 256-column kernel, which uses all 512 registers, came out with 40-60
-// spilled registers and reloads inside its tile loop; alone it spills two, outside the loop.
+// spilled registers and reloads inside its tile loop; alone and in its padded form only it spills none.
 template <typename T, bool PAD, bool PRE, int KG>
 void launch_direct(int dp, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
   switch (dp) {

@@ -257,7 +257,9 @@ size_t fa2_bwd_workspace_bytes(int batch, int nheads, int seqlen_q, int seqlen_k
  * order and writes it once.  There are no atomics, so results are bit-identical from run to run in
  * both modes (the reference's sequence-parallel mode, _triton_kernels_v2.py:336-339, allows
  * run-to-run differences but does not require them); fa2_bwd_workspace_bytes is 0 and `workspace`
- * may be NULL.
+ * may be NULL.  The order of the sums is that of the kernel forms that run, which depend on the
+ * whole call's sizes (fa2_launch_info_get): a head computed in calls of different batch * nheads may
+ * differ by the rounding of fp32 sums taken in another order, as the forward's may.
  * The reference's sequence-parallel formulation itself - one kernel per key tile that also adds its
  * dQ contributions into an fp32 accumulator with global atomics (_triton_kernels_v2.py:336-339,
  * 466-494), then dq = accumulator (flash_attention_2.py:277) - is the set of table rows with

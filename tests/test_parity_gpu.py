@@ -79,7 +79,7 @@ SMALL_CASES = [
     (1, 2, 333, 200, 192, torch.float16, 1.0),
     (2, 2, 300, 300, 256, torch.bfloat16, 1.0),
     (1, 1, 130, 130, 250, torch.float16, 1.0),    # above 128 and not a multiple of 8
-    # several tiles at head dims above 128 (LDS-direct forward with rows of 256 in LDS, generic backward)
+    # several tiles at head dims above 128 (LDS-direct kernels with rows of 256 in LDS, the paired dK/dV kernel)
     (1, 2, 450, 200, 256, torch.bfloat16, 1.0),
     (1, 2, 200, 450, 192, torch.float16, 1.0),
     (2, 1, 333, 333, 200, torch.bfloat16, 1.0),   # padded into the row of 256
