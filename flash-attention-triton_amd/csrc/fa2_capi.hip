@@ -72,12 +72,19 @@ const fa2_config_info kTable[] = {
 };
 constexpr int kTableRows = sizeof(kTable) / sizeof(kTable[0]);
 
-// Heads dispatched together by the forward and dQ kernels: the table's group size, evened out over
-// the heads there are (fa2::equal_head_groups).
-int head_group(int cfg, int64_t heads) { return fa2::equal_head_groups(kTable[cfg].head_group, heads); }
-
-// Size of a grid that fits the chip at once (0 otherwise), for kernels that share a CU `wg_per_cu` times.
-int resident_grid(int64_t nwg, int wg_per_cu) { return nwg <= (int64_t)fa2::kCUs * wg_per_cu ? (int)nwg : 0; }
+// Order of a grid of `nwg` workgroups that share a CU `wg_per_cu` times: the heads dispatched together (`group`, unless the
+// balanced walk needs others) and, where the grid fits the chip at once and may be balanced over the CUs, its size.
+template <typename Params>
+void plan_order(Params &p, int cfg, int64_t nwg, int wg_per_cu, int group) {
+  p.head_group = group;
+  p.resident_grid = nwg <= (int64_t)fa2::kCUs * wg_per_cu ? (int)nwg : 0;
+  if (p.resident_grid <= fa2::kCUs) return;  // not resident, or one round: nothing to balance
+  const fa2::ResidentWalk walk = fa2::resident_walk(kTable[cfg].head_group, (int64_t)p.batch * p.nheads);
+  if (walk.balanced)
+    p.head_group = walk.head_group;
+  else
+    p.resident_grid = 0;
+}
 
 // The row FA2_CONFIG_AUTO stands for: the first plain row wide enough for the head dimension.
 int pick_config(int headdim) {
@@ -161,34 +168,32 @@ bool good_scale(float s) { return s > 0.f && std::isfinite(s); }
 int64_t plan_fwd(int cfg, fa2::FwdParams &p) {
   const int64_t bh = (int64_t)p.batch * p.nheads;
   const int block_q = kFwdBlockQ / fa2::fwd_key_groups(kTable[cfg].headdim_padded, p);
-  p.head_group = head_group(cfg, bh);
   p.n_qtiles = (p.seqlen_q + block_q - 1) / block_q;
   const int64_t nwg = p.n_qtiles * bh;
-  p.resident_grid = resident_grid(nwg, kTable[cfg].fwd_wg_per_cu);
+  // The table's group size, evened out over the heads there are.
+  plan_order(p, cfg, nwg, kTable[cfg].fwd_wg_per_cu, fa2::equal_head_groups(kTable[cfg].head_group, bh));
   return nwg;
 }
 
 // The same for the two kernels of a backward.
 int64_t plan_dkdv(int cfg, fa2::BwdParams &p) {
   const int dp = kTable[cfg].headdim_padded;
-  // The dK/dV kernel keeps the table's group size at every head count: with one or two workgroups
-  // per CU its drain is short either way, and measured at 96 heads the single group is 1-2 % slower.
-  p.head_group = kTable[cfg].head_group;
   const int block_kv = kTable[cfg].dq_atomic ? kDkvBlockKV : fa2::dkdv_block_kv(dp, p);
   p.n_tiles = (p.seqlen_k + block_kv - 1) / block_kv;
-  const int64_t nwg = p.n_tiles * ((int64_t)p.batch * p.nheads);
+  const int64_t bh = (int64_t)p.batch * p.nheads, nwg = p.n_tiles * bh;
   const bool pair = block_kv == fa2::kDkvPairBlockKV;
-  p.resident_grid = resident_grid(nwg, pair ? fa2::dkdv_pair_wg_per_cu(dp) : kTable[cfg].dkdv_wg_per_cu);
+  // The dK/dV kernel keeps the table's group size where the grid does not fit the chip: with one or two
+  // workgroups per CU its drain is short either way, and measured at 96 heads the single group is 1-2 % slower.
+  plan_order(p, cfg, nwg, pair ? fa2::dkdv_pair_wg_per_cu(dp) : kTable[cfg].dkdv_wg_per_cu, kTable[cfg].head_group);
   return nwg;
 }
 
 int64_t plan_dq(int cfg, fa2::BwdParams &p) {
   const int64_t bh = (int64_t)p.batch * p.nheads;
   const int block_q = kDqBlockQ / fa2::dq_key_groups(kTable[cfg].headdim_padded, p);
-  p.head_group = head_group(cfg, bh);
   p.n_tiles = (p.seqlen_q + block_q - 1) / block_q;
   const int64_t nwg = p.n_tiles * bh;
-  p.resident_grid = resident_grid(nwg, kTable[cfg].dq_wg_per_cu);
+  plan_order(p, cfg, nwg, kTable[cfg].dq_wg_per_cu, fa2::equal_head_groups(kTable[cfg].head_group, bh));
   return nwg;
 }
 

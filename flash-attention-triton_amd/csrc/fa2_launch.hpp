@@ -106,6 +106,23 @@ inline int equal_head_groups(int group, int64_t heads) {
   const int64_t per_group = (heads + n_groups - 1) / n_groups;
   return (int)((per_group + 7) / 8 * 8);
 }
+// Whether the balanced walk (balanced_index) may reorder a grid that fits the chip at once, and in which head groups;
+// `group` is the table's.  The walk pairs rounds of the grid as if the whole of it were ordered heaviest tile first.  Over
+// several head groups it is not, and heavy tiles came to lie beside heavy ones.  Sharing in L2 does not need the groups
+// there, since all tiles run at once, so all heads form one.  Time in the groups over that in one, bf16, forward / dQ:
+//   walked      1.27 (232 x 384, 32 columns), 1.17 / 1.08 (184 x 256, 64 columns), 1.08 / 1.01 (64 x 512, 128 columns)
+//   in order    1.16 / 1.11 (136 x 700, 32 columns), 1.04 / 1.04 (184 x 512, 64 columns), 1.16 / 1.05 (64 x 512)
+// One group of heads that are no multiple of 8 spreads a head's tiles over the XCDs.  Up to twice the table's group
+// that still pays on the whole (dK/dV, walked in the groups over one group: 1.0-1.13 on 34 to 123 heads, but 0.91 at
+// 59 x 384 and 0.89 at 55 x 512, 128 columns).  Beyond, it is 0.9 to 1.3 with no rule to it, and walking over the groups
+// 0.91 to 1.09 of going in order: these grids run in their groups, in order.
+struct ResidentWalk {
+  bool balanced;
+  int head_group;
+};
+inline ResidentWalk resident_walk(int group, int64_t heads) {
+  return {heads % 8 == 0 || heads < 2 * group, (int)((heads + 7) / 8 * 8)};
+}
 
 // bf16 != 0 selects the bf16 kernels, otherwise fp16.
 // folded: the LDS-direct forward takes its exponents straight from the score MFMAs (Q fragments

@@ -111,7 +111,7 @@ typedef enum fa2_form {
 /*
  * What a call launches.  A table row leaves some of it open: the rules in csrc/fa2_launch.hpp choose by
  * grid, length and alignment, and this record says what they chose.  `resident` is 1 where all workgroups
- * fit the chip at once (their order is then balanced over the CUs).
+ * fit the chip at once and their order is balanced over the CUs.
  */
 typedef struct fa2_launch_part {
   int form;         /* fa2_form */

@@ -116,6 +116,31 @@ int check_balanced_index() {
   return bad;
 }
 
+// Grids that are reordered by balanced_index are ordered heaviest tile first as a whole, and a head stays on its XCD where
+// the heads divide by 8.
+int check_resident_walk() {
+  int bad = 0, walked = 0;
+  for (int group : {32, 64})
+    for (int heads = 1; heads <= 4 * fa2::kCUs; heads++)
+      for (int tiles = 1; tiles * heads <= 4 * fa2::kCUs; tiles++) {
+        const fa2::ResidentWalk walk = fa2::resident_walk(group, heads);
+        if (!walk.balanced) {
+          bad += heads % 8 == 0 || heads < 2 * group;
+          continue;
+        }
+        walked++;
+        int last = 0;
+        for (int i = 0; i < tiles * heads; i++) {
+          int bh, rank;
+          fa2::map_workgroup(i, heads, tiles, walk.head_group, bh, rank);
+          bad += rank < last || bh < 0 || bh >= heads || rank >= tiles || (heads % 8 == 0 && bh % 8 != i % 8);
+          last = rank;
+        }
+      }
+  printf("resident walk, %d grids: %s\n", walked, bad ? "FAILED" : "ok");
+  return bad;
+}
+
 // The paired dK/dV kernel has twice the workgroups of the others: it is not picked where only they make a grid
 // that can be launched.
 int check_launchable_grids() {
@@ -142,6 +167,7 @@ int check_launchable_grids() {
 int main() {
   int bad = check_mapping();
   bad += check_balanced_index();
+  bad += check_resident_walk();
   bad += check_launchable_grids();
   bad += check<32>();
   bad += check<64>();

@@ -32,5 +32,7 @@ def test_loader_slots_match_fragment_reads_and_reads_are_conflict_free(tmp_path)
     assert len(mapping) == 1 and mapping[0].endswith("ok"), run.stdout
     balanced = [l for l in run.stdout.splitlines() if l.startswith("balanced index")]
     assert len(balanced) == 1 and balanced[0].endswith("ok"), run.stdout
+    walk = [l for l in run.stdout.splitlines() if l.startswith("resident walk")]
+    assert len(walk) == 1 and walk[0].endswith("ok"), run.stdout
     grids = [l for l in run.stdout.splitlines() if l.startswith("launchable grids")]
     assert len(grids) == 1 and grids[0].endswith("ok"), run.stdout
