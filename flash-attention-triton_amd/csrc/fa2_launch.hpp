@@ -5,6 +5,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <climits>
+
 #include "fa2_params.hpp"
 
 namespace fa2 {
@@ -25,39 +27,56 @@ inline bool direct_headdim_wide(int dp, int headdim) {
 // waves share 32 of them, one taking the even and the other the odd 32-key blocks; they merge their results
 // through LDS at the end.  Every wave's chain of blocks is half as long and the grid has twice the
 // workgroups, but every K and V tile is loaded for half the rows and every block ends at a barrier.  So two
-// groups win while the grid leaves CUs idle.  Time of one group over two, bf16, (batch, head) pairs x
-// tokens, forward / dQ, by workgroups of 128 rows:
-//   to 128      1.06-1.2 / 1.03-1.15 (128, 256 tokens), 1.3-1.7 / 1.25-1.65 beyond, any head dimension
-//   to 256      128 columns 1.14 / 1.04 (64 x 512), 1.30 / 1.24 (8 x 4096); 64 columns 1.23 / 1.09, 1.46 / 1.35;
-//               but 0.96 / 0.84 (200 x 128, 128 columns).  192 and 256 columns (one workgroup per CU either
-//               way): 1.09 / 1.04 (32 x 1024), 0.95 / 0.91 (64 x 512)
-//   to 384      64 columns 1.17 / 1.09 (96 x 512); 96 columns 1.10 / 1.08 (24 x 2048); 128 columns
-//               1.11 / 1.04 (12 x 4096), 1.07 / 0.94 (24 x 2048)
-//   to 512      32 columns 1.11 / 1.06 (64 x 1024), 1.23 / 1.10 (16 x 4096); 64 columns 1.07 / 1.01 (16 x 4096),
-//               0.94 / 0.86 (64 x 1024); 128 columns 0.98 / 0.94 (16 x 4096)
+// groups win while the grid leaves CUs idle.  Heads that do not divide by 8 have their tiles spread over the XCDs, so
+// that the same K and V tiles are fetched into several L2s: with odd numbers of heads the doubled loads cost more.
+// Time of one group over two, bf16, (batch, head) pairs x tokens, forward / dQ, by workgroups of 128 rows:
+//   to 128      0.94-1.00 / 0.80-1.00 (64 tokens: half the workgroups would have no rows); from 65 tokens on
+//               1.04-1.2 / 0.99-1.2 (but dQ at 256 columns 0.95 at 65, 1.10 at 100), 1.3-1.7 / 1.25-1.65 beyond
+//   to 256      32 columns 1.20 / 1.12 (128 x 256); 64 columns 1.15 / 1.00 (128 x 256), 1.13 / 0.94 (77 x 333);
+//               96 columns 1.11 / 1.06 (128 x 256), 1.09 / 0.99 (59 x 333), 0.94 / 1.02 (77 x 384), 1.08 / 1.15 (58 x 512);
+//               128 columns 1.06 / 0.98 (128 x 256), 0.96 / 0.92 (116 x 256), 1.16 / 1.00 (72 x 384), 0.92 / 0.97
+//               (59 x 384), 0.96 / 0.98 (39 x 512), 0.92 / 1.01 (51 x 512), 0.91 (47 x 640), 1.05 / 1.07 (29 x 1024);
+//               192 and 256 columns (one workgroup per CU either way) 1.02 / 1.02 and 1.08 / 0.99 (32 x 1024),
+//               0.94 / 0.97 and 0.94 / 0.88 (29 x 1024), 1.18 / 1.21 and 1.25 / 1.14 (14 x 2048)
+//   to 384      32 columns 1.11 / 1.10 (from 512 tokens); 64 columns 1.09 / 1.01 (96 x 512), 0.92 / 0.97 (75 x 512),
+//               1.07 / 1.05 (43 x 1024); 96 columns 1.10 / 1.06 (24 x 2048), 0.96 / 1.00 at 1024 tokens;
+//               128 columns 1.14 / 1.04 (12 x 4096), 1.08 / 0.94 (24 x 2048)
+//   to 512      32 columns 1.08 / 1.03 (from 1024 tokens); 64 columns 1.04 / 1.01 (16 x 4096), 0.98 / 0.95 (2048 tokens);
+//               128 columns 0.98 / 0.94 (16 x 4096)
 //   beyond      0.75-0.98
-inline int key_groups(int dp, int64_t heads, int seqlen_q) {
+inline int key_groups(int dp, int64_t heads, int seqlen_q, bool dq) {
   const int64_t wgs = heads * ((seqlen_q + kFwdBlockQ - 1) / kFwdBlockQ);
-  static_assert(kFwdBlockQ == kDqBlockQ, "one rule for both kernels");
-  const bool two = wgs <= kCUs / 2       ? true
-                   : wgs <= kCUs         ? seqlen_q >= (dp > 128 ? 1024 : 256)
-                   : wgs <= 3 * kCUs / 2 ? dp <= 128 && seqlen_q >= (dp == 128 ? 4096 : dp == 96 ? 2048 : 512)
-                   : wgs <= 2 * kCUs     ? dp <= 64 && seqlen_q >= (dp == 64 ? 4096 : 1024)
-                                         : false;
-  return two ? 2 : 1;
+  static_assert(kFwdBlockQ == kDqBlockQ, "the same grid for both kernels");
+  const bool odd = heads % 2 != 0;
+  int from = INT_MAX;  // query rows from which two groups win
+  if (wgs <= kCUs / 2) {
+    from = dq && dp == 256 ? 97 : 65;
+  } else if (wgs <= kCUs) {
+    if (dp > 128)
+      from = odd && wgs > kCUs * 3 / 4 ? 2048 : 1024;
+    else if (dp == 128)
+      from = (odd && wgs > kCUs * 9 / 16) || (heads % 8 != 0 && wgs > kCUs * 13 / 16) ? 1024 : dq ? 384 : 256;
+    else
+      from = odd && ((dp == 96 && (dq || wgs > kCUs * 3 / 4)) || (dp == 64 && dq)) ? 512 : 256;
+  } else if (wgs <= 3 * kCUs / 2 && dp <= 128) {
+    from = dp == 128 ? 4096 : dp == 96 ? 2048 : dp == 64 && odd ? 1024 : 512;
+  } else if (wgs <= 2 * kCUs && dp <= 64) {
+    from = dp == 64 ? 4096 : 1024;
+  }
+  return seqlen_q >= from ? 2 : 1;
 }
 inline bool fwd_direct_ok(int dp, const FwdParams &p) {
   return p.vec && direct_headdim_wide(dp, p.headdim) && direct_stride_ok(p.q) && direct_stride_ok(p.k) &&
          direct_stride_ok(p.v);
 }
 inline int fwd_key_groups(int dp, const FwdParams &p) {
-  return fwd_direct_ok(dp, p) ? key_groups(dp, (int64_t)p.batch * p.nheads, p.seqlen_q) : 1;
+  return fwd_direct_ok(dp, p) ? key_groups(dp, (int64_t)p.batch * p.nheads, p.seqlen_q, false) : 1;
 }
 inline bool dq_direct_ok(int dp, const BwdParams &p) {
   return p.vec && direct_headdim_wide(dp, p.headdim) && direct_stride_ok(p.k) && direct_stride_ok(p.v);
 }
 inline int dq_key_groups(int dp, const BwdParams &p) {
-  return dq_direct_ok(dp, p) ? key_groups(dp, (int64_t)p.batch * p.nheads, p.seqlen_q) : 1;
+  return dq_direct_ok(dp, p) ? key_groups(dp, (int64_t)p.batch * p.nheads, p.seqlen_q, true) : 1;
 }
 inline bool dkdv_direct_ok(int dp, const BwdParams &p) {
   return p.vec && direct_headdim(dp, p.headdim) && dp != 96 && direct_stride_ok(p.q) && direct_stride_ok(p.d_o) &&

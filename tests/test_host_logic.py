@@ -415,6 +415,20 @@ def test_launch_info_says_what_a_call_launches(capi, workloads):
         capi.launch_info(1, 1, 1, 1, 64, 99)
 
 
+@pytest.mark.parametrize("heads,n,d,fwd,dq", [
+    (60, 64, 128, 1, 1), (60, 65, 128, 2, 2), (8, 65, 256, 2, 1), (8, 97, 256, 2, 2),  # at most 128 workgroups of 128 rows
+    (128, 256, 32, 2, 2), (77, 333, 64, 2, 1), (128, 256, 64, 2, 2), (59, 333, 96, 2, 1), (77, 384, 96, 1, 1), (58, 512, 96, 2, 2),  # 256
+    (72, 256, 128, 2, 1), (116, 256, 128, 1, 1), (59, 384, 128, 1, 1), (51, 512, 128, 1, 1), (64, 512, 128, 2, 2),
+    (33, 500, 128, 2, 2), (47, 640, 128, 1, 1), (29, 1024, 128, 2, 2), (29, 1024, 256, 1, 1), (32, 1024, 256, 2, 2), (17, 1024, 192, 2, 2), (15, 2048, 192, 2, 2),
+    (75, 512, 32, 2, 2), (75, 512, 64, 1, 1), (96, 512, 64, 2, 2), (43, 1024, 64, 2, 2), (24, 2048, 96, 2, 2),  # 384
+    (24, 2048, 128, 1, 1), (12, 4096, 128, 2, 2), (10, 4096, 256, 1, 1),
+    (64, 1024, 32, 2, 2), (16, 4096, 64, 2, 2), (64, 1024, 64, 1, 1), (16, 4096, 128, 1, 1), (17, 4096, 32, 1, 1)])  # 512
+def test_two_key_groups_only_where_they_measured_faster(capi, heads, n, d, fwd, dq):
+    """The forward's and dQ's key groups on both sides of every line of the rule."""
+    info = capi.launch_info(1, heads, n, n, d)
+    assert (info["fwd"]["key_groups"], info["dq"]["key_groups"]) == (fwd, dq)
+
+
 def test_traffic_stamp_ignores_comments_and_follows_code(tmp_path, monkeypatch):
     """bench.py drops the measured HBM traffic when the kernel sources have changed since the
     counter run.  The stamp it compares must not move when comments or layout change (nobody should
