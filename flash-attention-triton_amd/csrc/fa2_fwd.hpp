@@ -477,9 +477,10 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
       // The second key group's first block is block 1, which may hold nothing but keys above the diagonal or
       // keys that a bias hides (-inf, or the type's lowest value).  Its rows start from block 0's maximum, as
       // the first group's and those of a launch with one group do: the same probabilities, rounded to half
-      // precision at the same scale, whatever the grid.  One score chain more in this prologue costs less
-      // than the timing's noise (B=1 H=16 N=333 D=128, bf16: 9.20 us with the group's own maximum, 9.17 us so;
-      // B=1 H=8 N=4096 D=128, forward and backward: 186.1 and 186.2 us).
+      // precision at the same scale, whatever the grid.  The score chain more is 0.2 to 0.5 us per launch, which
+      // short forwards show (bf16, D=128, with the group's own maximum and so: B=1 H=72 N=256 8.1 and 8.6 us,
+      // H=48 N=640 12.4 and 12.8, H=16 N=333 9.0 and 9.2) and long ones do not (B=1 H=8 N=4096, forward and
+      // backward: 186.3 and 186.0 us).
       f32x16 s0 = zero;
 #pragma unroll
       for (int ks = 0; ks < KS; ks++) s0 = Elem<T>::mfma(lds_read_128(kcur[ks] - BLK * LP), qf[ks], s0);

@@ -93,7 +93,8 @@ inline bool dkdv_direct_ok(int dp, const BwdParams &p) {
 //   64 columns        1.56 (4 x 4096), 1.31 (64 x 512), 1.13 (4 x 16384) while the other kernel's workgroups
 //                     are all resident (512); 1.16 (256 x 512), 1.09 (256 x 1024), 1.06 (64 x 2048) while
 //                     they are short or few; 0.97 (256 x 2048), 0.93 (64 x 4096) beyond
-//   32 columns        1.72 (4 x 4096), 1.28 (16 x 4096), 1.03 (1024 x 512); 0.96 (256 x 1024), 0.92 beyond
+//   32 columns        1.72 (4 x 4096), 1.28 (16 x 4096), 1.03 (1024 x 512); 0.96 (256 x 1024), 0.92 beyond;
+//                     of 128 tokens and fewer 1.05 to 1.3, but 0.92-1.0 at 640 to 768 workgroups (8 us kernels)
 inline bool dkdv_pair_ok(int dp, const BwdParams &p) {
   if (!(p.vec && direct_headdim_wide(dp, p.headdim) && direct_stride_ok(p.q) && direct_stride_ok(p.d_o) &&
         direct_stride_ok(p.k) && direct_stride_ok(p.v)))
