@@ -28,15 +28,27 @@ void launch_atomic(int dp, const BwdParams &p, dim3 grid, dim3 block, hipStream_
   }
 }
 
-template <typename T, bool PAD>
+template <typename T, int DP, int COLS>
+void launch_pair_cols(const BwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
+  if (p.headdim == COLS)
+    hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, DP, false, COLS>), grid, block, 0, s, p);
+  else
+    hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, DP, true, COLS>), grid, block, 0, s, p);
+}
+
+template <typename T>
 void launch_pair(int dp, const BwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
-  switch (dp) {
-    case 32: hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 32, PAD>), grid, block, 0, s, p); break;
-    case 64: hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 64, PAD>), grid, block, 0, s, p); break;
-    case 96: hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 96, PAD>), grid, block, 0, s, p); break;
-    case 128: hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 128, PAD>), grid, block, 0, s, p); break;
-    case 192: hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 192, PAD>), grid, block, 0, s, p); break;
-    default: hipLaunchKernelGGL((bwd_dkdv_pair_kernel<T, 256, PAD>), grid, block, 0, s, p); break;
+  switch (direct_columns(dp, p.headdim)) {
+    case 32: launch_pair_cols<T, 32, 32>(p, grid, block, s); break;
+    case 48: launch_pair_cols<T, 64, 48>(p, grid, block, s); break;
+    case 64: launch_pair_cols<T, 64, 64>(p, grid, block, s); break;
+    case 80: launch_pair_cols<T, 96, 80>(p, grid, block, s); break;
+    case 96: launch_pair_cols<T, 96, 96>(p, grid, block, s); break;
+    case 128: launch_pair_cols<T, 128, 128>(p, grid, block, s); break;
+    case 160: launch_pair_cols<T, 192, 160>(p, grid, block, s); break;
+    case 192: launch_pair_cols<T, 192, 192>(p, grid, block, s); break;
+    case 224: launch_pair_cols<T, 256, 224>(p, grid, block, s); break;
+    default: launch_pair_cols<T, 256, 256>(p, grid, block, s); break;
   }
 }
 
@@ -48,10 +60,7 @@ void launch(int dp, const BwdParams &p, dim3 grid, hipStream_t s) {
     return;
   }
   if (dkdv_pair_ok(dp, p)) {  // always at 96 columns and above 128
-    if (p.headdim == dp)
-      launch_pair<T, false>(dp, p, grid, block, s);
-    else
-      launch_pair<T, true>(dp, p, grid, block, s);
+    launch_pair<T>(dp, p, grid, block, s);
     return;
   }
   if (dkdv_direct_ok(dp, p)) {

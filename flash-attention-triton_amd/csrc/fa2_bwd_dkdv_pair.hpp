@@ -26,6 +26,8 @@
 // long sequences the board's power limit takes the clock down by what the cycles gained (1.69 GHz against
 // 1.93).
 //
+// COLS (below): columns multiplied, as in the forward (fa2_fwd.hpp).
+//
 // The two roles are two instantiations of the loop selected once per wave.  With one loop and selects (or
 // branches) on the role inside it the kernel was 2 to 5 % slower (or spilled).  The barriers of the two
 // instantiations match one to one.
@@ -57,12 +59,12 @@ struct DkvPairLayout {
   static_assert(STAT_BASE >= PATCH_ELEMS, "the output patch overlays the stages");
 };
 
-template <typename T, int DP, bool PAD, int role>
+template <typename T, int DP, bool PAD, int role, int COLS>
 __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem) {
   using L = DkvPairLayout<DP>;
-  constexpr int BQ = L::BQ, KS = DP / 16, DB = DP / 32, LP = L::LP;
+  constexpr int BQ = L::BQ, KS = COLS / 16, DB = (COLS + 31) / 32, R = 2 * DB, LP = L::LP;
   constexpr int NTHREADS = 64 * kDkvWaves;
-  using Loader = TileLoader<DP, BQ, kDkvWaves, PAD>;
+  using Loader = TileLoader<DP, BQ, kDkvWaves, PAD || COLS != DP>;
   constexpr int LOADS = Loader::LOADS;
 
   const int tid = threadIdx.x;
@@ -85,7 +87,7 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem) {
   const float *LSE = p.lse + (int64_t)bh * p.seqlen_q_rounded;
   const float *DELTA = p.delta + (int64_t)bh * p.seqlen_q_rounded;
 
-  const int hdim = PAD ? p.headdim : DP;
+  const int hdim = PAD ? p.headdim : COLS;
   const Loader qload(uniform_ptr(Q), (int64_t)uniform64((uint64_t)p.q.stride_seq), hdim / 8),
       gload(uniform_ptr(DO), (int64_t)uniform64((uint64_t)p.d_o.stride_seq), hdim / 8);
   const int seqlen_q = p.seqlen_q;
@@ -205,7 +207,7 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem) {
       vf[ks] = lds_read_128(lds0 + (int)(V_AT / 2) + swz_off<LP>(r, 2 * ks + h));
     }
   }
-  s16x8 ring[KS];
+  s16x8 ring[R];
 #pragma unroll
   for (int ks = 0; ks < KS; ks++) ring[ks] = lds_read_128(qrow[ks]);
   // Every wave has its K and V fragments: stage 1 is free for its tile.
@@ -255,6 +257,7 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem) {
     for (int ks = 0; ks < KS; ks++) {
       dp = Elem<T>::mfma(ring[ks], vf[ks], dp);
       ring[ks] = t_frag(ks, 0);
+      if (KS < R && ks == 0) ring[R - 1] = t_frag(R - 1, 0);  // the slot no dO row was in
 #pragma unroll
       for (int i = part(16, KS, ks); i < part(16, KS, ks + 1); i++) {
         float x = fast_exp2(s[i] * scale_log2 - l4[i >> 2][i & 3]);
@@ -289,12 +292,12 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem) {
       pack_ds();
     }
 #pragma unroll
-    for (int f = 0; f < KS; f++) {
+    for (int f = 0; f < R; f++) {
       acc[f % DB] = Elem<T>::mfma(ring[f], role ? df[f / DB] : pf[f / DB], acc[f % DB]);
       ring[f] = t_frag(f, other_block);
       if (role == 0) {
 #pragma unroll
-        for (int i = part(16, KS, f); i < part(16, KS, f + 1); i++) dp[i] = s[i] * dp[i];
+        for (int i = part(16, R, f); i < part(16, R, f + 1); i++) dp[i] = s[i] * dp[i];
         asm volatile("" : "+v"(dp));
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -315,12 +318,12 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem) {
     const unsigned ldst = lds_base + 2u * (unsigned)((t & 1) * L::STAGE_ELEMS);
     const int lrow0 = q_top - (t + 2) * BQ;
 #pragma unroll
-    for (int f = 0; f < KS; f++) {
+    for (int f = 0; f < R; f++) {
       acc[f % DB] = Elem<T>::mfma(ring[f], got[f / DB], acc[f % DB]);
-      ring[f] = lds_read_128(qrow[f]);
+      if (f < KS) ring[f] = lds_read_128(qrow[f]);
       if (SPREAD) {
 #pragma unroll
-        for (int i = part(2 * LOADS, KS, f); i < part(2 * LOADS, KS, f + 1); i++) {
+        for (int i = part(2 * LOADS, R, f); i < part(2 * LOADS, R, f + 1); i++) {
           if (i < LOADS) qload.issue_one(lrow0, ldst, i);
           else gload.issue_one(lrow0, ldst + 2u * L::TILE_ELEMS, i - LOADS);
         }
@@ -346,17 +349,17 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem) {
   const Tensor4 &out = role ? p.dk : p.dv;
   __syncthreads();
   short *patch = smem + wave * 32 * (DP + 8);
-  store_transposed_acc<T, DP, true>(acc, role ? p.scale : 1.0f, patch, grad_rows(p, out, b, hd, kv0w), out.stride_seq,
+  store_transposed_acc<T, COLS, true>(acc, role ? p.scale : 1.0f, patch, grad_rows(p, out, b, hd, kv0w), out.stride_seq,
                               p.seqlen_k - kv0w, hdim, true, p.grads_f32);
 }
 
-template <typename T, int DP, bool PAD>
+template <typename T, int DP, bool PAD, int COLS = DP>
 __global__ __launch_bounds__(64 * kDkvWaves, (dkdv_pair_wg_per_cu(DP))) void bwd_dkdv_pair_kernel(const BwdParams p) {
   __shared__ __attribute__((aligned(1024))) short smem[DkvPairLayout<DP>::TOTAL_ELEMS];
   if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 1)
-    bwd_dkdv_pair<T, DP, PAD, 1>(p, smem);
+    bwd_dkdv_pair<T, DP, PAD, 1, COLS>(p, smem);
   else
-    bwd_dkdv_pair<T, DP, PAD, 0>(p, smem);
+    bwd_dkdv_pair<T, DP, PAD, 0, COLS>(p, smem);
 }
 
 }  // namespace fa2

@@ -268,14 +268,15 @@ struct DqDirectLayout {
 // With FUSE_DELTA the kernel also computes delta = rowsum(O * dO) for its query rows (it holds
 // the dO rows anyway), uses it and writes it out for the dK/dV kernel, which then has to be
 // launched after this one; the separate preprocess launch disappears.
-// PAD: the head dimension is a multiple of 8 below DP; the columns beyond it are zeros in LDS and in
+// COLS: columns multiplied, as in the forward (fa2_fwd.hpp).
+// PAD: the head dimension is a multiple of 8 below COLS; the columns beyond it are zeros in LDS and in
 // the register fragments, and are not stored.
 // KG: key groups, as in the forward (fa2_fwd.hpp).  With two the waves' sums over the even and the odd
 // 32-key blocks are added at the end, in that order: B=1 H=8 N=4096 D=128, bf16: 72.5 -> 58.5 us.
-template <typename T, int DP, int BKV, bool FUSE_DELTA, bool PAD, int KG = 1>
+template <typename T, int DP, int BKV, bool FUSE_DELTA, bool PAD, int KG = 1, int COLS = DP>
 __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_direct_kernel(const BwdParams p) {
   using L = DqDirectLayout<DP, BKV>;
-  constexpr int KS = DP / 16, DB = DP / 32, LP = L::LP;
+  constexpr int KS = COLS / 16, DB = (COLS + 31) / 32, R = 2 * DB, LP = L::LP;
   constexpr int BLK = 32;
   static_assert(BKV == 2 * BLK, "written for 64-row key tiles of two 32-row blocks");
 
@@ -302,8 +303,9 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
   const short *V = (const short *)p.v.ptr + b * p.v.stride_batch + hd * p.v.stride_head;
   const short *DO = (const short *)p.d_o.ptr + b * p.d_o.stride_batch + hd * p.d_o.stride_head;
 
-  const int hdim = PAD ? p.headdim : DP;
-  const TileLoader<DP, BKV, kDqWaves, PAD> kload(K, p.k.stride_seq, hdim / 8), vload(V, p.v.stride_seq, hdim / 8);
+  const int hdim = PAD ? p.headdim : COLS;
+  using Loader = TileLoader<DP, BKV, kDqWaves, PAD || COLS != DP>;
+  const Loader kload(K, p.k.stride_seq, hdim / 8), vload(V, p.v.stride_seq, hdim / 8);
   const int seqlen_k = p.seqlen_k;
   const float scale_log2 = p.scale_log2;
 
@@ -408,7 +410,7 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
   __syncthreads();
 
   // Ring of A fragments, preloaded with the K rows of block 0.
-  s16x8 ring[KS];
+  s16x8 ring[R];
 #pragma unroll
   for (int ks = 0; ks < KS; ks++) ring[ks] = lds_read_128(knext[ks]);
 
@@ -417,7 +419,7 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
   //     A: S^T = K Q^T            ring <- V rows              (loads of V tile t+1 when SPREAD)
   //     B: dP^T = V dO^T          ring <- K^T fragments       exponentials of S; loads of K tile t+2
   //     C: dQ^T += K^T dS^T       ring <- next block's K rows second half of the dS arithmetic
-  constexpr int LOADS = TileLoader<DP, BKV, kDqWaves, PAD>::LOADS;
+  constexpr int LOADS = Loader::LOADS;
   constexpr int LOAD_EVERY = KS / LOADS;
   // INNER blocks lie in tiles that end before the workgroup's first query row: they are every
   // wave's own and need no mask, so the two tests fold away.
@@ -463,6 +465,10 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
         s16x4 a1 = lds_read_tr(khi[ks % DB] + HOFF + 16 * (ks / DB) * LP);
         ring[ks] = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
       }
+      if (KS < R && ks == 0) {  // the slot no V row was in
+        s16x4 a0 = lds_read_tr(klo[DB - 1] + HOFF + 16 * LP), a1 = lds_read_tr(khi[DB - 1] + HOFF + 16 * LP);
+        ring[R - 1] = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
+      }
 #pragma unroll
       for (int i = part(16, KS, ks); i < part(16, KS, ks + 1); i++) {
         s[i] = fast_exp2(s[i] * scale_log2 - lse2);
@@ -477,11 +483,11 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
     s16x8 dsf[2];
     dsf[0] = Elem<T>::pack8(lo);
 #pragma unroll
-    for (int slot = 0; slot < KS; slot++) {
-      constexpr int HALF_SLOTS = KS / 2;
+    for (int slot = 0; slot < R; slot++) {
+      constexpr int HALF_SLOTS = R / 2;
       const int ks2 = slot / DB, db = slot % DB;
       dqacc[db] = Elem<T>::mfma(ring[slot], dsf[ks2], dqacc[db]);
-      ring[slot] = lds_read_128(knext[slot] + (HALF == 0 && KG == 1 ? BLK * LP : 0));
+      if (slot < KS) ring[slot] = lds_read_128(knext[slot] + (HALF == 0 && KG == 1 ? BLK * LP : 0));
       if (slot < HALF_SLOTS) {
 #pragma unroll
         for (int i = part(8, HALF_SLOTS, slot); i < part(8, HALF_SLOTS, slot + 1); i++)
@@ -556,7 +562,7 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
       }
   }
   short *patch = smem + KG * MERGE_FLOATS * 2 + wave * 32 * (DP + 8);
-  store_transposed_acc<T, DP>(dqacc, p.scale, patch, grad_rows(p, p.dq, b, hd, q0w),
+  store_transposed_acc<T, COLS>(dqacc, p.scale, patch, grad_rows(p, p.dq, b, hd, q0w),
                               p.dq.stride_seq, p.seqlen_q - q0w, hdim, true, p.grads_f32);
 }
 

@@ -5,24 +5,28 @@
 namespace fa2 {
 namespace {
 
-template <typename T, bool FUSE_DELTA, bool PAD, int KG>
-void launch_direct_pad(int dp, const BwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
-  switch (dp) {
-    case 32: hipLaunchKernelGGL((bwd_dq_direct_kernel<T, 32, kDqBlockKV, FUSE_DELTA, PAD, KG>), grid, block, 0, s, p); break;
-    case 64: hipLaunchKernelGGL((bwd_dq_direct_kernel<T, 64, kDqBlockKV, FUSE_DELTA, PAD, KG>), grid, block, 0, s, p); break;
-    case 96: hipLaunchKernelGGL((bwd_dq_direct_kernel<T, 96, kDqBlockKV, FUSE_DELTA, PAD, KG>), grid, block, 0, s, p); break;
-    case 128: hipLaunchKernelGGL((bwd_dq_direct_kernel<T, 128, kDqBlockKV, FUSE_DELTA, PAD, KG>), grid, block, 0, s, p); break;
-    case 192: hipLaunchKernelGGL((bwd_dq_direct_kernel<T, 192, kDqBlockKV, FUSE_DELTA, PAD, KG>), grid, block, 0, s, p); break;
-    default: hipLaunchKernelGGL((bwd_dq_direct_kernel<T, 256, kDqBlockKV, FUSE_DELTA, PAD, KG>), grid, block, 0, s, p); break;
-  }
+template <typename T, bool FUSE_DELTA, int KG, int DP, int COLS>
+void launch_cols(const BwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
+  if (p.headdim == COLS)
+    hipLaunchKernelGGL((bwd_dq_direct_kernel<T, DP, kDqBlockKV, FUSE_DELTA, false, KG, COLS>), grid, block, 0, s, p);
+  else
+    hipLaunchKernelGGL((bwd_dq_direct_kernel<T, DP, kDqBlockKV, FUSE_DELTA, true, KG, COLS>), grid, block, 0, s, p);
 }
 
 template <typename T, bool FUSE_DELTA, int KG>
 void launch_direct_groups(int dp, const BwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
-  if (p.headdim == dp)
-    launch_direct_pad<T, FUSE_DELTA, false, KG>(dp, p, grid, block, s);
-  else
-    launch_direct_pad<T, FUSE_DELTA, true, KG>(dp, p, grid, block, s);
+  switch (direct_columns(dp, p.headdim)) {
+    case 32: launch_cols<T, FUSE_DELTA, KG, 32, 32>(p, grid, block, s); break;
+    case 48: launch_cols<T, FUSE_DELTA, KG, 64, 48>(p, grid, block, s); break;
+    case 64: launch_cols<T, FUSE_DELTA, KG, 64, 64>(p, grid, block, s); break;
+    case 80: launch_cols<T, FUSE_DELTA, KG, 96, 80>(p, grid, block, s); break;
+    case 96: launch_cols<T, FUSE_DELTA, KG, 96, 96>(p, grid, block, s); break;
+    case 128: launch_cols<T, FUSE_DELTA, KG, 128, 128>(p, grid, block, s); break;
+    case 160: launch_cols<T, FUSE_DELTA, KG, 192, 160>(p, grid, block, s); break;
+    case 192: launch_cols<T, FUSE_DELTA, KG, 192, 192>(p, grid, block, s); break;
+    case 224: launch_cols<T, FUSE_DELTA, KG, 256, 224>(p, grid, block, s); break;
+    default: launch_cols<T, FUSE_DELTA, KG, 256, 256>(p, grid, block, s); break;
+  }
 }
 
 template <typename T, bool FUSE_DELTA>

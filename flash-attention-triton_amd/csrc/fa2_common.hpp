@@ -201,22 +201,24 @@ __device__ __forceinline__ void store_chunk_widened(float *row, int d0, int head
   }
 }
 
-// Write a wave's transposed accumulator (DB blocks of 32 headdim rows x 32 sequence columns,
-// lane (c, h) holding sequence position c) to a (seqlen, headdim) tensor.  The values go through
-// a wave-private LDS patch of 32 x (DP + 8) elements so that global stores are 16-byte and
+// Write a wave's transposed accumulator (blocks of 32 headdim rows x 32 sequence columns, the last one cut off
+// at COLS; lane (c, h) holding sequence position c) to a (seqlen, headdim) tensor.  The values go through
+// a wave-private LDS patch of 32 x (whole blocks + 8) elements so that global stores are 16-byte and
 // row-contiguous.  The caller guarantees the patch is not in use by anyone else.  With `f32` (uniform)
 // the rows are fp32 and receive the rounded values widened.
-template <typename T, int DP, bool UNROLL_F32 = false>
-__device__ __forceinline__ void store_transposed_acc(const f32x16 (&acc)[DP / 32], float mult,
+template <typename T, int COLS, bool UNROLL_F32 = false>
+__device__ __forceinline__ void store_transposed_acc(const f32x16 (&acc)[(COLS + 31) / 32], float mult,
                                                      short *patch, void *dst_rows,
                                                      int64_t stride_seq, int rows_valid,
                                                      int headdim, bool vec, bool f32 = false) {
-  constexpr int LD = DP + 8;
-  constexpr int CPR = DP / 8;
+  constexpr int DB = (COLS + 31) / 32;
+  constexpr int LD = 32 * DB + 8;
+  constexpr int CPR = COLS / 8;
+  static_assert(COLS % 16 == 0, "a wave stores whole chunks");
   const int lane = threadIdx.x & 63;
   const int c = lane & 31, h = lane >> 5;
 #pragma unroll
-  for (int db = 0; db < DP / 32; db++) {
+  for (int db = 0; db < DB; db++) {
 #pragma unroll
     for (int g = 0; g < 4; g++) {
       f32x4 x = {acc[db][4 * g] * mult, acc[db][4 * g + 1] * mult, acc[db][4 * g + 2] * mult,

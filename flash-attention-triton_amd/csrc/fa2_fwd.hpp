@@ -252,8 +252,8 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_kerne
 }
 
 // ------------------------------------------------------------------------------------------
-// Fast path: 16-byte aligned rows and a head dimension that is a multiple of 8; instantiated for 32,
-// 64, 96, 128, 192 and 256 columns (two workgroups or more per CU up to 128; at 192 and 256 the
+// Fast path: 16-byte aligned rows and a head dimension that is a multiple of 8; instantiated for 32, 48, 64,
+// 80, 96, 128, 160, 192, 224 and 256 columns (two workgroups or more per CU up to 128; at 192 and 256 the
 // five tile stages fill the CU's 160 KiB of LDS and the output accumulator moves into accumulation
 // registers: one workgroup per CU, one wave per SIMD).
 //
@@ -268,7 +268,7 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_kerne
 //        Y(j): O^T += V_j^T P_j^T         interleaved with   P_{j+1} = exp2(scale*S_{j+1} - m), row sums
 //    One score buffer and one probability buffer are enough: each is consumed in the phase after
 //    the one that fills it.
-//  * MFMA operand fragments travel through a ring of DP/16 register sets that is refilled as it
+//  * MFMA operand fragments travel through a ring of COLS/16 register sets (rounded up to even) that is refilled as it
 //    is consumed (K fragments of block j+2 during Y(j), V fragments of block j during X(j)), so
 //    LDS latency hides behind the MFMAs.
 // ------------------------------------------------------------------------------------------
@@ -292,7 +292,12 @@ struct HalfTag {
   static constexpr bool inner = INNER;
 };
 
-// PAD: the head dimension is a multiple of 8 below DP; the columns beyond it are zeros in LDS and in
+// COLS: columns multiplied, DP or (direct_columns in fa2_launch.hpp) a step less; DP is then the LDS tiles' alone.  With
+// an odd number of 16-column steps (48, 80) S takes one MFMA per block less than P V, whose last block is half
+// empty.  Forward and
+// backward, bf16, padded to DP before, us: 2x16x4096 D=160 1008 -> 903, 1x8x4096 D=160 314 -> 278, 2x16x4096 D=224
+// 1273 -> 1172, 8x16x2048 D=80 525 -> 500, 32x16x512 D=48 153 -> 145.
+// PAD: the head dimension is a multiple of 8 below COLS; the columns beyond it are zeros in LDS and in
 // the register fragments, and are not stored.
 // KG: key groups.  With one, a wave multiplies both 32-key blocks of every tile by its 32 query rows.  With
 // two, waves 0, 1 take the first and waves 2, 3 the second block of every tile, for the same 64 rows, and the
@@ -304,13 +309,13 @@ struct HalfTag {
 // every score chain starts from minus the maximum in use (the MFMA's C operand), so that the score
 // MFMAs deliver the base-2 exponents themselves and no multiply-add is left in front of the
 // exponentials.
-template <typename T, int DP, int BKV, bool PAD, bool PRE, int KG = 1>
+template <typename T, int DP, int BKV, bool PAD, bool PRE, int KG = 1, int COLS = DP>
 __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direct_kernel(const FwdParams p) {
   using L = FwdDirectLayout<DP, BKV>;
-  constexpr int KS = DP / 16, DB = DP / 32, LP = L::LP;
+  constexpr int KS = COLS / 16, DB = (COLS + 31) / 32, R = 2 * DB, LP = L::LP;
   constexpr int NTHREADS = 64 * kFwdWaves;
   constexpr int BLK = 32;  // keys per pipeline block
-  static_assert(BKV == 2 * BLK && KS == 2 * DB, "schedule is written for 64-row tiles of two blocks");
+  static_assert(BKV == 2 * BLK && (KS == R || KS == R - 1), "schedule is written for 64-row tiles of two blocks");
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
   __shared__ __attribute__((aligned(1024))) short smem[L::TOTAL_ELEMS];
@@ -337,8 +342,9 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
   short *O = (short *)p.o.ptr + b * p.o.stride_batch + hd * p.o.stride_head;
   float *LSE = p.lse + (int64_t)bh * p.seqlen_q_rounded;
 
-  const int hdim = PAD ? p.headdim : DP;
-  const TileLoader<DP, BKV, kFwdWaves, PAD> kload(K, p.k.stride_seq, hdim / 8), vload(V, p.v.stride_seq, hdim / 8);
+  const int hdim = PAD ? p.headdim : COLS;
+  using Loader = TileLoader<DP, BKV, kFwdWaves, PAD || COLS != DP>;
+  const Loader kload(K, p.k.stride_seq, hdim / 8), vload(V, p.v.stride_seq, hdim / 8);
   const int seqlen_k = p.seqlen_k;
   const float scale_log2 = p.scale_log2;
 
@@ -379,7 +385,7 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
   constexpr unsigned Q_HI = 2u * (unsigned)(L::V_BASE + 1 * L::TILE_ELEMS);
   constexpr unsigned Q_LO = KG == 1 ? 2u * (unsigned)(L::K_BASE + 2 * L::TILE_ELEMS) : Q_HI;
   constexpr int K_AHEAD = KG == 1 ? 2 : 3;  // tile t loads K tile t + K_AHEAD
-  const TileLoader<DP, BKV, kFwdWaves, PAD> qload(Q + (int64_t)q0 * p.q.stride_seq, p.q.stride_seq, hdim / 8);
+  const Loader qload(Q + (int64_t)q0 * p.q.stride_seq, p.q.stride_seq, hdim / 8);
   const int q_rows = p.seqlen_q - q0;  // rows of this query tile that exist (>= 1)
   issue_k(0);
   if (q_rows >= BKV) qload.issue(0, lds_base + Q_LO); else qload.issue_clamped(0, q_rows, lds_base + Q_LO);
@@ -442,7 +448,7 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
   };
   // K_0 and Q have landed once at most the loads of V_0 (and K_1) are outstanding: loads complete
   // in the order they were issued.
-  constexpr int LOADS_PER_TILE = TileLoader<DP, BKV, kFwdWaves, PAD>::LOADS;
+  constexpr int LOADS_PER_TILE = Loader::LOADS;
   static_assert(3 * LOADS_PER_TILE < 64, "vmcnt field");
   if (KG > 1 && n_tiles > 2) wait_vmem<3 * LOADS_PER_TILE>();
   else if (n_tiles > 1) wait_vmem<2 * LOADS_PER_TILE>(); else wait_vmem<LOADS_PER_TILE>();
@@ -463,7 +469,7 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
 
   // ---- prologue: S_0, its row maximum, e_0 = exp2(scale*S_0 - scale*m), ring <- K fragments of
   // block 1 ---------------------------------------------------------------------------------
-  s16x8 ring[KS];
+  s16x8 ring[R];
   f32x16 sc;  // the score block in flight (S_{j+1} during step j)
   f32x16 e;   // unnormalised probabilities of the block whose P V product comes next
   {
@@ -551,7 +557,7 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
   // time between the units of tile t's first step.  Issued back to back by all waves at once they
   // queue up in the memory pipeline, and a wave whose load cannot issue cannot issue its MFMAs
   // either.
-  constexpr int LOADS = TileLoader<DP, BKV, kFwdWaves, PAD>::LOADS;
+  constexpr int LOADS = Loader::LOADS;
   constexpr int LOAD_EVERY = KS / LOADS;
   auto step = [&](int j, auto half_tag, auto spread_tag) {
     constexpr int HALF = decltype(half_tag)::value;
@@ -577,12 +583,13 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
       sc = Elem<T>::mfma(ring[ks], qf[ks], (PRE && ks == 0) ? negm : sc);
       if (SPREAD && ks % LOAD_EVERY == 0 && ks / LOAD_EVERY < LOADS) vload.issue_one(vt * BKV, vdst, ks / LOAD_EVERY);
       ring[ks] = v_frag(HALF, ks / DB, ks % DB);
+      if (KS < R && ks == 0) ring[R - 1] = v_frag(HALF, 1, DB - 1);  // the slot no K fragment was in
 #pragma unroll
       for (int i = part(8, KS, ks); i < part(8, KS, ks + 1); i++)  // probability pair (2i, 2i+1) of the block
         w[i / 4][i % 4] = Elem<T>::pack2(e[2 * i], e[2 * i + 1]);
       // Pin the arithmetic to this unit: without a use here the optimiser sinks it next to the
       // MFMAs that consume it.
-      if (ks == KS / 2 - 1) asm volatile("" : "+v"(w[0]));
+      if (ks == (KS + 1) / 2 - 1) asm volatile("" : "+v"(w[0]));
       if (ks == KS - 1) asm volatile("" : "+v"(w[1]));
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -599,9 +606,9 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
         const int slot = ks2 * DB + db;
         oacc[db] = Elem<T>::mfma(ring[slot], pf[ks2], oacc[db]);
         if (SPREAD && slot % LOAD_EVERY == 0 && slot / LOAD_EVERY < LOADS) kload.issue_one(kt * BKV, kdst, slot / LOAD_EVERY);
-        ring[slot] = k_frag(HALF, slot);
+        if (slot < KS) ring[slot] = k_frag(HALF, slot);
 #pragma unroll
-        for (int i = part(16, KS, slot); i < part(16, KS, slot + 1); i++) {
+        for (int i = part(16, R, slot); i < part(16, R, slot + 1); i++) {
           e[i] = PRE ? fast_exp2(sc[i]) : fast_exp2(sc[i] * scale_log2 - mc);
           lsum[i & 1] += e[i];
         }
@@ -721,7 +728,7 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
   }
   // The patch overlays the stages; the loop's last barrier already ordered it after all reads.
   short *patch = smem + KG * MERGE_FLOATS * 2 + wave * 32 * (DP + 8);
-  store_transposed_acc<T, DP>(oacc, inv_l, patch, O + (int64_t)q0w * p.o.stride_seq,
+  store_transposed_acc<T, COLS>(oacc, inv_l, patch, O + (int64_t)q0w * p.o.stride_seq,
                               p.o.stride_seq, p.seqlen_q - q0w, hdim, true);
 }
 

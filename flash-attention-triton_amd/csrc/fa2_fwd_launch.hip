@@ -22,25 +22,33 @@ void launch_generic(int dp, const FwdParams &p, dim3 grid, dim3 block, hipStream
 // kernels live in a translation unit of their own (fa2_fwd_launch_wide.hip): compiled beside the
 // narrower instantiations the 256-column kernel, which uses all 512 registers, came out with 40-60
 // spilled registers and reloads inside its tile loop; alone and in its padded form only it spills none.
-template <typename T, bool PAD, bool PRE, int KG>
+template <typename T, int DP, int COLS, bool PRE, int KG>
+void launch_cols(const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
+  if (p.headdim == COLS)
+    hipLaunchKernelGGL((fwd_direct_kernel<T, DP, kFwdBlockKV, false, PRE, KG, COLS>), grid, block, 0, s, p);
+  else
+    hipLaunchKernelGGL((fwd_direct_kernel<T, DP, kFwdBlockKV, true, PRE, KG, COLS>), grid, block, 0, s, p);
+}
+
+template <typename T, bool PRE, int KG>
 void launch_direct(int dp, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
-  switch (dp) {
-    case 32: hipLaunchKernelGGL((fwd_direct_kernel<T, 32, kFwdBlockKV, PAD, PRE, KG>), grid, block, 0, s, p); break;
-    case 64: hipLaunchKernelGGL((fwd_direct_kernel<T, 64, kFwdBlockKV, PAD, PRE, KG>), grid, block, 0, s, p); break;
-    case 96: hipLaunchKernelGGL((fwd_direct_kernel<T, 96, kFwdBlockKV, PAD, PRE, KG>), grid, block, 0, s, p); break;
-    case 128: hipLaunchKernelGGL((fwd_direct_kernel<T, 128, kFwdBlockKV, PAD, PRE, KG>), grid, block, 0, s, p); break;
-    default: launch_fwd_direct_wide(std::is_same<T, __bf16>::value, dp, PAD, KG, p, grid, block, s); break;
+  switch (direct_columns(dp, p.headdim)) {
+    case 32: launch_cols<T, 32, 32, PRE, KG>(p, grid, block, s); break;
+    case 48: launch_cols<T, 64, 48, PRE, KG>(p, grid, block, s); break;
+    case 64: launch_cols<T, 64, 64, PRE, KG>(p, grid, block, s); break;
+    case 80: launch_cols<T, 96, 80, PRE, KG>(p, grid, block, s); break;
+    case 96: launch_cols<T, 96, 96, PRE, KG>(p, grid, block, s); break;
+    case 128: launch_cols<T, 128, 128, PRE, KG>(p, grid, block, s); break;
+    default: launch_fwd_direct_wide(std::is_same<T, __bf16>::value, dp, KG, p, grid, block, s); break;
   }
 }
 
 template <typename T, int KG>
 void launch_groups(int dp, bool folded, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
-  const bool pad = p.headdim != dp;
-  if (folded) {
-    if (pad) launch_direct<T, true, true, KG>(dp, p, grid, block, s); else launch_direct<T, false, true, KG>(dp, p, grid, block, s);
-  } else {
-    if (pad) launch_direct<T, true, false, KG>(dp, p, grid, block, s); else launch_direct<T, false, false, KG>(dp, p, grid, block, s);
-  }
+  if (folded)
+    launch_direct<T, true, KG>(dp, p, grid, block, s);
+  else
+    launch_direct<T, false, KG>(dp, p, grid, block, s);
 }
 
 template <typename T>

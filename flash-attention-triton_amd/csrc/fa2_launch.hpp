@@ -23,6 +23,14 @@ inline bool direct_headdim(int dp, int headdim) {
 inline bool direct_headdim_wide(int dp, int headdim) {
   return direct_headdim(dp, headdim) || (headdim % 8 == 0 && headdim <= dp && (dp == 192 || dp == 256));
 }
+// Columns the forward, dQ and paired dK/dV kernels of a row multiply: the head dimension rounded up to a step of 16
+// up to 96 columns and of 32 above (measured in fa2_fwd.hpp).  The row's own number (64, 96, 192, 256) stays the pitch of the LDS tiles.  A
+// head dimension that is such a number needs no zero-filled tiles either: what lies behind a row is multiplied into
+// accumulator rows that are not stored.
+inline int direct_columns(int dp, int headdim) {
+  const int less = dp == 64 || dp == 96 ? dp - 16 : dp > 128 ? dp - 32 : dp;
+  return headdim <= less ? less : dp;
+}
 // Key groups of the forward and dQ kernels.  With two, a workgroup owns 64 query rows instead of 128 and two
 // waves share 32 of them, one taking the even and the other the odd 32-key blocks; they merge their results
 // through LDS at the end.  Every wave's chain of blocks is half as long and the grid has twice the
@@ -149,7 +157,7 @@ inline ResidentWalk resident_walk(int group, int64_t heads) {
 // multiplied by scale * log2(e) and rounded once); the generic forward ignores it.
 void launch_fwd(bool bf16, int dp, bool folded, const FwdParams &p, dim3 grid, hipStream_t s);
 // The 192- and 256-column LDS-direct forward kernels (dp is 192 or 256), instantiated apart from the others.
-void launch_fwd_direct_wide(bool bf16, int dp, bool pad, int key_groups, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s);
+void launch_fwd_direct_wide(bool bf16, int dp, int key_groups, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s);
 void launch_preprocess(bool bf16, const PreParams &p, dim3 grid, hipStream_t s);
 // fuse_delta: the fast dQ kernel also forms delta from O and dO (dq_direct_ok must hold).
 void launch_dq(bool bf16, int dp, const BwdParams &p, dim3 grid, bool fuse_delta, hipStream_t s);
