@@ -15,7 +15,7 @@ import threading
 # The in-tree build; FA2_GFX950_LIBRARY names another build of the same ABI (e.g. one under test).
 LIBRARY_PATH = pathlib.Path(os.environ.get("FA2_GFX950_LIBRARY") or
                             pathlib.Path(__file__).resolve().parent / "csrc" / "libfa2_gfx950.so")
-ABI_VERSION = 7
+ABI_VERSION = 8
 
 FA2_DTYPE_F16 = 0
 FA2_DTYPE_BF16 = 1
@@ -68,6 +68,12 @@ class FwdArgs(ctypes.Structure):
                 ("seqlen_q_rounded", _i), ("softmax_scale", _f), ("dtype", _i), ("config_id", _i)]
 
 
+class Cast(ctypes.Structure):
+    """Mirror of ``fa2_cast``."""
+
+    _fields_ = [("src", _p), ("dst", _p), ("n", _i64)]
+
+
 class BwdArgs(ctypes.Structure):
     """Mirror of ``fa2_bwd_args``."""
 
@@ -96,6 +102,8 @@ SIGNATURES = {
     "fa2_bwd_fused_noalloc": (_i, [_p] * 9 + [_i] * 6 + [_i64] * 24 + [_f, _i, _i, _i, _p]),
     "fa2_launch_info_get": (_i, [_i] * 6 + [ctypes.POINTER(LaunchInfo)]),
     "fa2_fwd_packed": (_i, [ctypes.POINTER(FwdArgs), _p]),
+    "fa2_fwd_packed_f32_out": (_i, [ctypes.POINTER(FwdArgs), _p, _p]),
+    "fa2_cast_f32_to_f16": (_i, [ctypes.POINTER(Cast), _i, _p]),
     "fa2_bwd_packed": (_i, [ctypes.POINTER(BwdArgs), _p]),
     "fa2_bwd_packed_f32_grads": (_i, [ctypes.POINTER(BwdArgs), _p]),
 }

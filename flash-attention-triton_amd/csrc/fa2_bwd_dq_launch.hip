@@ -1,5 +1,6 @@
-// Instantiates and launches the dQ kernels and the delta preprocess.
+// Instantiates and launches the dQ kernels, the delta preprocess and the fp32 casts.
 #include "fa2_bwd_dq.hpp"
+#include "fa2_cast.hpp"
 #include "fa2_launch.hpp"
 
 namespace fa2 {
@@ -64,6 +65,10 @@ void launch_dq(bool bf16, int dp, const BwdParams &p, dim3 grid, bool fuse_delta
     launch<__bf16>(dp, p, grid, fuse_delta, s);
   else
     launch<_Float16>(dp, p, grid, fuse_delta, s);
+}
+
+void launch_cast(const CastParams &p, dim3 grid, hipStream_t s) {
+  hipLaunchKernelGGL(cast_f16_kernel, grid, dim3(kCastThreads), 0, s, p);
 }
 
 void launch_preprocess(bool bf16, const PreParams &p, dim3 grid, hipStream_t s) {

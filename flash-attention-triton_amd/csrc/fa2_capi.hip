@@ -197,7 +197,7 @@ int64_t plan_dq(int cfg, fa2::BwdParams &p) {
   return nwg;
 }
 
-int fwd_impl(const fa2_fwd_args &a, void *stream) {
+int fwd_impl(const fa2_fwd_args &a, void *stream, float *o_f32 = nullptr) {
   int rc = check_common(a.batch, a.nheads, a.seqlen_q, a.seqlen_k, a.headdim, a.seqlen_q_rounded, a.dtype);
   if (rc) return rc;
   fa2::FwdParams p;
@@ -205,8 +205,10 @@ int fwd_impl(const fa2_fwd_args &a, void *stream) {
   p.k = tensor(a.k);
   p.v = tensor(a.v);
   p.o = tensor(a.o);
+  p.o_f32 = o_f32;
+  const bool want_o = o_f32 == nullptr || a.o.ptr != nullptr;
   if ((rc = check_tensor("q", p.q)) || (rc = check_tensor("k", p.k)) ||
-      (rc = check_tensor("v", p.v)) || (rc = check_tensor("o", p.o)))
+      (rc = check_tensor("v", p.v)) || (want_o && (rc = check_tensor("o", p.o))))
     return rc;
   if (a.lse == nullptr) return fail(FA2_ERR_NULL_POINTER, "lse is NULL");
   if (!good_scale(a.softmax_scale))
@@ -223,7 +225,8 @@ int fwd_impl(const fa2_fwd_args &a, void *stream) {
   p.seqlen_q_rounded = a.seqlen_q_rounded;
   p.scale = a.softmax_scale;
   p.scale_log2 = a.softmax_scale * fa2::kLog2e;
-  p.vec = vec_ok(p.q, a.headdim) && vec_ok(p.k, a.headdim) && vec_ok(p.v, a.headdim) && vec_ok(p.o, a.headdim);
+  p.vec = vec_ok(p.q, a.headdim) && vec_ok(p.k, a.headdim) && vec_ok(p.v, a.headdim) &&
+          (!want_o || vec_ok(p.o, a.headdim)) && reinterpret_cast<uintptr_t>(o_f32) % 16 == 0;
 
   const int64_t nwg = plan_fwd(cfg, p);
   if (nwg > fa2::kMaxWorkgroups)
@@ -516,6 +519,43 @@ int fa2_launch_info_get(int batch, int nheads, int seqlen_q, int seqlen_k, int h
 int fa2_fwd_packed(const fa2_fwd_args *args, void *stream) {
   if (args == nullptr) return fail(FA2_ERR_NULL_POINTER, "args is NULL");
   return fwd_impl(*args, stream);
+}
+
+int fa2_fwd_packed_f32_out(const fa2_fwd_args *args, float *o_f32, void *stream) {
+  if (args == nullptr) return fail(FA2_ERR_NULL_POINTER, "args is NULL");
+  if (o_f32 == nullptr) return fail(FA2_ERR_NULL_POINTER, "o_f32 is NULL");
+  if (reinterpret_cast<uintptr_t>(o_f32) % 4 != 0) return fail(FA2_ERR_BAD_STRIDE, "o_f32 is not 4-byte aligned");
+  return fwd_impl(*args, stream, o_f32);
+}
+
+int fa2_cast_f32_to_f16(const fa2_cast *arrays, int count, void *stream) {
+  if (arrays == nullptr) return fail(FA2_ERR_NULL_POINTER, "arrays is NULL");
+  if (count < 1 || count > fa2::kCastJobs)
+    return fail(FA2_ERR_BAD_SHAPE, "count must be 1 to %d, got %d", fa2::kCastJobs, count);
+  fa2::CastParams p;
+  int64_t blocks = 0;
+  for (int i = 0; i < count; i++) {
+    const fa2_cast &a = arrays[i];
+    if (a.src == nullptr || a.dst == nullptr) return fail(FA2_ERR_NULL_POINTER, "array %d: src or dst is NULL", i);
+    if (a.n <= 0) return fail(FA2_ERR_BAD_SHAPE, "array %d: n must be positive, got %lld", i, (long long)a.n);
+    if (reinterpret_cast<uintptr_t>(a.src) % 16 != 0 || reinterpret_cast<uintptr_t>(a.dst) % 8 != 0)
+      return fail(FA2_ERR_BAD_STRIDE, "array %d: src must be 16-byte and dst 8-byte aligned", i);
+    if (a.n > fa2::kMaxWorkgroups * fa2::kCastBlock) return fail(FA2_ERR_TOO_LARGE, "array %d too large", i);
+    p.src[i] = a.src;
+    p.dst[i] = a.dst;
+    p.n[i] = a.n;
+    p.first[i] = (unsigned)blocks;
+    blocks += (a.n + fa2::kCastBlock - 1) / fa2::kCastBlock;
+  }
+  if (blocks > fa2::kMaxWorkgroups) return fail(FA2_ERR_TOO_LARGE, "grid of %lld workgroups too large", (long long)blocks);
+  for (int i = count; i < fa2::kCastJobs; i++) {
+    p.src[i] = nullptr;
+    p.dst[i] = nullptr;
+    p.n[i] = 0;
+    p.first[i] = UINT_MAX;
+  }
+  fa2::launch_cast(p, dim3((unsigned)blocks), reinterpret_cast<hipStream_t>(stream));
+  return launch_status("fa2_cast launch");
 }
 
 int fa2_bwd_packed(const fa2_bwd_args *args, void *stream) {

@@ -205,16 +205,11 @@ __device__ __forceinline__ void store_chunk_widened(float *row, int d0, int head
 // at COLS; lane (c, h) holding sequence position c) to a (seqlen, headdim) tensor.  The values go through
 // a wave-private LDS patch of 32 x (whole blocks + 8) elements so that global stores are 16-byte and
 // row-contiguous.  The caller guarantees the patch is not in use by anyone else.  With `f32` (uniform)
-// the rows are fp32 and receive the rounded values widened.
-template <typename T, int COLS, bool UNROLL_F32 = false>
-__device__ __forceinline__ void store_transposed_acc(const f32x16 (&acc)[(COLS + 31) / 32], float mult,
-                                                     short *patch, void *dst_rows,
-                                                     int64_t stride_seq, int rows_valid,
-                                                     int headdim, bool vec, bool f32 = false) {
+// the rows are fp32 and receive the rounded values widened.  The two halves, for a caller that stores twice:
+template <typename T, int COLS>
+__device__ __forceinline__ void transposed_acc_to_patch(const f32x16 (&acc)[(COLS + 31) / 32], float mult, short *patch) {
   constexpr int DB = (COLS + 31) / 32;
   constexpr int LD = 32 * DB + 8;
-  constexpr int CPR = COLS / 8;
-  static_assert(COLS % 16 == 0, "a wave stores whole chunks");
   const int lane = threadIdx.x & 63;
   const int c = lane & 31, h = lane >> 5;
 #pragma unroll
@@ -229,6 +224,15 @@ __device__ __forceinline__ void store_transposed_acc(const f32x16 (&acc)[(COLS +
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <typename T, int COLS, bool UNROLL_F32 = false>
+__device__ __forceinline__ void store_patch(const short *patch, void *dst_rows, int64_t stride_seq, int rows_valid,
+                                            int headdim, bool vec, bool f32) {
+  constexpr int LD = 32 * ((COLS + 31) / 32) + 8;
+  constexpr int CPR = COLS / 8;
+  static_assert(COLS % 16 == 0, "a wave stores whole chunks");
+  const int lane = threadIdx.x & 63;
   if (f32) {
     // At 256 columns registers decide: unrolled, the addresses cost the dQ kernel 12 bytes of scratch per lane;
     // rolled, the loop costs the paired dK/dV kernel 20.  So chosen, neither uses any, padded or not.
@@ -249,6 +253,29 @@ __device__ __forceinline__ void store_transposed_acc(const f32x16 (&acc)[(COLS +
     s16x8 v = *reinterpret_cast<const s16x8 *>(patch + r * LD + cc * 8);
     store_chunk((short *)dst_rows + (int64_t)r * stride_seq, cc * 8, headdim, r < rows_valid, vec, v);
   }
+}
+
+template <typename T, int COLS, bool UNROLL_F32 = false>
+__device__ __forceinline__ void store_transposed_acc(const f32x16 (&acc)[(COLS + 31) / 32], float mult,
+                                                     short *patch, void *dst_rows,
+                                                     int64_t stride_seq, int rows_valid,
+                                                     int headdim, bool vec, bool f32 = false) {
+  transposed_acc_to_patch<T, COLS>(acc, mult, patch);
+  store_patch<T, COLS, UNROLL_F32>(patch, dst_rows, stride_seq, rows_valid, headdim, vec, f32);
+}
+
+// The same for the forward's wave of query rows row0 .. row0 + 31 of (batch, head) pair bh: to the tensor in the
+// inputs' type, to the fp32 one, or to both.
+template <typename T, int COLS>
+__device__ __forceinline__ void store_output(const FwdParams &p, const f32x16 (&acc)[(COLS + 31) / 32], float mult,
+                                             short *patch, int bh, int b, int hd, int row0, int headdim, bool vec) {
+  transposed_acc_to_patch<T, COLS>(acc, mult, patch);
+  const int rows = p.seqlen_q - row0;
+  if (p.o.ptr != nullptr)
+    store_patch<T, COLS>(patch, (short *)p.o.ptr + b * p.o.stride_batch + hd * p.o.stride_head + row0 * p.o.stride_seq,
+                         p.o.stride_seq, rows, headdim, vec, false);
+  if (p.o_f32 != nullptr)
+    store_patch<T, COLS>(patch, p.o_f32 + ((int64_t)bh * p.seqlen_q + row0) * headdim, headdim, rows, headdim, vec, true);
 }
 
 // Address of element (b, hd, row, col) of a gradient.

@@ -158,7 +158,6 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_kerne
   const short *Q = (const short *)p.q.ptr + b * p.q.stride_batch + hd * p.q.stride_head;
   const short *K = (const short *)p.k.ptr + b * p.k.stride_batch + hd * p.k.stride_head;
   const short *V = (const short *)p.v.ptr + b * p.v.stride_batch + hd * p.v.stride_head;
-  short *O = (short *)p.o.ptr + b * p.o.stride_batch + hd * p.o.stride_head;
   float *LSE = p.lse + (int64_t)bh * p.seqlen_q_rounded;
 
   // Q^T fragments (B operand of S^T = K Q^T): lane (c, h) holds Q[q0w + c][16 ks + 8 h + j].
@@ -247,8 +246,7 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_kerne
   }
   // All waves passed the loop's final barrier, so the K/V stages are free to reuse.
   short *patch = smem + wave * 32 * (DP + 8);
-  store_transposed_acc<T, DP>(oacc, inv_l, patch, O + (int64_t)q0w * p.o.stride_seq,
-                              p.o.stride_seq, p.seqlen_q - q0w, p.headdim, VEC);
+  store_output<T, DP>(p, oacc, inv_l, patch, bh, b, hd, q0w, p.headdim, VEC);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -339,7 +337,6 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
   const short *Q = (const short *)p.q.ptr + b * p.q.stride_batch + hd * p.q.stride_head;
   const short *K = (const short *)p.k.ptr + b * p.k.stride_batch + hd * p.k.stride_head;
   const short *V = (const short *)p.v.ptr + b * p.v.stride_batch + hd * p.v.stride_head;
-  short *O = (short *)p.o.ptr + b * p.o.stride_batch + hd * p.o.stride_head;
   float *LSE = p.lse + (int64_t)bh * p.seqlen_q_rounded;
 
   const int hdim = PAD ? p.headdim : COLS;
@@ -728,8 +725,7 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
   }
   // The patch overlays the stages; the loop's last barrier already ordered it after all reads.
   short *patch = smem + KG * MERGE_FLOATS * 2 + wave * 32 * (DP + 8);
-  store_transposed_acc<T, COLS>(oacc, inv_l, patch, O + (int64_t)q0w * p.o.stride_seq,
-                              p.o.stride_seq, p.seqlen_q - q0w, hdim, true);
+  store_output<T, COLS>(p, oacc, inv_l, patch, bh, b, hd, q0w, hdim, true);
 }
 
 }  // namespace fa2

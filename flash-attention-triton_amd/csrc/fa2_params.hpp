@@ -37,6 +37,7 @@ constexpr int kDkvBlockQ = 64;
 
 struct FwdParams {
   Tensor4 q, k, v, o;
+  float *o_f32;  // contiguous fp32 tensor that receives the output widened, or null; o.ptr may be null beside it
   float *lse;
   int batch, nheads, seqlen_q, seqlen_k, headdim, seqlen_q_rounded;
   int n_qtiles;
@@ -73,6 +74,16 @@ struct PreParams {
   int batch, nheads, seqlen_q, headdim, seqlen_q_rounded;
   unsigned n_tiles;  // tiles of 16 rows over all (batch, head) pairs
   int vec;
+};
+
+// Arrays of fp32 numbers to round to fp16, at most kCastJobs in one launch.
+constexpr int kCastJobs = 3;
+constexpr int kCastThreads = 256, kCastBlock = 16 * kCastThreads;  // elements per workgroup
+struct CastParams {
+  const float *src[kCastJobs];
+  void *dst[kCastJobs];
+  int64_t n[kCastJobs];
+  unsigned first[kCastJobs];  // first workgroup of an array
 };
 
 }  // namespace fa2

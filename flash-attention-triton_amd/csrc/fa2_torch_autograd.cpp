@@ -17,6 +17,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
+#include <array>
 #include <cmath>
 #include <stdexcept>
 #include <string>
@@ -58,6 +59,27 @@ at::Tensor readable(const at::Tensor &t) {
   return direct ? t : t.contiguous();
 }
 
+// fp32 tensors rounded to fp16, at most three in one launch, with the strides t.to(at::kHalf) would give.  Tensors
+// without gaps are arrays to the kernel whatever the order of their dimensions; any other is torch's.
+template <size_t N>
+std::array<at::Tensor, N> rounded_to_half(const std::array<at::Tensor, N> &in) {
+  std::array<at::Tensor, N> out;
+  std::array<fa2_cast, N> jobs;
+  int count = 0;
+  for (size_t i = 0; i < N; i++) {
+    const at::Tensor &t = in[i];
+    if (t.numel() > 0 && t.is_non_overlapping_and_dense() && !t.is_neg() && !t._is_zerotensor() &&
+        reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0) {
+      out[i] = at::empty_like(t, t.options().dtype(at::kHalf));
+      jobs[count++] = fa2_cast{t.data_ptr<float>(), out[i].data_ptr(), t.numel()};
+    } else {
+      out[i] = t.to(at::kHalf);
+    }
+  }
+  if (count > 0) check(fa2_cast_f32_to_f16(jobs.data(), count, current_stream(in[0])), "fa2_cast_f32_to_f16");
+  return out;
+}
+
 int64_t rounded(int64_t seqlen_q, int64_t max_headdim) {
   return (seqlen_q + max_headdim - 1) / max_headdim * max_headdim;
 }
@@ -71,20 +93,26 @@ struct FlashAttentionV2 : public torch::autograd::Function<FlashAttentionV2> {
     // fp32 tensors are computed in fp16, as the reference does.  The casts are the node's and not the
     // graph's so that the backward can hand out fp32 gradients: the kernels store them widened, which saves
     // a pass over each.  B=32 H=20 N=1024 D=96, forward + backward: 1205 us, with casts in the graph 1339 us.
+    // The kernel stores the output in fp32 as well, and q, k and v are rounded in one launch: 1193 -> 1144 us.
     const bool f32 = q_in.scalar_type() == at::kFloat;
-    auto operand = [&](const at::Tensor &t) { return readable(f32 ? t.to(at::kHalf) : t); };
-    const at::Tensor q = operand(q_in), k = operand(k_in), v = operand(v_in);
+    std::array<at::Tensor, 3> in = {q_in, k_in, v_in};
+    if (f32) in = rounded_to_half(in);
+    const at::Tensor q = readable(in[0]), k = readable(in[1]), v = readable(in[2]);
     const int64_t batch = q.size(0), nheads = q.size(1), seqlen_q = q.size(2), headdim = q.size(3);
     const int64_t seqlen_k = k.size(2);
     const int64_t seqlen_q_rounded = rounded(seqlen_q, max_headdim);
-    at::Tensor o = at::empty(q.sizes(), q.options());  // contiguous whatever the strides of q
+    // Contiguous whatever the strides of q.  With fp32 tensors the kernel stores the result in fp32, and in
+    // fp16 only where a backward will read that.
+    at::Tensor o, o_f32;
+    if (!f32 || !forward_only) o = at::empty(q.sizes(), q.options());
+    if (f32) o_f32 = at::empty(q.sizes(), q_in.options());
     at::Tensor lse = at::empty({batch, nheads, seqlen_q_rounded}, q.options().dtype(at::kFloat));
 
     fa2_fwd_args a;
     a.q = as_arg(q);
     a.k = as_arg(k);
     a.v = as_arg(v);
-    a.o = as_arg(o);
+    a.o = o.defined() ? as_arg(o) : fa2_tensor{nullptr, 0, 0, 0};
     a.lse = lse.data_ptr<float>();
     a.batch = (int)batch;
     a.nheads = (int)nheads;
@@ -98,13 +126,14 @@ struct FlashAttentionV2 : public torch::autograd::Function<FlashAttentionV2> {
     a.config_id = forward_only ? fa2_pick_config_forward_only(a.dtype, a.headdim, a.seqlen_q, a.seqlen_k)
                                : FA2_CONFIG_AUTO;
     if (forward_only && a.config_id < 0) check(-a.config_id, "fa2_pick_config_forward_only");
-    check(fa2_fwd_packed(&a, current_stream(q)), "fa2_fwd");
+    check(f32 ? fa2_fwd_packed_f32_out(&a, o_f32.data_ptr<float>(), current_stream(q))
+              : fa2_fwd_packed(&a, current_stream(q)), "fa2_fwd");
 
     ctx->save_for_backward({q, k, v, o, lse});
     ctx->saved_data["softmax_scale"] = softmax_scale;
     ctx->saved_data["deterministic"] = deterministic;
     ctx->saved_data["f32"] = f32;
-    return f32 ? o.to(at::kFloat) : o;
+    return f32 ? o_f32 : o;
   }
 
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx,
@@ -115,7 +144,11 @@ struct FlashAttentionV2 : public torch::autograd::Function<FlashAttentionV2> {
     // Like the reference (flash_attention_2.py:364) the backward is not differentiable.
     const at::NoGradGuard no_grad;
     at::Tensor d_o = grads[0];
-    if (d_o.scalar_type() != q.scalar_type()) d_o = d_o.to(q.scalar_type());
+    if (d_o.scalar_type() == at::kFloat && q.scalar_type() == at::kHalf && d_o.is_cuda()) {
+      d_o = rounded_to_half(std::array<at::Tensor, 1>{d_o})[0];
+    } else if (d_o.scalar_type() != q.scalar_type()) {
+      d_o = d_o.to(q.scalar_type());
+    }
     d_o = readable(d_o);
     // (empty_like keeps the order of a dense view's dimensions: the gradients of transposed projections come
     // out in the projections' own order.)

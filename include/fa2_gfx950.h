@@ -35,8 +35,8 @@ extern "C" {
 
 /* Raised with every entry point added or changed and every change of what a field means: 6 brought
  * fa2_bwd_packed_f32_grads and the paired dK/dV kernel (bwd_block_kv, lds_direct and dkdv_passes below), 7
- * fa2_launch_info_get. */
-#define FA2_ABI_VERSION 7
+ * fa2_launch_info_get, 8 fa2_fwd_packed_f32_out and fa2_cast_f32_to_f16. */
+#define FA2_ABI_VERSION 8
 
 /* Largest head dimension the kernels accept (the table's `max_headdim`). */
 #define FA2_MAX_HEADDIM 256
@@ -225,6 +225,26 @@ int fa2_fwd(const void *q, const void *k, const void *v, void *o, float *lse,
  * (flash_attention_2.py:61-144, _triton_kernels_v2.py:11-189).
  */
 int fa2_fwd_packed(const fa2_fwd_args *args, void *stream);
+
+/*
+ * fa2_fwd_packed that writes the output as an fp32 tensor too: o_f32, contiguous (batch, nheads, seqlen_q,
+ * headdim), receives the values of o widened, without the pass that a caller with fp32 tensors would run
+ * (flash_attention_2.py:339).  args->o.ptr may be NULL where no backward will read o.
+ */
+int fa2_fwd_packed_f32_out(const fa2_fwd_args *args, float *o_f32, void *stream);
+
+/* n fp32 numbers to be rounded (to nearest, ties to even) to n fp16 numbers; src 16-byte aligned, dst 8-byte. */
+typedef struct fa2_cast {
+  const float *src;
+  void *dst;
+  int64_t n;
+} fa2_cast;
+
+/*
+ * The casts in front of a call with fp32 tensors (flash_attention_2.py:313-316): one to three arrays in one
+ * launch.
+ */
+int fa2_cast_f32_to_f16(const fa2_cast *arrays, int count, void *stream);
 
 /*
  * Backward preprocess: delta[b,h,i] = sum_d O[b,h,i,d] * dO[b,h,i,d] in fp32.

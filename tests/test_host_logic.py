@@ -47,7 +47,7 @@ def test_library_exports_every_declared_symbol(capi):
 
 # sha256 (first 16 digits) of include/fa2_gfx950.h without comments, white space and the version itself, per ABI
 # version.  A change of the interface needs a new version and a line here.
-INTERFACES = {6: "94837833e0c9a376", 7: "f98a87f9170d5460"}
+INTERFACES = {6: "94837833e0c9a376", 7: "f98a87f9170d5460", 8: "6532f24f44a70406"}
 
 
 def test_abi_version_follows_the_interface(capi):
