@@ -332,8 +332,25 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
     const unsigned dst = lds_base + 2u * (unsigned)(L::V_BASE + (t % L::V_STAGES) * L::TILE_ELEMS);
     if (t < n_inside) vload.issue(t * BKV, dst); else vload.issue_clamped(t * BKV, seqlen_k, dst);
   };
-  // K_0, V_0 and K_1 are loaded here; after that tile t brings in K_{t+2} and V_{t+1}.
+  // K_0, the workgroup's Q rows, V_0 and K_1 are loaded here; after that tile t brings in K_{t+2} and V_{t+1}.  The
+  // Q rows travel as in the forward, like a K tile into the stages nothing else uses yet (rows 0..63 in the third K
+  // stage and 64..127 in the second V stage, or all 64 in the latter), because fragment loads straight into
+  // registers touch 32 rows each and keep the address path busy.  Rows beyond the sequence come from its last row:
+  // their results are not stored.  Forward and backward, bf16: 256x16x512 D=64 1205 -> 1176 us; fp32
+  // 32x20x1024 D=96 1161 -> 1144; long sequences alike.  From 128 columns on they are loaded into registers as dO is:
+  // none is left for this order (scratch memory per lane: 8 bytes at 128, 212 at 256; 1x8x4096 D=128 gained 0.8 %).
+  constexpr bool Q_STAGED = DP <= 96;
+  constexpr int Q_HI = L::V_BASE + L::TILE_ELEMS;
+  constexpr int Q_LO = KG == 1 ? L::K_BASE + 2 * L::TILE_ELEMS : Q_HI;
+  const Loader qload(Q + (int64_t)q0 * p.q.stride_seq, p.q.stride_seq, hdim / 8);
+  const int q_rows = p.seqlen_q - q0;  // query rows of this tile that exist (>= 1)
   issue_k(0);
+  if (Q_STAGED) {
+    if (q_rows >= BKV) qload.issue(0, lds_base + 2u * Q_LO); else qload.issue_clamped(0, q_rows, lds_base + 2u * Q_LO);
+  }
+  if (Q_STAGED && KG == 1) {
+    if (q_rows >= 2 * BKV) qload.issue(BKV, lds_base + 2u * Q_HI); else qload.issue_clamped(BKV, q_rows, lds_base + 2u * Q_HI);
+  }
   issue_v(0);
   if (n_tiles > 1) issue_k(1);
 
@@ -347,7 +364,7 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
     const short *gp = DO + (int64_t)row * p.d_o.stride_seq;
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
-      qf[ks] = load_chunk(qp, 16 * ks + 8 * h, hdim, ok, true);
+      if (!Q_STAGED) qf[ks] = load_chunk(qp, 16 * ks + 8 * h, hdim, ok, true);
       gf[ks] = load_chunk(gp, 16 * ks + 8 * h, hdim, ok, true);
     }
     if (ok) lse2 = p.lse[(int64_t)bh * p.seqlen_q_rounded + row] * kLog2e;
@@ -408,11 +425,21 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
 
   wait_vmem_all();
   __syncthreads();
+  if (Q_STAGED) {
+    const lds_cptr qrows = to_lds(smem) + ((rg >> 1) ? Q_HI : Q_LO);
+    const int r = 32 * (rg & 1) + c;
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) qf[ks] = lds_read_128(qrows + swz_off<LP>(r, 2 * ks + h));
+  }
 
   // Ring of A fragments, preloaded with the K rows of block 0.
   s16x8 ring[R];
 #pragma unroll
   for (int ks = 0; ks < KS; ks++) ring[ks] = lds_read_128(knext[ks]);
+  if (Q_STAGED) {  // every wave has its Q fragments: their stages are free for K_2 and V_1
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __syncthreads();
+  }
 
   // One 32-key block j = 2 t + HALF, three GEMMs of KS MFMAs, each unit = one MFMA, the LDS reads
   // that refill the ring slot it freed, and a share of the vector work:

@@ -81,7 +81,8 @@ inline int fwd_key_groups(int dp, const FwdParams &p) {
   return fwd_direct_ok(dp, p) ? key_groups(dp, (int64_t)p.batch * p.nheads, p.seqlen_q, false) : 1;
 }
 inline bool dq_direct_ok(int dp, const BwdParams &p) {
-  return p.vec && direct_headdim_wide(dp, p.headdim) && direct_stride_ok(p.k) && direct_stride_ok(p.v);
+  return p.vec && direct_headdim_wide(dp, p.headdim) && (dp > 96 || direct_stride_ok(p.q)) && direct_stride_ok(p.k) &&
+         direct_stride_ok(p.v);
 }
 inline int dq_key_groups(int dp, const BwdParams &p) {
   return dq_direct_ok(dp, p) ? key_groups(dp, (int64_t)p.batch * p.nheads, p.seqlen_q, true) : 1;
