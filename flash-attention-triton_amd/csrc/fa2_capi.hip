@@ -231,8 +231,9 @@ int fwd_impl(const fa2_fwd_args &a, void *stream, float *o_f32 = nullptr) {
   const int64_t nwg = plan_fwd(cfg, p);
   if (nwg > fa2::kMaxWorkgroups)
     return fail(FA2_ERR_TOO_LARGE, "grid of %lld workgroups too large", (long long)nwg);
-  fa2::launch_fwd(a.dtype == FA2_DTYPE_BF16, kTable[cfg].headdim_padded, kTable[cfg].fwd_exp_folded != 0, p,
-                  dim3((unsigned)nwg), reinterpret_cast<hipStream_t>(stream));
+  const auto launch = o_f32 == nullptr ? fa2::launch_fwd<false> : fa2::launch_fwd<true>;
+  launch(a.dtype == FA2_DTYPE_BF16, kTable[cfg].headdim_padded, kTable[cfg].fwd_exp_folded != 0, p,
+         dim3((unsigned)nwg), reinterpret_cast<hipStream_t>(stream));
   return launch_status("fa2_fwd launch");
 }
 

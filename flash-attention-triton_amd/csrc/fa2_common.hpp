@@ -264,18 +264,23 @@ __device__ __forceinline__ void store_transposed_acc(const f32x16 (&acc)[(COLS +
   store_patch<T, COLS, UNROLL_F32>(patch, dst_rows, stride_seq, rows_valid, headdim, vec, f32);
 }
 
-// The same for the forward's wave of query rows row0 .. row0 + 31 of (batch, head) pair bh: to the tensor in the
-// inputs' type, to the fp32 one, or to both.
-template <typename T, int COLS>
+// The same for the forward's wave of query rows row0 .. row0 + 31 of (batch, head) pair bh, whose rows in the inputs'
+// type start at O.  With F32 they go to the fp32 tensor and, unless o.ptr is null, to O.  F32 is a variant of the kernels
+// that only calls with an fp32 output launch: as a test of the pointers in every forward it took one or two registers
+// more, up to seven spilled scalars, and fifty to a hundred instructions (bf16, us, with the test and without: 4x16x2048
+// D=64 45.9 and 44.2, 2x32x4096 D=128 251.0 and 249.2, 1x16x512 D=256 19.6 and 19.1; 1x16x333 D=128 alike).
+template <typename T, int COLS, bool F32>
 __device__ __forceinline__ void store_output(const FwdParams &p, const f32x16 (&acc)[(COLS + 31) / 32], float mult,
-                                             short *patch, int bh, int b, int hd, int row0, int headdim, bool vec) {
-  transposed_acc_to_patch<T, COLS>(acc, mult, patch);
+                                             short *patch, short *O, int bh, int row0, int headdim, bool vec) {
+  short *o_rows = O + (int64_t)row0 * p.o.stride_seq;
   const int rows = p.seqlen_q - row0;
-  if (p.o.ptr != nullptr)
-    store_patch<T, COLS>(patch, (short *)p.o.ptr + b * p.o.stride_batch + hd * p.o.stride_head + row0 * p.o.stride_seq,
-                         p.o.stride_seq, rows, headdim, vec, false);
-  if (p.o_f32 != nullptr)
+  if constexpr (!F32) {
+    store_transposed_acc<T, COLS>(acc, mult, patch, o_rows, p.o.stride_seq, rows, headdim, vec);
+  } else {
+    transposed_acc_to_patch<T, COLS>(acc, mult, patch);
+    if (p.o.ptr != nullptr) store_patch<T, COLS>(patch, o_rows, p.o.stride_seq, rows, headdim, vec, false);
     store_patch<T, COLS>(patch, p.o_f32 + ((int64_t)bh * p.seqlen_q + row0) * headdim, headdim, rows, headdim, vec, true);
+  }
 }
 
 // Address of element (b, hd, row, col) of a gradient.

@@ -127,7 +127,7 @@ __device__ __forceinline__ void fwd_tile(const short *sk, const short *sv, const
   }
 }
 
-template <typename T, int DP, int BKV, bool VEC>
+template <typename T, int DP, int BKV, bool VEC, bool F32 = false>
 __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_kernel(const FwdParams p) {
   using L = FwdLayout<DP, BKV>;
   constexpr int KS = DP / 16;    // k-steps of Q K^T
@@ -158,6 +158,7 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_kerne
   const short *Q = (const short *)p.q.ptr + b * p.q.stride_batch + hd * p.q.stride_head;
   const short *K = (const short *)p.k.ptr + b * p.k.stride_batch + hd * p.k.stride_head;
   const short *V = (const short *)p.v.ptr + b * p.v.stride_batch + hd * p.v.stride_head;
+  short *O = (short *)p.o.ptr + b * p.o.stride_batch + hd * p.o.stride_head;
   float *LSE = p.lse + (int64_t)bh * p.seqlen_q_rounded;
 
   // Q^T fragments (B operand of S^T = K Q^T): lane (c, h) holds Q[q0w + c][16 ks + 8 h + j].
@@ -246,7 +247,7 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_kerne
   }
   // All waves passed the loop's final barrier, so the K/V stages are free to reuse.
   short *patch = smem + wave * 32 * (DP + 8);
-  store_output<T, DP>(p, oacc, inv_l, patch, bh, b, hd, q0w, p.headdim, VEC);
+  store_output<T, DP, F32>(p, oacc, inv_l, patch, O, bh, q0w, p.headdim, VEC);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -307,7 +308,8 @@ struct HalfTag {
 // every score chain starts from minus the maximum in use (the MFMA's C operand), so that the score
 // MFMAs deliver the base-2 exponents themselves and no multiply-add is left in front of the
 // exponentials.
-template <typename T, int DP, int BKV, bool PAD, bool PRE, int KG = 1, int COLS = DP>
+// F32: the output goes to an fp32 tensor as well, or only there: store_output (fa2_common.hpp).
+template <typename T, int DP, int BKV, bool PAD, bool PRE, int KG = 1, int COLS = DP, bool F32 = false>
 __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direct_kernel(const FwdParams p) {
   using L = FwdDirectLayout<DP, BKV>;
   constexpr int KS = COLS / 16, DB = (COLS + 31) / 32, R = 2 * DB, LP = L::LP;
@@ -337,6 +339,7 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
   const short *Q = (const short *)p.q.ptr + b * p.q.stride_batch + hd * p.q.stride_head;
   const short *K = (const short *)p.k.ptr + b * p.k.stride_batch + hd * p.k.stride_head;
   const short *V = (const short *)p.v.ptr + b * p.v.stride_batch + hd * p.v.stride_head;
+  short *O = (short *)p.o.ptr + b * p.o.stride_batch + hd * p.o.stride_head;
   float *LSE = p.lse + (int64_t)bh * p.seqlen_q_rounded;
 
   const int hdim = PAD ? p.headdim : COLS;
@@ -725,7 +728,7 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
   }
   // The patch overlays the stages; the loop's last barrier already ordered it after all reads.
   short *patch = smem + KG * MERGE_FLOATS * 2 + wave * 32 * (DP + 8);
-  store_output<T, COLS>(p, oacc, inv_l, patch, bh, b, hd, q0w, hdim, true);
+  store_output<T, COLS, F32>(p, oacc, inv_l, patch, O, bh, q0w, hdim, true);
 }
 
 }  // namespace fa2

@@ -1,19 +1,21 @@
-// Instantiates and launches the forward kernels.
+// Instantiates and launches the forward kernels: compiled twice, with FA2_F32_OUT 0 and 1 (kF32).
 #include "fa2_fwd.hpp"
 #include "fa2_launch.hpp"
 
 namespace fa2 {
 namespace {
 
+constexpr bool kF32 = FA2_F32_OUT;
+
 template <typename T, bool VEC>
 void launch_generic(int dp, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
   switch (dp) {
-    case 32: hipLaunchKernelGGL((fwd_kernel<T, 32, kFwdBlockKV, VEC>), grid, block, 0, s, p); break;
-    case 64: hipLaunchKernelGGL((fwd_kernel<T, 64, kFwdBlockKV, VEC>), grid, block, 0, s, p); break;
-    case 96: hipLaunchKernelGGL((fwd_kernel<T, 96, kFwdBlockKV, VEC>), grid, block, 0, s, p); break;
-    case 128: hipLaunchKernelGGL((fwd_kernel<T, 128, kFwdBlockKV, VEC>), grid, block, 0, s, p); break;
-    case 192: hipLaunchKernelGGL((fwd_kernel<T, 192, kFwdBlockKV, VEC>), grid, block, 0, s, p); break;
-    default: hipLaunchKernelGGL((fwd_kernel<T, 256, kFwdBlockKV, VEC>), grid, block, 0, s, p); break;
+    case 32: hipLaunchKernelGGL((fwd_kernel<T, 32, kFwdBlockKV, VEC, kF32>), grid, block, 0, s, p); break;
+    case 64: hipLaunchKernelGGL((fwd_kernel<T, 64, kFwdBlockKV, VEC, kF32>), grid, block, 0, s, p); break;
+    case 96: hipLaunchKernelGGL((fwd_kernel<T, 96, kFwdBlockKV, VEC, kF32>), grid, block, 0, s, p); break;
+    case 128: hipLaunchKernelGGL((fwd_kernel<T, 128, kFwdBlockKV, VEC, kF32>), grid, block, 0, s, p); break;
+    case 192: hipLaunchKernelGGL((fwd_kernel<T, 192, kFwdBlockKV, VEC, kF32>), grid, block, 0, s, p); break;
+    default: hipLaunchKernelGGL((fwd_kernel<T, 256, kFwdBlockKV, VEC, kF32>), grid, block, 0, s, p); break;
   }
 }
 
@@ -25,9 +27,9 @@ void launch_generic(int dp, const FwdParams &p, dim3 grid, dim3 block, hipStream
 template <typename T, int DP, int COLS, bool PRE, int KG>
 void launch_cols(const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
   if (p.headdim == COLS)
-    hipLaunchKernelGGL((fwd_direct_kernel<T, DP, kFwdBlockKV, false, PRE, KG, COLS>), grid, block, 0, s, p);
+    hipLaunchKernelGGL((fwd_direct_kernel<T, DP, kFwdBlockKV, false, PRE, KG, COLS, kF32>), grid, block, 0, s, p);
   else
-    hipLaunchKernelGGL((fwd_direct_kernel<T, DP, kFwdBlockKV, true, PRE, KG, COLS>), grid, block, 0, s, p);
+    hipLaunchKernelGGL((fwd_direct_kernel<T, DP, kFwdBlockKV, true, PRE, KG, COLS, kF32>), grid, block, 0, s, p);
 }
 
 template <typename T, bool PRE, int KG>
@@ -39,7 +41,7 @@ void launch_direct(int dp, const FwdParams &p, dim3 grid, dim3 block, hipStream_
     case 80: launch_cols<T, 96, 80, PRE, KG>(p, grid, block, s); break;
     case 96: launch_cols<T, 96, 96, PRE, KG>(p, grid, block, s); break;
     case 128: launch_cols<T, 128, 128, PRE, KG>(p, grid, block, s); break;
-    default: launch_fwd_direct_wide(std::is_same<T, __bf16>::value, dp, KG, p, grid, block, s); break;
+    default: launch_fwd_direct_wide<kF32>(std::is_same<T, __bf16>::value, dp, KG, p, grid, block, s); break;
   }
 }
 
@@ -69,7 +71,8 @@ void launch(int dp, bool folded, const FwdParams &p, dim3 grid, hipStream_t s) {
 
 }  // namespace
 
-void launch_fwd(bool bf16, int dp, bool folded, const FwdParams &p, dim3 grid, hipStream_t s) {
+template <>
+void launch_fwd<kF32>(bool bf16, int dp, bool folded, const FwdParams &p, dim3 grid, hipStream_t s) {
   if (bf16)
     launch<__bf16>(dp, folded, p, grid, s);
   else

@@ -6,6 +6,8 @@
 namespace fa2 {
 namespace {
 
+constexpr bool kF32 = FA2_F32_OUT;
+
 // At 256 columns only the padded variant is instantiated, also for a head dimension of exactly 256
 // (it then switches no lane off): with the number of columns a run-time value the compiler keeps the
 // kernel within its 512 registers, with a constant 256 it spills about forty of them, with reloads
@@ -13,9 +15,9 @@ namespace {
 template <typename T, int DP, int COLS, int KG, bool PADDED_ONLY>
 void launch_cols(const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
   if (!PADDED_ONLY && p.headdim == COLS)
-    hipLaunchKernelGGL((fwd_direct_kernel<T, DP, kFwdBlockKV, PADDED_ONLY, false, KG, COLS>), grid, block, 0, s, p);
+    hipLaunchKernelGGL((fwd_direct_kernel<T, DP, kFwdBlockKV, PADDED_ONLY, false, KG, COLS, kF32>), grid, block, 0, s, p);
   else
-    hipLaunchKernelGGL((fwd_direct_kernel<T, DP, kFwdBlockKV, true, false, KG, COLS>), grid, block, 0, s, p);
+    hipLaunchKernelGGL((fwd_direct_kernel<T, DP, kFwdBlockKV, true, false, KG, COLS, kF32>), grid, block, 0, s, p);
 }
 
 template <typename T, int KG>
@@ -38,7 +40,8 @@ void launch_groups(int dp, int key_groups, const FwdParams &p, dim3 grid, dim3 b
 
 }  // namespace
 
-void launch_fwd_direct_wide(bool bf16, int dp, int key_groups, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
+template <>
+void launch_fwd_direct_wide<kF32>(bool bf16, int dp, int key_groups, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
   if (bf16)
     launch_groups<__bf16>(dp, key_groups, p, grid, block, s);
   else

@@ -37,7 +37,6 @@ constexpr int kDkvBlockQ = 64;
 
 struct FwdParams {
   Tensor4 q, k, v, o;
-  float *o_f32;  // contiguous fp32 tensor that receives the output widened, or null; o.ptr may be null beside it
   float *lse;
   int batch, nheads, seqlen_q, seqlen_k, headdim, seqlen_q_rounded;
   int n_qtiles;
@@ -46,6 +45,7 @@ struct FwdParams {
   float scale;       // softmax scale (natural units)
   float scale_log2;  // scale * log2(e)
   int vec;           // 16-byte global accesses are legal for every tensor
+  float *o_f32;      // contiguous fp32 tensor that receives the output widened, or null; o.ptr may be null beside it
 };
 
 struct BwdParams {

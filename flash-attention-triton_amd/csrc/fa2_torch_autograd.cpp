@@ -95,9 +95,10 @@ struct FlashAttentionV2 : public torch::autograd::Function<FlashAttentionV2> {
     // a pass over each.  B=32 H=20 N=1024 D=96, forward + backward: 1205 us, with casts in the graph 1339 us.
     // The kernel stores the output in fp32 as well, and q, k and v are rounded in one launch: 1193 -> 1144 us.
     const bool f32 = q_in.scalar_type() == at::kFloat;
-    std::array<at::Tensor, 3> in = {q_in, k_in, v_in};
-    if (f32) in = rounded_to_half(in);
-    const at::Tensor q = readable(in[0]), k = readable(in[1]), v = readable(in[2]);
+    std::array<at::Tensor, 3> half;
+    if (f32) half = rounded_to_half(std::array<at::Tensor, 3>{q_in, k_in, v_in});
+    const at::Tensor q = readable(f32 ? half[0] : q_in), k = readable(f32 ? half[1] : k_in),
+                     v = readable(f32 ? half[2] : v_in);
     const int64_t batch = q.size(0), nheads = q.size(1), seqlen_q = q.size(2), headdim = q.size(3);
     const int64_t seqlen_k = k.size(2);
     const int64_t seqlen_q_rounded = rounded(seqlen_q, max_headdim);

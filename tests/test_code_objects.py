@@ -107,6 +107,21 @@ def test_lds_direct_kernels_do_not_spill(records):
     assert {("bwd_dkdv_pair_kernel", dp) for dp in PAIR_COLUMNS} <= seen
 
 
+def test_fp32_output_is_a_variant_of_the_forward(records):
+    """Every forward kernel exists twice, and the store of an fp32 output costs only the one that has it registers."""
+    forms: dict = {}
+    for r in records:
+        m = re.match(r"(_ZN3fa2\d+fwd_\w*kernelI.*)Lb([01])EEEvNS_9FwdParamsE", r["name"])
+        if m:
+            forms.setdefault(m.group(1), {})[m.group(2)] = r
+    assert sum("fwd_direct_kernel" in stem for stem in forms) >= 2 * 2 * len(PAIR_COLUMNS)
+    assert any("10fwd_kernel" in stem for stem in forms)
+    for stem, both in forms.items():
+        assert set(both) == {"0", "1"}, stem
+        for key in ("vgpr_count", "sgpr_count", "sgpr_spill_count"):
+            assert int(both["0"][key]) <= int(both["1"][key]), (stem, key)
+
+
 def test_registers_and_lds_leave_room_for_the_tables_workgroups(records):
     import importlib
 
