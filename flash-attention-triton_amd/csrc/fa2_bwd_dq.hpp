@@ -345,12 +345,14 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
   const Loader qload(Q + (int64_t)q0 * p.q.stride_seq, p.q.stride_seq, hdim / 8);
   const int q_rows = p.seqlen_q - q0;  // query rows of this tile that exist (>= 1)
   issue_k(0);
-  if (Q_STAGED) {
-    if (q_rows >= BKV) qload.issue(0, lds_base + 2u * Q_LO); else qload.issue_clamped(0, q_rows, lds_base + 2u * Q_LO);
-  }
-  if (Q_STAGED && KG == 1) {
-    if (q_rows >= 2 * BKV) qload.issue(BKV, lds_base + 2u * Q_HI); else qload.issue_clamped(BKV, q_rows, lds_base + 2u * Q_HI);
-  }
+  // Rows too far apart for a lane's 32-bit offset go by the clamped loads, whose addresses are 64-bit: any q row stride
+  // runs this kernel, as it does where the rows go straight into registers.
+  const bool q_near = direct_stride_ok(p.q);
+  auto issue_q = [&](int row0, unsigned dst) {
+    if (q_near && q_rows >= row0 + BKV) qload.issue(row0, dst); else qload.issue_clamped(row0, q_rows, dst);
+  };
+  if (Q_STAGED) issue_q(0, lds_base + 2u * Q_LO);
+  if (Q_STAGED && KG == 1) issue_q(BKV, lds_base + 2u * Q_HI);
   issue_v(0);
   if (n_tiles > 1) issue_k(1);
 

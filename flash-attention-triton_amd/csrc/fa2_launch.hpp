@@ -12,9 +12,8 @@
 namespace fa2 {
 
 // The fast kernels need a head dimension that is a multiple of 8 (whole 16-byte chunks), 16-byte aligned
-// rows and row offsets inside a tile that fit 32 bits.  A head dimension below the table row's padded one
+// rows and row offsets inside a tile that fit 32 bits (direct_stride_ok).  A head dimension below the table row's padded one
 // runs the padded variant of the kernel.
-inline bool direct_stride_ok(const Tensor4 &t) { return t.stride_seq < (int64_t(1) << 24); }
 inline bool direct_headdim(int dp, int headdim) {
   return headdim % 8 == 0 && headdim <= dp && (dp == 32 || dp == 64 || dp == 96 || dp == 128);
 }
@@ -81,8 +80,7 @@ inline int fwd_key_groups(int dp, const FwdParams &p) {
   return fwd_direct_ok(dp, p) ? key_groups(dp, (int64_t)p.batch * p.nheads, p.seqlen_q, false) : 1;
 }
 inline bool dq_direct_ok(int dp, const BwdParams &p) {
-  return p.vec && direct_headdim_wide(dp, p.headdim) && (dp > 96 || direct_stride_ok(p.q)) && direct_stride_ok(p.k) &&
-         direct_stride_ok(p.v);
+  return p.vec && direct_headdim_wide(dp, p.headdim) && direct_stride_ok(p.k) && direct_stride_ok(p.v);
 }
 inline int dq_key_groups(int dp, const BwdParams &p) {
   return dq_direct_ok(dp, p) ? key_groups(dp, (int64_t)p.batch * p.nheads, p.seqlen_q, true) : 1;

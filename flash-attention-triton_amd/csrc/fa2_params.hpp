@@ -18,6 +18,8 @@ struct Tensor4 {
   void *ptr;
   int64_t stride_batch, stride_head, stride_seq;
 };
+// Row offsets inside a 64-row tile of the tensor fit 32 bits.
+constexpr bool direct_stride_ok(const Tensor4 &t) { return t.stride_seq < (int64_t(1) << 24); }
 
 // Every MFMA kernel runs 4 waves per workgroup, each wave owning 32 rows of the operand that stays
 // in registers: 128 query rows (forward, dQ) or 128 key rows (dK/dV) per workgroup.

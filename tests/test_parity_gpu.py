@@ -9,6 +9,7 @@ run beside these).  Deterministic mode: bit-identical across reruns.
 
 from __future__ import annotations
 
+import ctypes
 import math
 
 import pytest
@@ -634,6 +635,40 @@ def test_rows_far_apart(fa, rows_apart):
         results.append([out, *torch.autograd.grad(out, leaves, d_o)])
     for got, want in zip(*results):
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("rows_apart", [(1 << 24) - 8, 1 << 24, (1 << 25) + 8])
+@pytest.mark.parametrize("heads,n,d", [(2, 70, 64), (600, 130, 64), (600, 63, 32), (600, 130, 72), (2, 130, 96), (2, 70, 128)])
+def test_dq_of_query_rows_far_apart(fa2_module, capi, heads, n, d, rows_apart):
+    """dQ and delta through the C ABI with only q's rows at the limit of 32-bit offsets and beyond it: the bits of a
+    contiguous q, so the same kernels."""
+    lib = capi.load()
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    q, k, v, d_o = (torch.randn(1, heads, n, d, generator=gen, device="cuda").bfloat16() for _ in range(4))
+    far = torch.empty((n - 1) * rows_apart + heads * d, dtype=q.dtype, device="cuda").as_strided(
+        q.shape, (heads * d, d, rows_apart, 1))
+    far.copy_(q)
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def arg(t):
+        return capi.Tensor(t.data_ptr(), *fa2_module._strides3(t))
+
+    o, lse = torch.empty_like(q), torch.empty((1, heads, 256), device="cuda")
+    sizes = (1, heads, n, n, d, 256, 0.11, capi.FA2_DTYPE_BF16)
+    fwd = capi.FwdArgs(arg(q), arg(k), arg(v), arg(o), lse.data_ptr(), *sizes, capi.FA2_CONFIG_AUTO)
+    capi.check(lib.fa2_fwd_packed(ctypes.byref(fwd), stream), "fa2_fwd_packed")
+    results = []
+    for queries in (far, q):
+        delta, (dq, dk, dv) = torch.empty_like(lse), (torch.empty_like(t) for t in (q, k, v))
+        bwd = capi.BwdArgs(arg(queries), arg(k), arg(v), arg(o), arg(d_o), arg(dq), arg(dk), arg(dv), lse.data_ptr(),
+                           delta.data_ptr(), None, *sizes, 0, capi.FA2_CONFIG_AUTO)
+        capi.check(lib.fa2_bwd_packed(ctypes.byref(bwd), stream), "fa2_bwd_packed")
+        torch.cuda.synchronize()
+        results.append((dq, delta, dk, dv))
+    (dq, delta, dk, dv), want = results
+    assert torch.equal(dq, want[0]) and torch.equal(delta, want[1])
+    _assert_close("dk", dk, want[2])
+    _assert_close("dv", dv, want[3])
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
