@@ -314,7 +314,8 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
   // 32-key blocks of this wave: with two key groups those in its group's half of the tiles.  The wave's
   // i-th block is key block block_at(i) of the sequence.
   const int n_below = min((kv_end + BLK - 1) / BLK, q0w / BLK + 1);
-  const int n_mine = KG == 1 ? n_below : (n_below - kg + 1) / 2;
+  // (none for a wave without query rows, which only takes part in the loads and barriers)
+  const int n_mine = q0w >= p.seqlen_q ? 0 : KG == 1 ? n_below : (n_below - kg + 1) / 2;
   auto block_at = [&](int i) { return KG == 1 ? i : 2 * i + kg; };
   const int n_full = min(q0w + 1, seqlen_k) / BLK;                   // leading blocks without mask
   const int n_inside = seqlen_k / BKV;
@@ -335,11 +336,15 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
   // K_0, the workgroup's Q rows, V_0 and K_1 are loaded here; after that tile t brings in K_{t+2} and V_{t+1}.  The
   // Q rows travel as in the forward, like a K tile into the stages nothing else uses yet (rows 0..63 in the third K
   // stage and 64..127 in the second V stage, or all 64 in the latter), because fragment loads straight into
-  // registers touch 32 rows each and keep the address path busy.  Rows beyond the sequence come from its last row:
-  // their results are not stored.  Forward and backward, bf16: 256x16x512 D=64 1205 -> 1176 us; fp32
-  // 32x20x1024 D=96 1161 -> 1144; long sequences alike.  From 128 columns on they are loaded into registers as dO is:
-  // none is left for this order (scratch memory per lane: 8 bytes at 128, 212 at 256; 1x8x4096 D=128 gained 0.8 %).
-  constexpr bool Q_STAGED = DP <= 96;
+  // registers touch 32 rows each and keep the address path busy.  Rows beyond the sequence come from its last row, and
+  // where the tile has no more than 64 rows the second stage is left as it is: their results are not stored.  Forward and
+  // backward, bf16: 256x16x512 D=64 1205 -> 1176 us; fp32 32x20x1024 D=96 1161 -> 1140; long sequences alike.
+  // Tiles without rows for every wave need the two other measures to stay as fast as with loads into registers, dQ in us,
+  // registers / all 128 rows staged / so: 2048x64 D=64 18.0 / 18.8 / 18.1, 4096x16 D=64 21.3 / 22.8 / 20.7, 2048x16 D=96
+  // 17.0 / 18.6 / 17.0.  At 32 columns a row is four chunks and the second barrier costs what the loads gain: 2048x64
+  // 10.3 / 10.7 / 9.8 (into registers), 300x777 35.1 / 35.8 / 35.1.  From 128 columns on no registers are left for this
+  // order (scratch memory per lane: 8 bytes at 128, 212 at 256; 1x8x4096 D=128 gained 0.8 %).
+  constexpr bool Q_STAGED = DP > 32 && DP <= 96;
   constexpr int Q_HI = L::V_BASE + L::TILE_ELEMS;
   constexpr int Q_LO = KG == 1 ? L::K_BASE + 2 * L::TILE_ELEMS : Q_HI;
   const Loader qload(Q + (int64_t)q0 * p.q.stride_seq, p.q.stride_seq, hdim / 8);
@@ -352,7 +357,7 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
     if (q_near && q_rows >= row0 + BKV) qload.issue(row0, dst); else qload.issue_clamped(row0, q_rows, dst);
   };
   if (Q_STAGED) issue_q(0, lds_base + 2u * Q_LO);
-  if (Q_STAGED && KG == 1) issue_q(BKV, lds_base + 2u * Q_HI);
+  if (Q_STAGED && KG == 1 && q_rows > BKV) issue_q(BKV, lds_base + 2u * Q_HI);
   issue_v(0);
   if (n_tiles > 1) issue_k(1);
 

@@ -671,6 +671,23 @@ def test_dq_of_query_rows_far_apart(fa2_module, capi, heads, n, d, rows_apart):
     _assert_close("dv", dv, want[3])
 
 
+@pytest.mark.parametrize("heads", [2, 300], ids=["few", "many"])
+@pytest.mark.parametrize("d", [32, 48, 64, 96, 128, 224])
+@pytest.mark.parametrize("nq,nk", [(1, 1), (16, 300), (32, 32), (33, 64), (64, 500), (65, 65), (96, 20), (129, 129), (161, 400), (193, 100)])
+def test_query_tiles_without_rows_for_every_wave(fa, nq, nk, d, heads):
+    """Lengths whose last query tile leaves one to three of the four waves without rows: those multiply nothing and
+    their stage of Q rows may not be loaded."""
+    gen = torch.Generator(device="cuda").manual_seed(nq + d)
+    q, d_o = (torch.randn(1, heads, nq, d, generator=gen, device="cuda").bfloat16() for _ in range(2))
+    k, v = (torch.randn(1, heads, nk, d, generator=gen, device="cuda").bfloat16() for _ in range(2))
+    leaves = [t.clone().requires_grad_(True) for t in (q, k, v)]
+    grads = torch.autograd.grad(fa.flash_attention_v2(*leaves), leaves, d_o)
+    _, *want = _gpu_fp32_oracle(*(t[:, heads - 1 :] for t in (q, k, v, d_o)), None)
+    for name, g, w in zip(("dq", "dk", "dv"), grads, want):
+        assert torch.isfinite(g).all(), name
+        _assert_close(name, g[:, heads - 1 :].reshape(w.shape), w)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
 def test_strided_views_made_in_inference_mode(fa, dtype):
     """k and v as transposed views of tensors made under torch.inference_mode, which autograd cannot save, beside
