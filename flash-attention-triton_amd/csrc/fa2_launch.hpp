@@ -100,6 +100,10 @@ inline bool dkdv_direct_ok(int dp, const BwdParams &p) {
 //   64 columns        1.56 (4 x 4096), 1.31 (64 x 512), 1.13 (4 x 16384) while the other kernel's workgroups
 //                     are all resident (512); 1.16 (256 x 512), 1.09 (256 x 1024), 1.06 (64 x 2048) while
 //                     they are short or few; 0.97 (256 x 2048), 0.93 (64 x 4096) beyond
+//   48 columns        (heads of 40 and 48 in rows of 64; the other kernel multiplies all 64) 1.78 (4 x 4096), 1.19
+//                     (4 x 16384) while that is resident; 1.04-1.06 to 1024 tokens (4096 x 640, 2048 x 1024); beyond them
+//                     1.02-1.12 up to 2.75 x 2^21 rows times workgroups (96 x 2048, 20 x 5000, 80 x 3000), 0.99 at 3 x 2^21
+//                     (48 x 4096, 12 x 8192), 0.95-1.03 above (32 x 8192, 16 x 8192).  40 columns within 3 % of that
 //   32 columns        1.72 (4 x 4096), 1.28 (16 x 4096), 1.03 (1024 x 512); 0.96 (256 x 1024), 0.92 beyond;
 //                     of 128 tokens and fewer 1.05 to 1.3, but 0.92-1.0 at 640 to 768 workgroups (8 us kernels)
 inline bool dkdv_pair_ok(int dp, const BwdParams &p) {
@@ -112,6 +116,7 @@ inline bool dkdv_pair_ok(int dp, const BwdParams &p) {
   if (dp > 128 || dp == 96) return true;
   const int64_t wgs = (int64_t)((p.seqlen_k + kDkvBlockKV - 1) / kDkvBlockKV) * p.batch * p.nheads;
   if (dp == 128) return wgs < 2 * kCUs || p.seqlen_q <= 4096;
+  if (direct_columns(dp, p.headdim) == 48) return wgs <= 2 * kCUs || p.seqlen_q <= 1024 || wgs * p.seqlen_q < 3 << 21;
   return wgs <= 2 * kCUs || p.seqlen_q <= 512 || (dp == 64 && wgs * p.seqlen_q <= (1 << 21));
 }
 // Key rows per workgroup of the dK/dV kernel that launch_dkdv picks (p.n_tiles follows from it).

@@ -429,6 +429,16 @@ def test_two_key_groups_only_where_they_measured_faster(capi, heads, n, d, fwd, 
     assert (info["fwd"]["key_groups"], info["dq"]["key_groups"]) == (fwd, dq)
 
 
+@pytest.mark.parametrize("heads,n,d,form", [
+    (4, 16384, 48, "paired"), (4096, 640, 48, "paired"), (2048, 1024, 48, "paired"), (2048, 1025, 48, "direct"),
+    (80, 3000, 48, "paired"), (80, 3000, 40, "paired"), (48, 4096, 48, "direct"), (32, 8192, 40, "direct"),
+    (256, 1024, 64, "paired"), (80, 3000, 64, "direct"), (80, 3000, 56, "direct"), (2048, 640, 64, "direct"),
+    (80, 3000, 32, "direct")])
+def test_paired_dkdv_kernel_only_where_it_measured_faster(capi, heads, n, d, form):
+    """The dK/dV kernel on both sides of the lines of the rows of 64 columns, whose 48-column form has its own."""
+    assert capi.launch_info(1, heads, n, n, d)["dkdv"]["form"] == form
+
+
 def test_traffic_stamp_ignores_comments_and_follows_code(tmp_path, monkeypatch):
     """bench.py drops the measured HBM traffic when the kernel sources have changed since the
     counter run.  The stamp it compares must not move when comments or layout change (nobody should
