@@ -39,19 +39,26 @@ inline int direct_columns(int dp, int headdim) {
 // Time of one group over two, bf16, (batch, head) pairs x tokens, forward / dQ, by workgroups of 128 rows:
 //   to 128      0.94-1.00 / 0.80-1.00 (64 tokens: half the workgroups would have no rows); from 65 tokens on
 //               1.04-1.2 / 0.99-1.2 (but dQ at 256 columns 0.95 at 65, 1.10 at 100), 1.3-1.7 / 1.25-1.65 beyond
-//   to 256      32 columns 1.20 / 1.12 (128 x 256); 64 columns 1.15 / 1.00 (128 x 256), 1.13 / 0.94 (77 x 333);
-//               96 columns 1.11 / 1.06 (128 x 256), 1.09 / 0.99 (59 x 333), 0.94 / 1.02 (77 x 384), 1.08 / 1.15 (58 x 512);
+//   to 256      32 columns 1.20 / 1.12 (128 x 256); 64 columns 1.15 / 1.10 (128 x 256), 1.13 (77 x 333);
+//               96 columns 1.11 / 1.12 (128 x 256), 1.09 / 1.01 (59 x 333), 0.94 / 0.96 (77 x 384), 1.08 / 1.15 (58 x 512);
 //               128 columns 1.06 / 0.98 (128 x 256), 0.96 / 0.92 (116 x 256), 1.16 / 1.00 (72 x 384), 0.92 / 0.97
 //               (59 x 384), 0.96 / 0.98 (39 x 512), 0.92 / 1.01 (51 x 512), 0.91 (47 x 640), 1.05 / 1.07 (29 x 1024);
 //               192 and 256 columns (one workgroup per CU either way) 1.02 / 1.02 and 1.08 / 0.99 (32 x 1024),
 //               0.94 / 0.97 and 0.94 / 0.88 (29 x 1024), 1.18 / 1.21 and 1.25 / 1.14 (14 x 2048)
-//   to 384      32 columns 1.11 / 1.10 (from 512 tokens); 64 columns 1.09 / 1.01 (96 x 512), 0.92 / 0.97 (75 x 512),
-//               1.07 / 1.05 (43 x 1024); 96 columns 1.10 / 1.06 (24 x 2048), 0.96 / 1.00 at 1024 tokens;
+//   to 384      32 columns 1.11 / 1.10 (from 512 tokens); 64 columns 1.09 / 1.08 (96 x 512), 0.92 / 0.95 (75 x 512),
+//               1.07 / 1.13 (43 x 1024); 96 columns 1.10 / 1.09 (24 x 2048), 0.96 / 0.95-1.08 at 1024 tokens;
 //               128 columns 1.14 / 1.04 (12 x 4096), 1.08 / 0.94 (24 x 2048)
-//   to 512      32 columns 1.08 / 1.03 (from 1024 tokens); 64 columns 1.04 / 1.01 (16 x 4096), 0.98 / 0.95 (2048 tokens);
+//   to 512      32 columns 1.08 / 1.03 (from 1024 tokens); 64 columns 1.04 / 1.05 (16 x 4096), 0.98 / 0.99-1.02 (2048 tokens);
 //               128 columns 0.98 / 0.94 (16 x 4096)
 //   beyond      0.75-0.98
-inline int key_groups(int dp, int64_t heads, int seqlen_q, bool dq) {
+// `cols` are the columns multiplied (direct_columns).  At 160 and 224 the lines of 192 and 256 hold.  Those of 64 and 96
+// hold at 48 and 80 but for dQ with odd heads to 256 workgroups, where fewer columns leave the doubled loads less to cost:
+//   48 columns  1.16 (59 x 333), 1.12 (77 x 333), 1.11 (85 x 257), 1.10 (63 x 500): as with even heads
+//   64 columns  1.16 (59 x 333), 1.10 (65 x 300), 1.11 (67 x 384), 1.04 (51 x 512) to 208 workgroups; above, 1.07 (77 x 333)
+//               and 1.09 (79 x 300), but 0.95 (83 x 384) and 0.89 (63 x 500)
+//   80 columns  1.10 (59 x 333) to 192 workgroups; above, 1.09 (65 x 300), 1.05 (67 x 384), but 0.97 (77 x 333, 83 x 384)
+//   96 columns  1.01 (59 x 333); above 192, 1.06 (65 x 300), 0.98 (67 x 384), 0.90-0.96 beyond
+inline int key_groups(int dp, int cols, int64_t heads, int seqlen_q, bool dq) {
   const int64_t wgs = heads * ((seqlen_q + kFwdBlockQ - 1) / kFwdBlockQ);
   static_assert(kFwdBlockQ == kDqBlockQ, "the same grid for both kernels");
   const bool odd = heads % 2 != 0;
@@ -64,7 +71,7 @@ inline int key_groups(int dp, int64_t heads, int seqlen_q, bool dq) {
     else if (dp == 128)
       from = (odd && wgs > kCUs * 9 / 16) || (heads % 8 != 0 && wgs > kCUs * 13 / 16) ? 1024 : dq ? 384 : 256;
     else
-      from = odd && ((dp == 96 && (dq || wgs > kCUs * 3 / 4)) || (dp == 64 && dq)) ? 512 : 256;
+      from = odd && ((dp == 96 && ((dq && cols == 96) || wgs > kCUs * 3 / 4)) || (cols == 64 && dq && wgs > kCUs * 13 / 16)) ? 512 : 256;
   } else if (wgs <= 3 * kCUs / 2 && dp <= 128) {
     from = dp == 128 ? 4096 : dp == 96 ? 2048 : dp == 64 && odd ? 1024 : 512;
   } else if (wgs <= 2 * kCUs && dp <= 64) {
@@ -77,13 +84,13 @@ inline bool fwd_direct_ok(int dp, const FwdParams &p) {
          direct_stride_ok(p.v);
 }
 inline int fwd_key_groups(int dp, const FwdParams &p) {
-  return fwd_direct_ok(dp, p) ? key_groups(dp, (int64_t)p.batch * p.nheads, p.seqlen_q, false) : 1;
+  return fwd_direct_ok(dp, p) ? key_groups(dp, direct_columns(dp, p.headdim), (int64_t)p.batch * p.nheads, p.seqlen_q, false) : 1;
 }
 inline bool dq_direct_ok(int dp, const BwdParams &p) {
   return p.vec && direct_headdim_wide(dp, p.headdim) && direct_stride_ok(p.k) && direct_stride_ok(p.v);
 }
 inline int dq_key_groups(int dp, const BwdParams &p) {
-  return dq_direct_ok(dp, p) ? key_groups(dp, (int64_t)p.batch * p.nheads, p.seqlen_q, true) : 1;
+  return dq_direct_ok(dp, p) ? key_groups(dp, direct_columns(dp, p.headdim), (int64_t)p.batch * p.nheads, p.seqlen_q, true) : 1;
 }
 inline bool dkdv_direct_ok(int dp, const BwdParams &p) {
   return p.vec && direct_headdim(dp, p.headdim) && dp != 96 && direct_stride_ok(p.q) && direct_stride_ok(p.d_o) &&

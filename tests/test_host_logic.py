@@ -429,6 +429,16 @@ def test_two_key_groups_only_where_they_measured_faster(capi, heads, n, d, fwd, 
     assert (info["fwd"]["key_groups"], info["dq"]["key_groups"]) == (fwd, dq)
 
 
+@pytest.mark.parametrize("heads,n,d,fwd,dq", [
+    (59, 333, 48, 2, 2), (63, 500, 48, 2, 2), (65, 255, 40, 1, 1), (59, 333, 64, 2, 2), (67, 384, 64, 2, 2),
+    (70, 300, 64, 2, 2), (63, 500, 64, 2, 1), (63, 500, 56, 2, 1), (59, 333, 80, 2, 2), (61, 333, 72, 2, 2),
+    (67, 384, 80, 1, 1), (61, 333, 96, 2, 1), (61, 333, 88, 2, 1), (17, 1024, 160, 2, 2), (29, 1024, 224, 1, 1)])
+def test_key_groups_go_by_the_columns_multiplied(capi, heads, n, d, fwd, dq):
+    """Odd numbers of heads at the column counts between the table's rows."""
+    info = capi.launch_info(1, heads, n, n, d)
+    assert (info["fwd"]["key_groups"], info["dq"]["key_groups"]) == (fwd, dq)
+
+
 @pytest.mark.parametrize("heads,n,d,form", [
     (4, 16384, 48, "paired"), (4096, 640, 48, "paired"), (2048, 1024, 48, "paired"), (2048, 1025, 48, "direct"),
     (80, 3000, 48, "paired"), (80, 3000, 40, "paired"), (48, 4096, 48, "direct"), (32, 8192, 40, "direct"),
