@@ -166,12 +166,20 @@ inline ResidentWalk resident_walk(int group, int64_t heads) {
 // bf16 != 0 selects the bf16 kernels, otherwise fp16.
 // folded: the LDS-direct forward takes its exponents straight from the score MFMAs (Q fragments
 // multiplied by scale * log2(e) and rounded once); the generic forward ignores it.
-// F32: the variants that store the output in fp32 (p.o_f32), compiled in objects of their own.
+// F32: the variants that store the output in fp32 (p.o_f32), each a specialisation defined in an object of its own.
 template <bool F32>
 void launch_fwd(bool bf16, int dp, bool folded, const FwdParams &p, dim3 grid, hipStream_t s);
-// The 192- and 256-column LDS-direct forward kernels (dp is 192 or 256), instantiated apart from the others.
+template <>
+void launch_fwd<false>(bool bf16, int dp, bool folded, const FwdParams &p, dim3 grid, hipStream_t s);
+template <>
+void launch_fwd<true>(bool bf16, int dp, bool folded, const FwdParams &p, dim3 grid, hipStream_t s);
+// The LDS-direct forward kernels of 160 to 256 columns (dp is 192 or 256), instantiated apart from the others.
 template <bool F32>
 void launch_fwd_direct_wide(bool bf16, int dp, int key_groups, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s);
+template <>
+void launch_fwd_direct_wide<false>(bool bf16, int dp, int key_groups, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s);
+template <>
+void launch_fwd_direct_wide<true>(bool bf16, int dp, int key_groups, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s);
 // Rounds fp32 arrays to fp16 (fa2_cast.hpp); one launch for all of them.
 void launch_cast(const CastParams &p, dim3 grid, hipStream_t s);
 void launch_preprocess(bool bf16, const PreParams &p, dim3 grid, hipStream_t s);
