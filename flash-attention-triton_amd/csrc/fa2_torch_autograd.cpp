@@ -69,9 +69,10 @@ std::array<at::Tensor, N> rounded_to_half(const std::array<at::Tensor, N> &in) {
   for (size_t i = 0; i < N; i++) {
     const at::Tensor &t = in[i];
     if (t.numel() > 0 && t.is_non_overlapping_and_dense() && !t.is_neg() && !t._is_zerotensor() &&
-        reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0) {
+        reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0) {
       out[i] = at::empty_like(t, t.options().dtype(at::kHalf));
-      jobs[count++] = fa2_cast{t.data_ptr<float>(), out[i].data_ptr(), t.numel()};
+      // (A const pointer: asked for a writable one, a lazily cloned tensor would copy itself first.)
+      jobs[count++] = fa2_cast{t.const_data_ptr<float>(), out[i].data_ptr(), t.numel()};
     } else {
       out[i] = t.to(at::kHalf);
     }

@@ -63,6 +63,17 @@ def test_output_may_change_before_the_backward(fa2_module):
         assert torch.equal(g, w)
 
 
+def test_lazily_cloned_inputs_stay_shared(fa2_module):
+    """Rounding only reads: a copy-on-write clone is not copied for it."""
+    tensors = _inputs((1, 2, 130, 64), "bhnd")
+    clones = [torch._lazy_clone(t) for t in tensors[:3]]
+    assert all(torch._C._is_cow_tensor(t) for t in clones)
+    with torch.no_grad():
+        got = fa2_module.flash_attention_v2(*clones)
+    assert all(torch._C._is_cow_tensor(t) for t in clones)
+    assert torch.equal(got, _pass(fa2_module, *tensors)[0])
+
+
 @pytest.mark.parametrize("sizes", [(1,), (4096,), (4095, 4097), (5, 8192, 12289), (4096, 3, 20000)], ids=str)
 def test_cast_rounds_as_torch_does(capi, sizes):
     lib = capi.load()
