@@ -164,11 +164,31 @@ int check_launchable_grids() {
   return bad;
 }
 
+// The columns a row's kernels multiply: enough for every head dimension, in one of the counts printed here.
+int check_columns() {
+  int bad = 0, below = 0;
+  for (int dp : {32, 64, 96, 128, 192, 256}) {
+    std::set<int> counts;
+    for (int d = 8; d <= dp; d += 8) {
+      const int cols = fa2::direct_columns(dp, d);
+      if (cols < d || cols > dp || cols % 16) bad++;
+      if (d > below) counts.insert(cols);  // (smaller ones come to this row only by its id)
+      else if (cols != fa2::direct_columns(dp, below + 8)) bad++;
+    }
+    printf("columns %d:", dp);
+    for (int c : counts) printf(" %d", c);
+    printf("\n");
+    below = dp;
+  }
+  return bad;
+}
+
 int main() {
   int bad = check_mapping();
   bad += check_balanced_index();
   bad += check_resident_walk();
   bad += check_launchable_grids();
+  bad += check_columns();
   bad += check<32>();
   bad += check<64>();
   bad += check<96>();

@@ -19,10 +19,14 @@ REGS_PER_LANE = 512  # VGPRs + accumulation registers per SIMD lane, shared by t
 
 # No LDS-direct kernel may spill to scratch memory.  (The forward at 256 columns is instantiated in its padded form
 # only: with the column count a compile-time 256 the compiler spilled about forty registers.)  Spills into
-# accumulation registers, which cost a copy each way but no memory access: (kernel, columns, padded) -> how many.
-KNOWN_SPILLS: dict = {("bwd_dkdv_pair_kernel", 256, False): 40, ("bwd_dkdv_pair_kernel", 256, True): 48}
-# Columns the paired dK/dV kernel exists at.
-PAIR_COLUMNS = (32, 64, 96, 128, 192, 256)
+# accumulation registers, which cost a copy each way but no memory access: (kernel, row, columns, padded) -> how many.
+KNOWN_SPILLS: dict = {("bwd_dkdv_pair_kernel", 256, 256, False): 40, ("bwd_dkdv_pair_kernel", 256, 256, True): 48,
+                      ("bwd_dkdv_pair_kernel", 256, 224, False): 4}
+# Table row -> columns its forward, dQ and paired dK/dV kernels multiply (direct_columns in fa2_launch.hpp, which
+# test_lds_layout.py holds to the same numbers).
+COLUMNS = {32: (32,), 64: (48, 64), 96: (80, 96), 128: (128,), 192: (160, 192), 256: (224, 256)}
+# Rows the paired dK/dV kernel exists at.
+PAIR_COLUMNS = tuple(COLUMNS)
 
 
 def _kernel_records(library: pathlib.Path, tmp: pathlib.Path) -> list[dict]:
@@ -54,19 +58,27 @@ def _kernel_records(library: pathlib.Path, tmp: pathlib.Path) -> list[dict]:
     return records
 
 
+# Template arguments behind <T, DP: place of PAD among the flags, and of COLS among the numbers (None: DP).
+#   fwd_direct<BKV, PAD, PRE, KG, COLS, F32>; bwd_dq_direct<BKV, FUSE_DELTA, PAD, KG, COLS>; bwd_dkdv_pair<PAD, COLS>;
+#   bwd_dkdv_direct<BQ, PAD, ATOMIC>
+TEMPLATES = {"fwd_direct_kernel": (0, 2), "bwd_dq_direct_kernel": (1, 2), "bwd_dkdv_pair_kernel": (0, 0),
+             "bwd_dkdv_direct_kernel": (0, None)}
+
+
 def _parse(name: str):
-    """(kernel, padded head dimension, padded variant?) from a mangled fa2 kernel name."""
+    """(kernel, padded head dimension of the row, columns multiplied, padded variant?, atomic dQ?) from a mangled
+    fa2 kernel name."""
     m = re.match(r"_ZN3fa2\d+(\w+?)I(?:DF16b|DF16_)Li(\d+)E((?:Li\d+E|Lb[01]E)*)", name)
     if not m:
         return None
     kernel, dp, rest = m.group(1), int(m.group(2)), m.group(3)
     flags = re.findall(r"Lb([01])E", rest)
-    # fwd_direct<T, DP, BKV, PAD>; bwd_dq_direct<T, DP, BKV, FUSE_DELTA, PAD>; bwd_dkdv_direct<T, DP, BQ, PAD, ATOMIC>;
-    # bwd_dkdv_pair<T, DP, PAD>
-    pad = {"fwd_direct_kernel": lambda f: f[0], "bwd_dq_direct_kernel": lambda f: f[1],
-           "bwd_dkdv_direct_kernel": lambda f: f[0], "bwd_dkdv_pair_kernel": lambda f: f[0]}.get(kernel, lambda f: "0")(flags) == "1" if flags else False
-    atomic = kernel == "bwd_dkdv_direct_kernel" and len(flags) > 1 and flags[1] == "1"
-    return kernel, dp, pad, atomic
+    numbers = [int(n) for n in re.findall(r"Li(\d+)E", rest)]
+    if kernel not in TEMPLATES:
+        return kernel, dp, dp, False, False
+    pad, cols = TEMPLATES[kernel]
+    atomic = kernel == "bwd_dkdv_direct_kernel" and flags[1] == "1"
+    return kernel, dp, dp if cols is None else numbers[cols], flags[pad] == "1", atomic
 
 
 @pytest.fixture(scope="module")
@@ -95,16 +107,17 @@ def test_lds_direct_kernels_do_not_spill(records):
         parsed = _parse(r["name"])
         if not parsed or not parsed[0].endswith(("_direct_kernel", "_pair_kernel")):
             continue
-        kernel, dp, pad, _ = parsed
-        seen.add((kernel, dp))
+        kernel, dp, cols, pad, _ = parsed
+        seen.add((kernel, dp, cols, pad))
         scratch = int(r["private_segment_fixed_size"])
         assert scratch == 0, f"{r['name']}: {scratch} bytes of scratch per lane"
-        allowed = KNOWN_SPILLS.get((kernel, dp, pad), 0)
+        allowed = KNOWN_SPILLS.get((kernel, dp, cols, pad), 0)
         assert int(r["vgpr_spill_count"]) <= allowed, f"{r['name']}: {r['vgpr_spill_count']} vector registers spilled"
-    for dp in (32, 64, 96, 128, 192, 256):
-        assert {("fwd_direct_kernel", dp), ("bwd_dq_direct_kernel", dp)} <= seen
-    assert {dp for kernel, dp in seen if kernel == "bwd_dkdv_direct_kernel"} == {32, 64, 128}
-    assert {("bwd_dkdv_pair_kernel", dp) for dp in PAIR_COLUMNS} <= seen
+    built = {k: {key[1:] for key in seen if key[0] == k} for k in TEMPLATES}
+    every = {(dp, cols, pad) for dp, widths in COLUMNS.items() for cols in widths for pad in (False, True)}
+    assert built["bwd_dq_direct_kernel"] == built["bwd_dkdv_pair_kernel"] == every
+    assert built["fwd_direct_kernel"] == every - {(256, 256, False)}  # above: in its padded form only
+    assert built["bwd_dkdv_direct_kernel"] == {(dp, dp, pad) for dp in (32, 64, 128) for pad in (False, True)}
 
 
 def test_fp32_output_is_a_variant_of_the_forward(records):
@@ -114,7 +127,8 @@ def test_fp32_output_is_a_variant_of_the_forward(records):
         m = re.match(r"(_ZN3fa2\d+fwd_\w*kernelI.*)Lb([01])EEEvNS_9FwdParamsE", r["name"])
         if m:
             forms.setdefault(m.group(1), {})[m.group(2)] = r
-    assert sum("fwd_direct_kernel" in stem for stem in forms) >= 2 * 2 * len(PAIR_COLUMNS)
+    direct = [stem for stem in forms if "fwd_direct_kernel" in stem]
+    assert {_parse(stem)[1:3] for stem in direct} == {(dp, cols) for dp, widths in COLUMNS.items() for cols in widths}
     assert any("10fwd_kernel" in stem for stem in forms)
     for stem, both in forms.items():
         assert set(both) == {"0", "1"}, stem
@@ -135,9 +149,9 @@ def test_registers_and_lds_leave_room_for_the_tables_workgroups(records):
     checked = 0
     for r in records:
         parsed = _parse(r["name"])
-        if not parsed or parsed[0] not in (*column, "bwd_dkdv_pair_kernel") or parsed[3]:
+        if not parsed or parsed[0] not in (*column, "bwd_dkdv_pair_kernel") or parsed[4]:
             continue
-        kernel, dp, _, _ = parsed
+        kernel, dp, *_ = parsed
         if kernel == "bwd_dkdv_direct_kernel" and dp > 128:
             continue
         regs = (int(r["vgpr_count"]) + 7) // 8 * 8  # the count includes the accumulation registers

@@ -93,3 +93,39 @@ def test_cast_rounds_as_torch_does(capi, sizes):
         assert torch.equal(d[:-8], s.half()) and (d[-8:] == 7).all()
     assert lib.fa2_cast_f32_to_f16(jobs, 4, ctypes.c_void_p(0)) != 0
     assert lib.fa2_cast_f32_to_f16(jobs, 0, ctypes.c_void_p(0)) != 0
+
+
+@pytest.mark.parametrize("shape", [(2, 3, 333, 64), (1, 8, 130, 128), (1, 2, 200, 224), (1, 3, 77, 33)], ids=lambda s: "x".join(map(str, s)))
+def test_f32_output_at_any_float_address(fa2_module, capi, shape):
+    """fa2_fwd_packed_f32_out where o_f32 is 16-byte aligned and where it is not (the generic kernel), with o and without
+    it.  The values are those of o, and the two kernels' differ by no more than a rounding or two of fp16."""
+    lib = capi.load()
+    b, h, n, d = shape
+    q, k, v = (t.half() for t in _inputs(shape, "bhnd")[:3])
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def arg(t):
+        return capi.Tensor(t.data_ptr(), *fa2_module._strides3(t)) if t is not None else capi.Tensor(None, 0, 0, 0)
+
+    def forward(floats_off, want_o):
+        o = torch.empty_like(q) if want_o else None
+        lse = torch.empty((b, h, 512), device="cuda")
+        buf = torch.full((q.numel() + 8,), 7.0, device="cuda")
+        args = capi.FwdArgs(arg(q), arg(k), arg(v), arg(o), lse.data_ptr(), b, h, n, n, d, 512, d**-0.5,
+                            capi.FA2_DTYPE_F16, capi.FA2_CONFIG_AUTO)
+        capi.check(lib.fa2_fwd_packed_f32_out(ctypes.byref(args), buf.data_ptr() + 4 * floats_off, stream), "fa2_fwd_packed_f32_out")
+        torch.cuda.synchronize()
+        out = buf[floats_off : floats_off + q.numel()].view(shape)
+        assert (buf[:floats_off] == 7).all() and (buf[floats_off + q.numel() :] == 7).all()
+        return out, o, lse
+
+    aligned, o, lse = forward(0, True)
+    assert torch.equal(aligned, o.float())
+    for off in (0, 1, 2, 4):
+        out, o2, lse2 = forward(off, True)
+        assert torch.equal(out, o2.float())
+        assert torch.equal(out, forward(off, False)[0])
+        # One rounding of P per product differs between the kernels (2^-11 of values of order 1), one of the result.
+        torch.testing.assert_close(out, aligned, atol=2e-3, rtol=2e-3)
+        torch.testing.assert_close(lse2, lse, atol=1e-4, rtol=1e-5)
+    assert lib.fa2_status_string(lib.fa2_fwd_packed_f32_out(None, 16, stream)).decode() == "FA2_ERR_NULL_POINTER"

@@ -180,6 +180,37 @@ def test_backward_entry_points_reject_bad_arguments(capi):
     assert "forward-only" in lib.fa2_last_error_string().decode()
 
 
+def test_fp32_entry_points_reject_bad_arguments(capi):
+    """fa2_fwd_packed_f32_out and fa2_cast_f32_to_f16: every refusal comes before anything is launched."""
+    lib = capi.load()
+
+    def fwd(o_f32, o=16, args=True):
+        t = capi.Tensor(16, 512, 512, 64)
+        a = capi.FwdArgs(t, t, t, capi.Tensor(o, 512, 512, 64), 16, 1, 1, 0, 8, 64, 128, 0.125, capi.FA2_DTYPE_F16,
+                         capi.FA2_CONFIG_AUTO)
+        return lib.fa2_status_string(lib.fa2_fwd_packed_f32_out(ctypes.byref(a) if args else None, o_f32, None)).decode()
+
+    assert fwd(16, args=False) == fwd(None) == "FA2_ERR_NULL_POINTER"
+    assert fwd(18) == "FA2_ERR_BAD_STRIDE"
+    assert fwd(20) == fwd(16, o=None) == "FA2_ERR_BAD_SHAPE"  # seqlen_q is 0; the pointers are fine
+    t = capi.Tensor(16, 512, 512, 64)
+    a = capi.FwdArgs(t, t, t, capi.Tensor(None, 0, 0, 0), 16, 1, 1, 8, 8, 64, 128, 0.125, capi.FA2_DTYPE_F16, capi.FA2_CONFIG_AUTO)
+    assert lib.fa2_status_string(lib.fa2_fwd_packed(ctypes.byref(a), None)).decode() == "FA2_ERR_NULL_POINTER"
+
+    def cast(*jobs, count=None):
+        arrays = (capi.Cast * max(1, len(jobs)))(*(capi.Cast(*j) for j in jobs))
+        n = len(jobs) if count is None else count
+        return lib.fa2_status_string(lib.fa2_cast_f32_to_f16(arrays if jobs else None, n, None)).decode()
+
+    good = (16, 16, 8)
+    assert cast(count=1) == "FA2_ERR_NULL_POINTER"
+    assert cast(good, count=0) == cast(good, count=4) == "FA2_ERR_BAD_SHAPE"
+    assert cast(good, (None, 16, 8)) == cast((16, None, 8)) == "FA2_ERR_NULL_POINTER"
+    assert cast((16, 16, 0)) == cast(good, good, (16, 16, -1)) == "FA2_ERR_BAD_SHAPE"
+    assert cast((24, 16, 8)) == cast((16, 20, 8)) == "FA2_ERR_BAD_STRIDE"
+    assert cast(good, (16, 16, 1 << 60)) == cast(*[(16, 16, 1 << 35)] * 3) == "FA2_ERR_TOO_LARGE"
+
+
 def test_missing_library_fails_loudly(capi, monkeypatch, tmp_path):
     monkeypatch.setattr(capi, "_lib", None)
     monkeypatch.setattr(capi, "LIBRARY_PATH", tmp_path / "libfa2_gfx950.so")

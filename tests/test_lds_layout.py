@@ -10,6 +10,8 @@ import subprocess
 
 import pytest
 
+from tests.test_code_objects import COLUMNS
+
 ROOT = pathlib.Path(__file__).resolve().parent.parent
 HIPCC = pathlib.Path("/opt/rocm/bin/hipcc")
 
@@ -36,3 +38,5 @@ def test_loader_slots_match_fragment_reads_and_reads_are_conflict_free(tmp_path)
     assert len(walk) == 1 and walk[0].endswith("ok"), run.stdout
     grids = [l for l in run.stdout.splitlines() if l.startswith("launchable grids")]
     assert len(grids) == 1 and grids[0].endswith("ok"), run.stdout
+    columns = dict(line.split(": ") for line in run.stdout.splitlines() if line.startswith("columns"))
+    assert {int(k.split()[1]): tuple(map(int, v.split())) for k, v in columns.items()} == COLUMNS, run.stdout
