@@ -283,7 +283,7 @@ def _cpu_baseline(w, workloads, heads: int):
     ``heads`` (batch, head) slices of the same seeded workload, forward + backward."""
     from oracle import naive_attention as oracle
 
-    # A one-GPU box's share of the host is 16 cores whatever os.cpu_count() shows there.
+    # 16 cores are one GPU's share of the host, whatever os.cpu_count() shows.
     threads = min(os.cpu_count() or 1, 16)
     torch.set_num_threads(threads)
     q, k, v, d_o = workloads.make_inputs(w, "cpu", heads=heads)
@@ -396,7 +396,7 @@ def main() -> int:
     args = ap.parse_args()
 
     if args.gpus != 1:
-        print("bench.py measures one GPU: every box of this build has one, and causal attention needs "
+        print("bench.py measures one GPU: causal attention needs "
               "no exchange between GPUs (batch and heads shard with no communication). Use --gpus 1.",
               file=sys.stderr)
         return 2

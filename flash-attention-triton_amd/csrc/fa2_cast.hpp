@@ -1,5 +1,5 @@
 // fp32 arrays rounded to fp16: what q, k and v (in one launch) and dO of an fp32 model pass through in front of the
-// attention kernels.  Memory bound: 6.5 TB/s on 32 x 20 x 1024 x 96 (four tensors in 233 us, 378 MB each; a device copy
+// attention kernels.  Memory bound: 6.7 TB/s on 32 x 20 x 1024 x 96 (four tensors in 226 us, 378 MB each; a device copy
 // reaches 4.9).  Four loads per thread before its first store keep enough in flight; they go past the caches, which
 // the rounded values should have.
 #pragma once

@@ -440,7 +440,7 @@ __device__ __forceinline__ void tile_barrier() { asm volatile("s_barrier" ::: "m
 
 // Zero `elems` halves of LDS (a multiple of 8 per thread step) with the whole workgroup.  The
 // padded kernels do this once before their first tile load: tile loads never touch the slots of
-// columns beyond the head dimension, which the MFMAs read as part of their DP-wide fragments.
+// columns beyond the head dimension, up to the columns multiplied (COLS), which the MFMAs read as part of their fragments.
 template <int NTHREADS>
 __device__ __forceinline__ void zero_lds(short *smem, int elems) {
   const fa2::s16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};

@@ -252,8 +252,8 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_kerne
 
 // ------------------------------------------------------------------------------------------
 // Fast path: 16-byte aligned rows and a head dimension that is a multiple of 8; instantiated for 32, 48, 64,
-// 80, 96, 128, 160, 192, 224 and 256 columns (two workgroups or more per CU up to 128; at 192 and 256 the
-// five tile stages fill the CU's 160 KiB of LDS and the output accumulator moves into accumulation
+// 80, 96, 128, 160, 192, 224 and 256 columns (two workgroups or more per CU up to 128; from 160 on the
+// five tile stages, of 256 halves a row, fill the CU's 160 KiB of LDS and the output accumulator moves into accumulation
 // registers: one workgroup per CU, one wave per SIMD).
 //
 //  * K and V tiles (64 rows) go straight from global memory into swizzled, unpadded LDS
@@ -292,9 +292,8 @@ struct HalfTag {
 };
 
 // COLS: columns multiplied, DP or (direct_columns in fa2_launch.hpp) a step less; DP is then the LDS tiles' alone.  With
-// an odd number of 16-column steps (48, 80) S takes one MFMA per block less than P V, whose last block is half
-// empty.  Forward and
-// backward, bf16, padded to DP before, us: 2x16x4096 D=160 1008 -> 903, 1x8x4096 D=160 314 -> 278, 2x16x4096 D=224
+// an odd number of 16-column steps (48, 80) S takes one MFMA per block less than P V, whose last block is half empty.
+// Forward and backward, bf16, padded to DP before, us: 2x16x4096 D=160 1008 -> 903, 1x8x4096 D=160 314 -> 278, 2x16x4096 D=224
 // 1273 -> 1172, 8x16x2048 D=80 525 -> 500, 32x16x512 D=48 153 -> 145.
 // PAD: the head dimension is a multiple of 8 below COLS; the columns beyond it are zeros in LDS and in
 // the register fragments, and are not stored.

@@ -12,8 +12,7 @@
 namespace fa2 {
 
 // The fast kernels need a head dimension that is a multiple of 8 (whole 16-byte chunks), 16-byte aligned
-// rows and row offsets inside a tile that fit 32 bits (direct_stride_ok).  A head dimension below the table row's padded one
-// runs the padded variant of the kernel.
+// rows and row offsets inside a tile that fit 32 bits (direct_stride_ok).
 inline bool direct_headdim(int dp, int headdim) {
   return headdim % 8 == 0 && headdim <= dp && (dp == 32 || dp == 64 || dp == 96 || dp == 128);
 }
@@ -23,9 +22,12 @@ inline bool direct_headdim_wide(int dp, int headdim) {
   return direct_headdim(dp, headdim) || (headdim % 8 == 0 && headdim <= dp && (dp == 192 || dp == 256));
 }
 // Columns the forward, dQ and paired dK/dV kernels of a row multiply: the head dimension rounded up to a step of 16
-// up to 96 columns and of 32 above (measured in fa2_fwd.hpp).  The row's own number (64, 96, 192, 256) stays the pitch of the LDS tiles.  A
-// head dimension that is such a number needs no zero-filled tiles either: what lies behind a row is multiplied into
-// accumulator rows that are not stored.
+// up to 96 columns and of 32 above (against the row's own number: fa2_fwd.hpp).  The row still gives the LDS tiles, of pitch
+// lds_pitch(dp) (32, 64, 128 or 256).  A head dimension that is one of these counts needs no zero-filled tiles: what lies behind
+// a row is multiplied into accumulator rows that are not stored.  Any other runs the padded variant of the next count.
+// Steps of 16 above 96 columns are not instantiated (each count is 36 to 52 kernels).  What they would save, time at the next
+// count over its own, forward / dQ / paired dK/dV, bf16: 112 columns 1.03 / 1.04 / 1.03 (32 x 4096) to 1.06 / 1.05 / 1.09
+// (256 x 512), 144 columns 1.05 / 1.03 / 1.05, 208 columns 1.05 / 1.04 / 1.04 (32 x 4096); 176 and 240 not measured.
 inline int direct_columns(int dp, int headdim) {
   const int less = dp == 64 || dp == 96 ? dp - 16 : dp > 128 ? dp - 32 : dp;
   return headdim <= less ? less : dp;

@@ -230,6 +230,8 @@ int fa2_fwd_packed(const fa2_fwd_args *args, void *stream);
  * fa2_fwd_packed that writes the output as an fp32 tensor too: o_f32, contiguous (batch, nheads, seqlen_q,
  * headdim), receives the values of o widened, without the pass that a caller with fp32 tensors would run
  * (flash_attention_2.py:339).  args->o.ptr may be NULL where no backward will read o.
+ * o_f32 has to be 4-byte aligned.  Where it is not 16-byte aligned the generic forward runs, as for operands that
+ * are not.
  */
 int fa2_fwd_packed_f32_out(const fa2_fwd_args *args, float *o_f32, void *stream);
 
