@@ -54,12 +54,13 @@ inline int direct_columns(int dp, int headdim) {
 //               128 columns 0.98 / 0.94 (16 x 4096)
 //   beyond      0.75-0.98
 // `cols` are the columns multiplied (direct_columns).  At 160 and 224 the lines of 192 and 256 hold.  Those of 64 and 96
-// hold at 48 and 80 but for dQ with odd heads to 256 workgroups, where fewer columns leave the doubled loads less to cost:
-//   48 columns  1.16 (59 x 333), 1.12 (77 x 333), 1.11 (85 x 257), 1.10 (63 x 500): as with even heads
-//   64 columns  1.16 (59 x 333), 1.10 (65 x 300), 1.11 (67 x 384), 1.04 (51 x 512) to 208 workgroups; above, 1.07 (77 x 333)
-//               and 1.09 (79 x 300), but 0.95 (83 x 384) and 0.89 (63 x 500)
-//   80 columns  1.10 (59 x 333) to 192 workgroups; above, 1.09 (65 x 300), 1.05 (67 x 384), but 0.97 (77 x 333, 83 x 384)
-//   96 columns  1.01 (59 x 333); above 192, 1.06 (65 x 300), 0.98 (67 x 384), 0.90-0.96 beyond
+// hold at 48 and 80 but for dQ with odd heads to 256 workgroups.  Time of the whole backward (delta formed by dQ), dQ with one
+// group over two:
+//   48 columns  1.03 (59 x 333), 1.00 (77 x 333), 1.02 (85 x 257), 1.04 (65 x 300), 1.02 (63 x 500): as with even heads
+//   64 columns  0.98 (59 x 333), 0.98 (77 x 333), 0.97 (65 x 300), 0.98 (83 x 384), 1.00 (67 x 384), 0.99 (63 x 500), although
+//               dQ by itself gains (1.15 at 59 x 333): the dK/dV kernel behind it takes longer by more
+//   80 columns  1.05 (59 x 333), 1.03 (77 x 333), 1.04 (65 x 300), 1.03 (83 x 384), 1.04 (63 x 500): as with even heads
+//   96 columns  1.02 (59 x 333), 1.01 (77 x 333), 1.01 (65 x 300), 1.01 (83 x 384), 1.00 (63 x 500), dQ by itself 0.92-1.06
 inline int key_groups(int dp, int cols, int64_t heads, int seqlen_q, bool dq) {
   const int64_t wgs = heads * ((seqlen_q + kFwdBlockQ - 1) / kFwdBlockQ);
   static_assert(kFwdBlockQ == kDqBlockQ, "the same grid for both kernels");
@@ -73,7 +74,7 @@ inline int key_groups(int dp, int cols, int64_t heads, int seqlen_q, bool dq) {
     else if (dp == 128)
       from = (odd && wgs > kCUs * 9 / 16) || (heads % 8 != 0 && wgs > kCUs * 13 / 16) ? 1024 : dq ? 384 : 256;
     else
-      from = odd && ((dp == 96 && ((dq && cols == 96) || wgs > kCUs * 3 / 4)) || (cols == 64 && dq && wgs > kCUs * 13 / 16)) ? 512 : 256;
+      from = odd && (dq ? cols == 64 || cols == 96 : dp == 96 && wgs > kCUs * 3 / 4) ? 512 : 256;
   } else if (wgs <= 3 * kCUs / 2 && dp <= 128) {
     from = dp == 128 ? 4096 : dp == 96 ? 2048 : dp == 64 && odd ? 1024 : 512;
   } else if (wgs <= 2 * kCUs && dp <= 64) {
