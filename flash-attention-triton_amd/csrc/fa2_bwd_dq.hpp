@@ -350,14 +350,11 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
   const Loader qload(Q + (int64_t)q0 * p.q.stride_seq, p.q.stride_seq, hdim / 8);
   const int q_rows = p.seqlen_q - q0;  // query rows of this tile that exist (>= 1)
   issue_k(0);
-  // Rows too far apart for a lane's 32-bit offset go by the clamped loads, whose addresses are 64-bit: any q row stride
-  // runs this kernel, as it does where the rows go straight into registers.
-  const bool q_near = direct_stride_ok(p.q);
-  auto issue_q = [&](int row0, unsigned dst) {
-    if (q_near && q_rows >= row0 + BKV) qload.issue(row0, dst); else qload.issue_clamped(row0, q_rows, dst);
-  };
-  if (Q_STAGED) issue_q(0, lds_base + 2u * Q_LO);
-  if (Q_STAGED && KG == 1 && q_rows > BKV) issue_q(BKV, lds_base + 2u * Q_HI);
+  // By the clamped loads, whose addresses are 64-bit: q's rows may lie any distance apart, as where they go straight into
+  // registers.  (Beside a choice between them and the loads by 32-bit offsets, short sequences paid for the longer
+  // prologue: 77x22 D=64 backward 8.29 us with it, 8.16 without and with loads into registers.)
+  if (Q_STAGED) qload.issue_clamped(0, q_rows, lds_base + 2u * Q_LO);
+  if (Q_STAGED && KG == 1 && q_rows > BKV) qload.issue_clamped(BKV, q_rows, lds_base + 2u * Q_HI);
   issue_v(0);
   if (n_tiles > 1) issue_k(1);
 
@@ -443,7 +440,7 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
   s16x8 ring[R];
 #pragma unroll
   for (int ks = 0; ks < KS; ks++) ring[ks] = lds_read_128(knext[ks]);
-  if (Q_STAGED) {  // every wave has its Q fragments: their stages are free for K_2 and V_1
+  if (Q_STAGED && n_tiles > 1) {  // every wave has its Q fragments: their stages are free for K_2 and V_1 (if there are any)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __syncthreads();
   }
