@@ -314,8 +314,11 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
   // 32-key blocks of this wave: with two key groups those in its group's half of the tiles.  The wave's
   // i-th block is key block block_at(i) of the sequence.
   const int n_below = min((kv_end + BLK - 1) / BLK, q0w / BLK + 1);
-  // (none for a wave without query rows, which only takes part in the loads and barriers)
-  const int n_mine = q0w >= p.seqlen_q ? 0 : KG == 1 ? n_below : (n_below - kg + 1) / 2;
+  // Up to 96 columns none for a wave without query rows, which only takes part in the loads and barriers (2048x64 D=64, dQ:
+  // 18.4 -> 18.1 us, 2048x33 14.7 -> 13.7).  Wider kernels have no gain from it and paid 0.5 to 2 % for the test on short
+  // sequences (17x320, backward: D=160 26.1 -> 26.4 us, D=192 30.8 -> 31.1).
+  const bool rowless = DP <= 96 && q0w >= p.seqlen_q;
+  const int n_mine = rowless ? 0 : KG == 1 ? n_below : (n_below - kg + 1) / 2;
   auto block_at = [&](int i) { return KG == 1 ? i : 2 * i + kg; };
   const int n_full = min(q0w + 1, seqlen_k) / BLK;                   // leading blocks without mask
   const int n_inside = seqlen_k / BKV;
