@@ -59,8 +59,9 @@ struct DkvPairLayout {
   static_assert(STAT_BASE >= PATCH_ELEMS, "the output patch overlays the stages");
 };
 
-template <typename T, int DP, bool PAD, int role, int COLS>
-__device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem) {
+// `place` gives the workgroup's place in the order of map_workgroup.
+template <typename T, int DP, bool PAD, int role, int COLS, typename Place>
+__device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem, Place place) {
   using L = DkvPairLayout<DP>;
   constexpr int BQ = L::BQ, KS = COLS / 16, DB = (COLS + 31) / 32, R = 2 * DB, LP = L::LP;
   constexpr int NTHREADS = 64 * kDkvWaves;
@@ -75,7 +76,7 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem) {
 
   const int BH = p.batch * p.nheads;
   int bh, kt;  // key tile 0 has the longest query range: rank == key tile
-  map_workgroup(p.resident_grid ? balanced_index(blockIdx.x, p.resident_grid) : blockIdx.x, BH, p.n_tiles, p.head_group, bh, kt);
+  map_workgroup(place(), BH, p.n_tiles, p.head_group, bh, kt);
   const int b = bh / p.nheads, hd = bh % p.nheads;
   const int kv0 = kt * L::KEYS;
   const int kv0w = kv0 + 32 * (wave >> 1);
@@ -356,10 +357,11 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem) {
 template <typename T, int DP, bool PAD, int COLS = DP>
 __global__ __launch_bounds__(64 * kDkvWaves, (dkdv_pair_wg_per_cu(DP))) void bwd_dkdv_pair_kernel(const BwdParams p) {
   __shared__ __attribute__((aligned(1024))) short smem[DkvPairLayout<DP>::TOTAL_ELEMS];
+  const auto place = [&]() -> int { return p.resident_grid ? balanced_index(blockIdx.x, p.resident_grid) : blockIdx.x; };
   if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 1)
-    bwd_dkdv_pair<T, DP, PAD, 1, COLS>(p, smem);
+    bwd_dkdv_pair<T, DP, PAD, 1, COLS>(p, smem, place);
   else
-    bwd_dkdv_pair<T, DP, PAD, 0, COLS>(p, smem);
+    bwd_dkdv_pair<T, DP, PAD, 0, COLS>(p, smem, place);
 }
 
 }  // namespace fa2

@@ -63,6 +63,36 @@ __global__ __launch_bounds__(256) void bwd_preprocess_kernel(const PreParams p) 
   }
 }
 
+// The same in front of a joint grid of dQ and dK/dV (fa2_bwd_joint.hpp), for rows of whole 16-byte chunks up to KS steps of 16
+// columns: two lanes per row, which sum the halves of every step one after the other, so that a row's delta has the bits the dQ
+// kernel gives it where it forms delta itself.  32 rows per workgroup of one wave, all loads in flight at once: these grids
+// are small (8 x 4096, D=128: 4 us between the other launches) and what they wait for is the first bytes.
+template <typename T, int KS>
+__global__ __launch_bounds__(64) void bwd_delta_kernel(const PreParams p) {
+  const int lane = threadIdx.x;
+  const int c = lane & 31, h = lane >> 5;
+  const int tiles = (p.seqlen_q_rounded + 31) / 32;
+  const int bh = blockIdx.x / tiles;
+  const int row = (blockIdx.x - bh * tiles) * 32 + c;
+  const int b = bh / p.nheads, hd = bh % p.nheads;
+  const bool ok = row < p.seqlen_q;
+  const short *op = (const short *)p.o.ptr + b * p.o.stride_batch + hd * p.o.stride_head + (int64_t)row * p.o.stride_seq;
+  const short *gp = (const short *)p.d_o.ptr + b * p.d_o.stride_batch + hd * p.d_o.stride_head + (int64_t)row * p.d_o.stride_seq;
+  s16x8 of[KS], gf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) {
+    of[ks] = load_chunk(op, 16 * ks + 8 * h, p.headdim, ok, true);
+    gf[ks] = load_chunk(gp, 16 * ks + 8 * h, p.headdim, ok, true);
+  }
+  float part = 0.f;
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+    for (int j = 0; j < 8; j++) part += Elem<T>::to_float(of[ks][j]) * Elem<T>::to_float(gf[ks][j]);
+  const float delta = sum_over_halves(part);  // 0 for rows beyond the sequence
+  if (h == 0 && row < p.seqlen_q_rounded) p.delta[(int64_t)bh * p.seqlen_q_rounded + row] = delta;
+}
+
 // ------------------------------------------------------------------------------------------
 // dQ kernel (query-tile parallel, fixed accumulation order).
 // ------------------------------------------------------------------------------------------
@@ -273,14 +303,15 @@ struct DqDirectLayout {
 // the register fragments, and are not stored.
 // KG: key groups, as in the forward (fa2_fwd.hpp).  With two the waves' sums over the even and the odd
 // 32-key blocks are added at the end, in that order: B=1 H=8 N=4096 D=128, bf16: 72.5 -> 58.5 us.
-template <typename T, int DP, int BKV, bool FUSE_DELTA, bool PAD, int KG = 1, int COLS = DP>
-__global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_direct_kernel(const BwdParams p) {
+// The work of one workgroup, for the kernel below and for the one that runs dK/dV beside it (fa2_bwd_joint.hpp): smem is
+// DqDirectLayout's LDS, `place` gives the workgroup's place in the order of map_workgroup.  (A call, and in the place where it
+// always was, and the parameters by value: so the kernel below comes out with the registers it had as one function.)
+template <typename T, int DP, int BKV, bool FUSE_DELTA, bool PAD, int KG, int COLS, typename Place>
+__device__ __forceinline__ void bwd_dq_direct(const BwdParams p, short *smem, Place place) {
   using L = DqDirectLayout<DP, BKV>;
   constexpr int KS = COLS / 16, DB = (COLS + 31) / 32, R = 2 * DB, LP = L::LP;
   constexpr int BLK = 32;
   static_assert(BKV == 2 * BLK, "written for 64-row key tiles of two 32-row blocks");
-
-  __shared__ __attribute__((aligned(1024))) short smem[L::TOTAL_ELEMS];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -290,7 +321,7 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
 
   const int BH = p.batch * p.nheads;
   int bh, rank;
-  map_workgroup(p.resident_grid ? balanced_index(blockIdx.x, p.resident_grid) : blockIdx.x, BH, p.n_tiles, p.head_group, bh, rank);
+  map_workgroup(place(), BH, p.n_tiles, p.head_group, bh, rank);
   const int qt = p.n_tiles - 1 - rank;  // the last query tile sees the most keys
   const int b = bh / p.nheads, hd = bh % p.nheads;
   constexpr int BQ = kDqBlockQ / KG;  // query rows of the workgroup
@@ -600,5 +631,11 @@ __global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_dir
                               p.dq.stride_seq, p.seqlen_q - q0w, hdim, true, p.grads_f32);
 }
 
+template <typename T, int DP, int BKV, bool FUSE_DELTA, bool PAD, int KG = 1, int COLS = DP>
+__global__ __launch_bounds__(64 * kDqWaves, (DP <= 128 ? 2 : 1)) void bwd_dq_direct_kernel(const BwdParams p) {
+  __shared__ __attribute__((aligned(1024))) short smem[DqDirectLayout<DP, BKV>::TOTAL_ELEMS];
+  bwd_dq_direct<T, DP, BKV, FUSE_DELTA, PAD, KG, COLS>(
+      p, smem, [&]() -> int { return p.resident_grid ? balanced_index(blockIdx.x, p.resident_grid) : blockIdx.x; });
+}
 
 }  // namespace fa2

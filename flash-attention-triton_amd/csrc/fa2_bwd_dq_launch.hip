@@ -78,4 +78,23 @@ void launch_preprocess(bool bf16, const PreParams &p, dim3 grid, hipStream_t s) 
     hipLaunchKernelGGL((bwd_preprocess_kernel<_Float16>), grid, dim3(256), 0, s, p);
 }
 
+template <typename T>
+static void launch_delta_steps(const PreParams &p, dim3 grid, hipStream_t s) {
+  if (p.headdim <= 32)
+    hipLaunchKernelGGL((bwd_delta_kernel<T, 2>), grid, dim3(64), 0, s, p);
+  else if (p.headdim <= 64)
+    hipLaunchKernelGGL((bwd_delta_kernel<T, 4>), grid, dim3(64), 0, s, p);
+  else if (p.headdim <= 128)
+    hipLaunchKernelGGL((bwd_delta_kernel<T, 8>), grid, dim3(64), 0, s, p);
+  else
+    hipLaunchKernelGGL((bwd_delta_kernel<T, 16>), grid, dim3(64), 0, s, p);
+}
+
+void launch_delta(bool bf16, const PreParams &p, dim3 grid, hipStream_t s) {
+  if (bf16)
+    launch_delta_steps<__bf16>(p, grid, s);
+  else
+    launch_delta_steps<_Float16>(p, grid, s);
+}
+
 }  // namespace fa2

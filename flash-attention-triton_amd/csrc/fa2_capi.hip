@@ -197,6 +197,25 @@ int64_t plan_dq(int cfg, fa2::BwdParams &p) {
   return nwg;
 }
 
+// One grid for both (fa2_bwd_joint.hpp): completes `j`, whose `both` holds the call's sizes, and returns the number of
+// workgroups.
+int64_t plan_joint(int cfg, int groups, fa2::JointParams &j) {
+  fa2::BwdParams &p = j.both;
+  const int64_t bh = (int64_t)p.batch * p.nheads;
+  const int block_q = kDqBlockQ / groups;
+  j.dq_tiles = (p.seqlen_q + block_q - 1) / block_q;
+  p.n_tiles = (p.seqlen_k + fa2::kDkvPairBlockKV - 1) / fa2::kDkvPairBlockKV;
+  p.head_group = fa2::equal_head_groups(kTable[cfg].head_group, bh);
+  const int64_t n_dq = j.dq_tiles * bh, n_dkdv = p.n_tiles * bh;
+  const int64_t nwg = fa2::joint_workgroups(n_dq, n_dkdv, fa2::joint_period(groups));
+  j.n_dq = (int)n_dq;
+  j.n_dkdv = (int)n_dkdv;
+  // Resident at once and more than one to a CU: walked as balanced_index does.
+  const int64_t slots = (int64_t)fa2::kCUs * fa2::dkdv_pair_wg_per_cu(kTable[cfg].headdim_padded);
+  p.resident_grid = nwg > fa2::kCUs && nwg <= slots ? (int)nwg : 0;
+  return nwg;
+}
+
 int fwd_impl(const fa2_fwd_args &a, void *stream, float *o_f32 = nullptr) {
   int rc = check_common(a.batch, a.nheads, a.seqlen_q, a.seqlen_k, a.headdim, a.seqlen_q_rounded, a.dtype);
   if (rc) return rc;
@@ -237,8 +256,9 @@ int fwd_impl(const fa2_fwd_args &a, void *stream, float *o_f32 = nullptr) {
   return launch_status("fa2_fwd launch");
 }
 
+// in_dq_order: with the bits the fast dQ kernel would give delta (where it could form it).
 int preprocess_impl(const fa2_tensor &o, const fa2_tensor &d_o, float *delta, int batch, int nheads,
-                    int seqlen_q, int headdim, int seqlen_q_rounded, int dtype, void *stream) {
+                    int seqlen_q, int headdim, int seqlen_q_rounded, int dtype, void *stream, bool in_dq_order = false) {
   int rc = check_common(batch, nheads, seqlen_q, 1, headdim, seqlen_q_rounded, dtype);
   if (rc) return rc;
   fa2::PreParams p;
@@ -253,6 +273,13 @@ int preprocess_impl(const fa2_tensor &o, const fa2_tensor &d_o, float *delta, in
   p.headdim = headdim;
   p.seqlen_q_rounded = seqlen_q_rounded;
   p.vec = vec_ok(p.o, headdim) && vec_ok(p.d_o, headdim);
+  if (in_dq_order && p.vec) {
+    const int64_t rows32 = (int64_t)((seqlen_q_rounded + 31) / 32) * batch * nheads;
+    if (rows32 <= fa2::kMaxWorkgroups) {
+      fa2::launch_delta(dtype == FA2_DTYPE_BF16, p, dim3((unsigned)rows32), reinterpret_cast<hipStream_t>(stream));
+      return launch_status("backward delta launch");
+    }
+  }
   const int64_t nwg = (int64_t)((seqlen_q_rounded + 15) / 16) * batch * nheads;
   if (nwg > 0x7fffffff) return fail(FA2_ERR_TOO_LARGE, "grid of %lld workgroups too large", (long long)nwg);
   p.n_tiles = (unsigned)nwg;
@@ -363,6 +390,21 @@ int bwd_impl(const fa2_bwd_args &a, void *stream, bool grads_f32 = false) {
     if ((rc = run_dkdv())) return rc;
     fa2::launch_dq_accum_convert(bf16, pk, s);
     return launch_status("dQ accumulator convert");
+  }
+
+  if (const int groups = want_dq && want_dkdv ? fa2::joint_key_groups(dp, p) : 0) {
+    // Both read delta.  On the smallest grids it has the bits that the dQ kernel by itself gives it.
+    if (fused) {
+      rc = preprocess_impl(a.o, a.d_o, a.delta, a.batch, a.nheads, a.seqlen_q, a.headdim, a.seqlen_q_rounded,
+                           a.dtype, stream, nwg_q <= fa2::kCUs);
+      if (rc) return rc;
+    }
+    fa2::JointParams j;
+    j.both = p;
+    const int64_t nwg = plan_joint(cfg, groups, j);
+    if (nwg > fa2::kMaxWorkgroups) return fail(FA2_ERR_TOO_LARGE, "grid of %lld workgroups too large", (long long)nwg);
+    (bf16 ? fa2::launch_joint<__bf16> : fa2::launch_joint<_Float16>)(dp, j, groups, dim3((unsigned)nwg), s);
+    return launch_status("backward dQ, dK and dV launch");
   }
 
   if (fused && fa2::dq_direct_ok(dp, pq) && vec_ok(p.o, a.headdim)) {

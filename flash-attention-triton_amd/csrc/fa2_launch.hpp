@@ -137,6 +137,55 @@ inline bool seqpar_atomic_ok(int dp, const BwdParams &p) {
   return dkdv_direct_ok(dp, p) && p.headdim == dp && (dp == 32 || dp == 64 || dp == 128);
 }
 
+// Whether dQ and dK/dV run in one grid (fa2_bwd_joint.hpp) behind a launch that forms delta, and with how many key groups
+// dQ: 0 where two launches are as fast, dQ forming delta for dK/dV.  Time of the two over that of delta and the joint grid,
+// bf16, (batch, head) pairs x tokens, by workgroups of 128 query rows; in brackets the other number of key groups:
+//   to 128      1.2-1.9 (16 x 64 and up), 64 columns 1.33 (32 x 512) [1.22], 128 columns 1.71 (4 x 512) [1.44], 1.39 (16 x 1024)
+//               [1.29], 256 columns 1.83 (2 x 1024) [1.51]; of 128 tokens and fewer 0.94-1.1 beyond 96 workgroups, at 160 columns
+//               and more beyond 64
+//   to 256      from 257 tokens 1.0-1.25: 64 columns 1.15 (32 x 1024) [1.02], 1.05 (64 x 512) [0.98], 128 columns 1.06 (16 x 2048),
+//               1.15 (8 x 4096) [1.03], 256 columns 1.13 (50 x 512) [0.88]; shorter ones 1.05-1.15 to 160, 0.79-1.0 beyond
+//   to 512      32 columns 1.17 (13 x 3000), 1.00 (32 x 2048); 48 and 64 columns from 1500 tokens 1.03-1.15, to 576 with heads
+//               that divide by 8, below 1500 0.88-1.05; 80 and 96 columns from 768 tokens 1.03-1.17, below 0.85-1.06; 128 columns
+//               1.19 (80 x 512), 1.08 (12 x 4096), 1.12 (43 x 1500), of 256 tokens and fewer 0.82-1.03; 192 columns 1.13 (160 x
+//               192), 1.04 (16 x 3000) to 384, 0.93-1.08 beyond; 256 columns 1.19 (80 x 512), 1.17 (320 x 64), 0.95 beyond 384
+//   beyond      80 and 96 columns 1.04-1.16 to 800 and 1100 tokens, 0.95-1.0 past them; 128 columns to 2048 tokens 1.02-1.15, 1.07
+//               (256 x 1024), 1.04 (512 x 512), past them 0.92-0.99; 160 columns from 1200 workgroups and 256 to 1024 tokens
+//               1.02-1.09; 256 columns 1.05-1.26 to 1100 tokens, 0.93-0.97 past them.  Padded heads (112, 224) and heads that do not
+//               divide by 8 0.93-1.03 there
+// The paired dK/dV kernel's conditions hold (below): where the other one is the better one, dK/dV is no part of such a grid.
+inline int joint_key_groups(int dp, const BwdParams &p) {
+  if (!dq_direct_ok(dp, p) || !dkdv_pair_ok(dp, p)) return 0;
+  const int64_t heads = (int64_t)p.batch * p.nheads, wgs = heads * ((p.seqlen_q + kDqBlockQ - 1) / kDqBlockQ);
+  const int n = p.seqlen_q;
+  if (wgs <= kCUs / 2) return n > 128 || wgs <= (dp > 128 ? 64 : 96) ? dq_key_groups(dp, p) : 0;
+  if (wgs <= kCUs) return n > (wgs <= 160 ? 128 : 256);
+  const bool large = wgs > 2 * kCUs;
+  if (large && (p.headdim != direct_columns(dp, p.headdim) || (heads % 8 != 0 && wgs > 4 * kCUs))) return 0;
+  if (dp <= 64) return wgs <= (dp == 32 ? 336 : heads % 8 ? 400 : 576) && n >= 1500;
+  if (dp == 96) return large ? wgs <= 800 && n > 160 && n <= 1100 : n >= 768;
+  if (dp == 128) return large ? n >= 128 && n <= 2048 : n > 256;
+  if (dp == 192) return large ? wgs >= 1200 && n > 192 && n <= 1100 : wgs <= 384 && n > 128;
+  return n >= 96 && (large ? n <= 1100 : wgs <= 384);
+}
+// The order of a joint grid, in runs of 8 workgroups that keep heads on their XCDs: every joint_period-th run is of dQ.  A
+// workgroup of dQ has twice the rows of one of dK/dV, or with two key groups as many.
+__host__ __device__ constexpr int joint_period(int key_groups) { return key_groups == 1 ? 3 : 2; }
+constexpr int64_t joint_workgroups(int64_t n_dq, int64_t n_dkdv, int period) {
+  const int64_t rounds_dq = (n_dq + 7) / 8, rounds_dkdv = (n_dkdv + 8 * (period - 1) - 1) / (8 * (period - 1));
+  return (rounds_dq > rounds_dkdv ? rounds_dq : rounds_dkdv) * 8 * period;
+}
+// Workgroup i's place in the order of its own kind (which may lie beyond the end of that).
+struct JointPlace {
+  bool dq;
+  int index;
+};
+__host__ __device__ constexpr JointPlace joint_place(int i, int period) {
+  const int run = i / 8, turn = run % period, round = run / period;
+  const bool dq = turn == period - 1;
+  return {dq, (dq ? round : round * (period - 1) + turn) * 8 + i % 8};
+}
+
 // Size of the head groups map_workgroup is given, for `heads` (batch, head) pairs and a table group
 // size `group`: the heads are split into floor(heads / group) groups of (nearly) equal size, each a
 // multiple of 8 so that a head stays on one XCD.  Equal groups, because a small last group would start
@@ -186,10 +235,19 @@ void launch_fwd_direct_wide<true>(bool bf16, int dp, int key_groups, const FwdPa
 // Rounds fp32 arrays to fp16 (fa2_cast.hpp); one launch for all of them.
 void launch_cast(const CastParams &p, dim3 grid, hipStream_t s);
 void launch_preprocess(bool bf16, const PreParams &p, dim3 grid, hipStream_t s);
+// delta with the bits of the fast dQ kernel's own, for rows of whole chunks (p.vec); p.n_tiles is not read.
+void launch_delta(bool bf16, const PreParams &p, dim3 grid, hipStream_t s);
 // fuse_delta: the fast dQ kernel also forms delta from O and dO (dq_direct_ok must hold).
 void launch_dq(bool bf16, int dp, const BwdParams &p, dim3 grid, bool fuse_delta, hipStream_t s);
 // With p.dq_accum set the sequence-parallel kernel runs: dK, dV and atomic dQ contributions.
 void launch_dkdv(bool bf16, int dp, const BwdParams &p, dim3 grid, hipStream_t s);
+// dQ (from p.dq, reading delta) and dK/dV (from p.dkdv) in one grid, which joint_grid gives; a specialisation for each type.
+template <typename T>
+void launch_joint(int dp, const JointParams &p, int key_groups, dim3 grid, hipStream_t s);
+template <>
+void launch_joint<__bf16>(int dp, const JointParams &p, int key_groups, dim3 grid, hipStream_t s);
+template <>
+void launch_joint<_Float16>(int dp, const JointParams &p, int key_groups, dim3 grid, hipStream_t s);
 void launch_dq_accum_zero(float *acc, int64_t floats, hipStream_t s);
 void launch_dq_accum_convert(bool bf16, const BwdParams &p, hipStream_t s);
 

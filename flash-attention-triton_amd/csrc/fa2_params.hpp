@@ -70,6 +70,14 @@ struct BwdParams {
   bool grads_f32;  // dq, dk and dv are fp32 tensors (strides in fp32 elements)
 };
 
+// dQ and dK/dV in one grid: n_tiles and resident_grid of `both` are dK/dV's and the whole grid's.  (One record for both: a
+// second one, 340 bytes more to hand over, showed in the host time of a launch.)
+struct JointParams {
+  BwdParams both;
+  int dq_tiles;      // query tiles per (batch, head) pair
+  int n_dq, n_dkdv;  // workgroups of each
+};
+
 struct PreParams {
   Tensor4 o, d_o;
   float *delta;

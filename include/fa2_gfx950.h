@@ -190,6 +190,9 @@ int fa2_pick_config(int dtype, int headdim, int seqlen_q, int seqlen_k, int dete
 
 /*
  * The kernels a forward and a backward of these sizes launch, for 16-byte aligned contiguous tensors.
+ * dq and dkdv are those of launches of their own, as when only one of them is asked for; a backward that
+ * wants all of dq, dk and dv runs both kinds of workgroup in one grid where that is faster
+ * (joint_key_groups in csrc/fa2_launch.hpp), dQ with the key groups that rule gives.
  * Touches no device.  No counterpart in the reference.  A forward-only row (fwd_exp_folded) has no
  * backward: dq and dkdv come back all zero.
  */

@@ -1,0 +1,73 @@
+"""dQ, dK and dV in one grid (csrc/fa2_bwd_joint.hpp): the order of its workgroups and what the compiler made of the kernel,
+on the CPU, and gradients at the edges of the rule that picks it (joint_key_groups in csrc/fa2_launch.hpp)."""
+
+from __future__ import annotations
+
+import math
+import pathlib
+import re
+import subprocess
+
+import pytest
+import torch
+
+from oracle import naive_attention as oracle
+from tests.test_code_objects import COLUMNS, LDS_PER_CU, REGS_PER_LANE, records  # noqa: F401
+
+ROOT = pathlib.Path(__file__).resolve().parent.parent
+HIPCC = pathlib.Path("/opt/rocm/bin/hipcc")
+ATOL, RTOL = 2e-2, 1e-2
+
+
+def test_every_workgroup_of_either_kind_once(tmp_path):
+    if not HIPCC.exists():
+        pytest.skip("hipcc not installed")
+    exe = tmp_path / "joint_grid_check"
+    build = subprocess.run(
+        [str(HIPCC), "-x", "hip", "--cuda-host-only", "-O1", "-std=c++17", "-Wno-unused-command-line-argument",
+         f"-I{ROOT / 'flash-attention-triton_amd' / 'csrc'}", f"-I{ROOT / 'include'}",
+         "-o", str(exe), str(ROOT / "tests" / "joint_grid_check.hip")], capture_output=True, text=True, timeout=300)
+    assert build.returncode == 0, build.stderr[-2000:]
+    run = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert run.returncode == 0 and run.stdout.endswith("ok\n"), run.stdout + run.stderr
+
+
+def test_joint_kernels_share_a_cu_like_their_parts(records):  # noqa: F811
+    """As many workgroups to a CU as the paired dK/dV kernel has, and no scratch memory but for the values kept across the
+    choice of the kind."""
+    seen = set()
+    for r in records:
+        m = re.match(r"_ZN3fa216bwd_joint_kernelI(DF16b|DF16_)Li(\d+)ELb([01])ELi([12])ELi(\d+)E", r["name"])
+        if not m:
+            continue
+        dtype, dp, pad, groups, cols = m.group(1), *map(int, m.groups()[1:])
+        seen.add((dtype, dp, pad, groups, cols))
+        waves = REGS_PER_LANE // ((int(r["vgpr_count"]) + 7) // 8 * 8)
+        assert min(waves, LDS_PER_CU // int(r["group_segment_fixed_size"])) >= (3 if dp <= 64 else 2 if dp <= 128 else 1), r["name"]
+        assert int(r["private_segment_fixed_size"]) <= (0 if dp < 128 or dp == 192 else 24 if dp == 128 else 52), r["name"]
+    assert seen == {(t, dp, pad, kg, cols) for t in ("DF16b", "DF16_") for dp, widths in COLUMNS.items() for cols in widths
+                    for pad in (0, 1) for kg in (1, 2)}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,nq,nk,d,dtype", [
+    (1, 1, 1, 64, torch.bfloat16), (96, 64, 64, 128, torch.float16), (97, 64, 64, 128, torch.bfloat16),  # one key group, 32 or fewer tokens
+    (3, 129, 700, 40, torch.bfloat16), (3, 700, 129, 128, torch.bfloat16), (2, 65, 1, 256, torch.float16),  # kinds of unlike number
+    (64, 192, 192, 48, torch.bfloat16), (65, 160, 160, 48, torch.bfloat16), (9, 1000, 1000, 104, torch.bfloat16),  # 128 workgroups and more
+    (41, 300, 333, 32, torch.bfloat16), (32, 1024, 1024, 64, torch.float16), (27, 1153, 1100, 72, torch.bfloat16),
+    (11, 3000, 3000, 96, torch.bfloat16), (43, 500, 500, 256, torch.bfloat16), (60, 200, 200, 176, torch.bfloat16),
+    (136, 520, 520, 128, torch.bfloat16), (136, 520, 520, 120, torch.bfloat16), (200, 512, 500, 80, torch.bfloat16),  # more than 512
+    (300, 100, 260, 160, torch.bfloat16), (520, 120, 120, 256, torch.bfloat16)], ids=lambda x: str(x).replace("torch.", ""))
+def test_gradients_at_the_edges_of_the_rule(fa, heads, nq, nk, d, dtype):
+    gen = torch.Generator(device="cuda").manual_seed(nq + heads)
+    q, d_o = (torch.randn(1, heads, nq, d, generator=gen, device="cuda").to(dtype) for _ in range(2))
+    k, v = (torch.randn(1, heads, nk, d, generator=gen, device="cuda").to(dtype) for _ in range(2))
+    leaves = [t.requires_grad_(True) for t in (q, k, v)]
+    grads = torch.autograd.grad(fa.flash_attention_v2(*leaves), leaves, d_o)
+    for at in {0, heads // 2, heads - 1}:
+        one = [t.detach()[:, at : at + 1].float() for t in (q, k, v, d_o)]
+        _, *want = oracle.naive_backward(*one, 1.0 / math.sqrt(d), torch.float32)
+        for name, got, ref in zip(("dq", "dk", "dv"), grads, want):
+            assert torch.isfinite(got).all(), name
+            err = (got[:, at : at + 1].float() - ref).abs()
+            assert (err <= ATOL + RTOL * ref.abs()).all(), f"{name}, head {at}: max abs err {err.max().item():.3e}"
