@@ -80,6 +80,8 @@ def _measured_traffic(workload: str) -> tuple[dict, str]:
 
 def kernel_name(launch: dict, part: str) -> str:
     """Name of the kernel a part of a call runs, from the library's own account of it (capi.launch_info)."""
+    if part == "fwd" and launch[part]["key_groups"] == 4:
+        return "fwd_quad_kernel"
     suffix = {"generic": "kernel", "direct": "direct_kernel", "paired": "pair_kernel"}[launch[part]["form"]]
     return {"fwd": "fwd_", "dq": "bwd_dq_", "dkdv": "bwd_dkdv_"}[part] + suffix
 

@@ -164,14 +164,18 @@ int launch_status(const char *what) {
 
 bool good_scale(float s) { return s > 0.f && std::isfinite(s); }
 
+int fwd_wg_per_cu(int cfg, int groups) {
+  return groups == 4 ? fa2::fwd_quad_wg_per_cu(kTable[cfg].headdim_padded) : kTable[cfg].fwd_wg_per_cu;
+}
+
 // Kernel form, tiles and grid of a forward: completes `p` and returns the number of workgroups.
 int64_t plan_fwd(int cfg, fa2::FwdParams &p) {
   const int64_t bh = (int64_t)p.batch * p.nheads;
-  const int block_q = kFwdBlockQ / fa2::fwd_key_groups(kTable[cfg].headdim_padded, p);
+  const int groups = fa2::fwd_key_groups(kTable[cfg].headdim_padded, p), block_q = kFwdBlockQ / groups;
   p.n_qtiles = (p.seqlen_q + block_q - 1) / block_q;
   const int64_t nwg = p.n_qtiles * bh;
   // The table's group size, evened out over the heads there are.
-  plan_order(p, cfg, nwg, kTable[cfg].fwd_wg_per_cu, fa2::equal_head_groups(kTable[cfg].head_group, bh));
+  plan_order(p, cfg, nwg, fwd_wg_per_cu(cfg, groups), fa2::equal_head_groups(kTable[cfg].head_group, bh));
   return nwg;
 }
 
@@ -544,7 +548,7 @@ int fa2_launch_info_get(int batch, int nheads, int seqlen_q, int seqlen_k, int h
   int64_t nwg = plan_fwd(cfg, f);
   int groups = fa2::fwd_key_groups(dp, f);
   out->fwd = part(fa2::fwd_direct_ok(dp, f) ? FA2_FORM_DIRECT : FA2_FORM_GENERIC, kFwdBlockQ / groups, groups,
-                  row.fwd_wg_per_cu, f.resident_grid, nwg);
+                  fwd_wg_per_cu(cfg, groups), f.resident_grid, nwg);
   if (row.fwd_exp_folded) return FA2_OK;
   nwg = plan_dkdv(cfg, k);
   const bool pair = !row.dq_atomic && fa2::dkdv_pair_ok(dp, k);

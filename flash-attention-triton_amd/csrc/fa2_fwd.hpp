@@ -300,7 +300,7 @@ struct HalfTag {
 // KG: key groups.  With one, a wave multiplies both 32-key blocks of every tile by its 32 query rows.  With
 // two, waves 0, 1 take the first and waves 2, 3 the second block of every tile, for the same 64 rows, and the
 // results are merged at the end: half the blocks per wave, for grids that do not fill the chip (key_groups
-// in fa2_launch.hpp has the rule).  B=1 H=8 N=4096 D=128, bf16: 62.6 -> 48.0 us; B=2 H=4 N=512 D=64, fp16:
+// in fa2_launch.hpp has the rule; four: fwd_quad_kernel below).  B=1 H=8 N=4096 D=128, bf16: 62.6 -> 48.0 us; B=2 H=4 N=512 D=64, fp16:
 // 9.9 -> 7.1 us.  There a wave's own chain is what takes the time: QK^T, softmax and PV of one block after
 // the other at 0.5 us each, with at most one other wave on its SIMD.
 // PRE: the Q fragments are multiplied by scale * log2(e) and rounded to half precision once, and
@@ -308,16 +308,15 @@ struct HalfTag {
 // MFMAs deliver the base-2 exponents themselves and no multiply-add is left in front of the
 // exponentials.
 // F32: the output goes to an fp32 tensor as well, or only there: store_output (fa2_common.hpp).
-template <typename T, int DP, int BKV, bool PAD, bool PRE, int KG = 1, int COLS = DP, bool F32 = false>
-__global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direct_kernel(const FwdParams p) {
+// The work of one workgroup: smem is FwdDirectLayout's LDS, `place` gives the workgroup's place in the order of map_workgroup.
+template <typename T, int DP, int BKV, bool PAD, bool PRE, int KG, int COLS, bool F32, typename Place>
+__device__ __forceinline__ void fwd_direct(const FwdParams p, short *smem, Place place) {
   using L = FwdDirectLayout<DP, BKV>;
   constexpr int KS = COLS / 16, DB = (COLS + 31) / 32, R = 2 * DB, LP = L::LP;
   constexpr int NTHREADS = 64 * kFwdWaves;
   constexpr int BLK = 32;  // keys per pipeline block
-  static_assert(BKV == 2 * BLK && (KS == R || KS == R - 1), "schedule is written for 64-row tiles of two blocks");
+  static_assert(BKV == (KG == 4 ? 4 : 2) * BLK && (KS == R || KS == R - 1), "schedule is written for tiles of two blocks, or of one per key group");
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-
-  __shared__ __attribute__((aligned(1024))) short smem[L::TOTAL_ELEMS];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -327,7 +326,7 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
 
   const int BH = p.batch * p.nheads;
   int bh, rank;
-  map_workgroup(p.resident_grid ? balanced_index(blockIdx.x, p.resident_grid) : blockIdx.x, BH, p.n_qtiles, p.head_group, bh, rank);
+  map_workgroup(place(), BH, p.n_qtiles, p.head_group, bh, rank);
   const int qt = p.n_qtiles - 1 - rank;  // the last query tile sees the most keys
   const int b = bh / p.nheads, hd = bh % p.nheads;
   constexpr int BQ = kFwdBlockQ / KG;  // query rows of the workgroup
@@ -353,8 +352,8 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
   // groups) lie in the half of the tiles that is its group's.  The wave's i-th block is key block
   // block_at(i) of the sequence.
   const int n_below = min((kv_end + BLK - 1) / BLK, q0w / BLK + 1);
-  const int n_mine = KG == 1 ? n_below : (n_below - kg + 1) / 2;
-  auto block_at = [&](int i) { return KG == 1 ? i : 2 * i + kg; };
+  const int n_mine = KG == 1 ? n_below : (n_below - kg + KG - 1) / KG;
+  auto block_at = [&](int i) { return KG == 1 ? i : KG * i + kg; };
   // Leading blocks that need no mask (entirely at or below the wave's first row, inside the keys).
   const int n_full = min(q0w + 1, seqlen_k) / BLK;
   const int n_inside = seqlen_k / BKV;  // tiles whose every row exists
@@ -379,17 +378,18 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
   // fragments.  Loaded straight into registers, a wave's fragment loads touch 32 different rows
   // each, eight times over, and keep the CU's address path busy for a microsecond per workgroup.
   // Rows beyond the sequence are read from its last row: finite values whose results are never stored.
-  // With two key groups, whose waves take one block per tile, tile t brings in K_{t+3}, K_2 is loaded here
-  // as well and the 64 query rows go through the second V stage.
+  // With more key groups, whose waves take one block per tile, tile t brings in K_{t+3}, K_2 is loaded here
+  // as well and the 64 (four groups: 32) query rows go through the second V stage.
   constexpr unsigned Q_HI = 2u * (unsigned)(L::V_BASE + 1 * L::TILE_ELEMS);
   constexpr unsigned Q_LO = KG == 1 ? 2u * (unsigned)(L::K_BASE + 2 * L::TILE_ELEMS) : Q_HI;
   constexpr int K_AHEAD = KG == 1 ? 2 : 3;  // tile t loads K tile t + K_AHEAD
-  const Loader qload(Q + (int64_t)q0 * p.q.stride_seq, p.q.stride_seq, hdim / 8);
+  constexpr int QROWS = KG == 4 && DP > 32 ? 32 : 64;  // (rows of 32 halves: a tile of 32 is less than one load per wave)
+  const TileLoader<DP, QROWS, kFwdWaves, PAD || COLS != DP> qload(Q + (int64_t)q0 * p.q.stride_seq, p.q.stride_seq, hdim / 8);
   const int q_rows = p.seqlen_q - q0;  // rows of this query tile that exist (>= 1)
   issue_k(0);
-  if (q_rows >= BKV) qload.issue(0, lds_base + Q_LO); else qload.issue_clamped(0, q_rows, lds_base + Q_LO);
+  if (q_rows >= QROWS) qload.issue(0, lds_base + Q_LO); else qload.issue_clamped(0, q_rows, lds_base + Q_LO);
   if (KG == 1) {
-    if (q_rows >= 2 * BKV) qload.issue(BKV, lds_base + Q_HI); else qload.issue_clamped(BKV, q_rows, lds_base + Q_HI);
+    if (q_rows >= 2 * QROWS) qload.issue(QROWS, lds_base + Q_HI); else qload.issue_clamped(QROWS, q_rows, lds_base + Q_HI);
   }
   issue_v(0);
   if (n_tiles > 1) issue_k(1);
@@ -478,8 +478,8 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) sc = Elem<T>::mfma(ring[ks], qf[ks], sc);
     if (block_at(0) >= n_full) apply_mask(sc, block_at(0) * BLK);
-    if (KG > 1 && kg == 1) {
-      // The second key group's first block is block 1, which may hold nothing but keys above the diagonal or
+    if (KG > 1 && kg > 0) {
+      // The second key group's first block is block 1 (and so on), which may hold nothing but keys above the diagonal or
       // keys that a bias hides (-inf, or the type's lowest value).  Its rows start from block 0's maximum, as
       // the first group's and those of a launch with one group do: the same probabilities, rounded to half
       // precision at the same scale, whatever the grid.  The score chain more is 0.2 to 0.5 us per launch, which
@@ -488,7 +488,7 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
       // backward: 186.3 and 186.0 us).
       f32x16 s0 = zero;
 #pragma unroll
-      for (int ks = 0; ks < KS; ks++) s0 = Elem<T>::mfma(lds_read_128(kcur[ks] - BLK * LP), qf[ks], s0);
+      for (int ks = 0; ks < KS; ks++) s0 = Elem<T>::mfma(lds_read_128(kcur[ks] - (KG == 2 ? 1 : kg) * BLK * LP), qf[ks], s0);
       if (n_full < 1) apply_mask(s0, 0);
       m_ref = row_max(s0);
     } else {
@@ -505,7 +505,7 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
     };
     exponentials();
     // Block 1 far above block 0's maximum: what a step does then (below), with nothing accumulated yet.
-    if (KG > 1 && kg == 1 && __builtin_amdgcn_ballot_w64(!(l_run <= kSumTrigger)) != 0) {
+    if (KG > 1 && kg > 0 && __builtin_amdgcn_ballot_w64(!(l_run <= kSumTrigger)) != 0) {
       m_ref = fmaxf(m_ref, row_max(sc));
       exponentials();
     }
@@ -557,7 +557,10 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
   // queue up in the memory pipeline, and a wave whose load cannot issue cannot issue its MFMAs
   // either.
   constexpr int LOADS = Loader::LOADS;
-  constexpr int LOAD_EVERY = KS / LOADS;
+  // The wave-loads of a tile that go with unit u: every LOAD_EVERY-th unit takes one, or, of more loads than units, each its share.
+  constexpr int LOAD_EVERY = KS >= LOADS ? KS / LOADS : 1;
+  constexpr auto first_load = [](int u) { return KS >= LOADS ? min((u + LOAD_EVERY - 1) / LOAD_EVERY, LOADS) : part(LOADS, KS, min(u, KS)); };
+  constexpr auto tile_of = [](int j) { return KG == 1 ? j / 2 : j; };
   auto step = [&](int j, auto half_tag, auto spread_tag) {
     constexpr int HALF = decltype(half_tag)::value;
     constexpr bool SPREAD = decltype(spread_tag)::value;
@@ -566,12 +569,12 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
     constexpr bool INNER = decltype(spread_tag)::value || decltype(half_tag)::inner;
     if (!INNER && j >= n_mine) {
       if (SPREAD) {  // not reached: the skipped blocks lie in the last two tiles, which load nothing
-        issue_k(j / (2 / KG) + K_AHEAD);
-        issue_v(j / (2 / KG) + 1);
+        issue_k(tile_of(j) + K_AHEAD);
+        issue_v(tile_of(j) + 1);
       }
       return;
     }
-    const int kt = j / (2 / KG) + K_AHEAD, vt = j / (2 / KG) + 1;  // tiles loaded during this step (SPREAD)
+    const int kt = tile_of(j) + K_AHEAD, vt = tile_of(j) + 1;  // tiles loaded during this step (SPREAD)
     const unsigned kdst = lds_base + 2u * (unsigned)(L::K_BASE + (kt % L::K_STAGES) * L::TILE_ELEMS);
     const unsigned vdst = lds_base + 2u * (unsigned)(L::V_BASE + (vt % L::V_STAGES) * L::TILE_ELEMS);
     typedef unsigned u32x4v __attribute__((ext_vector_type(4)));
@@ -580,7 +583,10 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
       sc = Elem<T>::mfma(ring[ks], qf[ks], (PRE && ks == 0) ? negm : sc);
-      if (SPREAD && ks % LOAD_EVERY == 0 && ks / LOAD_EVERY < LOADS) vload.issue_one(vt * BKV, vdst, ks / LOAD_EVERY);
+      if (SPREAD) {
+#pragma unroll
+        for (int i = first_load(ks); i < first_load(ks + 1); i++) vload.issue_one(vt * BKV, vdst, i);
+      }
       ring[ks] = v_frag(HALF, ks / DB, ks % DB);
       if (KS < R && ks == 0) ring[R - 1] = v_frag(HALF, 1, DB - 1);  // the slot no K fragment was in
 #pragma unroll
@@ -604,7 +610,10 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
       for (int db = 0; db < DB; db++) {
         const int slot = ks2 * DB + db;
         oacc[db] = Elem<T>::mfma(ring[slot], pf[ks2], oacc[db]);
-        if (SPREAD && slot % LOAD_EVERY == 0 && slot / LOAD_EVERY < LOADS) kload.issue_one(kt * BKV, kdst, slot / LOAD_EVERY);
+        if (SPREAD) {
+#pragma unroll
+          for (int i = first_load(slot); i < first_load(slot + 1); i++) kload.issue_one(kt * BKV, kdst, i);
+        }
         if (slot < KS) ring[slot] = k_frag(HALF, slot);
 #pragma unroll
         for (int i = part(16, R, slot); i < part(16, R, slot + 1); i++) {
@@ -687,14 +696,15 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
     end_tile(t);
   }
   float l_tot = sum_over_halves(l_run);
-  // Two key groups: the second hands its maximum, sum and accumulator to the first, which merges them with
-  // the rescale of an online-softmax step and stores.  The areas overlay the stages: the loop's last
+  // More key groups than one: the others hand their maximum, sum and accumulator to the first, which merges them one after
+  // the other with the rescale of an online-softmax step and stores.  The areas overlay the stages: the loop's last
   // barrier ordered them after all reads.
-  constexpr int MERGE_FLOATS = KG == 1 ? 0 : (DB * 16 + 2) * 64;  // per row group
-  static_assert(KG == 1 || 2 * MERGE_FLOATS * 2 + 2 * 32 * (DP + 8) <= L::TOTAL_ELEMS, "merge area and patch overlay the stages");
+  constexpr int AREAS = (KG - 1) * (kFwdWaves / KG);
+  constexpr int MERGE_FLOATS = KG == 1 ? 0 : (DB * 16 + 2) * 64;  // per row group and other key group
+  static_assert(KG == 1 || AREAS * MERGE_FLOATS * 2 + kFwdWaves / KG * 32 * (DP + 8) <= L::TOTAL_ELEMS, "merge areas and patch overlay the stages");
   if constexpr (KG > 1) {
-    float *area = reinterpret_cast<float *>(smem) + rg * MERGE_FLOATS + 4 * lane;
-    if (kg == 1) {
+    float *area = reinterpret_cast<float *>(smem) + (KG == 2 ? rg : max(kg - 1, 0)) * MERGE_FLOATS + 4 * lane;
+    if (kg > 0) {
 #pragma unroll
       for (int db = 0; db < DB; db++)
 #pragma unroll
@@ -705,20 +715,23 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
       area[DB * 1024 - 3 * lane + 64] = l_tot;
     }
     __syncthreads();
-    if (kg == 1) return;
-    const float m1 = area[DB * 1024 - 3 * lane], l1 = area[DB * 1024 - 3 * lane + 64];
-    const float m_new = fmaxf(m_ref, m1), unit = PRE ? 1.f : scale_log2;
-    const float a0 = fast_exp2((m_ref - m_new) * unit), a1 = fast_exp2((m1 - m_new) * unit);
-    m_ref = m_new;
-    l_tot = l_tot * a0 + l1 * a1;
+    if (kg > 0) return;
+#pragma unroll 1
+    for (int other = 1; other < KG; other++, area += MERGE_FLOATS) {
+      const float m1 = area[DB * 1024 - 3 * lane], l1 = area[DB * 1024 - 3 * lane + 64];
+      const float m_new = fmaxf(m_ref, m1), unit = PRE ? 1.f : scale_log2;
+      const float a0 = fast_exp2((m_ref - m_new) * unit), a1 = fast_exp2((m1 - m_new) * unit);
+      m_ref = m_new;
+      l_tot = l_tot * a0 + l1 * a1;
 #pragma unroll
-    for (int db = 0; db < DB; db++)
+      for (int db = 0; db < DB; db++)
 #pragma unroll
-      for (int g = 0; g < 4; g++) {
-        const f32x4 x = *reinterpret_cast<const f32x4 *>(area + (db * 4 + g) * 256);
+        for (int g = 0; g < 4; g++) {
+          const f32x4 x = *reinterpret_cast<const f32x4 *>(area + (db * 4 + g) * 256);
 #pragma unroll
-        for (int e2 = 0; e2 < 4; e2++) oacc[db][4 * g + e2] = oacc[db][4 * g + e2] * a0 + x[e2] * a1;
-      }
+          for (int e2 = 0; e2 < 4; e2++) oacc[db][4 * g + e2] = oacc[db][4 * g + e2] * a0 + x[e2] * a1;
+        }
+    }
   }
   const float inv_l = 1.f / l_tot;
   if (h == 0 && q0w + c < p.seqlen_q) LSE[q0w + c] = m_ref * (PRE ? kLn2 : p.scale) + __logf(l_tot);
@@ -726,8 +739,28 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
     for (int r = p.seqlen_q + tid; r < p.seqlen_q_rounded; r += NTHREADS / KG) LSE[r] = 0.f;
   }
   // The patch overlays the stages; the loop's last barrier already ordered it after all reads.
-  short *patch = smem + KG * MERGE_FLOATS * 2 + wave * 32 * (DP + 8);
+  short *patch = smem + AREAS * MERGE_FLOATS * 2 + wave * 32 * (DP + 8);
   store_output<T, COLS, F32>(p, oacc, inv_l, patch, O, bh, q0w, hdim, true);
+}
+
+template <typename T, int DP, int BKV, bool PAD, bool PRE, int KG = 1, int COLS = DP, bool F32 = false>
+__global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direct_kernel(const FwdParams p) {
+  __shared__ __attribute__((aligned(1024))) short smem[FwdDirectLayout<DP, BKV>::TOTAL_ELEMS];
+  fwd_direct<T, DP, BKV, PAD, PRE, KG, COLS, F32>(
+      p, smem, [&]() -> int { return p.resident_grid ? balanced_index(blockIdx.x, p.resident_grid) : blockIdx.x; });
+}
+
+// Four key groups: a wave for each, 32 query rows, tiles of 128 keys.  For grids of so few workgroups that the chain of blocks of
+// one wave is what the launch takes (fwd_quad in fa2_launch.hpp has the rule): bf16, 2 x 4096 D=64 29.0 -> 19.6 us, 2 x 4096 D=80
+// 39.4 -> 29.6, 1 x 8192 D=128 89.4 -> 69.3.  At 128 columns three K and two V tiles are all of a CU's LDS, and the 160 KiB they
+// take to fill before the first block eat the gain below 1500 tokens.  (Compiled for two waves per SIMD although one fits: with all
+// 512 registers allowed, the compiler moves the accumulators through accumulation registers.)
+template <typename T, int DP, bool PAD, bool PRE, bool F32, int COLS = DP>
+__global__ __launch_bounds__(64 * kFwdWaves, 2) void fwd_quad_kernel(const FwdParams p) {
+  constexpr int BKV = 4 * 32;
+  __shared__ __attribute__((aligned(1024))) short smem[FwdDirectLayout<DP, BKV>::TOTAL_ELEMS];
+  fwd_direct<T, DP, BKV, PAD, PRE, 4, COLS, F32>(
+      p, smem, [&]() -> int { return p.resident_grid ? balanced_index(blockIdx.x, p.resident_grid) : blockIdx.x; });
 }
 
 }  // namespace fa2

@@ -26,7 +26,12 @@ void launch_generic(int dp, const FwdParams &p, dim3 grid, dim3 block, hipStream
 // spilled registers and reloads inside its tile loop; alone and in its padded form only it spills none.
 template <typename T, int DP, int COLS, bool PRE, int KG>
 void launch_cols(const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
-  if (p.headdim == COLS)
+  if constexpr (KG == 4) {
+    if (p.headdim == COLS)
+      hipLaunchKernelGGL((fwd_quad_kernel<T, DP, false, PRE, kF32, COLS>), grid, block, 0, s, p);
+    else
+      hipLaunchKernelGGL((fwd_quad_kernel<T, DP, true, PRE, kF32, COLS>), grid, block, 0, s, p);
+  } else if (p.headdim == COLS)
     hipLaunchKernelGGL((fwd_direct_kernel<T, DP, kFwdBlockKV, false, PRE, KG, COLS, kF32>), grid, block, 0, s, p);
   else
     hipLaunchKernelGGL((fwd_direct_kernel<T, DP, kFwdBlockKV, true, PRE, KG, COLS, kF32>), grid, block, 0, s, p);
@@ -41,7 +46,9 @@ void launch_direct(int dp, const FwdParams &p, dim3 grid, dim3 block, hipStream_
     case 80: launch_cols<T, 96, 80, PRE, KG>(p, grid, block, s); break;
     case 96: launch_cols<T, 96, 96, PRE, KG>(p, grid, block, s); break;
     case 128: launch_cols<T, 128, 128, PRE, KG>(p, grid, block, s); break;
-    default: launch_fwd_direct_wide<kF32>(std::is_same<T, __bf16>::value, dp, KG, p, grid, block, s); break;
+    default:  // (there are two key groups at most)
+      launch_fwd_direct_wide<kF32>(std::is_same<T, __bf16>::value, dp, KG, p, grid, block, s);
+      break;
   }
 }
 
@@ -57,7 +64,10 @@ template <typename T>
 void launch(int dp, bool folded, const FwdParams &p, dim3 grid, hipStream_t s) {
   const dim3 block(64 * kFwdWaves);
   if (fwd_direct_ok(dp, p)) {
-    if (fwd_key_groups(dp, p) == 2)
+    const int groups = fwd_key_groups(dp, p);
+    if (groups == 4)
+      launch_groups<T, 4>(dp, folded, p, grid, block, s);
+    else if (groups == 2)
       launch_groups<T, 2>(dp, folded, p, grid, block, s);
     else
       launch_groups<T, 1>(dp, folded, p, grid, block, s);

@@ -86,8 +86,29 @@ inline bool fwd_direct_ok(int dp, const FwdParams &p) {
   return p.vec && direct_headdim_wide(dp, p.headdim) && direct_stride_ok(p.q) && direct_stride_ok(p.k) &&
          direct_stride_ok(p.v);
 }
+// Four key groups (fwd_quad_kernel), to 128 columns: 32 query rows to a workgroup, again half the chain for twice the loads per
+// row, in tiles of 128 keys that leave room for four workgroups per CU at 32 columns, two at 64 and one from 80 on.  Time of the other
+// forms over its own, bf16, by workgroups of 32 rows: while they are all resident it grows with the chain, and past that it is lost.
+//   32 columns        to 512 1.03 (32 x 512), 1.20 (16 x 1024), 1.47 (4 x 4096); to 768 1.06 (24 x 1024), 0.96 (31 x 777); to 1024
+//                     1.12 (16 x 2048), 0.95 (32 x 1024); 0.88-1.0 beyond, 1.34 at 5 x 8192
+//   48, 64 columns    to 512 1.03 (32 x 512), 1.22 (16 x 1024), 1.47 (4 x 4096), 1.0-1.1 below 512 tokens; to 640 1.08 (10 x 2048),
+//                     0.84 (20 x 1024); to 768 1.07 (8 x 3000), 0.97 (12 x 2048); 0.5-0.95 beyond
+//   80, 96 columns    to 256 1.10 (8 x 1024), 1.19-1.23 (4 x 2048), 1.41 (1 x 8192), 0.98 (16 x 512); to 384 1.20 (3 x 4096), 0.92 (6 x
+//                     2048); 0.9-1.0 beyond
+//   128 columns       to 256 1.05 (5 x 1500), 1.16 (2 x 4096), 1.25 (1 x 8192), 0.97 (8 x 1024); to 384 1.17 (3 x 4096), 0.92 (4 x
+//                     3000); 0.8 beyond
+inline bool fwd_quad(int dp, int64_t heads, int seqlen_q) {
+  const int64_t wgs = heads * ((seqlen_q + 31) / 32);
+  const int n = seqlen_q;
+  if (dp == 32) return n > 512 && wgs <= (n >= 2048 ? 1024 : n >= 1024 ? 768 : 512);
+  if (dp == 64) return n > 512 && wgs <= (n >= 3000 ? 768 : n >= 2048 ? 640 : 512);
+  if (dp == 96) return n >= 768 && wgs <= (n >= 4096 ? 384 : 256);
+  return dp == 128 && n >= 1500 && wgs <= (n >= 4096 ? 384 : 256);
+}
 inline int fwd_key_groups(int dp, const FwdParams &p) {
-  return fwd_direct_ok(dp, p) ? key_groups(dp, direct_columns(dp, p.headdim), (int64_t)p.batch * p.nheads, p.seqlen_q, false) : 1;
+  if (!fwd_direct_ok(dp, p)) return 1;
+  const int64_t heads = (int64_t)p.batch * p.nheads;
+  return fwd_quad(dp, heads, p.seqlen_q) ? 4 : key_groups(dp, direct_columns(dp, p.headdim), heads, p.seqlen_q, false);
 }
 inline bool dq_direct_ok(int dp, const BwdParams &p) {
   return p.vec && direct_headdim_wide(dp, p.headdim) && direct_stride_ok(p.k) && direct_stride_ok(p.v);

@@ -32,6 +32,9 @@ constexpr int kDkvBlockKV = 32 * kDkvWaves;
 constexpr int kDkvPairBlockKV = 64;  // key rows per workgroup of the paired dK/dV kernel (two waves share 32)
 // Its workgroups per CU: registers and LDS leave room for three up to 64 columns, two up to 128.
 constexpr int dkdv_pair_wg_per_cu(int dp) { return dp <= 64 ? 3 : dp <= 128 ? 2 : 1; }
+// Workgroups per CU of the forward with four key groups, whose tiles of 128 keys take 80 KiB of LDS at 64 columns and all 160 at 96
+// and 128.
+constexpr int fwd_quad_wg_per_cu(int dp) { return dp <= 32 ? 4 : dp <= 64 ? 2 : 1; }
 // Rows of the streamed operand per LDS tile.
 constexpr int kFwdBlockKV = 64;
 constexpr int kDqBlockKV = 64;

@@ -104,7 +104,7 @@ typedef struct fa2_config_info {
 /* Kernel forms.  FA2_FORM_GENERIC is the fallback for operands the LDS-direct kernels cannot read. */
 typedef enum fa2_form {
   FA2_FORM_GENERIC = 0, /* fwd_kernel, bwd_dq_kernel, bwd_dkdv_kernel */
-  FA2_FORM_DIRECT = 1,  /* fwd_direct_kernel, bwd_dq_direct_kernel, bwd_dkdv_direct_kernel */
+  FA2_FORM_DIRECT = 1,  /* fwd_direct_kernel (fwd_quad_kernel), bwd_dq_direct_kernel, bwd_dkdv_direct_kernel */
   FA2_FORM_PAIRED = 2   /* bwd_dkdv_pair_kernel */
 } fa2_form;
 
@@ -116,7 +116,8 @@ typedef enum fa2_form {
 typedef struct fa2_launch_part {
   int form;         /* fa2_form */
   int block_rows;   /* query rows (forward, dQ) or key rows (dK/dV) per workgroup */
-  int key_groups;   /* forward and dQ: 2 when two waves share 32 query rows and split the keys, else 1 */
+  int key_groups;   /* forward and dQ: 2 when two waves share 32 query rows and split the keys, 4 when four do
+                       (forward, fwd_quad_kernel), else 1 */
   int wg_per_cu;    /* workgroups that share a CU (0: not stated, for the generic kernels) */
   int resident;
   int64_t workgroups;
