@@ -325,6 +325,7 @@ __global__ __launch_bounds__(64 * kDkvWaves, (DP <= 64 && !ATOMIC_DQ ? 2 : 1)) v
   // others, and the atomic rows have one workgroup per CU.)
   const int index = DP == 32 && !ATOMIC_DQ && p.resident_grid ? balanced_index(blockIdx.x, p.resident_grid) : blockIdx.x;
   map_workgroup(index, BH, p.n_tiles, p.head_group, bh, kt);
+  if (p.last_heads_first) bh = from_the_end(bh, BH);
   const int b = bh / p.nheads, hd = bh % p.nheads;
   const int kv0 = kt * kDkvBlockKV;
   const int kv0w = kv0 + 32 * wave;

@@ -77,6 +77,7 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem, P
   const int BH = p.batch * p.nheads;
   int bh, kt;  // key tile 0 has the longest query range: rank == key tile
   map_workgroup(place(), BH, p.n_tiles, p.head_group, bh, kt);
+  if (p.last_heads_first) bh = from_the_end(bh, BH);
   const int b = bh / p.nheads, hd = bh % p.nheads;
   const int kv0 = kt * L::KEYS;
   const int kv0w = kv0 + 32 * (wave >> 1);

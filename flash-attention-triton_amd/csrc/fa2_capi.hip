@@ -354,6 +354,7 @@ int bwd_impl(const fa2_bwd_args &a, void *stream, bool grads_f32 = false) {
   const int dp = kTable[cfg].headdim_padded;
   const int64_t bh = (int64_t)a.batch * a.nheads;
   p.grads_f32 = grads_f32;
+  p.last_heads_first = false;
   p.dq_accum = nullptr;
   p.dq_accum_rows = 0;
 
@@ -415,6 +416,7 @@ int bwd_impl(const fa2_bwd_args &a, void *stream, bool grads_f32 = false) {
     // dQ first: it writes delta, which the dK/dV kernel reads.
     fa2::launch_dq(bf16, dp, pq, dim3((unsigned)nwg_q), true, s);
     if ((rc = launch_status("backward dQ launch (delta fused)"))) return rc;
+    pk.last_heads_first = true;
     return run_dkdv();
   }
   if (fused) {

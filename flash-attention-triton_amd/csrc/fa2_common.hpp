@@ -309,6 +309,14 @@ __host__ __device__ __forceinline__ void map_workgroup(int i, int heads, int til
   rank = r / gsize;
 }
 
+// The heads in the opposite order, whole runs of 8 where their number allows it, so that a head stays on its XCD.  What the
+// dQ kernel read last is still in the memory-side cache when the dK/dV kernel behind it starts, so that starts with those
+// heads.  Forward and backward in turn with heads from the front, us: 256x16x512 D=64 1166.5 -> 1158.8, fp32 32x20x1024 D=96 1135.6
+// -> 1130.4, 2x32x4096 D=128 1134.7 -> 1127.1; where everything fits that cache, alike.
+__host__ __device__ __forceinline__ int from_the_end(int bh, int heads) {
+  return heads % 8 ? heads - 1 - bh : (heads - 8 - (bh & ~7)) + (bh & 7);
+}
+
 // Order in which a grid that fits the chip at once takes its tiles.  Workgroups i, i + kCUs, i + 2 kCUs ...
 // of such a grid share a CU (they are handed out round-robin, all before the first one ends; read back from
 // the hardware id registers), and with tiles ordered by weight every CU would get the tiles of one weight

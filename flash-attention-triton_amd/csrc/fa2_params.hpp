@@ -71,6 +71,7 @@ struct BwdParams {
   float scale, scale_log2;
   int vec;
   bool grads_f32;  // dq, dk and dv are fp32 tensors (strides in fp32 elements)
+  bool last_heads_first;  // the dK/dV kernel takes the heads from the end: see from_the_end
 };
 
 // dQ and dK/dV in one grid: n_tiles and resident_grid of `both` are dK/dV's and the whole grid's.  (One record for both: a
