@@ -171,6 +171,15 @@ int fwd_wg_per_cu(int cfg, int groups) {
 // Kernel form, tiles and grid of a forward: completes `p` and returns the number of workgroups.
 int64_t plan_fwd(int cfg, fa2::FwdParams &p) {
   const int64_t bh = (int64_t)p.batch * p.nheads;
+  const int pairs = fa2::fwd_mixed_pairs(kTable[cfg].headdim_padded, p);
+  p.mixed_singles = 0;
+  if (pairs > 0) {
+    p.n_qtiles = (p.seqlen_q + 63) / 64;
+    p.mixed_singles = p.n_qtiles - 2 * pairs;
+    p.head_group = (int)((bh + 7) / 8 * 8);
+    p.resident_grid = 0;
+    return (p.mixed_singles + pairs) * bh;
+  }
   const int groups = fa2::fwd_key_groups(kTable[cfg].headdim_padded, p), block_q = kFwdBlockQ / groups;
   p.n_qtiles = (p.seqlen_q + block_q - 1) / block_q;
   const int64_t nwg = p.n_qtiles * bh;

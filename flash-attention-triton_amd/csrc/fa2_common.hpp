@@ -331,6 +331,24 @@ __host__ __device__ __forceinline__ int balanced_index(int i, int total) {
   return r / 8 < steps ? base + (steps - 1 - r / 8) * 8 + r % 8 : i;
 }
 
+// Order of a head's tiles in fwd_mixed_kernel, the longest first by the chain of a wave: of `tiles` tiles of 64 rows the last
+// `singles` are taken as they are, tile i with a chain of i + 1 blocks of 32 keys, and those in front two at a time, pair i
+// with a chain of 4 (i + 1).
+struct MixedPlace {
+  bool single;
+  int rank;  // among its own kind
+};
+__host__ __device__ __forceinline__ MixedPlace mixed_place(int pos, int tiles, int singles) {
+  const int pairs = (tiles - singles) / 2, lead = tiles - 4 * pairs;
+  const int first_singles = min(max(lead, 0), singles), first_pairs = max(-lead, 0) / 4;
+  if (pos < first_singles) return {true, pos};
+  if (pos < first_pairs) return {false, pos};
+  // Then a pair and four singles in turn, until there are no more singles.
+  const int left = singles - first_singles, i = pos - first_singles - first_pairs;
+  if (i >= left + (left + 3) / 4) return {false, pos - singles};
+  return i % 5 == 0 ? MixedPlace{false, first_pairs + i / 5} : MixedPlace{true, first_singles + i / 5 * 4 + i % 5 - 1};
+}
+
 }  // namespace fa2
 
 // ------------------------------------------------------------------------------------------

@@ -750,6 +750,27 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
       p, smem, [&]() -> int { return p.resident_grid ? balanced_index(blockIdx.x, p.resident_grid) : blockIdx.x; });
 }
 
+// One and two key groups in one grid: the last quarter of the rows, whose chains of blocks are the longest, in tiles of 64 with two
+// groups, the rows in front in tiles of 128 with one.  For grids of one to two rounds (fwd_mixed_pairs in fa2_launch.hpp): there the
+// launch lasts as long as the last tile's chain, beside which most CUs have nothing left, while two groups for all rows load every
+// K and V tile twice as often.  Heaviest first; what is not resident at once are the shortest tiles.  bf16, us: 10 x 5001 D=80
+// 69.7 -> 60.2, 12 x 5001 81.4 -> 73.4, 16 x 4096 D=96 71.0 -> 65.8, 16 x 4096 D=128 79.9 -> 76.4, 25 x 2048 D=64 27.1 -> 25.0.
+template <typename T, int DP, bool PRE, bool F32, int COLS = DP>
+__global__ __launch_bounds__(64 * kFwdWaves, 2) void fwd_mixed_kernel(const FwdParams p) {
+  __shared__ __attribute__((aligned(1024))) short smem[FwdDirectLayout<DP, kFwdBlockKV>::TOTAL_ELEMS];
+  const int heads = p.batch * p.nheads;
+  const int pos = blockIdx.x / heads, bh = blockIdx.x - pos * heads;
+  const MixedPlace at = mixed_place(pos, p.n_qtiles, p.mixed_singles);
+  const int index = at.rank * heads + bh;
+  if (at.single) {
+    fwd_direct<T, DP, kFwdBlockKV, false, PRE, 2, COLS, F32>(p, smem, [=]() { return index; });
+  } else {
+    FwdParams front = p;
+    front.n_qtiles = (p.n_qtiles - p.mixed_singles) / 2;
+    fwd_direct<T, DP, kFwdBlockKV, false, PRE, 1, COLS, F32>(front, smem, [=]() { return index; });
+  }
+}
+
 // Four key groups: a wave for each, 32 query rows, tiles of 128 keys.  For grids of so few workgroups that the chain of blocks of
 // one wave is what the launch takes (fwd_quad in fa2_launch.hpp has the rule): bf16, 2 x 4096 D=64 29.0 -> 19.6 us, 2 x 4096 D=80
 // 39.4 -> 29.6, 1 x 8192 D=128 89.4 -> 69.3.  At 128 columns three K and two V tiles are all of a CU's LDS, and the 160 KiB they

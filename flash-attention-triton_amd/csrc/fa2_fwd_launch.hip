@@ -52,6 +52,16 @@ void launch_direct(int dp, const FwdParams &p, dim3 grid, dim3 block, hipStream_
   }
 }
 
+template <typename T, bool PRE>
+void launch_mixed(const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
+  switch (p.headdim) {
+    case 64: hipLaunchKernelGGL((fwd_mixed_kernel<T, 64, PRE, kF32>), grid, block, 0, s, p); break;
+    case 80: hipLaunchKernelGGL((fwd_mixed_kernel<T, 96, PRE, kF32, 80>), grid, block, 0, s, p); break;
+    case 96: hipLaunchKernelGGL((fwd_mixed_kernel<T, 96, PRE, kF32>), grid, block, 0, s, p); break;
+    default: hipLaunchKernelGGL((fwd_mixed_kernel<T, 128, PRE, kF32>), grid, block, 0, s, p); break;
+  }
+}
+
 template <typename T, int KG>
 void launch_groups(int dp, bool folded, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
   if (folded)
@@ -63,6 +73,13 @@ void launch_groups(int dp, bool folded, const FwdParams &p, dim3 grid, dim3 bloc
 template <typename T>
 void launch(int dp, bool folded, const FwdParams &p, dim3 grid, hipStream_t s) {
   const dim3 block(64 * kFwdWaves);
+  if (p.mixed_singles > 0) {
+    if (folded)
+      launch_mixed<T, true>(p, grid, block, s);
+    else
+      launch_mixed<T, false>(p, grid, block, s);
+    return;
+  }
   if (fwd_direct_ok(dp, p)) {
     const int groups = fwd_key_groups(dp, p);
     if (groups == 4)

@@ -110,6 +110,30 @@ inline int fwd_key_groups(int dp, const FwdParams &p) {
   const int64_t heads = (int64_t)p.batch * p.nheads;
   return fwd_quad(dp, heads, p.seqlen_q) ? 4 : key_groups(dp, direct_columns(dp, p.headdim), heads, p.seqlen_q, false);
 }
+// One and two key groups in one grid (fwd_mixed_kernel): how many pairs of 64-row tiles of a head one group takes, 0 where all tiles
+// are of one kind.  Three eighths of the tiles, a little more on the larger grids, whose last round the smaller tiles would make
+// longer.  Time of one group over it, bf16, by workgroups of 128 rows; where two groups are the better ones (key_groups) it is
+// 0.94-1.05 of theirs:
+//   64 columns       to 512 1.02-1.11 (25 x 2048 1.08, 28 x 2048 1.11, 64 x 1024 1.02) to 3000 tokens; 0.97-1.0 from 4096 on and at 700
+//   80, 96 columns   to 456 1.01-1.04 at 1024 and 1500 tokens, 1.04-1.16 from 2048 on (10 x 5001 1.16, 17 x 3000 1.12, 14 x 4096 1.06);
+//                    to 520 0.92-0.96 to 1500 tokens, 1.01-1.09 from 2048 on (16 x 4096 1.05, 13 x 5001 1.09); to 576 (13/32 of the
+//                    tiles) 1.03-1.08 from 4096 on, 0.98-1.05 below; 0.83-1.01 beyond
+//   128 columns      to 520 1.03-1.09 from 4096 tokens on (10 x 5001 1.09, 16 x 4096 1.05), 0.95-1.06 below; to 576 1.01-1.05 from 4096
+//                    on; 0.87-1.0 beyond
+// At 32 columns 0.85-1.07 with no rule to it.  Padded heads and 48 columns have no such kernel.
+inline int fwd_mixed_pairs(int dp, const FwdParams &p) {
+  const int n = p.seqlen_q;
+  const int64_t heads = (int64_t)p.batch * p.nheads, wgs = heads * ((n + kFwdBlockQ - 1) / kFwdBlockQ);
+  if (wgs <= 3 * kCUs / 2 || wgs > 576 || !fwd_direct_ok(dp, p) || fwd_key_groups(dp, p) != 1) return 0;
+  bool mixed = false;
+  if (p.headdim == 64)
+    mixed = wgs <= 512 && n >= 1024 && n <= 3000;
+  else if (p.headdim == 80 || p.headdim == 96)
+    mixed = n >= (wgs <= 456 ? 1024 : wgs <= 520 ? 2048 : 4096);
+  else if (p.headdim == 128)
+    mixed = n >= 4096;
+  return mixed ? (n + 63) / 64 * (wgs <= 520 ? 12 : 13) / 32 : 0;
+}
 inline bool dq_direct_ok(int dp, const BwdParams &p) {
   return p.vec && direct_headdim_wide(dp, p.headdim) && direct_stride_ok(p.k) && direct_stride_ok(p.v);
 }

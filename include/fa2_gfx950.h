@@ -117,7 +117,8 @@ typedef struct fa2_launch_part {
   int form;         /* fa2_form */
   int block_rows;   /* query rows (forward, dQ) or key rows (dK/dV) per workgroup */
   int key_groups;   /* forward and dQ: 2 when two waves share 32 query rows and split the keys, 4 when four do
-                       (forward, fwd_quad_kernel), else 1 */
+                       (forward, fwd_quad_kernel), else 1; a forward grid that mixes one and two
+                       (fwd_mixed_kernel) states the tiles of one, and all of its workgroups */
   int wg_per_cu;    /* workgroups that share a CU (0: not stated, for the generic kernels) */
   int resident;
   int64_t workgroups;
