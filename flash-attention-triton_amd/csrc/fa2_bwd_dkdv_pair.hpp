@@ -15,9 +15,9 @@
 // instead, forms S and dP twice and waits for its staging registers: B=2 H=8 N=4096 D=256, bf16,
 // 756 -> 275 us (1000 TFLOP/s over the four products, 72 % of a large library matmul's rate on the same
 // card); D=192 (in one pass) 337 -> 220 us.  What bounds it now: one wave per SIMD, whose exponentials,
-// dS and exchange have only the wave's own MFMAs to hide under, and at 256 columns some fifty copies per
-// tile between the two halves of the register file (40 values live in accumulation registers that the
-// vector instructions cannot reach, 48 in the padded kernel; none in scratch memory).
+// dS and exchange have only the wave's own MFMAs to hide under.  K and V fragments and the accumulator fill the
+// accumulation registers (ResidentB in fa2_common.hpp); the loop copies nothing between the two halves of the register file
+// (463 instructions for its 64 MFMAs at 256 columns).
 //
 // At 128 columns and below one accumulator per wave lets two (three at 64) workgroups share a CU, and
 // workgroups of 64 keys fill the chip from fewer heads: dkdv_pair_ok (fa2_launch.hpp) says where that beats
@@ -154,15 +154,16 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem, P
   // next (the dO tile sits TILE_ELEMS behind); tlo, thi: transposed fragments of the tile this wave
   // contracts with (dO for role 0, Q for role 1), the wave's own block first.
   const lds_cptr lds0 = to_lds(smem);
-  lds_cptr qrow[KS], tlo[DB], thi[DB];
+  constexpr int NK = kept_addresses(LP, KS, 2), ND = kept_addresses(LP, DB, 4);
+  lds_cptr qrow[NK], tlo[ND], thi[ND];
 #pragma unroll
-  for (int ks = 0; ks < KS; ks++) qrow[ks] = lds0 + role * 32 * LP + swz_off<LP>(c, 2 * ks + h);
+  for (int ks = 0; ks < NK; ks++) qrow[ks] = lds0 + role * 32 * LP + swz_off<LP>(c, 2 * ks + h);
   {
     const int rowlo = 4 * h + (i16 >> 2);
     const int sub = (i16 & 1) * 4;
     const lds_cptr t0 = lds0 + (role ? 32 * LP : L::TILE_ELEMS);
 #pragma unroll
-    for (int db = 0; db < DB; db++) {
+    for (int db = 0; db < ND; db++) {
       const int chunk = 4 * db + 2 * g2 + ((i16 & 3) >> 1);
       tlo[db] = t0 + swz_off<LP>(rowlo, chunk) + sub;
       thi[db] = t0 + swz_off<LP>(rowlo + 8, chunk) + sub;
@@ -211,18 +212,19 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem, P
   }
   s16x8 ring[R];
 #pragma unroll
-  for (int ks = 0; ks < KS; ks++) ring[ks] = lds_read_128(qrow[ks]);
+  for (int ks = 0; ks < KS; ks++) ring[ks] = lds_read_128(qrow[ks % NK] + ks / NK * 128);
   // Every wave has its K and V fragments: stage 1 is free for its tile.
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __syncthreads();
   if (n_tiles > 1) issue_tile(1);
 
   auto t_frag = [&](int f, int block) -> s16x8 {
-    s16x4 a0 = lds_read_tr(tlo[f % DB] + block + 16 * (f / DB) * LP);
-    s16x4 a1 = lds_read_tr(thi[f % DB] + block + 16 * (f / DB) * LP);
+    s16x4 a0 = lds_read_tr(tlo[f % DB % ND] + f % DB / ND * 128 + block + 16 * (f / DB) * LP);
+    s16x4 a1 = lds_read_tr(thi[f % DB % ND] + f % DB / ND * 128 + block + 16 * (f / DB) * LP);
     return __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
   };
 
+  constexpr bool WIDE = DP > 128;  // one wave per SIMD: ResidentB
   // One 64-row query tile.  One barrier in its middle (two with a single exchange buffer):
   //     A: S = Q K^T of the own block         ring <- dO rows
   //     B: dP = dO V^T                        ring <- transposed fragments, own block; exponentials
@@ -238,11 +240,17 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem, P
     f32x16 s, dp;
     f32x4 l4[4], d4[4];
 #pragma unroll
-    for (int i = 0; i < 16; i++) s[i] = 0.f;
+    for (int i = 0; i < 16 && !WIDE; i++) s[i] = 0.f;
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
-      s = Elem<T>::mfma(ring[ks], kf[ks], s);
-      ring[ks] = lds_read_128(qrow[ks] + L::TILE_ELEMS);
+      if constexpr (WIDE) {
+        if (ks == 0) ResidentB<T>::zero(s, ring[ks], kf[ks]);
+        else if (SPREAD) ResidentB<T>::next_loaded(s, ring[ks], kf[ks]);
+        else ResidentB<T>::next(s, ring[ks], kf[ks]);
+      } else {
+        s = Elem<T>::mfma(ring[ks], kf[ks], s);
+      }
+      ring[ks] = lds_read_128(qrow[ks % NK] + ks / NK * 128 + L::TILE_ELEMS);
 #pragma unroll
       for (int g = part(4, KS, ks); g < part(4, KS, ks + 1); g++) {
         l4[g] = *reinterpret_cast<stat4_ptr>(stat + 8 * g);
@@ -257,9 +265,15 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem, P
                                  6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
-      dp = Elem<T>::mfma(ring[ks], vf[ks], dp);
+      if constexpr (WIDE) {
+        if (SPREAD && ks > 0) ResidentB<T>::next_loaded(dp, ring[ks], vf[ks]);
+        else ResidentB<T>::next(dp, ring[ks], vf[ks]);
+      } else {
+        dp = Elem<T>::mfma(ring[ks], vf[ks], dp);
+      }
       ring[ks] = t_frag(ks, 0);
       if (KS < R && ks == 0) ring[R - 1] = t_frag(R - 1, 0);  // the slot no dO row was in
+      if (WIDE && ks == 0) chain_end(s);
 #pragma unroll
       for (int i = part(16, KS, ks); i < part(16, KS, ks + 1); i++) {
         float x = fast_exp2(s[i] * scale_log2 - l4[i >> 2][i & 3]);
@@ -269,9 +283,10 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem, P
       asm volatile("" : "+v"(s));
       __builtin_amdgcn_sched_barrier(0);
     }
+    if (WIDE && role == 1) chain_end(dp);  // (role 0 takes dP up behind the first MFMA of its accumulator)
     // The own block is consumed; the row pointers move on to the next tile.
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) qrow[ks] += dstage;
+    for (int ks = 0; ks < NK; ks++) qrow[ks] += dstage;
     const s16x8 pf[2] = {Elem<T>::pack8(f32x8{s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7]}),
                          Elem<T>::pack8(f32x8{s[8], s[9], s[10], s[11], s[12], s[13], s[14], s[15]})};
     const int xoff = L::XBUFS == 2 ? (t & 1) * kDkvWaves * L::XCHG_WAVE : 0;
@@ -297,6 +312,7 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem, P
     for (int f = 0; f < R; f++) {
       acc[f % DB] = Elem<T>::mfma(ring[f], role ? df[f / DB] : pf[f / DB], acc[f % DB]);
       ring[f] = t_frag(f, other_block);
+      if (WIDE && role == 0 && f == 0) chain_end(dp);
       if (role == 0) {
 #pragma unroll
         for (int i = part(16, R, f); i < part(16, R, f + 1); i++) dp[i] = s[i] * dp[i];
@@ -322,7 +338,7 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem, P
 #pragma unroll
     for (int f = 0; f < R; f++) {
       acc[f % DB] = Elem<T>::mfma(ring[f], got[f / DB], acc[f % DB]);
-      if (f < KS) ring[f] = lds_read_128(qrow[f]);
+      if (f < KS) ring[f] = lds_read_128(qrow[f % NK] + f / NK * 128);
       if (SPREAD) {
 #pragma unroll
         for (int i = part(2 * LOADS, R, f); i < part(2 * LOADS, R, f + 1); i++) {
@@ -333,7 +349,7 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem, P
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
-    for (int db = 0; db < DB; db++) {
+    for (int db = 0; db < ND; db++) {
       tlo[db] += dstage;
       thi[db] += dstage;
     }

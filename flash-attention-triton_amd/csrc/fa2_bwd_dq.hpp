@@ -429,9 +429,10 @@ __device__ __forceinline__ void bwd_dq_direct(const BwdParams p, short *smem, Pl
   // Swizzled fragment addresses (32-bit LDS pointers).  knext: K rows of the tile the next block
   // lies in; vrow: V rows of the current tile; klo/khi: transposed K fragments of the current tile.
   const lds_cptr lds0 = to_lds(smem) + kg * BLK * LP;  // the key group's half of every tile
-  lds_cptr knext[KS], vrow[KS], klo[DB], khi[DB];
+  constexpr int NK = kept_addresses(LP, KS, 2), ND = kept_addresses(LP, DB, 4);
+  lds_cptr knext[NK], vrow[NK], klo[ND], khi[ND];
 #pragma unroll
-  for (int ks = 0; ks < KS; ks++) {
+  for (int ks = 0; ks < NK; ks++) {
     knext[ks] = lds0 + L::K_BASE + swz_off<LP>(c, 2 * ks + h);
     vrow[ks] = lds0 + L::V_BASE + swz_off<LP>(c, 2 * ks + h);
   }
@@ -439,7 +440,7 @@ __device__ __forceinline__ void bwd_dq_direct(const BwdParams p, short *smem, Pl
     const int rowlo = 4 * h + (i16 >> 2);
     const int sub = (i16 & 1) * 4;
 #pragma unroll
-    for (int db = 0; db < DB; db++) {
+    for (int db = 0; db < ND; db++) {
       const int chunk = 4 * db + 2 * g2 + ((i16 & 3) >> 1);
       klo[db] = lds0 + L::K_BASE + swz_off<LP>(rowlo, chunk) + sub;
       khi[db] = lds0 + L::K_BASE + swz_off<LP>(rowlo + 8, chunk) + sub;
@@ -459,7 +460,10 @@ __device__ __forceinline__ void bwd_dq_direct(const BwdParams p, short *smem, Pl
 
   // The dP chain of every block starts from -delta instead of zero (the MFMA's C operand), so that
   // dS = P * dP needs no subtraction.  Costs sixteen registers (255 of 256 in use at 128 columns).
-  const f32x16 dp_start = splat16(-delta);
+  // At 256 columns there are no sixteen registers left for that: there delta is subtracted.
+  constexpr bool LATE_DELTA = COLS == 256;
+  f32x16 dp_start;
+  if (!LATE_DELTA) dp_start = splat16(-delta);
 
   wait_vmem_all();
   __syncthreads();
@@ -473,7 +477,7 @@ __device__ __forceinline__ void bwd_dq_direct(const BwdParams p, short *smem, Pl
   // Ring of A fragments, preloaded with the K rows of block 0.
   s16x8 ring[R];
 #pragma unroll
-  for (int ks = 0; ks < KS; ks++) ring[ks] = lds_read_128(knext[ks]);
+  for (int ks = 0; ks < KS; ks++) ring[ks] = lds_read_128(knext[ks % NK] + ks / NK * 128);
   if (Q_STAGED && n_tiles > 1) {  // every wave has its Q fragments: their stages are free for K_2 and V_1 (if there are any)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __syncthreads();
@@ -486,6 +490,11 @@ __device__ __forceinline__ void bwd_dq_direct(const BwdParams p, short *smem, Pl
   //     C: dQ^T += K^T dS^T       ring <- next block's K rows second half of the dS arithmetic
   constexpr int LOADS = Loader::LOADS;
   constexpr int LOAD_EVERY = KS / LOADS;
+  constexpr bool WIDE = DP > 128;  // one wave per SIMD: ResidentB
+  // dO fragments that lie in accumulation registers: beside the Q rows and the accumulator half of them at 224 columns, none at
+  // 256.  (With more the compiler had no register left to move a value through: all of them at 256 columns were 324 bytes of scratch
+  // memory per lane.)
+  constexpr int G_AGPRS = COLS == 256 ? 0 : COLS > 192 ? KS / 2 : KS;
   // INNER blocks lie in tiles that end before the workgroup's first query row: they are every
   // wave's own and need no mask, so the two tests fold away.
   auto block = [&](int j, auto half_tag, auto spread_tag, auto inner_tag) __attribute__((always_inline)) {
@@ -503,12 +512,19 @@ __device__ __forceinline__ void bwd_dq_direct(const BwdParams p, short *smem, Pl
     const unsigned kdst = lds_base + 2u * (unsigned)(L::K_BASE + (kt % L::K_STAGES) * L::TILE_ELEMS);
     const unsigned vdst = lds_base + 2u * (unsigned)(L::V_BASE + (vt % L::V_STAGES) * L::TILE_ELEMS);
     constexpr int HOFF = HALF * BLK * LP;
-    f32x16 s = zero, dp;
+    f32x16 s, dp;
+    if (!WIDE) s = zero;
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
-      s = Elem<T>::mfma(ring[ks], qf[ks], s);
+      if constexpr (WIDE) {
+        if (ks == 0) ResidentB<T>::zero(s, ring[ks], qf[ks]);
+        else if (INNER) ResidentB<T>::next_loaded(s, ring[ks], qf[ks]);
+        else ResidentB<T>::next(s, ring[ks], qf[ks]);
+      } else {
+        s = Elem<T>::mfma(ring[ks], qf[ks], s);
+      }
       if (SPREAD && ks % LOAD_EVERY == 0 && ks / LOAD_EVERY < LOADS) vload.issue_one(vt * BKV, vdst, ks / LOAD_EVERY);
-      ring[ks] = lds_read_128(vrow[ks] + HOFF);
+      ring[ks] = lds_read_128(vrow[ks % NK] + ks / NK * 128 + HOFF);
       __builtin_amdgcn_sched_barrier(0);
     }
     if (!INNER && block_at(j) >= n_full) {
@@ -516,6 +532,7 @@ __device__ __forceinline__ void bwd_dq_direct(const BwdParams p, short *smem, Pl
       // statement keeps this a branch that interior blocks skip (the test is cheap enough that the
       // optimiser would otherwise run it for every block).
       asm volatile("");
+      if (WIDE) chain_end(s);
       const int lim = key_limit - block_at(j) * BLK;
 #pragma unroll
       for (int i = 0; i < 16; i++)
@@ -523,17 +540,27 @@ __device__ __forceinline__ void bwd_dq_direct(const BwdParams p, short *smem, Pl
     }
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
-      dp = Elem<T>::mfma(ring[ks], gf[ks], ks == 0 ? dp_start : dp);
+      if constexpr (WIDE) {
+        using G = ResidentB<T, (G_AGPRS > 0)>;
+        if (ks == 0 && LATE_DELTA) G::zero(dp, ring[ks], gf[ks]);
+        else if (ks == 0) G::from(dp, ring[ks], gf[ks], dp_start);
+        else if (ks >= G_AGPRS) INNER ? ResidentB<T, false>::next_loaded(dp, ring[ks], gf[ks]) : ResidentB<T, false>::next(dp, ring[ks], gf[ks]);
+        else INNER ? G::next_loaded(dp, ring[ks], gf[ks]) : G::next(dp, ring[ks], gf[ks]);
+      } else {
+        dp = Elem<T>::mfma(ring[ks], gf[ks], ks == 0 ? dp_start : dp);
+      }
       if (SPREAD && ks % LOAD_EVERY == 0 && ks / LOAD_EVERY < LOADS) kload.issue_one(kt * BKV, kdst, ks / LOAD_EVERY);
       {
-        s16x4 a0 = lds_read_tr(klo[ks % DB] + HOFF + 16 * (ks / DB) * LP);
-        s16x4 a1 = lds_read_tr(khi[ks % DB] + HOFF + 16 * (ks / DB) * LP);
+        s16x4 a0 = lds_read_tr(klo[ks % DB % ND] + ks % DB / ND * 128 + HOFF + 16 * (ks / DB) * LP);
+        s16x4 a1 = lds_read_tr(khi[ks % DB % ND] + ks % DB / ND * 128 + HOFF + 16 * (ks / DB) * LP);
         ring[ks] = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
       }
       if (KS < R && ks == 0) {  // the slot no V row was in
-        s16x4 a0 = lds_read_tr(klo[DB - 1] + HOFF + 16 * LP), a1 = lds_read_tr(khi[DB - 1] + HOFF + 16 * LP);
+        constexpr int AT = (DB - 1) % ND, FAR = (DB - 1) / ND * 128;
+        s16x4 a0 = lds_read_tr(klo[AT] + FAR + HOFF + 16 * LP), a1 = lds_read_tr(khi[AT] + FAR + HOFF + 16 * LP);
         ring[R - 1] = __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7);
       }
+      if (WIDE && ks == 0) chain_end(s);
 #pragma unroll
       for (int i = part(16, KS, ks); i < part(16, KS, ks + 1); i++) {
         s[i] = fast_exp2(s[i] * scale_log2 - lse2);
@@ -541,10 +568,11 @@ __device__ __forceinline__ void bwd_dq_direct(const BwdParams p, short *smem, Pl
       asm volatile("" : "+v"(s));
       __builtin_amdgcn_sched_barrier(0);
     }
+    if (WIDE) chain_end(dp);
     // dS of the first 16 keys before the dQ MFMAs that need them, the rest beside those MFMAs.
     f32x8 lo, hi;
 #pragma unroll
-    for (int i = 0; i < 8; i++) lo[i] = s[i] * dp[i];
+    for (int i = 0; i < 8; i++) lo[i] = s[i] * (LATE_DELTA ? dp[i] - delta : dp[i]);
     s16x8 dsf[2];
     dsf[0] = Elem<T>::pack8(lo);
 #pragma unroll
@@ -552,11 +580,11 @@ __device__ __forceinline__ void bwd_dq_direct(const BwdParams p, short *smem, Pl
       constexpr int HALF_SLOTS = R / 2;
       const int ks2 = slot / DB, db = slot % DB;
       dqacc[db] = Elem<T>::mfma(ring[slot], dsf[ks2], dqacc[db]);
-      if (slot < KS) ring[slot] = lds_read_128(knext[slot] + (HALF == 0 && KG == 1 ? BLK * LP : 0));
+      if (slot < KS) ring[slot] = lds_read_128(knext[slot % NK] + slot / NK * 128 + (HALF == 0 && KG == 1 ? BLK * LP : 0));
       if (slot < HALF_SLOTS) {
 #pragma unroll
         for (int i = part(8, HALF_SLOTS, slot); i < part(8, HALF_SLOTS, slot + 1); i++)
-          hi[i] = s[8 + i] * dp[8 + i];
+          hi[i] = s[8 + i] * (LATE_DELTA ? dp[8 + i] - delta : dp[8 + i]);
         asm volatile("" : "+v"(hi));
         if (slot == HALF_SLOTS - 1) dsf[1] = Elem<T>::pack8(hi);
       }
@@ -573,9 +601,9 @@ __device__ __forceinline__ void bwd_dq_direct(const BwdParams p, short *smem, Pl
     const int dk = k_step(t);
     const int dv = ((t + 1) % L::V_STAGES == 0) ? -(L::V_STAGES - 1) * L::TILE_ELEMS : L::TILE_ELEMS;
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) vrow[ks] += dv;
+    for (int ks = 0; ks < NK; ks++) vrow[ks] += dv;
 #pragma unroll
-    for (int db = 0; db < DB; db++) {
+    for (int db = 0; db < ND; db++) {
       klo[db] += dk;
       khi[db] += dk;
     }
@@ -585,7 +613,7 @@ __device__ __forceinline__ void bwd_dq_direct(const BwdParams p, short *smem, Pl
     // knext -> K tile t+1 before the tile's last block prefetches from it.
     const int dk = k_step(t);
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) knext[ks] += dk;
+    for (int ks = 0; ks < NK; ks++) knext[ks] += dk;
     if constexpr (KG == 1) block(2 * t + 1, std::integral_constant<int, 1>{}, std::false_type{}, spread_tag);
     else block(t, std::integral_constant<int, 0>{}, spread_tag, spread_tag);
     end_tile(t);

@@ -80,6 +80,42 @@ struct Elem<_Float16> {
   }
 };
 
+// The score and dP products of the kernels that run one wave per SIMD (from 160 columns on): the B operand, a fragment that stays
+// for the whole launch, lies in accumulation registers, where the MFMA reads it directly, and the result in vector registers.
+// Left to itself the compiler gives every MFMA result there accumulation registers and parks the fragments in others: per MFMA
+// four copies out of them for B, and one for each element of the result.  It does not know these are MFMAs.  An MFMA may read a
+// register two wait states after a vector instruction has written it: the s_nop 1 of the first one of a chain, and of all but
+// `next_loaded`, which is for loops whose operands come from LDS or were there before (tests/test_resident_fragments.py reads
+// the code for that).  `chain_end` supplies those that an 8-pass MFMA's result needs before a vector instruction reads it (11; the
+// s_nop gives 12).  One wave issues an instruction in 5 to 8 cycles, whatever its kind, so the copies were time.  bf16, us, forward /
+// backward: 16x4096 D=256 182.0 -> 163.9 / 479.9 -> 469.7, D=224 139.5 -> 126.6 / 433.3 -> 416.0, D=192 118.2 -> 114.7 / 384.7 ->
+// 371.4, D=160 112.2 -> 109.5 / 341.1 -> 327.6, 256x512 D=256 82.7 -> 77.2 / 264.4 -> 243.9.
+// (AGPR false: B in vector registers after all, where the accumulation registers are full.)
+template <typename T, bool AGPR = true>
+struct ResidentB;
+#define FA2_RESIDENT_B(T, AGPR, reg, op)                                                                           \
+  template <>                                                                                                      \
+  struct ResidentB<T, AGPR> {                                                                                      \
+    static __device__ __forceinline__ void zero(f32x16 &d, s16x8 a, s16x8 b) {                                     \
+      asm volatile("s_nop 1\n\t" op " %0, %1, %2, 0" : "=&v"(d) : "v"(a), reg(b));                                 \
+    }                                                                                                              \
+    static __device__ __forceinline__ void from(f32x16 &d, s16x8 a, s16x8 b, const f32x16 &c) {                    \
+      asm volatile("s_nop 1\n\t" op " %0, %1, %2, %3" : "=&v"(d) : "v"(a), reg(b), "v"(c));                        \
+    }                                                                                                              \
+    static __device__ __forceinline__ void next(f32x16 &d, s16x8 a, s16x8 b) {                                     \
+      asm volatile("s_nop 1\n\t" op " %0, %1, %2, %0" : "+v"(d) : "v"(a), reg(b));                                 \
+    }                                                                                                              \
+    static __device__ __forceinline__ void next_loaded(f32x16 &d, s16x8 a, s16x8 b) {                              \
+      asm volatile(op " %0, %1, %2, %0" : "+v"(d) : "v"(a), reg(b));                                               \
+    }                                                                                                              \
+  };
+FA2_RESIDENT_B(__bf16, true, "a", "v_mfma_f32_32x32x16_bf16")
+FA2_RESIDENT_B(__bf16, false, "v", "v_mfma_f32_32x32x16_bf16")
+FA2_RESIDENT_B(_Float16, true, "a", "v_mfma_f32_32x32x16_f16")
+FA2_RESIDENT_B(_Float16, false, "v", "v_mfma_f32_32x32x16_f16")
+#undef FA2_RESIDENT_B
+__device__ __forceinline__ void chain_end(f32x16 &d) { asm volatile("s_nop 11" : "+v"(d)); }
+
 // 32-bit pointer into LDS.
 typedef const __attribute__((address_space(3))) short *lds_cptr;
 __device__ __forceinline__ lds_cptr to_lds(const short *p) {
@@ -452,6 +488,11 @@ __device__ __forceinline__ void wait_vmem() {
 // needs a power-of-two number of 16-byte chunks per row, so 96 columns live in rows of 128: the
 // last four chunk slots of a row are never loaded and never read.
 constexpr int lds_pitch(int dp) { return dp == 96 ? 128 : dp == 192 ? 256 : dp; }
+
+// Fragment addresses a kernel keeps for `n` 16-column steps (two chunks each) or 32-column blocks (four) of a row.  In rows of 256
+// halves the swizzle changes the lower four bits of a chunk's number only, so that what lies 16 chunks further on is 128 halves
+// away, an immediate: half of the registers, and of the additions when the addresses move on to the next tile.
+constexpr int kept_addresses(int pitch, int n, int chunks_each) { return pitch == 256 && n > 16 / chunks_each ? 16 / chunks_each : n; }
 
 // Items [part(n, units, u), part(n, units, u + 1)) are unit u's share of n items spread as evenly
 // as integers allow over `units` units (equal shares when units divides n).

@@ -398,27 +398,28 @@ __device__ __forceinline__ void fwd_direct(const FwdParams p, short *smem, Place
   // Fragment addresses (swizzled, 32-bit LDS pointers).  kcur points into the stage of the K tile
   // after the current one, vcur into the stage of the current V tile; both advance by a uniform
   // amount per tile, and half-tile offsets are immediates.
-  lds_cptr kcur[KS], vlo[DB], vhi[DB];
+  constexpr int NK = kept_addresses(LP, KS, 2), ND = kept_addresses(LP, DB, 4);
+  lds_cptr kcur[NK], vlo[ND], vhi[ND];
   const lds_cptr lds0 = to_lds(smem);
   const lds_cptr half0 = lds0 + kg * BLK * LP;  // the key group's half of every tile
 #pragma unroll
-  for (int ks = 0; ks < KS; ks++) kcur[ks] = half0 + L::K_BASE + swz_off<LP>(c, 2 * ks + h);
+  for (int ks = 0; ks < NK; ks++) kcur[ks] = half0 + L::K_BASE + swz_off<LP>(c, 2 * ks + h);
   {
     const int rowlo = 4 * h + (i16 >> 2);
     const int sub = (i16 & 1) * 4;
 #pragma unroll
-    for (int db = 0; db < DB; db++) {
+    for (int db = 0; db < ND; db++) {
       const int chunk = 4 * db + 2 * g2 + ((i16 & 3) >> 1);
       vlo[db] = half0 + L::V_BASE + swz_off<LP>(rowlo, chunk) + sub;
       vhi[db] = half0 + L::V_BASE + swz_off<LP>(rowlo + 8, chunk) + sub;
     }
   }
   // K fragment ks of the half-tile `half` of the tile kcur points at.
-  auto k_frag = [&](int half, int ks) { return lds_read_128(kcur[ks] + half * BLK * LP); };
+  auto k_frag = [&](int half, int ks) { return lds_read_128(kcur[ks % NK] + ks / NK * 128 + half * BLK * LP); };
   // V^T fragment (k-step ks2 in {0,1} of half-tile `half`, head-dim block db) of the tile vcur points at.
   auto v_frag = [&](int half, int ks2, int db) -> s16x8 {
-    s16x4 lo = lds_read_tr(vlo[db] + half * BLK * LP + 16 * ks2 * LP);
-    s16x4 hi = lds_read_tr(vhi[db] + half * BLK * LP + 16 * ks2 * LP);
+    s16x4 lo = lds_read_tr(vlo[db % ND] + db / ND * 128 + half * BLK * LP + 16 * ks2 * LP);
+    s16x4 hi = lds_read_tr(vhi[db % ND] + db / ND * 128 + half * BLK * LP + 16 * ks2 * LP);
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   };
 
@@ -466,6 +467,17 @@ __device__ __forceinline__ void fwd_direct(const FwdParams p, short *smem, Place
     }
   }
 
+  constexpr bool WIDE = DP > 128;
+  static_assert(!(WIDE && PRE), "score chains of the wide kernels start from zero");
+  auto score_chain = [&](f32x16 &s, auto a) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+      if (ks == 0) ResidentB<T>::zero(s, a(ks), qf[ks]);
+      else ResidentB<T>::next(s, a(ks), qf[ks]);
+    }
+    chain_end(s);
+  };
+
   // ---- prologue: S_0, its row maximum, e_0 = exp2(scale*S_0 - scale*m), ring <- K fragments of
   // block 1 ---------------------------------------------------------------------------------
   s16x8 ring[R];
@@ -474,9 +486,13 @@ __device__ __forceinline__ void fwd_direct(const FwdParams p, short *smem, Place
   {
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) ring[ks] = k_frag(0, ks);
-    sc = zero;
+    if constexpr (WIDE) {
+      score_chain(sc, [&](int ks) { return ring[ks]; });
+    } else {
+      sc = zero;
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) sc = Elem<T>::mfma(ring[ks], qf[ks], sc);
+      for (int ks = 0; ks < KS; ks++) sc = Elem<T>::mfma(ring[ks], qf[ks], sc);
+    }
     if (block_at(0) >= n_full) apply_mask(sc, block_at(0) * BLK);
     if (KG > 1 && kg > 0) {
       // The second key group's first block is block 1 (and so on), which may hold nothing but keys above the diagonal or
@@ -487,8 +503,11 @@ __device__ __forceinline__ void fwd_direct(const FwdParams p, short *smem, Place
       // H=48 N=640 12.4 and 12.8, H=16 N=333 9.0 and 9.2) and long ones do not (B=1 H=8 N=4096, forward and
       // backward: 186.3 and 186.0 us).
       f32x16 s0 = zero;
+      if constexpr (WIDE) {
+        score_chain(s0, [&](int ks) { return lds_read_128(kcur[ks % NK] + ks / NK * 128 - (KG == 2 ? 1 : kg) * BLK * LP); });
+      } else
 #pragma unroll
-      for (int ks = 0; ks < KS; ks++) s0 = Elem<T>::mfma(lds_read_128(kcur[ks] - (KG == 2 ? 1 : kg) * BLK * LP), qf[ks], s0);
+      for (int ks = 0; ks < KS; ks++) s0 = Elem<T>::mfma(lds_read_128(kcur[ks % NK] + ks / NK * 128 - (KG == 2 ? 1 : kg) * BLK * LP), qf[ks], s0);
       if (n_full < 1) apply_mask(s0, 0);
       m_ref = row_max(s0);
     } else {
@@ -515,7 +534,7 @@ __device__ __forceinline__ void fwd_direct(const FwdParams p, short *smem, Place
     }
     // From here on kcur addresses K tile 1 (the tile after the current one).
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) kcur[ks] += L::TILE_ELEMS;
+    for (int ks = 0; ks < NK; ks++) kcur[ks] += L::TILE_ELEMS;
   }
   // V_0 and K_1 have landed, and every wave has taken its Q fragments out of the two stages that
   // the first tile's loads (K_2, V_1) are about to overwrite.
@@ -523,10 +542,9 @@ __device__ __forceinline__ void fwd_direct(const FwdParams p, short *smem, Place
   __syncthreads();
   if (KG > 1) {  // the next block is the group's half of tile 1; kcur moves on to tile 2
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-      ring[ks] = k_frag(0, ks);
-      kcur[ks] += L::TILE_ELEMS;
-    }
+    for (int ks = 0; ks < KS; ks++) ring[ks] = k_frag(0, ks);
+#pragma unroll
+    for (int ks = 0; ks < NK; ks++) kcur[ks] += L::TILE_ELEMS;
   }
 
   // PRE: the C operand every later score chain starts from.
@@ -579,10 +597,16 @@ __device__ __forceinline__ void fwd_direct(const FwdParams p, short *smem, Place
     const unsigned vdst = lds_base + 2u * (unsigned)(L::V_BASE + (vt % L::V_STAGES) * L::TILE_ELEMS);
     typedef unsigned u32x4v __attribute__((ext_vector_type(4)));
     u32x4v w[2];  // packed probabilities, two per word: w[0] = k-step 0, w[1] = k-step 1
-    if (!PRE) sc = zero;
+    if (!PRE && !WIDE) sc = zero;
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
-      sc = Elem<T>::mfma(ring[ks], qf[ks], (PRE && ks == 0) ? negm : sc);
+      if constexpr (WIDE) {
+        if (ks == 0) ResidentB<T>::zero(sc, ring[ks], qf[ks]);
+        else if (INNER) ResidentB<T>::next_loaded(sc, ring[ks], qf[ks]);
+        else ResidentB<T>::next(sc, ring[ks], qf[ks]);
+      } else {
+        sc = Elem<T>::mfma(ring[ks], qf[ks], (PRE && ks == 0) ? negm : sc);
+      }
       if (SPREAD) {
 #pragma unroll
         for (int i = first_load(ks); i < first_load(ks + 1); i++) vload.issue_one(vt * BKV, vdst, i);
@@ -600,7 +624,10 @@ __device__ __forceinline__ void fwd_direct(const FwdParams p, short *smem, Place
     }
     // S_{j+1} of a SPREAD step is the second half of a tile that ends before the workgroup's first
     // query row: never masked.  (The step after it may produce the first block of the diagonal.)
-    if (!SPREAD && block_at(j + 1) >= n_full) apply_mask(sc, block_at(j + 1) * BLK);
+    if (!SPREAD && block_at(j + 1) >= n_full) {
+      if (WIDE) chain_end(sc);
+      apply_mask(sc, block_at(j + 1) * BLK);
+    }
     const s16x8 pf[2] = {__builtin_bit_cast(s16x8, w[0]), __builtin_bit_cast(s16x8, w[1])};
     const float mc = m_ref * scale_log2;
     float lsum[2] = {0.f, 0.f};  // this lane's sum of the new probabilities, in two chains
@@ -615,6 +642,7 @@ __device__ __forceinline__ void fwd_direct(const FwdParams p, short *smem, Place
           for (int i = first_load(slot); i < first_load(slot + 1); i++) kload.issue_one(kt * BKV, kdst, i);
         }
         if (slot < KS) ring[slot] = k_frag(HALF, slot);
+        if (WIDE && slot == 0) chain_end(sc);
 #pragma unroll
         for (int i = part(16, R, slot); i < part(16, R, slot + 1); i++) {
           e[i] = PRE ? fast_exp2(sc[i]) : fast_exp2(sc[i] * scale_log2 - mc);
@@ -664,9 +692,9 @@ __device__ __forceinline__ void fwd_direct(const FwdParams p, short *smem, Place
     const int dk = ((t + K_AHEAD) % L::K_STAGES == 0) ? -(L::K_STAGES - 1) * L::TILE_ELEMS : L::TILE_ELEMS;
     const int dv = ((t + 1) % L::V_STAGES == 0) ? -(L::V_STAGES - 1) * L::TILE_ELEMS : L::TILE_ELEMS;
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) kcur[ks] += dk;
+    for (int ks = 0; ks < NK; ks++) kcur[ks] += dk;
 #pragma unroll
-    for (int db = 0; db < DB; db++) {
+    for (int db = 0; db < ND; db++) {
       vlo[db] += dv;
       vhi[db] += dv;
     }

@@ -1,0 +1,83 @@
+"""The inline-assembly MFMAs of the kernels from 160 columns on (ResidentB in csrc/fa2_common.hpp), which the compiler's hazard
+recogniser does not see: in the code it made, no MFMA reads a register that one of the two wait states before it wrote on the
+vector unit, and no vector instruction reads a score chain's result before its wait states are over."""
+
+from __future__ import annotations
+
+import pathlib
+import re
+import subprocess
+
+import pytest
+
+from tests.test_code_objects import LLVM, _kernel_records
+
+OBJDUMP = LLVM / "llvm-objdump"
+SOURCES = r"[va]\[?\d+(?::\d+)?\]?"
+
+
+def _registers(operand: str) -> set:
+    m = re.fullmatch(r"([va])(?:(\d+)|\[(\d+):(\d+)\])", operand)
+    if not m:
+        return set()
+    first = int(m.group(2) or m.group(3))
+    return {(m.group(1), i) for i in range(first, int(m.group(4) or first) + 1)}
+
+
+def _operands(line: str) -> list[str]:
+    return re.findall(SOURCES, line.split("//")[0].partition(" ")[2])
+
+
+def _hazards(lines: list[str]) -> list[str]:
+    """`lines`: one kernel's instructions in order.  Branches are not followed: what a block starts with has its s_nop."""
+    found = []
+    written: list[tuple[int, set]] = []  # (wait state, registers) of vector instructions
+    chain: list = []  # [registers, wait state of issue] of the last result in vector registers
+    now = 0
+    for text in lines:
+        op = text.split()[0]
+        if op == "s_nop":
+            now += int(text.split()[1], 0) + 1
+            continue
+        operands = _operands(text)
+        if op.startswith("v_mfma_f32_32x32x16"):
+            reads = set().union(*(_registers(o) for o in operands[1:]))
+            if any(now - at <= 2 and regs & reads for at, regs in written[-3:]):
+                found.append(f"written too late for: {text}")
+            chain = [_registers(operands[0]), now] if operands[0].startswith("v") else []
+        elif op.startswith("v_"):
+            if chain and now - chain[1] <= 11 and set().union(set(), *(_registers(o) for o in operands)) & chain[0]:
+                found.append(f"result not there yet: {text}")
+            if operands:
+                written.append((now, _registers(operands[0])))
+        now += 1
+    return found
+
+
+def test_the_check_sees_both_mistakes():
+    mfma = "v_mfma_f32_32x32x16_bf16 v[0:15], v[16:19], a[0:3], v[0:15]"
+    assert _hazards(["v_accvgpr_write_b32 a3, v40", mfma]) and _hazards(["v_mov_b32_e32 v16, v40", "s_nop 0", mfma])
+    assert not _hazards(["v_accvgpr_write_b32 a3, v40", "s_nop 1", mfma]) and not _hazards(["v_mov_b32_e32 v20, v40", mfma])
+    assert _hazards([mfma, "s_nop 9", "v_exp_f32_e32 v50, v3"]) and not _hazards([mfma, "s_nop 11", "v_exp_f32_e32 v50, v3"])
+
+
+def test_no_operand_is_written_too_late_and_no_result_read_too_early(tmp_path):
+    import importlib
+
+    capi = importlib.import_module("flash-attention-triton_amd._capi")
+    if not capi.LIBRARY_PATH.exists() or not OBJDUMP.exists():
+        pytest.skip("library not built, or no ROCm LLVM tools")
+    _kernel_records(capi.LIBRARY_PATH, tmp_path)  # unbundles the code objects
+    wide = re.compile(r"<(_ZN3fa2\d+\w*kernelI(?:DF16b|DF16_)Li(?:192|256)E\w*)>:")
+    checked = 0
+    for obj in sorted(tmp_path.glob("code*.o")):
+        listing = subprocess.run([str(OBJDUMP), "-d", "--no-show-raw-insn", "--no-leading-addr", str(obj)], check=True,
+                                 capture_output=True, text=True).stdout
+        for part in re.split(r"\n(?=(?:[0-9a-f]+ )?<_ZN3fa2)", listing):
+            name = wide.search(part[:400])
+            if not name or not re.search(r"fwd_direct_kernel|fwd_full_kernel|dq_direct_kernel|pair_kernel|joint_kernel", name.group(1)):
+                continue
+            lines = [s for s in (line.strip() for line in part.split("\n")[1:]) if s and not s.startswith("<")]
+            assert not (bad := _hazards(lines)), (name.group(1), bad[:3])
+            checked += sum(s.startswith("v_mfma_f32_32x32x16") for s in lines) > 0
+    assert checked >= 100
