@@ -778,6 +778,17 @@ __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direc
       p, smem, [&]() -> int { return p.resident_grid ? balanced_index(blockIdx.x, p.resident_grid) : blockIdx.x; });
 }
 
+// A head dimension of exactly 256.  The padded kernel, which these took too, switches the lanes of every tile load on and off by
+// a register, with a branch around the load: a fifth of its loop's instructions, and instructions are what one wave per SIMD is
+// bound by.  (Before ResidentB this form spilled about forty registers.)  bf16, us: 16x4096
+// 163.9 -> 155.7, 256x512 77.2 -> 73.7, 8x2048 42.6 -> 39.2, 100x200 20.9 -> 18.7.
+template <typename T, int KG, bool F32, int COLS = 256>
+__global__ __launch_bounds__(64 * kFwdWaves, 1) void fwd_full_kernel(const FwdParams p) {
+  __shared__ __attribute__((aligned(1024))) short smem[FwdDirectLayout<COLS, kFwdBlockKV>::TOTAL_ELEMS];
+  fwd_direct<T, COLS, kFwdBlockKV, false, false, KG, COLS, F32>(
+      p, smem, [&]() -> int { return p.resident_grid ? balanced_index(blockIdx.x, p.resident_grid) : blockIdx.x; });
+}
+
 // One and two key groups in one grid: the last quarter of the rows, whose chains of blocks are the longest, in tiles of 64 with two
 // groups, the rows in front in tiles of 128 with one.  For grids of one to two rounds (fwd_mixed_pairs in fa2_launch.hpp): there the
 // launch lasts as long as the last tile's chain, beside which most CUs have nothing left, while two groups for all rows load every

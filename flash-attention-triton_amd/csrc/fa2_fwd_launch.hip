@@ -19,11 +19,8 @@ void launch_generic(int dp, const FwdParams &p, dim3 grid, dim3 block, hipStream
   }
 }
 
-// PRE (exponents straight from the score MFMAs) is instantiated up to 128 columns: the sixteen registers
-// of the chain's start value are more than the 256-column kernel has left.  The 192- and 256-column
-// kernels live in a translation unit of their own (fa2_fwd_launch_wide.hip): compiled beside the
-// narrower instantiations the 256-column kernel, which uses all 512 registers, came out with 40-60
-// spilled registers and reloads inside its tile loop; alone and in its padded form only it spills none.
+// PRE (exponents straight from the score MFMAs) is instantiated up to 128 columns.  The kernels of 160 columns and more live in a
+// translation unit of their own (fa2_fwd_launch_wide.hip), for the time that they take to compile.
 template <typename T, int DP, int COLS, bool PRE, int KG>
 void launch_cols(const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
   if constexpr (KG == 4) {

@@ -8,25 +8,27 @@ namespace {
 
 constexpr bool kF32 = FA2_F32_OUT;
 
-// At 256 columns only the padded variant is instantiated, also for a head dimension of exactly 256
-// (it then switches no lane off): with the number of columns a run-time value the compiler keeps the
-// kernel within its 512 registers, with a constant 256 it spills about forty of them, with reloads
-// inside the tile loop, where they queue behind the tile loads (same counter).
-template <typename T, int DP, int COLS, int KG, bool PADDED_ONLY>
+template <typename T, int DP, int COLS, int KG>
 void launch_cols(const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
-  if (!PADDED_ONLY && p.headdim == COLS)
-    hipLaunchKernelGGL((fwd_direct_kernel<T, DP, kFwdBlockKV, PADDED_ONLY, false, KG, COLS, kF32>), grid, block, 0, s, p);
-  else
-    hipLaunchKernelGGL((fwd_direct_kernel<T, DP, kFwdBlockKV, true, false, KG, COLS, kF32>), grid, block, 0, s, p);
+  if constexpr (COLS == 256) {
+    if (p.headdim == COLS) {
+      hipLaunchKernelGGL((fwd_full_kernel<T, KG, kF32>), grid, block, 0, s, p);
+      return;
+    }
+  } else if (p.headdim == COLS) {
+    hipLaunchKernelGGL((fwd_direct_kernel<T, DP, kFwdBlockKV, false, false, KG, COLS, kF32>), grid, block, 0, s, p);
+    return;
+  }
+  hipLaunchKernelGGL((fwd_direct_kernel<T, DP, kFwdBlockKV, true, false, KG, COLS, kF32>), grid, block, 0, s, p);
 }
 
 template <typename T, int KG>
 void launch_wide(int dp, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
   switch (direct_columns(dp, p.headdim)) {
-    case 160: launch_cols<T, 192, 160, KG, false>(p, grid, block, s); break;
-    case 192: launch_cols<T, 192, 192, KG, false>(p, grid, block, s); break;
-    case 224: launch_cols<T, 256, 224, KG, false>(p, grid, block, s); break;
-    default: launch_cols<T, 256, 256, KG, true>(p, grid, block, s); break;
+    case 160: launch_cols<T, 192, 160, KG>(p, grid, block, s); break;
+    case 192: launch_cols<T, 192, 192, KG>(p, grid, block, s); break;
+    case 224: launch_cols<T, 256, 224, KG>(p, grid, block, s); break;
+    default: launch_cols<T, 256, 256, KG>(p, grid, block, s); break;
   }
 }
 

@@ -4,11 +4,13 @@ vector unit, and no vector instruction reads a score chain's result before its w
 
 from __future__ import annotations
 
+import math
 import pathlib
 import re
 import subprocess
 
 import pytest
+import torch
 
 from tests.test_code_objects import LLVM, _kernel_records
 
@@ -67,7 +69,8 @@ def test_no_operand_is_written_too_late_and_no_result_read_too_early(tmp_path):
     capi = importlib.import_module("flash-attention-triton_amd._capi")
     if not capi.LIBRARY_PATH.exists() or not OBJDUMP.exists():
         pytest.skip("library not built, or no ROCm LLVM tools")
-    _kernel_records(capi.LIBRARY_PATH, tmp_path)  # unbundles the code objects
+    full = [r for r in _kernel_records(capi.LIBRARY_PATH, tmp_path) if "fwd_full_kernel" in r["name"]]  # (unbundles the code objects)
+    assert len(full) == 8 and all(int(r["private_segment_fixed_size"]) == 0 and int(r["vgpr_count"]) <= 512 for r in full)
     wide = re.compile(r"<(_ZN3fa2\d+\w*kernelI(?:DF16b|DF16_)Li(?:192|256)E\w*)>:")
     checked = 0
     for obj in sorted(tmp_path.glob("code*.o")):
@@ -81,3 +84,34 @@ def test_no_operand_is_written_too_late_and_no_result_read_too_early(tmp_path):
             assert not (bad := _hazards(lines)), (name.group(1), bad[:3])
             checked += sum(s.startswith("v_mfma_f32_32x32x16") for s in lines) > 0
     assert checked >= 100
+
+
+# fp16 rounds P and O to 11 bits, bf16 to 8: a relative 2-norm below one unit, 5e-4 and 4e-3; gradients, whose dS is a difference of
+# rounded values, twice that.
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,nq,nk,d,dtype", [
+    (300, 129, 129, 256, torch.bfloat16), (16, 333, 300, 256, torch.float16), (3, 65, 1, 256, torch.float32), (70, 512, 520, 256, torch.float16),
+    (33, 1100, 1100, 224, torch.bfloat16), (16, 700, 650, 216, torch.float16), (40, 1025, 1025, 192, torch.bfloat16),
+    (16, 2000, 129, 160, torch.float16)], ids=lambda x: str(x).replace("torch.", ""))
+def test_wide_heads_match_64_bits(heads, nq, nk, d, dtype):
+    import flash_attention_triton_amd as fa
+
+    gen = torch.Generator(device="cuda").manual_seed(d + nq)
+    q, k, v, g = (torch.randn((1, heads, n, d), generator=gen, device="cuda").to(dtype) for n in (nq, nk, nk, nq))
+    for x in (q, k, v):
+        x.requires_grad_(True)
+    out = fa.flash_attention_v2(q, k, v)
+    got = [out.detach(), *torch.autograd.grad(out, (q, k, v), g)]
+    at = [0, heads - 1]
+    qd, kd, vd = (x[0, at].detach().double().requires_grad_(True) for x in (q, k, v))
+    s = qd @ kd.transpose(1, 2).contiguous() / math.sqrt(d)
+    s = s.masked_fill(torch.arange(nk, device="cuda")[None] > torch.arange(nq, device="cuda")[:, None], -math.inf)
+    o = torch.softmax(s, -1) @ vd
+    want = [o.detach(), *torch.autograd.grad(o, (qd, kd, vd), g[0, at].double())]
+    unit = 4e-3 if dtype == torch.bfloat16 else 5e-4
+    for name, x, w in zip(("o", "dq", "dk", "dv"), got, want):
+        if nk == 1 and name in ("dq", "dk"):  # a softmax of one key has no gradient: rounding against the size of its summands
+            assert x[0, at].double().abs().max() < 1e-2
+            continue
+        err = (x[0, at].double() - w).norm() / w.norm()
+        assert err < unit * (1 if name == "o" else 2), (name, err.item())
