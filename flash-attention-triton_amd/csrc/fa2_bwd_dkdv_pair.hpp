@@ -65,7 +65,7 @@ __device__ __forceinline__ void bwd_dkdv_pair(const BwdParams &p, short *smem, P
   using L = DkvPairLayout<DP>;
   constexpr int BQ = L::BQ, KS = COLS / 16, DB = (COLS + 31) / 32, R = 2 * DB, LP = L::LP;
   constexpr int NTHREADS = 64 * kDkvWaves;
-  using Loader = TileLoader<DP, BQ, kDkvWaves, PAD || COLS != DP>;
+  using Loader = TileLoader<DP, BQ, kDkvWaves, PAD>;
   constexpr int LOADS = Loader::LOADS;
 
   const int tid = threadIdx.x;

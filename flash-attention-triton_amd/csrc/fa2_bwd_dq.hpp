@@ -335,7 +335,7 @@ __device__ __forceinline__ void bwd_dq_direct(const BwdParams p, short *smem, Pl
   const short *DO = (const short *)p.d_o.ptr + b * p.d_o.stride_batch + hd * p.d_o.stride_head;
 
   const int hdim = PAD ? p.headdim : COLS;
-  using Loader = TileLoader<DP, BKV, kDqWaves, PAD || COLS != DP>;
+  using Loader = TileLoader<DP, BKV, kDqWaves, PAD>;
   const Loader kload(K, p.k.stride_seq, hdim / 8), vload(V, p.v.stride_seq, hdim / 8);
   const int seqlen_k = p.seqlen_k;
   const float scale_log2 = p.scale_log2;

@@ -516,9 +516,12 @@ __device__ __forceinline__ void zero_lds(short *smem, int elems) {
 
 // Streams ROWS x DP tiles of a (seqlen, headdim) matrix into swizzled LDS (row pitch lds_pitch(DP))
 // with LDS-direct loads.  All NW waves of the workgroup take part; each wave issues LOADS loads of
-// 1 KiB of LDS per tile.  A lane owns one 16-byte slot of a row; lanes whose slot holds no data
-// (DP < pitch, or with PAD a head dimension of `chunks` 16-byte chunks below DP) are switched off
-// for the load.
+// 1 KiB of LDS per tile.  A lane owns one 16-byte slot of a row.  With PAD (a head dimension of `chunks` 16-byte chunks below the
+// columns multiplied) lanes whose slot holds no data are switched off for the load: their slots stay zero.  Without, what lies
+// behind a row's `chunks` is not multiplied, or into rows that are not stored, and those lanes load the row's last chunk once
+// more, from a line that the load touches anyway: no branch around each load, no mask to set and restore.  (Switched off like those
+// of PAD before: bf16, us, forward / backward: 640x1024 D=96 fp16 218 -> 209 / 622 -> 618, 64x2048 D=80 58.6 -> 57.4 / 181 -> 178,
+// 2048x512 D=48 111 -> 111 / 364 -> 349, 16x4096 D=160 113.5 -> 103.1 / 336 -> 321, D=192 114.8 -> 112.7 / 365 -> 358.)
 template <int DP, int ROWS, int NW, bool PAD = false>
 struct TileLoader {
   static constexpr int LP = lds_pitch(DP);
@@ -546,7 +549,7 @@ struct TileLoader {
   unsigned voff_odd;
   bool active_odd;
 
-  static constexpr bool ALL_ACTIVE = LP == DP && !PAD;  // every slot of a row holds data
+  static constexpr bool ALL_ACTIVE = !PAD;
 
   // Wave-load i of wave `wave` fills LDS bytes [(i * NW + wave) * 1024, + 1024) of the tile, lane l
   // the 16 bytes at 16 * l: slot l % CPR of tile row i * NW * RPL + wave * RPL + l / CPR.  This is the
@@ -562,10 +565,14 @@ struct TileLoader {
     wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     row_in = wave * RPL + lane / CPR;
     chunk = (lane % CPR) ^ swz<LP>(row_in);  // == chunk_of(lane, wave, 0)
-    active = ALL_ACTIVE || chunk < (PAD ? chunks : DP / 8);
-    voff = 2u * (unsigned)(row_in * (int)stride + chunk * 8);
     chunk_odd = BY_PARITY ? chunk ^ 2 : chunk;  // == chunk_of(lane, wave, odd i), see BY_PARITY
-    active_odd = ALL_ACTIVE || chunk_odd < (PAD ? chunks : DP / 8);
+    active = ALL_ACTIVE || chunk < chunks;
+    active_odd = ALL_ACTIVE || chunk_odd < chunks;
+    if (!PAD) {
+      chunk = min(chunk, chunks - 1);
+      chunk_odd = min(chunk_odd, chunks - 1);
+    }
+    voff = 2u * (unsigned)(row_in * (int)stride + chunk * 8);
     voff_odd = 2u * (unsigned)(row_in * (int)stride + chunk_odd * 8);
   }
 

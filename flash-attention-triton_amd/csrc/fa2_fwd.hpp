@@ -341,7 +341,7 @@ __device__ __forceinline__ void fwd_direct(const FwdParams p, short *smem, Place
   float *LSE = p.lse + (int64_t)bh * p.seqlen_q_rounded;
 
   const int hdim = PAD ? p.headdim : COLS;
-  using Loader = TileLoader<DP, BKV, kFwdWaves, PAD || COLS != DP>;
+  using Loader = TileLoader<DP, BKV, kFwdWaves, PAD>;
   const Loader kload(K, p.k.stride_seq, hdim / 8), vload(V, p.v.stride_seq, hdim / 8);
   const int seqlen_k = p.seqlen_k;
   const float scale_log2 = p.scale_log2;
@@ -384,7 +384,7 @@ __device__ __forceinline__ void fwd_direct(const FwdParams p, short *smem, Place
   constexpr unsigned Q_LO = KG == 1 ? 2u * (unsigned)(L::K_BASE + 2 * L::TILE_ELEMS) : Q_HI;
   constexpr int K_AHEAD = KG == 1 ? 2 : 3;  // tile t loads K tile t + K_AHEAD
   constexpr int QROWS = KG == 4 && DP > 32 ? 32 : 64;  // (rows of 32 halves: a tile of 32 is less than one load per wave)
-  const TileLoader<DP, QROWS, kFwdWaves, PAD || COLS != DP> qload(Q + (int64_t)q0 * p.q.stride_seq, p.q.stride_seq, hdim / 8);
+  const TileLoader<DP, QROWS, kFwdWaves, PAD> qload(Q + (int64_t)q0 * p.q.stride_seq, p.q.stride_seq, hdim / 8);
   const int q_rows = p.seqlen_q - q0;  // rows of this query tile that exist (>= 1)
   issue_k(0);
   if (q_rows >= QROWS) qload.issue(0, lds_base + Q_LO); else qload.issue_clamped(0, q_rows, lds_base + Q_LO);
