@@ -415,8 +415,7 @@ int bwd_impl(const fa2_bwd_args &a, void *stream, bool grads_f32 = false) {
     }
     fa2::JointParams j;
     j.both = p;
-    const int64_t nwg = plan_joint(cfg, groups, j);
-    if (nwg > fa2::kMaxWorkgroups) return fail(FA2_ERR_TOO_LARGE, "grid of %lld workgroups too large", (long long)nwg);
+    const int64_t nwg = plan_joint(cfg, groups, j);  // (joint_fits: no more than can be launched)
     (bf16 ? fa2::launch_joint<__bf16> : fa2::launch_joint<_Float16>)(dp, j, groups, dim3((unsigned)nwg), s);
     return launch_status("backward dQ, dK and dV launch");
   }

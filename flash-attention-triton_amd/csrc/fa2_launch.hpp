@@ -182,6 +182,13 @@ inline bool seqpar_atomic_ok(int dp, const BwdParams &p) {
   return dkdv_direct_ok(dp, p) && p.headdim == dp && (dp == 32 || dp == 64 || dp == 128);
 }
 
+// The order of a joint grid, in runs of 8 workgroups that keep heads on their XCDs: every joint_period-th run is of dQ.  A
+// workgroup of dQ has twice the rows of one of dK/dV, or with two key groups as many.
+__host__ __device__ constexpr int joint_period(int key_groups) { return key_groups == 1 ? 3 : 2; }
+constexpr int64_t joint_workgroups(int64_t n_dq, int64_t n_dkdv, int period) {
+  const int64_t rounds_dq = (n_dq + 7) / 8, rounds_dkdv = (n_dkdv + 8 * (period - 1) - 1) / (8 * (period - 1));
+  return (rounds_dq > rounds_dkdv ? rounds_dq : rounds_dkdv) * 8 * period;
+}
 // Whether dQ and dK/dV run in one grid (fa2_bwd_joint.hpp) behind a launch that forms delta, and with how many key groups
 // dQ: 0 where two launches are as fast, dQ forming delta for dK/dV.  Time of the two over that of delta and the joint grid,
 // bf16, (batch, head) pairs x tokens, by workgroups of 128 query rows; in brackets the other number of key groups:
@@ -199,7 +206,7 @@ inline bool seqpar_atomic_ok(int dp, const BwdParams &p) {
 //               1.02-1.09; 256 columns 1.05-1.26 to 1100 tokens, 0.93-0.97 past them.  Padded heads (112, 224) and heads that do not
 //               divide by 8 0.93-1.03 there
 // The paired dK/dV kernel's conditions hold (below): where the other one is the better one, dK/dV is no part of such a grid.
-inline int joint_key_groups(int dp, const BwdParams &p) {
+inline int joint_key_groups_by_size(int dp, const BwdParams &p) {
   if (!dq_direct_ok(dp, p) || !dkdv_pair_ok(dp, p)) return 0;
   const int64_t heads = (int64_t)p.batch * p.nheads, wgs = heads * ((p.seqlen_q + kDqBlockQ - 1) / kDqBlockQ);
   const int n = p.seqlen_q;
@@ -213,12 +220,18 @@ inline int joint_key_groups(int dp, const BwdParams &p) {
   if (dp == 192) return large ? wgs >= 1200 && n > 192 && n <= 1100 : wgs <= 384 && n > 128;
   return n >= 96 && (large ? n <= 1100 : wgs <= 384);
 }
-// The order of a joint grid, in runs of 8 workgroups that keep heads on their XCDs: every joint_period-th run is of dQ.  A
-// workgroup of dQ has twice the rows of one of dK/dV, or with two key groups as many.
-__host__ __device__ constexpr int joint_period(int key_groups) { return key_groups == 1 ? 3 : 2; }
-constexpr int64_t joint_workgroups(int64_t n_dq, int64_t n_dkdv, int period) {
-  const int64_t rounds_dq = (n_dq + 7) / 8, rounds_dkdv = (n_dkdv + 8 * (period - 1) - 1) / (8 * (period - 1));
-  return (rounds_dq > rounds_dkdv ? rounds_dq : rounds_dkdv) * 8 * period;
+// Whether such a grid can be launched, and the one that forms delta in front of it: a joint grid has up to three times the workgroups
+// of its larger kind.  Where not, two launches run, each with a limit of its own.
+inline bool joint_fits(const BwdParams &p, int key_groups) {
+  const int64_t heads = (int64_t)p.batch * p.nheads;
+  const int64_t n_dq = heads * ((p.seqlen_q + kDqBlockQ / key_groups - 1) / (kDqBlockQ / key_groups));
+  const int64_t n_dkdv = heads * ((p.seqlen_k + kDkvPairBlockKV - 1) / kDkvPairBlockKV);
+  return joint_workgroups(n_dq, n_dkdv, joint_period(key_groups)) <= kMaxWorkgroups &&
+         heads * (((int64_t)p.seqlen_q_rounded + 15) / 16) <= INT_MAX;
+}
+inline int joint_key_groups(int dp, const BwdParams &p) {
+  const int groups = joint_key_groups_by_size(dp, p);
+  return groups > 0 && joint_fits(p, groups) ? groups : 0;
 }
 // Workgroup i's place in the order of its own kind (which may lie beyond the end of that).
 struct JointPlace {

@@ -19,17 +19,44 @@ HIPCC = pathlib.Path("/opt/rocm/bin/hipcc")
 ATOL, RTOL = 2e-2, 1e-2
 
 
-def test_every_workgroup_of_either_kind_once(tmp_path):
+def _host_program(source: str, tmp_path) -> str:
     if not HIPCC.exists():
         pytest.skip("hipcc not installed")
-    exe = tmp_path / "joint_grid_check"
+    exe = tmp_path / source.partition(".")[0]
     build = subprocess.run(
         [str(HIPCC), "-x", "hip", "--cuda-host-only", "-O1", "-std=c++17", "-Wno-unused-command-line-argument",
          f"-I{ROOT / 'flash-attention-triton_amd' / 'csrc'}", f"-I{ROOT / 'include'}",
-         "-o", str(exe), str(ROOT / "tests" / "joint_grid_check.hip")], capture_output=True, text=True, timeout=300)
+         "-o", str(exe), str(ROOT / "tests" / source)], capture_output=True, text=True, timeout=300)
     assert build.returncode == 0, build.stderr[-2000:]
-    run = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    return str(exe)
+
+
+def test_every_workgroup_of_either_kind_once(tmp_path):
+    run = subprocess.run([_host_program("joint_grid_check.hip", tmp_path)], capture_output=True, text=True, timeout=60)
     assert run.returncode == 0 and run.stdout.endswith("ok\n"), run.stdout + run.stderr
+
+
+@pytest.fixture(scope="module")
+def rule(tmp_path_factory):
+    """(heads, seqlen_q, seqlen_k, headdim[, seqlen_q_rounded]) ... -> (key groups of dQ by itself, of the joint grid, its workgroups) ..."""
+    program = _host_program("joint_rule.hip", tmp_path_factory.mktemp("rule"))
+
+    def of(sizes):
+        lines = "".join(f"{h} {nq} {nk} {rest[0] if rest else nq} {d}\n" for h, nq, nk, d, *rest in sizes)
+        out = subprocess.run([program], input=lines, check=True, capture_output=True, text=True, timeout=60).stdout
+        return [tuple(map(int, line.split())) for line in out.splitlines()]
+
+    return of
+
+
+def test_a_grid_too_large_to_launch_is_two_launches(rule):
+    """Sizes whose dQ and dK/dV grids can each be launched (16.7 million workgroups), but not the joint one; and rows of delta
+    beyond what the launch in front of it takes, where dQ can form delta by itself."""
+    assert [groups for _, groups, _ in rule([
+        (1, 100, 540_000_000, 8), (8_000_000, 128, 128, 128), (6_000_000, 128, 128, 256), (17, 1000, 1000, 64, 2**31 - 1)])] == [0] * 4
+    for _, groups, workgroups in rule([(h, n, nk, d) for h in (8, 1 << 16, 1 << 20, 3 << 20, 1 << 22, 8_000_000, 12_000_000)
+                                       for n in (96, 128, 700) for nk in (1, 128, 700, 100_000) for d in (64, 96, 128, 256)]):
+        assert workgroups <= 0xFFFFFFFF // 256
 
 
 def test_joint_kernels_share_a_cu_like_their_parts(records):  # noqa: F811
