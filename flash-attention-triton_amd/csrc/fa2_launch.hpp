@@ -206,15 +206,32 @@ constexpr int64_t joint_workgroups(int64_t n_dq, int64_t n_dkdv, int period) {
 //               1.02-1.09; 256 columns 1.05-1.26 to 1100 tokens, 0.93-0.97 past them.  Padded heads (112, 224) and heads that do not
 //               divide by 8 0.93-1.03 there
 // The paired dK/dV kernel's conditions hold (below): where the other one is the better one, dK/dV is no part of such a grid.
+// dQ takes the key groups it takes by itself (dq_key_groups), so that a call for part of the gradient gives the bits of a call for all
+// of it.  With two groups on 129 workgroups and more the joint grid loads K and V twice as often as with one:
+//   to 208      32 to 64 columns 1.06-1.42 (48 x 256 tokens 1.00), 128 columns 1.00-1.36; 80 and 96 columns to 160 1.01-1.32, to 208 1.05-
+//               1.20 beyond 512 tokens, 0.96-1.03 below; 160 columns and more to 144 1.12-1.35, 0.85-1.05 beyond
+//   to 256      1.01-1.17 at 32 to 64 columns from 1500 tokens on, 0.88-1.02 below; 128 columns 1.02-1.09 from 2048 on, 0.94-1.05 below;
+//               80 and 96 columns 0.94-1.00
+//   to 320      32 columns 1.03-1.17 from 1500 tokens on, 0.90-1.0 below and 0.88-1.01 beyond; the others 0.88-1.02
 inline int joint_key_groups_by_size(int dp, const BwdParams &p) {
   if (!dq_direct_ok(dp, p) || !dkdv_pair_ok(dp, p)) return 0;
   const int64_t heads = (int64_t)p.batch * p.nheads, wgs = heads * ((p.seqlen_q + kDqBlockQ - 1) / kDqBlockQ);
-  const int n = p.seqlen_q;
-  if (wgs <= kCUs / 2) return n > 128 || wgs <= (dp > 128 ? 64 : 96) ? dq_key_groups(dp, p) : 0;
+  const int n = p.seqlen_q, groups = dq_key_groups(dp, p);
+  if (wgs <= kCUs / 2) return n > 128 || wgs <= (dp > 128 ? 64 : 96) ? groups : 0;
+  if (groups == 2) {
+    bool joint = wgs <= 144;
+    if (dp <= 64)
+      joint = wgs <= (n < 1500 ? 208 : dp == 32 ? 320 : 256);
+    else if (dp == 96)
+      joint = wgs <= (n > 512 ? 208 : 160);
+    else if (dp == 128)
+      joint = wgs <= (n < 2048 ? 208 : 256);
+    return joint ? 2 : 0;
+  }
   if (wgs <= kCUs) return n > (wgs <= 160 ? 128 : 256);
   const bool large = wgs > 2 * kCUs;
   if (large && (p.headdim != direct_columns(dp, p.headdim) || (heads % 8 != 0 && wgs > 4 * kCUs))) return 0;
-  if (dp <= 64) return wgs <= (dp == 32 ? 336 : heads % 8 ? 400 : 576) && n >= 1500;
+  if (dp <= 64) return dp == 64 && wgs <= (heads % 8 ? 400 : 576) && n >= 1500;
   if (dp == 96) return large ? wgs <= 800 && n > 160 && n <= 1100 : n >= 768;
   if (dp == 128) return large ? n >= 128 && n <= 2048 : n > 256;
   if (dp == 192) return large ? wgs >= 1200 && n > 192 && n <= 1100 : wgs <= 384 && n > 128;

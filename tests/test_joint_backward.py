@@ -3,6 +3,7 @@ on the CPU, and gradients at the edges of the rule that picks it (joint_key_grou
 
 from __future__ import annotations
 
+import ctypes
 import math
 import pathlib
 import re
@@ -59,6 +60,15 @@ def test_a_grid_too_large_to_launch_is_two_launches(rule):
         assert workgroups <= 0xFFFFFFFF // 256
 
 
+def test_dq_takes_the_key_groups_it_takes_by_itself(rule):
+    """The joint grid's dQ sums in the order of a dQ launch of its own: the same bits, whatever part of the gradient is asked for."""
+    sizes = [(h, n, n, d) for d in (32, 40, 48, 64, 72, 80, 96, 104, 128, 160, 176, 192, 224, 256)
+             for n in (64, 100, 129, 256, 333, 512, 640, 1000, 1500, 2048, 3000, 4096, 5000, 8192) for h in (*range(1, 70), 80, 96, 128, 200, 512, 1024)]
+    got = rule(sizes)
+    assert all(joint in (0, alone) for alone, joint, _ in got)
+    assert {joint for _, joint, _ in got} == {0, 1, 2}
+
+
 def test_joint_kernels_share_a_cu_like_their_parts(records):  # noqa: F811
     """As many workgroups to a CU as the paired dK/dV kernel has, and no scratch memory but for the values kept across the
     choice of the kind."""
@@ -74,6 +84,37 @@ def test_joint_kernels_share_a_cu_like_their_parts(records):  # noqa: F811
         assert int(r["private_segment_fixed_size"]) <= (0 if dp < 128 or dp == 192 else 24 if dp == 128 else 52), r["name"]
     assert seen == {(t, dp, pad, kg, cols) for t in ("DF16b", "DF16_") for dp, widths in COLUMNS.items() for cols in widths
                     for pad in (0, 1) for kg in (1, 2)}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,n,d,dtype", [
+    (8, 4096, 128, torch.bfloat16), (64, 512, 64, torch.float16), (16, 2048, 64, torch.bfloat16), (12, 2500, 120, torch.bfloat16),  # up to 256
+    (24, 1024, 96, torch.bfloat16), (17, 1024, 192, torch.float16), (9, 2000, 224, torch.bfloat16), (32, 1024, 256, torch.bfloat16),
+    (13, 3000, 32, torch.float16), (12, 4096, 128, torch.bfloat16), (50, 700, 48, torch.bfloat16),  # workgroups of 128 rows and beyond
+    (33, 1000, 128, torch.bfloat16), (31, 2000, 128, torch.bfloat16), (33, 500, 128, torch.bfloat16), (61, 500, 128, torch.bfloat16),
+    (56, 500, 128, torch.bfloat16), (9, 3700, 96, torch.bfloat16), (11, 1900, 96, torch.bfloat16)],  # (second rounds walked backwards)
+    ids=lambda x: str(x).replace("torch.", ""))
+def test_part_of_the_gradient_has_the_bits_of_all_of_it(capi, heads, n, d, dtype):
+    """fa2_bwd with dq == NULL, or dk == dv == NULL, launches one of the two kernels by itself."""
+    gen = torch.Generator(device="cuda").manual_seed(heads + d)
+    q, k, v, d_o = (torch.randn((1, heads, n, d), generator=gen, device="cuda").to(dtype) for _ in range(4))
+    lse = torch.logsumexp((q.float() @ k.float().transpose(-1, -2).contiguous() / math.sqrt(d)).masked_fill(
+        ~torch.ones(n, n, dtype=torch.bool, device="cuda").tril(), -math.inf), -1) if n <= 1100 else torch.full((1, heads, n), 8.0, device="cuda")
+    delta = torch.randn((1, heads, n), generator=gen, device="cuda")
+
+    def run(*wanted):
+        out = {name: torch.full_like(q, 7.0) for name in ("dq", "dk", "dv")}
+        a = capi.BwdArgs(lse=lse.data_ptr(), delta=delta.data_ptr(), workspace=None, batch=1, nheads=heads, seqlen_q=n, seqlen_k=n, headdim=d,
+                         seqlen_q_rounded=n, softmax_scale=1 / math.sqrt(d), deterministic=1, config_id=capi.FA2_CONFIG_AUTO,
+                         dtype=capi.FA2_DTYPE_BF16 if dtype == torch.bfloat16 else capi.FA2_DTYPE_F16)
+        for name, t in {"q": q, "k": k, "v": v, "d_o": d_o, **{x: out[x] for x in wanted}}.items():
+            setattr(a, name, capi.Tensor(t.data_ptr(), *t.stride()[:3]))
+        capi.check(capi.load().fa2_bwd_packed(ctypes.byref(a), torch.cuda.current_stream().cuda_stream), "fa2_bwd_packed")
+        return out
+
+    full, only_dq, only_dkdv = run("dq", "dk", "dv"), run("dq"), run("dk", "dv")
+    assert torch.equal(only_dq["dq"], full["dq"]) and torch.equal(only_dkdv["dk"], full["dk"]) and torch.equal(only_dkdv["dv"], full["dv"])
+    assert all((t == 7).all() for t in (only_dq["dk"], only_dq["dv"], only_dkdv["dq"]))
 
 
 @pytest.mark.gpu
