@@ -213,10 +213,16 @@ constexpr int64_t joint_workgroups(int64_t n_dq, int64_t n_dkdv, int period) {
 //   to 256      1.01-1.17 at 32 to 64 columns from 1500 tokens on, 0.88-1.02 below; 128 columns 1.02-1.09 from 2048 on, 0.94-1.05 below;
 //               80 and 96 columns 0.94-1.00
 //   to 320      32 columns 1.03-1.17 from 1500 tokens on, 0.90-1.0 below and 0.88-1.01 beyond; the others 0.88-1.02
+// The order of the grid takes the two sequences to be of one length.  With many more keys than queries most workgroups of dK/dV see no
+// query, and it is padded with ones of dQ that do not exist: 32 x 512, 4096 keys 0.69 (192 columns) to 0.93 (64), 24 x 1024, 8192 keys 0.78
+// (96) to 0.85 (128), 64 x 192, 1536 keys 0.73 (192) to 0.94 (128), 1.5 times the keys 1.0-1.4.  Grids of more than 512 workgroups lose
+// with fewer keys too: 128 columns 0.90 (1024 x 192, 19 keys), 0.96 (128 x 1024, 819 keys), 256 columns 0.92 (256 x 1024, 102 keys).
 inline int joint_key_groups_by_size(int dp, const BwdParams &p) {
   if (!dq_direct_ok(dp, p) || !dkdv_pair_ok(dp, p)) return 0;
   const int64_t heads = (int64_t)p.batch * p.nheads, wgs = heads * ((p.seqlen_q + kDqBlockQ - 1) / kDqBlockQ);
   const int n = p.seqlen_q, groups = dq_key_groups(dp, p);
+  const int64_t nk = p.seqlen_k;
+  if (wgs > 2 * kCUs ? nk < n || nk > n + n / 4 : nk > n + n / 2) return 0;
   if (wgs <= kCUs / 2) return n > 128 || wgs <= (dp > 128 ? 64 : 96) ? groups : 0;
   if (groups == 2) {
     bool joint = wgs <= 144;

@@ -69,6 +69,13 @@ def test_dq_takes_the_key_groups_it_takes_by_itself(rule):
     assert {joint for _, joint, _ in got} == {0, 1, 2}
 
 
+def test_unlike_lengths_are_two_launches(rule):
+    """On both sides of each line of seqlen_k; what the sizes measured is at joint_key_groups."""
+    sizes = [(32, 512, 768, 192), (32, 512, 769, 192), (32, 512, 4096, 64), (32, 512, 1, 64),  # 128 workgroups of 128 rows
+             (24, 1024, 1536, 96), (24, 1024, 8192, 96), (256, 512, 512, 256), (256, 512, 511, 256), (256, 512, 640, 256), (256, 512, 641, 256)]
+    assert [groups for _, groups, _ in rule(sizes)] == [2, 0, 0, 2, 2, 0, 1, 0, 1, 0]
+
+
 def test_joint_kernels_share_a_cu_like_their_parts(records):  # noqa: F811
     """As many workgroups to a CU as the paired dK/dV kernel has, and no scratch memory but for the values kept across the
     choice of the kind."""
