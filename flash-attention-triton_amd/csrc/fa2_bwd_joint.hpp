@@ -4,8 +4,8 @@
 // it do, and a kernel starts when the one before it has drained.  Two launches are two chains; in one grid the two kinds of
 // workgroup share the chip and the longer chain hides the other (bf16, backward: 2 x 3968 D=128 102 -> 61 us, 16 x 333 D=128
 // 20.2 -> 12.7, 4 x 1024 D=256 62.7 -> 34.2).  On grids of one to two rounds the second kind fills the CUs that the end of the
-// first leaves idle (8 x 4096 D=128 125 -> 109, 16 x 2048 D=64 45.6 -> 39.2), and at 128 and 256 columns also on
-// larger ones.  The price is the launch in front, since dQ can no longer form delta for dK/dV.  The heaviest workgroups of both
+// first leaves idle (40 x 1024 D=128 61.5 -> 52.3, 16 x 2048 D=64 48.6 -> 45.9), and at 128 and 256 columns also on
+// larger ones (200 x 512 D=256 218 -> 195).  The price is the launch in front, since dQ can no longer form delta for dK/dV.  The heaviest workgroups of both
 // kinds come first.  Where each is the faster one: joint_key_groups.
 //
 // Registers and LDS are the larger of the two kernels', whose workgroups share a CU equally often.  The compiler keeps a

@@ -189,59 +189,78 @@ constexpr int64_t joint_workgroups(int64_t n_dq, int64_t n_dkdv, int period) {
   const int64_t rounds_dq = (n_dq + 7) / 8, rounds_dkdv = (n_dkdv + 8 * (period - 1) - 1) / (8 * (period - 1));
   return (rounds_dq > rounds_dkdv ? rounds_dq : rounds_dkdv) * 8 * period;
 }
-// Whether dQ and dK/dV run in one grid (fa2_bwd_joint.hpp) behind a launch that forms delta, and with how many key groups
-// dQ: 0 where two launches are as fast, dQ forming delta for dK/dV.  Time of the two over that of delta and the joint grid,
-// bf16, (batch, head) pairs x tokens, by workgroups of 128 query rows; in brackets the other number of key groups:
-//   to 128      1.2-1.9 (16 x 64 and up), 64 columns 1.33 (32 x 512) [1.22], 128 columns 1.71 (4 x 512) [1.44], 1.39 (16 x 1024)
-//               [1.29], 256 columns 1.83 (2 x 1024) [1.51]; of 128 tokens and fewer 0.94-1.1 beyond 96 workgroups, at 160 columns
-//               and more beyond 64
-//   to 256      from 257 tokens 1.0-1.25: 64 columns 1.15 (32 x 1024) [1.02], 1.05 (64 x 512) [0.98], 128 columns 1.06 (16 x 2048),
-//               1.15 (8 x 4096) [1.03], 256 columns 1.13 (50 x 512) [0.88]; shorter ones 1.05-1.15 to 160, 0.79-1.0 beyond
-//   to 512      32 columns 1.17 (13 x 3000), 1.00 (32 x 2048); 48 and 64 columns from 1500 tokens 1.03-1.15, to 576 with heads
-//               that divide by 8, below 1500 0.88-1.05; 80 and 96 columns from 768 tokens 1.03-1.17, below 0.85-1.06; 128 columns
-//               1.19 (80 x 512), 1.08 (12 x 4096), 1.12 (43 x 1500), of 256 tokens and fewer 0.82-1.03; 192 columns 1.13 (160 x
-//               192), 1.04 (16 x 3000) to 384, 0.93-1.08 beyond; 256 columns 1.19 (80 x 512), 1.17 (320 x 64), 0.95 beyond 384
-//   beyond      80 and 96 columns 1.04-1.16 to 800 and 1100 tokens, 0.95-1.0 past them; 128 columns to 2048 tokens 1.02-1.15, 1.07
-//               (256 x 1024), 1.04 (512 x 512), past them 0.92-0.99; 160 columns from 1200 workgroups and 256 to 1024 tokens
-//               1.02-1.09; 256 columns 1.05-1.26 to 1100 tokens, 0.93-0.97 past them.  Padded heads (112, 224) and heads that do not
-//               divide by 8 0.93-1.03 there
-// The paired dK/dV kernel's conditions hold (below): where the other one is the better one, dK/dV is no part of such a grid.
-// dQ takes the key groups it takes by itself (dq_key_groups), so that a call for part of the gradient gives the bits of a call for all
-// of it.  With two groups on 129 workgroups and more the joint grid loads K and V twice as often as with one:
-//   to 208      32 to 64 columns 1.06-1.42 (48 x 256 tokens 1.00), 128 columns 1.00-1.36; 80 and 96 columns to 160 1.01-1.32, to 208 1.05-
-//               1.20 beyond 512 tokens, 0.96-1.03 below; 160 columns and more to 144 1.12-1.35, 0.85-1.05 beyond
-//   to 256      1.01-1.17 at 32 to 64 columns from 1500 tokens on, 0.88-1.02 below; 128 columns 1.02-1.09 from 2048 on, 0.94-1.05 below;
-//               80 and 96 columns 0.94-1.00
-//   to 320      32 columns 1.03-1.17 from 1500 tokens on, 0.90-1.0 below and 0.88-1.01 beyond; the others 0.88-1.02
+// Whether dQ and dK/dV run in one grid (fa2_bwd_joint.hpp) behind a launch that forms delta: 0 where two launches are as fast, dQ
+// forming delta for dK/dV, else the key groups of dQ.  Those are the groups it takes by itself (dq_key_groups), so that a call for part
+// of the gradient gives the bits of a call for all of it.  Time of the two launches over that of delta and the joint grid, bf16, keys
+// from 1 to 1.5 times the queries, by workgroups of 128 query rows (4000 sizes; the table over sizes: profiles/joint_backward_sweep.txt).
+// Inside the lines 0.96 to 1.71, in the geometric mean 1.26 to 512 workgroups; 1.06 beyond, where two launches fill the chip as well and
+// what is gained is the end of the first.
+//   to 128      to 128 columns 1.13-1.70, of 128 tokens and fewer to 96 1.08-1.45 (beyond 1.11-1.23, not taken); 160 columns and more 1.01-1.71
+//               from 257 tokens on, to 256 1.03-1.67 (beyond 96 workgroups 0.97-1.08), to 128 1.29-1.48 (beyond 64 0.84-1.3)
+//   one group   to 160     129 tokens and more 1.10-1.41; 160 columns and more from 256 on 1.05-1.29, below 0.86-0.94
+//               to 208     128 columns from 257 tokens on 1.09-1.25, 32 to 64 columns likewise, 160 and more from 768 on 1.01-1.14; below
+//                          those, and 80 and 96 columns to 512, 0.81-1.20
+//               to 256     0.68-1.12
+//               to 512     48 and 64 columns from 1500 tokens on 1.05-1.16 (to 576 with heads that divide by 8 1.04-1.09), below 0.74-1.17;
+//                          80 and 96 from 768 on 1.00-1.23, below 0.73-1.13; 128 from 1500 on 1.02-1.31, below to 448 0.98-1.27 (padded
+//                          heads 0.93-1.17); 256 to 328 1.02-1.26, to 384 1.02-1.27 to 128 and from 3000 tokens on (between 0.99-1.18),
+//                          beyond 0.87-1.18; 160 to 224 to 328 from 2048 tokens on 1.05-1.18, to 384 from 3000 on 0.99-1.11, else 0.80-1.27
+//   two groups  (the joint grid loads K and V twice as often as with one)
+//               to 208     32 to 64 and 128 columns 1.00-1.55; 80 and 96 to 160 1.01-1.49, beyond from 513 tokens on 1.05-1.41 (below 0.96-
+//                          1.04); 160 and more to 144 1.05-1.29, beyond 0.84-1.08
+//               to 256     32 to 64 columns from 1500 tokens on 1.04-1.31, below 0.88-1.02; 128 from 2048 on 1.02-1.20, below 0.94-1.05; 80 and
+//                          96 0.90-1.03
+//               to 320     32 columns from 1500 tokens on 1.03-1.17, below 0.90-0.95 and beyond 0.87-1.01; the others 0.88-1.10
+//   beyond 512  (not padded heads, and to 1024 unless the heads divide by 8)
+//               80, 96     to 800 from 161 to 1100 tokens 0.98-1.20 (0.96 at 192 x 384, 128 x 768), else 0.85-1.10
+//               128        128 tokens 1.05-1.20; to 1300 workgroups, and from 1100 tokens on, to 2048 tokens 0.98-1.20; else 0.93-1.09
+//               256        96 to 128 tokens 1.05-1.29, 193 to 1100 0.98-1.16; 129 to 192 0.95-1.16, beyond 4096 workgroups from 513 tokens
+//                          on 0.95-1.04, past 1100 tokens 0.88-1.05
+//               others     32 columns 0.63-0.99, 48 and 64 0.74-1.17, 160 0.89-1.10, 192 0.91-1.12, 224 0.89-1.19, with no line to them
 // The order of the grid takes the two sequences to be of one length.  With many more keys than queries most workgroups of dK/dV see no
 // query, and it is padded with ones of dQ that do not exist: 32 x 512, 4096 keys 0.69 (192 columns) to 0.93 (64), 24 x 1024, 8192 keys 0.78
 // (96) to 0.85 (128), 64 x 192, 1536 keys 0.73 (192) to 0.94 (128), 1.5 times the keys 1.0-1.4.  Grids of more than 512 workgroups lose
 // with fewer keys too: 128 columns 0.90 (1024 x 192, 19 keys), 0.96 (128 x 1024, 819 keys), 256 columns 0.92 (256 x 1024, 102 keys).
+// The paired dK/dV kernel's conditions hold (above): where the other one is the better one, dK/dV is no part of such a grid.
 inline int joint_key_groups_by_size(int dp, const BwdParams &p) {
   if (!dq_direct_ok(dp, p) || !dkdv_pair_ok(dp, p)) return 0;
   const int64_t heads = (int64_t)p.batch * p.nheads, wgs = heads * ((p.seqlen_q + kDqBlockQ - 1) / kDqBlockQ);
   const int n = p.seqlen_q, groups = dq_key_groups(dp, p);
   const int64_t nk = p.seqlen_k;
-  if (wgs > 2 * kCUs ? nk < n || nk > n + n / 4 : nk > n + n / 2) return 0;
-  if (wgs <= kCUs / 2) return n > 128 || wgs <= (dp > 128 ? 64 : 96) ? groups : 0;
-  if (groups == 2) {
-    bool joint = wgs <= 144;
+  if (wgs > 2 * kCUs) {
+    if (p.headdim != direct_columns(dp, p.headdim) || (heads % 8 != 0 && wgs > 4 * kCUs) || nk < n || nk > n + n / 4) return 0;
+    if (dp == 64) return wgs <= 576 && n >= 1500 && heads % 8 == 0;
+    if (dp == 96) return wgs <= 800 && n > 160 && n <= 1100;
+    if (dp == 128) return n >= 128 && n <= 2048 && (n == 128 || n >= 1100 || wgs <= 1300);
+    return p.headdim == 256 && n >= 96 && (n <= 128 || n > 192) && n <= (wgs <= 4096 ? 1100 : 512);
+  }
+  if (nk > n + n / 2) return 0;
+  bool joint;
+  if (wgs <= kCUs / 2) {
+    joint = dp > 128 ? wgs <= 64 || n > (wgs <= 96 ? 128 : 256) : wgs <= 96 || n > 128;
+  } else if (groups == 2) {
     if (dp <= 64)
       joint = wgs <= (n < 1500 ? 208 : dp == 32 ? 320 : 256);
     else if (dp == 96)
       joint = wgs <= (n > 512 ? 208 : 160);
     else if (dp == 128)
       joint = wgs <= (n < 2048 ? 208 : 256);
-    return joint ? 2 : 0;
+    else
+      joint = wgs <= 144;
+  } else if (wgs <= kCUs) {
+    joint = wgs <= 160 ? n > (dp > 128 ? 255 : 128) : wgs <= 208 && n > (dp > 128 ? 767 : dp == 96 ? 512 : 256);
+  } else if (dp <= 64) {
+    joint = dp == 64 && n >= 1500 && (wgs <= 400 || heads % 8 == 0);
+  } else if (dp == 96) {
+    joint = n >= 768 && nk >= n;
+  } else if (dp == 128) {
+    joint = n >= 1500 || (p.headdim == 128 && n > 256 && wgs <= 448);
+  } else if (p.headdim == 256) {
+    joint = n >= 96 && wgs <= (n <= 128 || n >= 3000 ? 384 : 328);
+  } else {
+    joint = nk >= n && (wgs <= 328 ? n >= 2048 : wgs <= 384 && n >= 3000);
   }
-  if (wgs <= kCUs) return n > (wgs <= 160 ? 128 : 256);
-  const bool large = wgs > 2 * kCUs;
-  if (large && (p.headdim != direct_columns(dp, p.headdim) || (heads % 8 != 0 && wgs > 4 * kCUs))) return 0;
-  if (dp <= 64) return dp == 64 && wgs <= (heads % 8 ? 400 : 576) && n >= 1500;
-  if (dp == 96) return large ? wgs <= 800 && n > 160 && n <= 1100 : n >= 768;
-  if (dp == 128) return large ? n >= 128 && n <= 2048 : n > 256;
-  if (dp == 192) return large ? wgs >= 1200 && n > 192 && n <= 1100 : wgs <= 384 && n > 128;
-  return n >= 96 && (large ? n <= 1100 : wgs <= 384);
+  return joint ? groups : 0;
 }
 // Whether such a grid can be launched, and the one that forms delta in front of it: a joint grid has up to three times the workgroups
 // of its larger kind.  Where not, two launches run, each with a limit of its own.

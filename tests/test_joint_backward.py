@@ -76,6 +76,22 @@ def test_unlike_lengths_are_two_launches(rule):
     assert [groups for _, groups, _ in rule(sizes)] == [2, 0, 0, 2, 2, 0, 1, 0, 1, 0]
 
 
+@pytest.mark.parametrize("heads,n,d,groups", [
+    (96, 128, 64, 2), (97, 64, 64, 0), (64, 128, 256, 2), (65, 64, 192, 0), (48, 129, 160, 2), (64, 200, 224, 0), (64, 192, 256, 0), (42, 300, 192, 2),  # 128
+    (80, 192, 128, 1), (80, 192, 160, 0), (80, 256, 160, 1), (67, 300, 128, 1), (84, 256, 128, 0), (34, 768, 192, 1), (48, 512, 256, 0), (64, 512, 160, 0),  # 256
+    (80, 256, 64, 2), (56, 512, 64, 0), (32, 1024, 64, 0), (16, 2048, 64, 2), (64, 512, 128, 0), (8, 4096, 128, 2), (32, 1024, 128, 0),
+    (20, 1024, 96, 2), (24, 1024, 80, 2), (64, 333, 80, 0), (32, 1024, 96, 0), (17, 1024, 192, 2), (20, 1024, 160, 0),
+    (12, 3000, 32, 2), (16, 3000, 32, 0), (24, 2048, 64, 0), (32, 2048, 64, 1), (33, 2048, 64, 0), (24, 2048, 96, 0), (32, 2048, 80, 1),  # 512
+    (12, 4096, 128, 0), (112, 512, 128, 1), (128, 512, 128, 0), (96, 320, 112, 0), (32, 2048, 112, 1), (160, 192, 192, 0), (20, 2048, 192, 1),
+    (24, 2048, 192, 0), (12, 4096, 192, 1), (80, 512, 224, 0), (80, 512, 256, 1), (96, 512, 256, 0), (384, 64, 256, 0), (384, 128, 256, 1),
+    (256, 512, 224, 0), (640, 200, 224, 0), (1280, 192, 224, 0), (1280, 256, 160, 0), (1280, 256, 192, 0), (640, 160, 96, 0), (640, 161, 96, 0),  # beyond
+    (200, 512, 80, 1), (224, 512, 96, 0), (1024, 128, 128, 1), (1024, 256, 128, 0), (1024, 1024, 128, 0), (256, 1100, 128, 1), (4096, 512, 128, 0),
+    (520, 192, 256, 0), (520, 256, 256, 1), (1024, 512, 256, 1), (1024, 700, 256, 0), (1024, 1024, 64, 0), (4096, 512, 64, 0), (512, 2048, 32, 0)])
+def test_joint_only_where_it_measured_faster(rule, heads, n, d, groups):
+    """Both sides of the lines of joint_key_groups."""
+    assert rule([(heads, n, n, d)])[0][1] == groups
+
+
 def test_joint_kernels_share_a_cu_like_their_parts(records):  # noqa: F811
     """As many workgroups to a CU as the paired dK/dV kernel has, and no scratch memory but for the values kept across the
     choice of the kind."""
@@ -131,7 +147,7 @@ def test_part_of_the_gradient_has_the_bits_of_all_of_it(capi, heads, n, d, dtype
     (64, 192, 192, 48, torch.bfloat16), (65, 160, 160, 48, torch.bfloat16), (9, 1000, 1000, 104, torch.bfloat16),  # 128 workgroups and more
     (41, 300, 333, 32, torch.bfloat16), (32, 1024, 1024, 64, torch.float16), (27, 1153, 1100, 72, torch.bfloat16),
     (11, 3000, 3000, 96, torch.bfloat16), (43, 500, 500, 256, torch.bfloat16), (60, 200, 200, 176, torch.bfloat16),
-    (136, 520, 520, 128, torch.bfloat16), (136, 520, 520, 120, torch.bfloat16), (200, 512, 500, 80, torch.bfloat16),  # more than 512
+    (136, 520, 520, 128, torch.bfloat16), (136, 520, 520, 120, torch.bfloat16), (200, 512, 500, 80, torch.bfloat16), (200, 512, 520, 80, torch.float16),  # more than 512
     (300, 100, 260, 160, torch.bfloat16), (520, 120, 120, 256, torch.bfloat16)], ids=lambda x: str(x).replace("torch.", ""))
 def test_gradients_at_the_edges_of_the_rule(fa, heads, nq, nk, d, dtype):
     gen = torch.Generator(device="cuda").manual_seed(nq + heads)
