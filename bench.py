@@ -82,7 +82,7 @@ def kernel_name(launch: dict, part: str) -> str:
     """Name of the kernel a part of a call runs, from the library's own account of it (capi.launch_info)."""
     if part == "fwd" and launch[part]["key_groups"] == 4:
         return "fwd_quad_kernel"
-    suffix = {"generic": "kernel", "direct": "direct_kernel", "paired": "pair_kernel"}[launch[part]["form"]]
+    suffix = {"generic": "kernel", "direct": "direct_kernel", "paired": "pair_kernel", "mixed": "mixed_kernel"}[launch[part]["form"]]
     return {"fwd": "fwd_", "dq": "bwd_dq_", "dkdv": "bwd_dkdv_"}[part] + suffix
 
 

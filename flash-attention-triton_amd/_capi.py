@@ -15,7 +15,7 @@ import threading
 # The in-tree build; FA2_GFX950_LIBRARY names another build of the same ABI (e.g. one under test).
 LIBRARY_PATH = pathlib.Path(os.environ.get("FA2_GFX950_LIBRARY") or
                             pathlib.Path(__file__).resolve().parent / "csrc" / "libfa2_gfx950.so")
-ABI_VERSION = 8
+ABI_VERSION = 9
 
 FA2_DTYPE_F16 = 0
 FA2_DTYPE_BF16 = 1
@@ -46,6 +46,9 @@ class LaunchPart(ctypes.Structure):
 
     _fields_ = [*((name, _i) for name in ("form", "block_rows", "key_groups", "wg_per_cu", "resident")),
                 ("workgroups", _i64)]
+
+    def as_dict(self) -> dict:
+        return {**{name: getattr(self, name) for name, *_ in self._fields_}, "form": FORMS[self.form]}
 
 
 class LaunchInfo(ctypes.Structure):
@@ -101,6 +104,7 @@ SIGNATURES = {
     "fa2_bwd_fused": (_i, [_p] * 11 + [_i] * 6 + [_i64] * 24 + [_f, _i, _i, _i, _p]),
     "fa2_bwd_fused_noalloc": (_i, [_p] * 9 + [_i] * 6 + [_i64] * 24 + [_f, _i, _i, _i, _p]),
     "fa2_launch_info_get": (_i, [_i] * 6 + [ctypes.POINTER(LaunchInfo)]),
+    "fa2_joint_info_get": (_i, [_i] * 6 + [ctypes.POINTER(LaunchPart)]),
     "fa2_fwd_packed": (_i, [ctypes.POINTER(FwdArgs), _p]),
     "fa2_fwd_packed_f32_out": (_i, [ctypes.POINTER(FwdArgs), _p, _p]),
     "fa2_cast_f32_to_f16": (_i, [ctypes.POINTER(Cast), _i, _p]),
@@ -157,7 +161,7 @@ def config_table() -> list[dict]:
     return rows
 
 
-FORMS = ("generic", "direct", "paired")
+FORMS = ("generic", "direct", "paired", "mixed", "joint")
 
 
 def launch_info(batch: int, nheads: int, seqlen_q: int, seqlen_k: int, headdim: int,
@@ -168,6 +172,14 @@ def launch_info(batch: int, nheads: int, seqlen_q: int, seqlen_k: int, headdim: 
           "fa2_launch_info_get")
     out = {"config_id": info.config_id}
     for part in ("fwd", "dq", "dkdv"):
-        out[part] = {name: getattr(getattr(info, part), name) for name, *_ in LaunchPart._fields_}
-        out[part]["form"] = FORMS[out[part]["form"]]
+        out[part] = getattr(info, part).as_dict()
     return out
+
+
+def joint_info(batch: int, nheads: int, seqlen_q: int, seqlen_k: int, headdim: int,
+               config_id: int = FA2_CONFIG_AUTO) -> dict | None:
+    """The grid in which a backward of these sizes forms dq, dk and dv, None where two launches do (fa2_joint_info_get)."""
+    part = LaunchPart()
+    check(load().fa2_joint_info_get(batch, nheads, seqlen_q, seqlen_k, headdim, config_id, ctypes.byref(part)),
+          "fa2_joint_info_get")
+    return part.as_dict() if part.workgroups > 0 else None

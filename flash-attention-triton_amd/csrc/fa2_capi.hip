@@ -440,6 +440,28 @@ int bwd_impl(const fa2_bwd_args &a, void *stream, bool grads_f32 = false) {
   return FA2_OK;
 }
 
+// The parameters of a forward and a backward on contiguous, 16-byte aligned tensors, without their pointers, and the table row.
+int contiguous_call(int batch, int nheads, int seqlen_q, int seqlen_k, int headdim, int config_id, fa2::FwdParams *f,
+                    fa2::BwdParams *b, int *cfg) {
+  int rc = check_common(batch, nheads, seqlen_q, seqlen_k, headdim, seqlen_q, FA2_DTYPE_F16);
+  if (rc || (rc = resolve_config(config_id, headdim, cfg))) return rc;
+  auto contiguous = [&](int seqlen) {
+    return fa2::Tensor4{nullptr, (int64_t)nheads * seqlen * headdim, (int64_t)seqlen * headdim, headdim};
+  };
+  *f = fa2::FwdParams{};
+  *b = fa2::BwdParams{};
+  f->q = f->o = b->q = b->o = b->d_o = b->dq = contiguous(seqlen_q);
+  f->k = f->v = b->k = b->v = b->dk = b->dv = contiguous(seqlen_k);
+  f->batch = b->batch = batch;
+  f->nheads = b->nheads = nheads;
+  f->seqlen_q = b->seqlen_q = seqlen_q;
+  f->seqlen_k = b->seqlen_k = seqlen_k;
+  b->seqlen_q_rounded = seqlen_q;
+  f->headdim = b->headdim = headdim;
+  f->vec = b->vec = headdim % 8 == 0;
+  return FA2_OK;
+}
+
 fa2_tensor make_tensor(const void *ptr, int64_t sb, int64_t sh, int64_t ss) { return fa2_tensor{ptr, sb, sh, ss}; }
 
 // ---- delta scratch of fa2_bwd_fused_noalloc ---------------------------------------------------
@@ -528,25 +550,12 @@ int fa2_pick_config_forward_only(int dtype, int headdim, int seqlen_q, int seqle
 int fa2_launch_info_get(int batch, int nheads, int seqlen_q, int seqlen_k, int headdim, int config_id,
                         fa2_launch_info *out) {
   if (out == nullptr) return fail(FA2_ERR_NULL_POINTER, "out is NULL");
-  int rc = check_common(batch, nheads, seqlen_q, seqlen_k, headdim, seqlen_q, FA2_DTYPE_F16);
+  fa2::FwdParams f;
+  fa2::BwdParams k;
   int cfg;
-  if (rc || (rc = resolve_config(config_id, headdim, &cfg))) return rc;
+  if (int rc = contiguous_call(batch, nheads, seqlen_q, seqlen_k, headdim, config_id, &f, &k, &cfg)) return rc;
   const fa2_config_info &row = kTable[cfg];
   const int dp = row.headdim_padded;
-  auto contiguous = [&](int seqlen) {
-    return fa2::Tensor4{nullptr, (int64_t)nheads * seqlen * headdim, (int64_t)seqlen * headdim, headdim};
-  };
-  const fa2::Tensor4 tq = contiguous(seqlen_q), tk = contiguous(seqlen_k);
-  fa2::FwdParams f = {};
-  fa2::BwdParams k = {};
-  f.q = f.o = k.q = k.o = k.d_o = k.dq = tq;
-  f.k = f.v = k.k = k.v = k.dk = k.dv = tk;
-  f.batch = k.batch = batch;
-  f.nheads = k.nheads = nheads;
-  f.seqlen_q = k.seqlen_q = seqlen_q;
-  f.seqlen_k = k.seqlen_k = seqlen_k;
-  f.headdim = k.headdim = headdim;
-  f.vec = k.vec = headdim % 8 == 0;
   fa2::BwdParams q = k;
   auto part = [](int form, int block_rows, int key_groups, int wg_per_cu, int resident, int64_t nwg) {
     const bool fast = form != FA2_FORM_GENERIC;
@@ -557,7 +566,8 @@ int fa2_launch_info_get(int batch, int nheads, int seqlen_q, int seqlen_k, int h
   out->config_id = cfg;
   int64_t nwg = plan_fwd(cfg, f);
   int groups = fa2::fwd_key_groups(dp, f);
-  out->fwd = part(fa2::fwd_direct_ok(dp, f) ? FA2_FORM_DIRECT : FA2_FORM_GENERIC, kFwdBlockQ / groups, groups,
+  out->fwd = part(f.mixed_singles > 0 ? FA2_FORM_MIXED : fa2::fwd_direct_ok(dp, f) ? FA2_FORM_DIRECT : FA2_FORM_GENERIC,
+                  kFwdBlockQ / groups, groups,
                   fwd_wg_per_cu(cfg, groups), f.resident_grid, nwg);
   if (row.fwd_exp_folded) return FA2_OK;
   nwg = plan_dkdv(cfg, k);
@@ -570,6 +580,25 @@ int fa2_launch_info_get(int batch, int nheads, int seqlen_q, int seqlen_k, int h
   groups = fa2::dq_key_groups(dp, q);
   out->dq = part(fa2::dq_direct_ok(dp, q) ? FA2_FORM_DIRECT : FA2_FORM_GENERIC, kDqBlockQ / groups, groups,
                  row.dq_wg_per_cu, q.resident_grid, nwg);
+  return FA2_OK;
+}
+
+int fa2_joint_info_get(int batch, int nheads, int seqlen_q, int seqlen_k, int headdim, int config_id,
+                       fa2_launch_part *out) {
+  if (out == nullptr) return fail(FA2_ERR_NULL_POINTER, "out is NULL");
+  fa2::FwdParams f;
+  fa2::JointParams j = {};
+  int cfg;
+  if (int rc = contiguous_call(batch, nheads, seqlen_q, seqlen_k, headdim, config_id, &f, &j.both, &cfg)) return rc;
+  *out = fa2_launch_part{};
+  const fa2_config_info &row = kTable[cfg];
+  const int dp = row.headdim_padded;
+  if (row.fwd_exp_folded || row.dq_atomic) return FA2_OK;
+  const int groups = fa2::joint_key_groups(dp, j.both);
+  if (groups == 0) return FA2_OK;
+  const int64_t nwg = plan_joint(cfg, groups, j);
+  const int wg_per_cu = fa2::dkdv_pair_wg_per_cu(dp);
+  *out = fa2_launch_part{FA2_FORM_JOINT, kDqBlockQ / groups, groups, wg_per_cu, nwg <= fa2::kCUs * wg_per_cu, nwg};
   return FA2_OK;
 }
 

@@ -35,8 +35,9 @@ extern "C" {
 
 /* Raised with every entry point added or changed and every change of what a field means: 6 brought
  * fa2_bwd_packed_f32_grads and the paired dK/dV kernel (bwd_block_kv, lds_direct and dkdv_passes below), 7
- * fa2_launch_info_get, 8 fa2_fwd_packed_f32_out and fa2_cast_f32_to_f16. */
-#define FA2_ABI_VERSION 8
+ * fa2_launch_info_get, 8 fa2_fwd_packed_f32_out and fa2_cast_f32_to_f16, 9 fa2_joint_info_get and the forms
+ * FA2_FORM_MIXED and FA2_FORM_JOINT. */
+#define FA2_ABI_VERSION 9
 
 /* Largest head dimension the kernels accept (the table's `max_headdim`). */
 #define FA2_MAX_HEADDIM 256
@@ -105,7 +106,9 @@ typedef struct fa2_config_info {
 typedef enum fa2_form {
   FA2_FORM_GENERIC = 0, /* fwd_kernel, bwd_dq_kernel, bwd_dkdv_kernel */
   FA2_FORM_DIRECT = 1,  /* fwd_direct_kernel (fwd_quad_kernel), bwd_dq_direct_kernel, bwd_dkdv_direct_kernel */
-  FA2_FORM_PAIRED = 2   /* bwd_dkdv_pair_kernel */
+  FA2_FORM_PAIRED = 2,  /* bwd_dkdv_pair_kernel */
+  FA2_FORM_MIXED = 3,   /* fwd_mixed_kernel: tiles of one and of two key groups in one grid */
+  FA2_FORM_JOINT = 4    /* bwd_joint_kernel: dQ and dK/dV in one grid */
 } fa2_form;
 
 /*
@@ -117,8 +120,8 @@ typedef struct fa2_launch_part {
   int form;         /* fa2_form */
   int block_rows;   /* query rows (forward, dQ) or key rows (dK/dV) per workgroup */
   int key_groups;   /* forward and dQ: 2 when two waves share 32 query rows and split the keys, 4 when four do
-                       (forward, fwd_quad_kernel), else 1; a forward grid that mixes one and two
-                       (fwd_mixed_kernel) states the tiles of one, and all of its workgroups */
+                       (forward, fwd_quad_kernel), else 1; FA2_FORM_MIXED states the tiles of one, and all
+                       of its workgroups */
   int wg_per_cu;    /* workgroups that share a CU (0: not stated, for the generic kernels) */
   int resident;
   int64_t workgroups;
@@ -193,13 +196,23 @@ int fa2_pick_config(int dtype, int headdim, int seqlen_q, int seqlen_k, int dete
 /*
  * The kernels a forward and a backward of these sizes launch, for 16-byte aligned contiguous tensors.
  * dq and dkdv are those of launches of their own, as when only one of them is asked for; a backward that
- * wants all of dq, dk and dv runs both kinds of workgroup in one grid where that is faster
- * (joint_key_groups in csrc/fa2_launch.hpp), dQ with the key groups that rule gives.
+ * wants all of dq, dk and dv may run both kinds of workgroup in one grid (fa2_joint_info_get).
  * Touches no device.  No counterpart in the reference.  A forward-only row (fwd_exp_folded) has no
  * backward: dq and dkdv come back all zero.
  */
 int fa2_launch_info_get(int batch, int nheads, int seqlen_q, int seqlen_k, int headdim, int config_id,
                         fa2_launch_info *out);
+
+/*
+ * The one grid in which a backward of these sizes forms dq, dk and dv where that is faster than two launches
+ * (joint_key_groups in csrc/fa2_launch.hpp), for 16-byte aligned contiguous tensors: form FA2_FORM_JOINT, the
+ * query rows and the key groups of its dQ workgroups (those of dK/dV take what dkdv states), and all of its
+ * workgroups.  All zero where two launches run, those of fa2_launch_info_get.  Where delta is formed on the
+ * way, a launch in front of the joint grid forms it: bwd_delta_kernel where dQ by itself has at most 256
+ * workgroups, else bwd_preprocess_kernel.  Touches no device.  No counterpart in the reference.
+ */
+int fa2_joint_info_get(int batch, int nheads, int seqlen_q, int seqlen_k, int headdim, int config_id,
+                       fa2_launch_part *out);
 
 /*
  * The row for a forward whose log-sum-exp no backward will read (inference, evaluation under

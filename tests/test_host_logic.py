@@ -47,7 +47,7 @@ def test_library_exports_every_declared_symbol(capi):
 
 # sha256 (first 16 digits) of include/fa2_gfx950.h without comments, white space and the version itself, per ABI
 # version.  A change of the interface needs a new version and a line here.
-INTERFACES = {6: "94837833e0c9a376", 7: "f98a87f9170d5460", 8: "6532f24f44a70406"}
+INTERFACES = {6: "94837833e0c9a376", 7: "f98a87f9170d5460", 8: "6532f24f44a70406", 9: "1aebc81505efa417"}
 
 
 def test_abi_version_follows_the_interface(capi):
@@ -444,6 +444,30 @@ def test_launch_info_says_what_a_call_launches(capi, workloads):
         capi.launch_info(0, 1, 1, 1, 64)
     with pytest.raises(RuntimeError, match="FA2_ERR_BAD_CONFIG"):
         capi.launch_info(1, 1, 1, 1, 64, 99)
+
+
+def test_launch_info_knows_grids_of_two_kinds(capi):
+    """The forward that mixes one and two key groups, and the backward's joint grid: its runs of 8 workgroups, of which every third
+    (two key groups: every second) is of dQ, cover both kinds."""
+    import importlib
+
+    bench = importlib.import_module("bench")
+    for config in (capi.FA2_CONFIG_AUTO, capi.load().fa2_pick_config_forward_only(capi.FA2_DTYPE_BF16, 128, 4096, 4096)):
+        info = capi.launch_info(1, 16, 4096, 4096, 128, config)  # 64 tiles of 64 rows per head: 24 pairs and 16 by themselves
+        assert info["fwd"] == dict(form="mixed", block_rows=128, key_groups=1, wg_per_cu=2, resident=0, workgroups=16 * 40)
+        assert bench.kernel_name(info, "fwd") == "fwd_mixed_kernel"
+    assert capi.launch_info(1, 16, 4095, 4095, 128)["fwd"]["form"] == "direct"
+    part = dict(form="joint", block_rows=64, key_groups=2, wg_per_cu=3, resident=1, workgroups=128)
+    assert capi.joint_info(2, 4, 512, 512, 64) == part  # 64 workgroups of 64 rows and 64 of 64 keys
+    assert capi.joint_info(1, 32, 2048, 2048, 64) == {**part, "block_rows": 128, "key_groups": 1, "resident": 0, "workgroups": 3 * 512}
+    assert capi.joint_info(1, 8, 4096, 4096, 128) == {**part, "wg_per_cu": 2, "resident": 0, "workgroups": 2 * 512}
+    for sizes in [(2, 32, 4096, 4096, 128), (2, 4, 512, 769, 64), (1, 8, 100, 100, 50)]:  # large; longer keys; no 16-byte rows
+        assert capi.joint_info(*sizes) is None
+    for row in capi.config_table():
+        if row["headdim_padded"] == 64 and (row["dq_atomic"] or row["fwd_exp_folded"]):
+            assert capi.joint_info(2, 4, 512, 512, 64, row["id"]) is None
+    with pytest.raises(RuntimeError, match="FA2_ERR_BAD_SHAPE"):
+        capi.joint_info(0, 1, 1, 1, 64)
 
 
 @pytest.mark.parametrize("heads,n,d,fwd,dq", [
