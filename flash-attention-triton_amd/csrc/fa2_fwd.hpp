@@ -771,21 +771,13 @@ __device__ __forceinline__ void fwd_direct(const FwdParams p, short *smem, Place
   store_output<T, COLS, F32>(p, oacc, inv_l, patch, O, bh, q0w, hdim, true);
 }
 
+// The padded form (PAD) switches the lanes of every tile load on and off by a register, with a branch around the load: at 256 columns
+// a fifth of its loop's instructions, and instructions are what one wave per SIMD is bound by.  A head dimension of exactly 256,
+// padded -> not, bf16, us: 16x4096 163.9 -> 155.7, 256x512 77.2 -> 73.7, 8x2048 42.6 -> 39.2, 100x200 20.9 -> 18.7.
 template <typename T, int DP, int BKV, bool PAD, bool PRE, int KG = 1, int COLS = DP, bool F32 = false>
 __global__ __launch_bounds__(64 * kFwdWaves, (DP <= 128 ? 2 : 1)) void fwd_direct_kernel(const FwdParams p) {
   __shared__ __attribute__((aligned(1024))) short smem[FwdDirectLayout<DP, BKV>::TOTAL_ELEMS];
   fwd_direct<T, DP, BKV, PAD, PRE, KG, COLS, F32>(
-      p, smem, [&]() -> int { return p.resident_grid ? balanced_index(blockIdx.x, p.resident_grid) : blockIdx.x; });
-}
-
-// A head dimension of exactly 256.  The padded kernel, which these took too, switches the lanes of every tile load on and off by
-// a register, with a branch around the load: a fifth of its loop's instructions, and instructions are what one wave per SIMD is
-// bound by.  (Before ResidentB this form spilled about forty registers.)  bf16, us: 16x4096
-// 163.9 -> 155.7, 256x512 77.2 -> 73.7, 8x2048 42.6 -> 39.2, 100x200 20.9 -> 18.7.
-template <typename T, int KG, bool F32, int COLS = 256>
-__global__ __launch_bounds__(64 * kFwdWaves, 1) void fwd_full_kernel(const FwdParams p) {
-  __shared__ __attribute__((aligned(1024))) short smem[FwdDirectLayout<COLS, kFwdBlockKV>::TOTAL_ELEMS];
-  fwd_direct<T, COLS, kFwdBlockKV, false, false, KG, COLS, F32>(
       p, smem, [&]() -> int { return p.resident_grid ? balanced_index(blockIdx.x, p.resident_grid) : blockIdx.x; });
 }
 

@@ -10,16 +10,10 @@ constexpr bool kF32 = FA2_F32_OUT;
 
 template <typename T, int DP, int COLS, int KG>
 void launch_cols(const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
-  if constexpr (COLS == 256) {
-    if (p.headdim == COLS) {
-      hipLaunchKernelGGL((fwd_full_kernel<T, KG, kF32>), grid, block, 0, s, p);
-      return;
-    }
-  } else if (p.headdim == COLS) {
+  if (p.headdim == COLS)
     hipLaunchKernelGGL((fwd_direct_kernel<T, DP, kFwdBlockKV, false, false, KG, COLS, kF32>), grid, block, 0, s, p);
-    return;
-  }
-  hipLaunchKernelGGL((fwd_direct_kernel<T, DP, kFwdBlockKV, true, false, KG, COLS, kF32>), grid, block, 0, s, p);
+  else
+    hipLaunchKernelGGL((fwd_direct_kernel<T, DP, kFwdBlockKV, true, false, KG, COLS, kF32>), grid, block, 0, s, p);
 }
 
 template <typename T, int KG>

