@@ -243,7 +243,7 @@ __global__ __launch_bounds__(64 * kDkvWaves, 1) void bwd_dkdv_kernel(const BwdPa
 // chains are written out by hand with vector-register accumulators (dK and dV, which are only
 // read at the very end, stay in accumulation registers).  The compiler does not know these are
 // MFMAs: `settle` supplies the wait states an 8-pass MFMA result needs before vector
-// instructions may read it (11; the s_nop gives 12) and ties them to the value.
+// instructions may read it (12 on gfx950, none to spare) and ties them to the value.
 template <typename T>
 struct VgprMfma;
 template <>

@@ -86,8 +86,8 @@ struct Elem<_Float16> {
 // four copies out of them for B, and one for each element of the result.  It does not know these are MFMAs.  An MFMA may read a
 // register two wait states after a vector instruction has written it: the s_nop 1 of the first one of a chain, and of all but
 // `next_loaded`, which is for loops whose operands come from LDS or were there before (tests/test_resident_fragments.py reads
-// the code for that).  `chain_end` supplies those that an 8-pass MFMA's result needs before a vector instruction reads it (11; the
-// s_nop gives 12).  One wave issues an instruction in 5 to 8 cycles, whatever its kind, so the copies were time.  bf16, us, forward /
+// the code for that).  `chain_end` supplies those that an 8-pass MFMA's result needs before a vector instruction reads it (12 on
+// gfx950, none to spare).  One wave issues an instruction in 5 to 8 cycles, whatever its kind, so the copies were time.  bf16, us, forward /
 // backward: 16x4096 D=256 182.0 -> 163.9 / 479.9 -> 469.7, D=224 139.5 -> 126.6 / 433.3 -> 416.0, D=192 118.2 -> 114.7 / 384.7 ->
 // 371.4, D=160 112.2 -> 109.5 / 341.1 -> 327.6, 256x512 D=256 82.7 -> 77.2 / 264.4 -> 243.9.
 // (AGPR false: B in vector registers after all, where the accumulation registers are full.)
