@@ -170,6 +170,7 @@ int fwd_wg_per_cu(int cfg, int groups) {
 
 // Kernel form, tiles and grid of a forward: completes `p` and returns the number of workgroups.
 int64_t plan_fwd(int cfg, fa2::FwdParams &p) {
+  p.folded = kTable[cfg].fwd_exp_folded;
   const int64_t bh = (int64_t)p.batch * p.nheads;
   const int pairs = fa2::fwd_mixed_pairs(kTable[cfg].headdim_padded, p);
   p.mixed_singles = 0;
@@ -264,7 +265,7 @@ int fwd_impl(const fa2_fwd_args &a, void *stream, float *o_f32 = nullptr) {
   if (nwg > fa2::kMaxWorkgroups)
     return fail(FA2_ERR_TOO_LARGE, "grid of %lld workgroups too large", (long long)nwg);
   const auto launch = o_f32 == nullptr ? fa2::launch_fwd<false> : fa2::launch_fwd<true>;
-  launch(a.dtype == FA2_DTYPE_BF16, kTable[cfg].headdim_padded, kTable[cfg].fwd_exp_folded != 0, p,
+  launch(a.dtype == FA2_DTYPE_BF16, kTable[cfg].headdim_padded, p,
          dim3((unsigned)nwg), reinterpret_cast<hipStream_t>(stream));
   return launch_status("fa2_fwd launch");
 }

@@ -60,18 +60,18 @@ void launch_mixed(const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
 }
 
 template <typename T, int KG>
-void launch_groups(int dp, bool folded, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
-  if (folded)
+void launch_groups(int dp, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
+  if (p.folded)
     launch_direct<T, true, KG>(dp, p, grid, block, s);
   else
     launch_direct<T, false, KG>(dp, p, grid, block, s);
 }
 
 template <typename T>
-void launch(int dp, bool folded, const FwdParams &p, dim3 grid, hipStream_t s) {
+void launch(int dp, const FwdParams &p, dim3 grid, hipStream_t s) {
   const dim3 block(64 * kFwdWaves);
   if (p.mixed_singles > 0) {
-    if (folded)
+    if (p.folded)
       launch_mixed<T, true>(p, grid, block, s);
     else
       launch_mixed<T, false>(p, grid, block, s);
@@ -80,11 +80,11 @@ void launch(int dp, bool folded, const FwdParams &p, dim3 grid, hipStream_t s) {
   if (fwd_direct_ok(dp, p)) {
     const int groups = fwd_key_groups(dp, p);
     if (groups == 4)
-      launch_groups<T, 4>(dp, folded, p, grid, block, s);
+      launch_groups<T, 4>(dp, p, grid, block, s);
     else if (groups == 2)
-      launch_groups<T, 2>(dp, folded, p, grid, block, s);
+      launch_groups<T, 2>(dp, p, grid, block, s);
     else
-      launch_groups<T, 1>(dp, folded, p, grid, block, s);
+      launch_groups<T, 1>(dp, p, grid, block, s);
     return;
   }
   if (p.vec)
@@ -96,11 +96,11 @@ void launch(int dp, bool folded, const FwdParams &p, dim3 grid, hipStream_t s) {
 }  // namespace
 
 template <>
-void launch_fwd<kF32>(bool bf16, int dp, bool folded, const FwdParams &p, dim3 grid, hipStream_t s) {
+void launch_fwd<kF32>(bool bf16, int dp, const FwdParams &p, dim3 grid, hipStream_t s) {
   if (bf16)
-    launch<__bf16>(dp, folded, p, grid, s);
+    launch<__bf16>(dp, p, grid, s);
   else
-    launch<_Float16>(dp, folded, p, grid, s);
+    launch<_Float16>(dp, p, grid, s);
 }
 
 }  // namespace fa2

@@ -87,39 +87,54 @@ inline bool fwd_direct_ok(int dp, const FwdParams &p) {
          direct_stride_ok(p.v);
 }
 // Four key groups (fwd_quad_kernel), to 128 columns: 32 query rows to a workgroup, again half the chain for twice the loads per
-// row, in tiles of 128 keys that leave room for four workgroups per CU at 32 columns, two at 64 and one from 80 on.  Time of the other
-// forms over its own, bf16, by workgroups of 32 rows: while they are all resident it grows with the chain, and past that it is lost.
-//   32 columns        to 512 1.03 (32 x 512), 1.20 (16 x 1024), 1.47 (4 x 4096); to 768 1.06 (24 x 1024), 0.96 (31 x 777); to 1024
-//                     1.12 (16 x 2048), 0.95 (32 x 1024); 0.88-1.0 beyond, 1.34 at 5 x 8192
-//   48, 64 columns    to 512 1.03 (32 x 512), 1.22 (16 x 1024), 1.47 (4 x 4096), 1.0-1.1 below 512 tokens; to 640 1.08 (10 x 2048),
-//                     0.84 (20 x 1024); to 768 1.07 (8 x 3000), 0.97 (12 x 2048); 0.5-0.95 beyond
-//   80, 96 columns    to 256 1.10 (8 x 1024), 1.19-1.23 (4 x 2048), 1.41 (1 x 8192), 0.98 (16 x 512); to 384 1.20 (3 x 4096), 0.92 (6 x
-//                     2048); 0.9-1.0 beyond
-//   128 columns       to 256 1.05 (5 x 1500), 1.16 (2 x 4096), 1.25 (1 x 8192), 0.97 (8 x 1024); to 384 1.17 (3 x 4096), 0.92 (4 x
-//                     3000); 0.8 beyond
-inline bool fwd_quad(int dp, int64_t heads, int seqlen_q) {
-  const int64_t wgs = heads * ((seqlen_q + 31) / 32);
-  const int n = seqlen_q;
+// row, in tiles of 128 keys that leave room for four workgroups per CU at 32 columns, two at 64 and one from 80 on.  Time of the faster
+// of the other forms over its own, bf16, by workgroups of 32 rows, the row a backward follows / the folded one (the sizes:
+// profiles/forward_forms_sweep.txt): while they are all resident it grows with the chain, and past that it is lost.
+//   32 columns        to 512 1.02-1.65 / 1.01-1.52, to 768 from 1024 tokens on 1.02-1.50 / 1.00-1.40, to 1024 from 2048 on 1.17-1.36; 0.88-1.0
+//                     beyond
+//   48, 64 columns    to 512 1.02-1.63 / 1.02-1.55, to 640 from 2048 on 1.02-1.39 / 0.99-1.39, to 768 from 3000 on 1.01-1.55 / 0.99-1.55; to 768
+//                     of 1024 to 2500 tokens 0.75-1.33 / 0.74-1.28
+//   40, 56 columns    to 512 1.00-1.56 / 1.00-1.52, but 0.97-1.00 / 0.98-1.01 of up to 600 tokens beyond 256; to 576 from 2048 on 1.09-1.40 / 1.08-
+//                     1.37, to 640 from 2500 on 1.05-1.42 / 1.05-1.39 (of 2048 0.93-0.99), to 704 from 3000 on 1.09-1.35 / 1.10-1.33, to 768
+//                     from 3500 on 1.03-1.52 (of 3000 0.95-0.98)
+//   80, 96 columns    to 256 from 2048 on 1.00-1.13 / 0.95-1.03, 1500 and 1750 0.97-1.01 / 0.93-0.95, below 0.92-0.97 / 0.87-0.92; to 384 from
+//                     4096 on 1.05-1.29 / 0.99-1.23, below 0.66-1.18
+//   72, 88 columns    to 256 from 1000 on 1.02-1.38 / from 1500 on 1.05-1.30, 768 and 900 0.96-1.00 / 0.94-0.96; to 384 from 4096 on 1.21-1.42 /
+//                     1.15-1.27
+//   128 columns       to 256 from 1500 on 1.02-1.36 / from 2048 on 1.02-1.28 (1500 and 1750 0.98-1.01); to 384 from 4096 on 1.17-1.39 / 1.09-1.31,
+//                     below 0.65-1.31
+//   104 to 120        to 256 from 1500 on 1.10-1.35 / 1.06-1.30; to 384 from 4096 on 1.28-1.50 / 1.23-1.33
+// The folded forward has fewer instructions to a block, so that a shorter chain saves it less.
+constexpr int fwd_quad_limit_64(int n, bool padded) {
+  if (!padded) return n >= 3000 ? 768 : n >= 2048 ? 640 : 512;
+  return n >= 3500 ? 768 : n >= 3000 ? 704 : n >= 2500 ? 640 : n >= 2048 ? 576 : 512;
+}
+inline bool fwd_quad(int dp, const FwdParams &p) {
+  const int n = p.seqlen_q;
+  const int64_t wgs = (int64_t)p.batch * p.nheads * ((n + 31) / 32);
+  const bool padded = p.headdim != direct_columns(dp, p.headdim);
   if (dp == 32) return n > 512 && wgs <= (n >= 2048 ? 1024 : n >= 1024 ? 768 : 512);
-  if (dp == 64) return n > 512 && wgs <= (n >= 3000 ? 768 : n >= 2048 ? 640 : 512);
-  if (dp == 96) return n >= 768 && wgs <= (n >= 4096 ? 384 : 256);
-  return dp == 128 && n >= 1500 && wgs <= (n >= 4096 ? 384 : 256);
+  if (dp == 64) return n > (padded && wgs > 256 ? 600 : 512) && wgs <= fwd_quad_limit_64(n, padded);
+  if (dp == 96 && !padded && p.folded) return n >= 4096 && wgs > 256 && wgs <= 384;
+  const int shortest = dp == 96 ? (padded ? (p.folded ? 1500 : 1000) : 2048) : !padded && p.folded ? 2048 : 1500;
+  return dp <= 128 && n >= shortest && wgs <= (n >= 4096 ? 384 : 256);
 }
 inline int fwd_key_groups(int dp, const FwdParams &p) {
   if (!fwd_direct_ok(dp, p)) return 1;
   const int64_t heads = (int64_t)p.batch * p.nheads;
-  return fwd_quad(dp, heads, p.seqlen_q) ? 4 : key_groups(dp, direct_columns(dp, p.headdim), heads, p.seqlen_q, false);
+  return fwd_quad(dp, p) ? 4 : key_groups(dp, direct_columns(dp, p.headdim), heads, p.seqlen_q, false);
 }
 // One and two key groups in one grid (fwd_mixed_kernel): how many pairs of 64-row tiles of a head one group takes, 0 where all tiles
 // are of one kind.  Three eighths of the tiles, a little more on the larger grids, whose last round the smaller tiles would make
-// longer.  Time of one group over it, bf16, by workgroups of 128 rows; where two groups are the better ones (key_groups) it is
-// 0.94-1.05 of theirs:
-//   64 columns       to 512 1.02-1.11 (25 x 2048 1.08, 28 x 2048 1.11, 64 x 1024 1.02) to 3000 tokens; 0.97-1.0 from 4096 on and at 700
-//   80, 96 columns   to 456 1.01-1.04 at 1024 and 1500 tokens, 1.04-1.16 from 2048 on (10 x 5001 1.16, 17 x 3000 1.12, 14 x 4096 1.06);
-//                    to 520 0.92-0.96 to 1500 tokens, 1.01-1.09 from 2048 on (16 x 4096 1.05, 13 x 5001 1.09); to 576 (13/32 of the
-//                    tiles) 1.03-1.08 from 4096 on, 0.98-1.05 below; 0.83-1.01 beyond
-//   128 columns      to 520 1.03-1.09 from 4096 tokens on (10 x 5001 1.09, 16 x 4096 1.05), 0.95-1.06 below; to 576 1.01-1.05 from 4096
-//                    on; 0.87-1.0 beyond
+// longer.  Time of one group over it, bf16, by workgroups of 128 rows, the row a backward follows / the folded one (the sizes:
+// profiles/forward_forms_sweep.txt); where two groups are the better ones (key_groups) it is 0.94-1.05 of theirs:
+//   64 columns       of 1024 to 3000 tokens to 448 1.05-1.16 / 1.00-1.15; to 512 from 1700 on 1.00-1.10 / 0.99-1.10, below with an even number
+//                    of heads 1.01-1.09 / 0.98-1.06, with an odd one 0.97-1.03 / 0.94-0.99; from 4096 on two groups are the better ones
+//   80, 96 columns   to 456 from 1700 on 1.01-1.13 / 0.97-1.13, of 1300 and 1500 tokens with an even number of heads 1.02-1.12 / 0.99-1.16, an odd
+//                    one 0.97-1.02 / 0.96-0.97, of 1024 and 1100 0.89-1.06 / 0.91-1.03; to 480 from 2048 on 1.00-1.07 / 0.97-1.09; to 520
+//                    from 2500 on 0.98-1.12 / 0.98-1.07, of 2048 0.98-1.00; to 576 (13/32 of the tiles) from 4096 on 1.03-1.09 / 1.02-
+//                    1.09, below 0.81-1.04
+//   128 columns      to 520 from 4096 on 1.01-1.13 / 0.97-1.13; to 576 1.02-1.07; below 4096 0.78-1.10
 // At 32 columns 0.85-1.07 with no rule to it.  Padded heads and 48 columns have no such kernel.
 inline int fwd_mixed_pairs(int dp, const FwdParams &p) {
   const int n = p.seqlen_q;
@@ -127,9 +142,9 @@ inline int fwd_mixed_pairs(int dp, const FwdParams &p) {
   if (wgs <= 3 * kCUs / 2 || wgs > 576 || !fwd_direct_ok(dp, p) || fwd_key_groups(dp, p) != 1) return 0;
   bool mixed = false;
   if (p.headdim == 64)
-    mixed = wgs <= 512 && n >= 1024 && n <= 3000;
+    mixed = n >= 1024 && n <= 3000 && wgs <= (n >= 1700 || heads % 2 == 0 ? 512 : 448);
   else if (p.headdim == 80 || p.headdim == 96)
-    mixed = n >= (wgs <= 456 ? 1024 : wgs <= 520 ? 2048 : 4096);
+    mixed = n >= (wgs > 520 ? 4096 : wgs > 480 ? 2500 : wgs > 456 ? 2048 : heads % 2 == 0 ? 1300 : 1700);
   else if (p.headdim == 128)
     mixed = n >= 4096;
   return mixed ? (n + 63) / 64 * (wgs <= 520 ? 12 : 13) / 32 : 0;
@@ -228,13 +243,13 @@ inline int joint_key_groups_by_size(int dp, const BwdParams &p) {
   const int n = p.seqlen_q, groups = dq_key_groups(dp, p);
   const int64_t nk = p.seqlen_k;
   if (wgs > 2 * kCUs) {
-    if (p.headdim != direct_columns(dp, p.headdim) || (heads % 8 != 0 && wgs > 4 * kCUs) || nk < n || nk > n + n / 4) return 0;
+    if (p.headdim != direct_columns(dp, p.headdim) || (heads % 8 != 0 && wgs > 4 * kCUs) || nk < n || nk > n + (int64_t)n / 4) return 0;
     if (dp == 64) return wgs <= 576 && n >= 1500 && heads % 8 == 0;
     if (dp == 96) return wgs <= 800 && n > 160 && n <= 1100;
     if (dp == 128) return n >= 128 && n <= 2048 && (n == 128 || n >= 1100 || wgs <= 1300);
     return p.headdim == 256 && n >= 96 && (n <= 128 || n > 192) && n <= (wgs <= 4096 ? 1100 : 512);
   }
-  if (nk > n + n / 2) return 0;
+  if (nk > n + (int64_t)n / 2) return 0;
   bool joint;
   if (wgs <= kCUs / 2) {
     joint = dp > 128 ? wgs <= 64 || n > (wgs <= 96 ? 128 : 256) : wgs <= 96 || n > 128;
@@ -316,15 +331,15 @@ inline ResidentWalk resident_walk(int group, int64_t heads) {
 }
 
 // bf16 != 0 selects the bf16 kernels, otherwise fp16.
-// folded: the LDS-direct forward takes its exponents straight from the score MFMAs (Q fragments
+// p.folded: the LDS-direct forward takes its exponents straight from the score MFMAs (Q fragments
 // multiplied by scale * log2(e) and rounded once); the generic forward ignores it.
 // F32: the variants that store the output in fp32 (p.o_f32), each a specialisation defined in an object of its own.
 template <bool F32>
-void launch_fwd(bool bf16, int dp, bool folded, const FwdParams &p, dim3 grid, hipStream_t s);
+void launch_fwd(bool bf16, int dp, const FwdParams &p, dim3 grid, hipStream_t s);
 template <>
-void launch_fwd<false>(bool bf16, int dp, bool folded, const FwdParams &p, dim3 grid, hipStream_t s);
+void launch_fwd<false>(bool bf16, int dp, const FwdParams &p, dim3 grid, hipStream_t s);
 template <>
-void launch_fwd<true>(bool bf16, int dp, bool folded, const FwdParams &p, dim3 grid, hipStream_t s);
+void launch_fwd<true>(bool bf16, int dp, const FwdParams &p, dim3 grid, hipStream_t s);
 // The LDS-direct forward kernels of 160 to 256 columns (dp is 192 or 256), instantiated apart from the others.
 template <bool F32>
 void launch_fwd_direct_wide(bool bf16, int dp, int key_groups, const FwdParams &p, dim3 grid, dim3 block, hipStream_t s);
@@ -341,7 +356,7 @@ void launch_delta(bool bf16, const PreParams &p, dim3 grid, hipStream_t s);
 void launch_dq(bool bf16, int dp, const BwdParams &p, dim3 grid, bool fuse_delta, hipStream_t s);
 // With p.dq_accum set the sequence-parallel kernel runs: dK, dV and atomic dQ contributions.
 void launch_dkdv(bool bf16, int dp, const BwdParams &p, dim3 grid, hipStream_t s);
-// dQ (from p.dq, reading delta) and dK/dV (from p.dkdv) in one grid, which joint_grid gives; a specialisation for each type.
+// dQ (of p.dq_tiles tiles) and dK/dV in one grid of joint_workgroups, both reading delta; a specialisation for each type.
 template <typename T>
 void launch_joint(int dp, const JointParams &p, int key_groups, dim3 grid, hipStream_t s);
 template <>

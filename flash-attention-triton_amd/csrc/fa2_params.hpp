@@ -51,6 +51,7 @@ struct FwdParams {
   float scale_log2;  // scale * log2(e)
   int vec;           // 16-byte global accesses are legal for every tensor
   int mixed_singles;  // fwd_mixed_kernel: tiles of 64 rows per head that it takes as they are (else 0); n_qtiles counts all of them
+  int folded;        // a row with fwd_exp_folded, for the host: see launch_fwd (fa2_launch.hpp)
   float *o_f32;      // contiguous fp32 tensor that receives the output widened, or null; o.ptr may be null beside it
 };
 

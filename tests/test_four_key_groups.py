@@ -17,14 +17,23 @@ ATOL, RTOL = 2e-2, 1e-2
 
 @pytest.mark.parametrize("heads,n,d,groups", [
     (24, 640, 32, 4), (32, 513, 32, 2), (24, 1024, 32, 4), (32, 1024, 32, 2), (16, 2048, 32, 4), (17, 2048, 32, 2), (8, 512, 64, 2),
-    (16, 1024, 64, 4), (17, 1024, 64, 2), (10, 2048, 48, 4), (11, 2048, 40, 2), (8, 3072, 64, 4), (8, 1024, 96, 4), (8, 1024, 80, 4),
-    (9, 1024, 72, 2), (10, 767, 96, 2), (3, 4096, 96, 4), (5, 1500, 128, 4), (5, 1499, 128, 2), (3, 4096, 104, 4), (4, 4096, 128, 2),
+    (16, 1024, 64, 4), (17, 1024, 64, 2), (10, 2048, 48, 4), (11, 2048, 40, 2), (8, 3072, 64, 4), (8, 1024, 96, 2), (8, 1024, 80, 2),  # (0.95 of two groups' rate)
+    (4, 2048, 80, 4), (4, 2047, 96, 2), (8, 1000, 72, 4), (8, 999, 88, 2), (15, 601, 40, 4), (16, 600, 56, 2), (8, 576, 40, 4), (9, 2048, 40, 4),
+    (10, 2048, 56, 2), (8, 3000, 48, 4), (8, 3000, 40, 2), (9, 1024, 72, 2), (10, 767, 96, 2), (3, 4096, 96, 4), (5, 1500, 128, 4), (5, 1499, 128, 2), (3, 4096, 104, 4), (4, 4096, 128, 2),
     (1, 8192, 160, 2)])
 def test_four_key_groups_only_where_they_measured_faster(capi, heads, n, d, groups):
     info = capi.launch_info(1, heads, n, n, d)["fwd"]
     assert info["key_groups"] == groups and info["block_rows"] == 128 // groups
     if groups == 4:
         assert info["workgroups"] == heads * math.ceil(n / 32) and info["wg_per_cu"] == {32: 4, 40: 2, 48: 2, 64: 2}.get(d, 1)
+
+
+@pytest.mark.parametrize("heads,n,d,groups", [
+    (5, 1500, 128, 2), (4, 2047, 128, 2), (4, 2048, 128, 4), (5, 1500, 104, 4), (4, 2048, 80, 2), (1, 8192, 96, 2), (3, 4096, 96, 4), (3, 4096, 80, 4),
+    (3, 4000, 96, 2), (5, 1499, 72, 2), (5, 1500, 88, 4), (16, 1024, 64, 4), (16, 2048, 32, 4)])
+def test_the_folded_row_has_lines_of_its_own(capi, heads, n, d, groups):
+    row = capi.load().fa2_pick_config_forward_only(capi.FA2_DTYPE_BF16, d, n, n)
+    assert capi.launch_info(1, heads, n, n, d, row)["fwd"]["key_groups"] == groups
 
 
 def test_four_key_groups_fit_a_cu(records):  # noqa: F811

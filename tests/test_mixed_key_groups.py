@@ -70,6 +70,19 @@ def test_every_row_once_and_longest_first(tmp_path):
     assert run.returncode == 0 and run.stdout == "ok\n", run.stdout + run.stderr
 
 
+@pytest.mark.parametrize("heads,n,d,mixed", [
+    (54, 1024, 64, True), (64, 1024, 64, True), (57, 1024, 64, False), (33, 1300, 64, False), (41, 1500, 64, False), (35, 1700, 64, True), (29, 2048, 64, True),
+    (36, 1300, 80, True), (38, 1500, 96, True), (39, 1300, 80, False), (33, 1500, 96, False), (57, 1024, 80, False), (50, 1024, 96, False), (32, 1700, 96, True),
+    (34, 1700, 80, False), (29, 2048, 80, True), (32, 2048, 96, False), (26, 2500, 80, True), (16, 4096, 96, True), (18, 4096, 80, True), (18, 4000, 80, False),
+    (16, 4096, 128, True), (16, 4095, 128, False), (20, 3000, 128, False), (16, 4096, 104, False), (40, 1300, 48, False)])
+def test_mixed_only_where_it_measured_faster(heads, n, d, mixed):
+    """Both sides of the lines of fwd_mixed_pairs."""
+    import importlib
+
+    capi = importlib.import_module("flash-attention-triton_amd._capi")
+    assert (capi.launch_info(1, heads, n, n, d)["fwd"]["form"] == "mixed") == mixed
+
+
 def test_mixed_kernels_share_a_cu_like_their_parts(records):  # noqa: F811
     seen = set()
     for r in records:
@@ -94,7 +107,7 @@ REL = {torch.bfloat16: 4e-3, torch.float16: 5e-4, torch.float32: 2e-3}
 @pytest.mark.parametrize("heads,nq,nk,d,dtype", [
     (43, 1025, 1025, 64, torch.bfloat16), (64, 1024, 900, 64, torch.float16), (17, 2999, 3100, 64, torch.bfloat16),
     (49, 1024, 1024, 80, torch.float16), (10, 5001, 5001, 80, torch.bfloat16), (25, 2100, 700, 96, torch.bfloat16),
-    (32, 2048, 2048, 96, torch.float32), (12, 6000, 64, 80, torch.bfloat16), (17, 4097, 4097, 96, torch.float16),
+    (32, 2048, 2048, 96, torch.float32), (12, 6000, 64, 80, torch.bfloat16), (17, 4097, 4097, 96, torch.float16), (36, 1300, 1300, 80, torch.bfloat16), (26, 2500, 2500, 96, torch.float32),
     (12, 4097, 4000, 128, torch.bfloat16), (16, 4500, 4500, 128, torch.float16), (1, 65000, 130, 128, torch.bfloat16)],
     ids=lambda x: str(x).replace("torch.", ""))
 @pytest.mark.parametrize("grad", (False, True))
