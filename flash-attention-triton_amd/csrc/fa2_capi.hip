@@ -425,7 +425,7 @@ int bwd_impl(const fa2_bwd_args &a, void *stream, bool grads_f32 = false) {
     // dQ first: it writes delta, which the dK/dV kernel reads.
     fa2::launch_dq(bf16, dp, pq, dim3((unsigned)nwg_q), true, s);
     if ((rc = launch_status("backward dQ launch (delta fused)"))) return rc;
-    pk.last_heads_first = true;
+    pk.last_heads_first = fa2::dkdv_from_the_end(dp, bh);
     return run_dkdv();
   }
   if (fused) {

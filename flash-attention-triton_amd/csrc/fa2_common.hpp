@@ -347,8 +347,7 @@ __host__ __device__ __forceinline__ void map_workgroup(int i, int heads, int til
 
 // The heads in the opposite order, whole runs of 8 where their number allows it, so that a head stays on its XCD.  What the
 // dQ kernel read last is still in the memory-side cache when the dK/dV kernel behind it starts, so that starts with those
-// heads.  Forward and backward in turn with heads from the front, us: 256x16x512 D=64 1166.5 -> 1158.8, fp32 32x20x1024 D=96 1135.6
-// -> 1130.4, 2x32x4096 D=128 1134.7 -> 1127.1; where everything fits that cache, alike.
+// heads where there are many (dkdv_from_the_end in fa2_launch.hpp).
 __host__ __device__ __forceinline__ int from_the_end(int bh, int heads) {
   return heads % 8 ? heads - 1 - bh : (heads - 8 - (bh & ~7)) + (bh & 7);
 }
@@ -486,7 +485,7 @@ __device__ __forceinline__ void wait_vmem() {
 
 // Row pitch, in elements, of the LDS tiles of the fast kernels for head dimension DP.  The swizzle
 // needs a power-of-two number of 16-byte chunks per row, so 96 columns live in rows of 128: the
-// last four chunk slots of a row are never loaded and never read.
+// last four chunk slots of a row hold nothing that is read (TileLoader fills them with copies of the row's last chunk).
 constexpr int lds_pitch(int dp) { return dp == 96 ? 128 : dp == 192 ? 256 : dp; }
 
 // Fragment addresses a kernel keeps for `n` 16-column steps (two chunks each) or 32-column blocks (four) of a row.  In rows of 256

@@ -197,6 +197,12 @@ inline bool seqpar_atomic_ok(int dp, const BwdParams &p) {
   return dkdv_direct_ok(dp, p) && p.headdim == dp && (dp == 32 || dp == 64 || dp == 128);
 }
 
+// Whether the dK/dV kernel behind a dQ kernel starts with the last heads (from_the_end).  Time of a backward with the heads from the front
+// over that from the end, bf16, in turn in one process: 128 heads and more of 300 to 2048 tokens 1.00-1.07 (4096 x 512 D=64 1.012-1.016,
+// 640 x 1024 D=96 1.014-1.023, 2048 x 300 D=48 1.04-1.08, 512 x 1024 D=128 1.015-1.022), beyond 1.00-1.01; fewer 0.986-1.007, in the
+// geometric mean 0.998, since the heads that dQ works on at its end are then most of them; but at 128 columns from 64 heads on 1.002-
+// 1.013 (64 x 4096 1.012).
+inline bool dkdv_from_the_end(int dp, int64_t heads) { return heads >= (dp == 128 ? 64 : 128); }
 // The order of a joint grid, in runs of 8 workgroups that keep heads on their XCDs: every joint_period-th run is of dQ.  A
 // workgroup of dQ has twice the rows of one of dK/dV, or with two key groups as many.
 __host__ __device__ constexpr int joint_period(int key_groups) { return key_groups == 1 ? 3 : 2; }

@@ -1,4 +1,5 @@
-"""The order of heads that the dK/dV kernel takes behind the dQ kernel (from_the_end in csrc/fa2_common.hpp): every head once."""
+"""The order of heads that the dK/dV kernel takes behind the dQ kernel (from_the_end in csrc/fa2_common.hpp): every head once, and from the
+end only where there are many."""
 
 from __future__ import annotations
 
@@ -14,7 +15,11 @@ SOURCE = """
 #include <cstdio>
 #include <vector>
 #include "fa2_common.hpp"
+#include "fa2_launch.hpp"
 int main() {
+  for (int dp : {32, 64, 96, 128, 192, 256})
+    for (int heads : {1, 16, 63, 64, 127, 128, 4096})
+      if (fa2::dkdv_from_the_end(dp, heads) != (heads >= (dp == 128 ? 64 : 128))) return std::printf("%d columns, %d heads\\n", dp, heads), 1;
   for (int heads : {1, 2, 7, 8, 9, 16, 17, 24, 640, 641, 4096}) {
     std::vector<int> seen(heads, 0);
     for (int i = 0; i < heads; i++) {
