@@ -292,9 +292,9 @@ size_t fa2_bwd_workspace_bytes(int batch, int nheads, int seqlen_q, int seqlen_k
  * Replaces _flash_attention_backward's main launch, the dQ zero-fill pre-hook and the final
  * dq.copy_(dq_accum) (flash_attention_2.py:235-277, _configurators_v2.py:81-93,
  * _triton_kernels_v2.py:192-529).
- * With FA2_CONFIG_AUTO both values of `deterministic` run the same two kernels: a key-tile-parallel
- * kernel for dK and dV and a query-tile-parallel kernel that accumulates dQ in registers in a fixed
- * order and writes it once.  There are no atomics, so results are bit-identical from run to run in
+ * With FA2_CONFIG_AUTO both values of `deterministic` run the same kernels: workgroups that each own a
+ * key tile form dK and dV, workgroups that each own a query tile accumulate dQ in registers in a fixed
+ * order and write it once.  There are no atomics, so results are bit-identical from run to run in
  * both modes (the reference's sequence-parallel mode, _triton_kernels_v2.py:336-339, allows
  * run-to-run differences but does not require them); fa2_bwd_workspace_bytes is 0 and `workspace`
  * may be NULL.  The order of the sums is that of the kernel forms that run, which depend on the
@@ -308,10 +308,11 @@ size_t fa2_bwd_workspace_bytes(int batch, int nheads, int seqlen_q, int seqlen_k
  * aligned tensors (FA2_ERR_BAD_CONFIG otherwise), needs dq, dk and dv together, and its dq may
  * differ in the last bits from run to run.  The table never picks it: on MI355X the L2 retires
  * about 1.35 TB/s of fp32 atomic adds whatever their locality, so it is 2-3 times slower than the
- * two-kernel backward.
- * dK/dV and dQ are computed by two kernels launched back to back on `stream`.  A caller that
- * needs only part of the gradient (or wants to time one kernel) may pass dq == NULL to skip the
- * dQ kernel, or dk == dv == NULL to skip the dK/dV kernel; dk and dv are given or omitted
+ * backward above.
+ * dK/dV and dQ are computed by two kernels launched back to back on `stream`, or by workgroups of both
+ * kinds in one grid where that is faster (fa2_joint_info_get).  A caller that needs only part of the
+ * gradient (or wants to time one kernel) may pass dq == NULL to skip dQ, or dk == dv == NULL to skip dK
+ * and dV; what is left has the bits it has in a call for all of it.  dk and dv are given or omitted
  * together, and at least one of the two groups must be present.
  */
 int fa2_bwd(const void *q, const void *k, const void *v, const void *d_o,
@@ -334,7 +335,8 @@ int fa2_bwd(const void *q, const void *k, const void *v, const void *d_o,
  * `delta` is an output here: fp32 (batch, nheads, seqlen_q_rounded) scratch supplied by the caller,
  * filled like fa2_bwd_preprocess fills it.  When the fast dQ kernel applies, that kernel forms
  * delta from the O and dO rows it already holds and the dK/dV kernel runs after it, which saves
- * one launch and one pass over O and dO; otherwise the three kernels run as in the two-call path.
+ * one launch and one pass over O and dO; where one grid forms dq, dk and dv (fa2_joint_info_get) a
+ * launch in front of it forms delta; otherwise the three kernels run as in the two-call path.
  * dq, dk and dv must all be given.
  */
 int fa2_bwd_fused(const void *q, const void *k, const void *v, const void *o, const void *d_o,

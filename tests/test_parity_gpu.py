@@ -754,7 +754,9 @@ def test_grids_that_fit_the_chip_at_once(fa, capi, b, h, n, d):
     every tile of every head exactly once.  In the first four cases that is the forward and dQ (264 to 765
     workgroups) and at 32 columns the dK/dV kernel whose waves hold both accumulators; in the fifth none (522
     workgroups, 512 fit); in the last six the paired dK/dV kernel too, with a ragged second or third round (264,
-    488, 448, 330, 747 and 747 workgroups of 64 keys), at 61 heads that one alone (244 workgroups of 128 rows)."""
+    488, 448, 330, 747 and 747 workgroups of 64 keys), at 61 heads that one alone (244 workgroups of 128 rows).  That is
+    dQ and dK/dV by themselves; where the backward here runs both in one grid (33 and 31 heads, 11 x 1900),
+    test_joint_backward.py holds their launches by themselves to its bits."""
     info = capi.launch_info(b, h, n, n, d)
     reordered = [p for p in ("fwd", "dq", "dkdv") if info[p]["resident"] and info[p]["workgroups"] > 256]
     paired_too = n <= 520 or n == 1900
