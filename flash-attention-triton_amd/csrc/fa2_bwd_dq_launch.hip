@@ -31,21 +31,21 @@ void launch_direct_groups(int dp, const BwdParams &p, dim3 grid, dim3 block, hip
 }
 
 template <typename T, bool FUSE_DELTA>
-void launch_direct(int dp, const BwdParams &p, dim3 grid, dim3 block, hipStream_t s) {
-  if (dq_key_groups(dp, p) == 2)
+void launch_direct(int dp, const BwdParams &p, int key_groups, dim3 grid, dim3 block, hipStream_t s) {
+  if (key_groups == 2)
     launch_direct_groups<T, FUSE_DELTA, 2>(dp, p, grid, block, s);
   else
     launch_direct_groups<T, FUSE_DELTA, 1>(dp, p, grid, block, s);
 }
 
 template <typename T>
-void launch(int dp, const BwdParams &p, dim3 grid, bool fuse_delta, hipStream_t s) {
+void launch(int dp, const BwdParams &p, int key_groups, dim3 grid, bool fuse_delta, hipStream_t s) {
   const dim3 block(64 * kDqWaves);
   if (dq_direct_ok(dp, p)) {
     if (fuse_delta)
-      launch_direct<T, true>(dp, p, grid, block, s);
+      launch_direct<T, true>(dp, p, key_groups, grid, block, s);
     else
-      launch_direct<T, false>(dp, p, grid, block, s);
+      launch_direct<T, false>(dp, p, key_groups, grid, block, s);
     return;
   }
   switch (dp) {
@@ -60,11 +60,11 @@ void launch(int dp, const BwdParams &p, dim3 grid, bool fuse_delta, hipStream_t 
 
 }  // namespace
 
-void launch_dq(bool bf16, int dp, const BwdParams &p, dim3 grid, bool fuse_delta, hipStream_t s) {
+void launch_dq(bool bf16, int dp, const BwdParams &p, int key_groups, dim3 grid, bool fuse_delta, hipStream_t s) {
   if (bf16)
-    launch<__bf16>(dp, p, grid, fuse_delta, s);
+    launch<__bf16>(dp, p, key_groups, grid, fuse_delta, s);
   else
-    launch<_Float16>(dp, p, grid, fuse_delta, s);
+    launch<_Float16>(dp, p, key_groups, grid, fuse_delta, s);
 }
 
 void launch_cast(const CastParams &p, dim3 grid, hipStream_t s) {

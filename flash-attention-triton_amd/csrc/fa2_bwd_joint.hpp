@@ -4,7 +4,7 @@
 // it do, and a kernel starts when the one before it has drained.  Two launches are two chains; in one grid the two kinds of
 // workgroup share the chip and the longer chain hides the other (bf16, backward: 2 x 3968 D=128 102 -> 61 us, 16 x 333 D=128
 // 20.2 -> 12.7, 4 x 1024 D=256 62.7 -> 34.2).  On grids of one to two rounds the second kind fills the CUs that the end of the
-// first leaves idle (40 x 1024 D=128 61.5 -> 52.3, 16 x 2048 D=64 48.6 -> 45.9), and at 128 and 256 columns also on
+// first leaves idle (8 x 4096 D=128 132 -> 116, 40 x 1024 58.7 -> 50.7, 16 x 2048 D=64 45.2 -> 38.5), and at 128 and 256 columns also on
 // larger ones (200 x 512 D=256 218 -> 195).  The price is the launch in front, since dQ can no longer form delta for dK/dV.  The heaviest workgroups of both
 // kinds come first.  Where each is the faster one: joint_key_groups.
 //

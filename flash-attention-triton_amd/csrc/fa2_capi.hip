@@ -202,9 +202,9 @@ int64_t plan_dkdv(int cfg, fa2::BwdParams &p) {
   return nwg;
 }
 
-int64_t plan_dq(int cfg, fa2::BwdParams &p) {
+int64_t plan_dq(int cfg, int groups, fa2::BwdParams &p) {
   const int64_t bh = (int64_t)p.batch * p.nheads;
-  const int block_q = kDqBlockQ / fa2::dq_key_groups(kTable[cfg].headdim_padded, p);
+  const int block_q = kDqBlockQ / groups;
   p.n_tiles = (p.seqlen_q + block_q - 1) / block_q;
   const int64_t nwg = p.n_tiles * bh;
   plan_order(p, cfg, nwg, kTable[cfg].dq_wg_per_cu, fa2::equal_head_groups(kTable[cfg].head_group, bh));
@@ -369,7 +369,8 @@ int bwd_impl(const fa2_bwd_args &a, void *stream, bool grads_f32 = false) {
   p.dq_accum_rows = 0;
 
   fa2::BwdParams pk = p, pq = p;
-  const int64_t nwg_k = plan_dkdv(cfg, pk), nwg_q = plan_dq(cfg, pq);
+  const int dq_groups = kTable[cfg].dq_atomic ? 1 : fa2::dq_key_groups_of_call(dp, p);
+  const int64_t nwg_k = plan_dkdv(cfg, pk), nwg_q = plan_dq(cfg, dq_groups, pq);
   if (nwg_k > fa2::kMaxWorkgroups || nwg_q > fa2::kMaxWorkgroups)
     return fail(FA2_ERR_TOO_LARGE, "grid of %lld workgroups too large", (long long)std::max(nwg_k, nwg_q));
 
@@ -408,10 +409,11 @@ int bwd_impl(const fa2_bwd_args &a, void *stream, bool grads_f32 = false) {
   }
 
   if (const int groups = want_dq && want_dkdv ? fa2::joint_key_groups(dp, p) : 0) {
-    // Both read delta.  On the smallest grids it has the bits that the dQ kernel by itself gives it.
+    // Both read delta.  On the smallest grids it has the bits that the dQ kernel in front of a dK/dV kernel gives it.
     if (fused) {
+      fa2::BwdParams apart = p;
       rc = preprocess_impl(a.o, a.d_o, a.delta, a.batch, a.nheads, a.seqlen_q, a.headdim, a.seqlen_q_rounded,
-                           a.dtype, stream, nwg_q <= fa2::kCUs);
+                           a.dtype, stream, plan_dq(cfg, fa2::dq_key_groups(dp, p), apart) <= fa2::kCUs);
       if (rc) return rc;
     }
     fa2::JointParams j;
@@ -423,7 +425,7 @@ int bwd_impl(const fa2_bwd_args &a, void *stream, bool grads_f32 = false) {
 
   if (fused && fa2::dq_direct_ok(dp, pq) && vec_ok(p.o, a.headdim)) {
     // dQ first: it writes delta, which the dK/dV kernel reads.
-    fa2::launch_dq(bf16, dp, pq, dim3((unsigned)nwg_q), true, s);
+    fa2::launch_dq(bf16, dp, pq, dq_groups, dim3((unsigned)nwg_q), true, s);
     if ((rc = launch_status("backward dQ launch (delta fused)"))) return rc;
     pk.last_heads_first = fa2::dkdv_from_the_end(dp, bh);
     return run_dkdv();
@@ -435,7 +437,7 @@ int bwd_impl(const fa2_bwd_args &a, void *stream, bool grads_f32 = false) {
   }
   if (want_dkdv && (rc = run_dkdv())) return rc;
   if (want_dq) {
-    fa2::launch_dq(bf16, dp, pq, dim3((unsigned)nwg_q), false, s);
+    fa2::launch_dq(bf16, dp, pq, dq_groups, dim3((unsigned)nwg_q), false, s);
     if ((rc = launch_status("backward dQ launch"))) return rc;
   }
   return FA2_OK;
@@ -577,8 +579,8 @@ int fa2_launch_info_get(int batch, int nheads, int seqlen_q, int seqlen_k, int h
                    pair ? fa2::kDkvPairBlockKV : kDkvBlockKV, 1, pair ? fa2::dkdv_pair_wg_per_cu(dp) : row.dkdv_wg_per_cu,
                    k.resident_grid, nwg);
   if (row.dq_atomic) return FA2_OK;
-  nwg = plan_dq(cfg, q);
   groups = fa2::dq_key_groups(dp, q);
+  nwg = plan_dq(cfg, groups, q);
   out->dq = part(fa2::dq_direct_ok(dp, q) ? FA2_FORM_DIRECT : FA2_FORM_GENERIC, kDqBlockQ / groups, groups,
                  row.dq_wg_per_cu, q.resident_grid, nwg);
   return FA2_OK;

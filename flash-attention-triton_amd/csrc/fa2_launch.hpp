@@ -210,78 +210,56 @@ constexpr int64_t joint_workgroups(int64_t n_dq, int64_t n_dkdv, int period) {
   const int64_t rounds_dq = (n_dq + 7) / 8, rounds_dkdv = (n_dkdv + 8 * (period - 1) - 1) / (8 * (period - 1));
   return (rounds_dq > rounds_dkdv ? rounds_dq : rounds_dkdv) * 8 * period;
 }
-// Whether dQ and dK/dV run in one grid (fa2_bwd_joint.hpp) behind a launch that forms delta: 0 where two launches are as fast, dQ
-// forming delta for dK/dV, else the key groups of dQ.  Those are the groups it takes by itself (dq_key_groups), so that a call for part
-// of the gradient gives the bits of a call for all of it.  Time of the two launches over that of delta and the joint grid, bf16, keys
-// from 1 to 1.5 times the queries, by workgroups of 128 query rows (4000 sizes; the table over sizes: profiles/joint_backward_sweep.txt).
-// Inside the lines 0.96 to 1.71, in the geometric mean 1.26 to 512 workgroups; 1.06 beyond, where two launches fill the chip as well and
-// what is gained is the end of the first.
-//   to 128      to 128 columns 1.13-1.70, of 128 tokens and fewer to 96 1.08-1.45 (beyond 1.11-1.23, not taken); 160 columns and more 1.01-1.71
-//               from 257 tokens on, to 256 1.03-1.67 (beyond 96 workgroups 0.97-1.08), to 128 1.29-1.48 (beyond 64 0.84-1.3)
-//   one group   to 160     129 tokens and more 1.10-1.41; 160 columns and more from 256 on 1.05-1.29, below 0.86-0.94
-//               to 208     128 columns from 257 tokens on 1.09-1.25, 32 to 64 columns likewise, 160 and more from 768 on 1.01-1.14; below
-//                          those, and 80 and 96 columns to 512, 0.81-1.20
-//               to 256     0.68-1.12
-//               to 512     48 and 64 columns from 1500 tokens on 1.05-1.16 (to 576 with heads that divide by 8 1.04-1.09), below 0.74-1.17;
-//                          80 and 96 from 768 on 1.00-1.23, below 0.73-1.13; 128 from 1500 on 1.02-1.31, below to 448 0.98-1.27 (padded
-//                          heads 0.93-1.17); 256 to 328 1.02-1.26, to 384 1.02-1.27 to 128 and from 3000 tokens on (between 0.99-1.18),
-//                          beyond 0.87-1.18; 160 to 224 to 328 from 2048 tokens on 1.05-1.18, to 384 from 3000 on 0.99-1.11, else 0.80-1.27
-//   two groups  (the joint grid loads K and V twice as often as with one)
-//               to 208     32 to 64 and 128 columns 1.00-1.55; 80 and 96 to 160 1.01-1.49, beyond from 513 tokens on 1.05-1.41 (below 0.96-
-//                          1.04); 160 and more to 144 1.05-1.29, beyond 0.84-1.08
-//               to 256     32 to 64 columns from 1500 tokens on 1.04-1.31, below 0.88-1.02; 128 from 2048 on 1.02-1.20, below 0.94-1.05; 80 and
-//                          96 0.90-1.03
-//               to 320     32 columns from 1500 tokens on 1.03-1.17, below 0.90-0.95 and beyond 0.87-1.01; the others 0.88-1.10
-//   beyond 512  (not padded heads, and to 1024 unless the heads divide by 8)
-//               80, 96     to 800 from 161 to 1100 tokens 0.98-1.20 (0.96 at 192 x 384, 128 x 768), else 0.85-1.10
-//               128        128 tokens 1.05-1.20; to 1300 workgroups, and from 1100 tokens on, to 2048 tokens 0.98-1.20; else 0.93-1.09
-//               256        96 to 128 tokens 1.05-1.29, 193 to 1100 0.98-1.16; 129 to 192 0.95-1.16, beyond 4096 workgroups from 513 tokens
-//                          on 0.95-1.04, past 1100 tokens 0.88-1.05
-//               others     32 columns 0.63-0.99, 48 and 64 0.74-1.17, 160 0.89-1.10, 192 0.91-1.12, 224 0.89-1.19, with no line to them
-// The order of the grid takes the two sequences to be of one length.  With many more keys than queries most workgroups of dK/dV see no
-// query, and it is padded with ones of dQ that do not exist: 32 x 512, 4096 keys 0.69 (192 columns) to 0.93 (64), 24 x 1024, 8192 keys 0.78
-// (96) to 0.85 (128), 64 x 192, 1536 keys 0.73 (192) to 0.94 (128), 1.5 times the keys 1.0-1.4.  Grids of more than 512 workgroups lose
-// with fewer keys too: 128 columns 0.90 (1024 x 192, 19 keys), 0.96 (128 x 1024, 819 keys), 256 columns 0.92 (256 x 1024, 102 keys).
-// The paired dK/dV kernel's conditions hold (above): where the other one is the better one, dK/dV is no part of such a grid.
+// Whether dQ and dK/dV run in one grid (fa2_bwd_joint.hpp) behind a launch that forms delta, and with how many key groups dQ: 0 where
+// two launches are as fast, dQ forming delta for dK/dV.  Time of the two launches over that of delta and the joint grid,
+// bf16, in turn in one process (7700 sizes: profiles/joint_backward_sweep.txt), as the middle nine tenths of the sizes that the lines take (beside
+// them of those they leave), by workgroups of 128 query rows; keys as many as queries:
+//   columns    to 128       to 160              to 208              to 256              to 352              to 512
+//   32         1.30-1.48    1.13-1.53           1.09-1.43           1.01-1.40           1.08-1.25 (1.01)    - (0.86-1.15)
+//   48, 64     1.30-1.62    1.21-1.47           1.12-1.43           1.05-1.31           1.06-1.16 (1.00)    1.02-1.13 (0.85-1.13)
+//   80, 96     1.29-1.60    1.20-1.46           1.05-1.38           1.01-1.20 (0.94)    1.04-1.18 (1.01)    1.04-1.15 (0.91-1.07)
+//   112, 128   1.22-1.65    1.14-1.41           1.00-1.36           1.01-1.26 (0.93)    1.00-1.26           0.94-1.17 (0.87-1.09)
+//   160-224    1.05-1.58    1.03-1.37 (0.99)    0.97-1.20 (0.97)    0.97-1.05 (0.93)    0.98-1.20           0.99-1.08 (0.91-1.06)
+//   256        1.08-1.70    1.09-1.36           1.04-1.23           0.98-1.08 (0.96)    1.03-1.27           1.01-1.12 (0.95-1.13)
+// Sequences of up to 128 or 256 tokens beside the lines 0.8-1.2.  To 128 workgroups dQ has the key groups it takes in front of a dK/dV kernel,
+// beyond one: 64 rows to a workgroup would load K and V twice as often, and two groups are 0.75-1.0 of its rate there (up to 1.1 times at
+// 32 to 64 columns and 129 to 512 tokens).  Beyond 512 workgroups two launches fill the chip as well, and what is gained is the end of the
+// first: inside the lines 0.97-1.16, in the geometric mean 1.05; padded heads, numbers of heads that do not divide by 8, 32 and 160 columns,
+// more than 2000 or 3000 workgroups 0.82-1.09, below 1.0 on the average.
+// Unlike lengths, by keys over queries: to 512 workgroups 0.1 to 4 inside the lines 0.93-1.66, in the geometric mean 1.2, and with a fifth of
+// the keys and fewer (512 tokens and more) 1.0-1.3 beside them as well; to 128 workgroups from 160 columns on 0.79-0.95 where short sequences
+// have more keys (64 x 256, 1024 keys 0.79).  With many more keys most workgroups of dK/dV see no query, and the grid, whose order takes the
+// lengths to be alike, is padded with ones of dQ that do not exist: 32 x 512 D=192, 4096 keys 0.69.
 inline int joint_key_groups_by_size(int dp, const BwdParams &p) {
   if (!dq_direct_ok(dp, p) || !dkdv_pair_ok(dp, p)) return 0;
   const int64_t heads = (int64_t)p.batch * p.nheads, wgs = heads * ((p.seqlen_q + kDqBlockQ - 1) / kDqBlockQ);
-  const int n = p.seqlen_q, groups = dq_key_groups(dp, p);
-  const int64_t nk = p.seqlen_k;
+  const int64_t n = p.seqlen_q, nk = p.seqlen_k;
+  const int cols = direct_columns(dp, p.headdim);
+  const bool wide = dp > 128, padded = p.headdim != cols;
   if (wgs > 2 * kCUs) {
-    if (p.headdim != direct_columns(dp, p.headdim) || (heads % 8 != 0 && wgs > 4 * kCUs) || nk < n || nk > n + (int64_t)n / 4) return 0;
+    if (padded || (heads % 8 != 0 && wgs > 4 * kCUs)) return 0;
+    if (wgs <= 4 * kCUs ? nk > 4 * n : wgs <= 2000 ? nk > 4 * n || 2 * nk < n : nk < n || nk > n + n / 4) return 0;
     if (dp == 64) return wgs <= 576 && n >= 1500 && heads % 8 == 0;
     if (dp == 96) return wgs <= 800 && n > 160 && n <= 1100;
-    if (dp == 128) return n >= 128 && n <= 2048 && (n == 128 || n >= 1100 || wgs <= 1300);
-    return p.headdim == 256 && n >= 96 && (n <= 128 || n > 192) && n <= (wgs <= 4096 ? 1100 : 512);
+    if (dp == 128) return n >= 128 && n <= 2048 && (n == 128 || wgs <= (n <= 400 || n >= 1100 ? 3000 : 2000));
+    if (cols == 256) return n >= 96 && n <= 1100 && (n <= 128 || wgs <= (n <= 192 ? 640 : 2000));
+    return cols >= 192 && n >= 96 && n <= 1100 && (n <= 128 || (n > 200 && (wgs <= 576 || (wgs > 1100 && wgs <= 2000))));
   }
-  if (nk > n + (int64_t)n / 2) return 0;
-  bool joint;
   if (wgs <= kCUs / 2) {
-    joint = dp > 128 ? wgs <= 64 || n > (wgs <= 96 ? 128 : 256) : wgs <= 96 || n > 128;
-  } else if (groups == 2) {
-    if (dp <= 64)
-      joint = wgs <= (n < 1500 ? 208 : dp == 32 ? 320 : 256);
-    else if (dp == 96)
-      joint = wgs <= (n > 512 ? 208 : 160);
-    else if (dp == 128)
-      joint = wgs <= (n < 2048 ? 208 : 256);
-    else
-      joint = wgs <= 144;
-  } else if (wgs <= kCUs) {
-    joint = wgs <= 160 ? n > (dp > 128 ? 255 : 128) : wgs <= 208 && n > (dp > 128 ? 767 : dp == 96 ? 512 : 256);
-  } else if (dp <= 64) {
-    joint = dp == 64 && n >= 1500 && (wgs <= 400 || heads % 8 == 0);
-  } else if (dp == 96) {
-    joint = n >= 768 && nk >= n;
-  } else if (dp == 128) {
-    joint = n >= 1500 || (p.headdim == 128 && n > 256 && wgs <= 448);
-  } else if (p.headdim == 256) {
-    joint = n >= 96 && wgs <= (n <= 128 || n >= 3000 ? 384 : 328);
-  } else {
-    joint = nk >= n && (wgs <= 328 ? n >= 2048 : wgs <= 384 && n >= 3000);
+    if (nk > (!wide || wgs <= 64 || n > 512 ? 4 : wgs <= 96 || n > 256 ? 2 : 1) * n) return 0;
+    return n > 128 || wgs <= (wide ? 64 : 96) ? dq_key_groups(dp, p) : 0;
   }
-  return joint ? groups : 0;
+  if (nk > 4 * n) return 0;
+  if (n >= 512 && 5 * nk <= n) return 1;
+  if (wgs <= kCUs) {
+    if (n <= 256) return wgs <= 160 && n > (wide ? 255 : 128);
+    if (dp == 96 || (dp == 128 && padded) || cols == 256) return wgs <= 208 || n > 512;
+    return !wide || wgs <= 176 || (n > 512 && (wgs <= 208 || n <= 3100));
+  }
+  if (dp <= 64) return n >= 1500 && wgs <= (dp == 32 ? 336 : heads % 8 ? 400 : 512);
+  if (!wide) return dp == 96 ? n >= 768 : n > 256;
+  if (cols == 256) return n >= 96 && wgs <= 384;
+  return wgs <= 352 ? n >= 96 : wgs <= 384 && n >= 3000;
 }
 // Whether such a grid can be launched, and the one that forms delta in front of it: a joint grid has up to three times the workgroups
 // of its larger kind.  Where not, two launches run, each with a limit of its own.
@@ -295,6 +273,13 @@ inline bool joint_fits(const BwdParams &p, int key_groups) {
 inline int joint_key_groups(int dp, const BwdParams &p) {
   const int groups = joint_key_groups_by_size(dp, p);
   return groups > 0 && joint_fits(p, groups) ? groups : 0;
+}
+// The key groups of dQ in a call of these sizes, whatever part of the gradient is asked for: so a call for a part gives the bits of a
+// call for all of it.  (dQ by itself would rather have two where the joint grid has one: 8 x 4096 D=128 58.5 us with two, 72.5 with
+// one; the whole backward 132 and, in the joint grid, 116.)
+inline int dq_key_groups_of_call(int dp, const BwdParams &p) {
+  const int joint = joint_key_groups(dp, p);
+  return joint > 0 ? joint : dq_key_groups(dp, p);
 }
 // Workgroup i's place in the order of its own kind (which may lie beyond the end of that).
 struct JointPlace {
@@ -359,7 +344,7 @@ void launch_preprocess(bool bf16, const PreParams &p, dim3 grid, hipStream_t s);
 // delta with the bits of the fast dQ kernel's own, for rows of whole chunks (p.vec); p.n_tiles is not read.
 void launch_delta(bool bf16, const PreParams &p, dim3 grid, hipStream_t s);
 // fuse_delta: the fast dQ kernel also forms delta from O and dO (dq_direct_ok must hold).
-void launch_dq(bool bf16, int dp, const BwdParams &p, dim3 grid, bool fuse_delta, hipStream_t s);
+void launch_dq(bool bf16, int dp, const BwdParams &p, int key_groups, dim3 grid, bool fuse_delta, hipStream_t s);
 // With p.dq_accum set the sequence-parallel kernel runs: dK, dV and atomic dQ contributions.
 void launch_dkdv(bool bf16, int dp, const BwdParams &p, dim3 grid, hipStream_t s);
 // dQ (of p.dq_tiles tiles) and dK/dV in one grid of joint_workgroups, both reading delta; a specialisation for each type.

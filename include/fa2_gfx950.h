@@ -195,8 +195,8 @@ int fa2_pick_config(int dtype, int headdim, int seqlen_q, int seqlen_k, int dete
 
 /*
  * The kernels a forward and a backward of these sizes launch, for 16-byte aligned contiguous tensors.
- * dq and dkdv are those of launches of their own, as when only one of them is asked for; a backward that
- * wants all of dq, dk and dv may run both kinds of workgroup in one grid (fa2_joint_info_get).
+ * dq and dkdv are those of a backward in two launches.  Where one grid forms dq, dk and dv instead
+ * (fa2_joint_info_get), dQ has the key groups stated there, also in a call for dq alone.
  * Touches no device.  No counterpart in the reference.  A forward-only row (fwd_exp_folded) has no
  * backward: dq and dkdv come back all zero.
  */
@@ -208,8 +208,8 @@ int fa2_launch_info_get(int batch, int nheads, int seqlen_q, int seqlen_k, int h
  * (joint_key_groups in csrc/fa2_launch.hpp), for 16-byte aligned contiguous tensors: form FA2_FORM_JOINT, the
  * query rows and the key groups of its dQ workgroups (those of dK/dV take what dkdv states), and all of its
  * workgroups.  All zero where two launches run, those of fa2_launch_info_get.  Where delta is formed on the
- * way, a launch in front of the joint grid forms it: bwd_delta_kernel where dQ by itself has at most 256
- * workgroups, else bwd_preprocess_kernel.  Touches no device.  No counterpart in the reference.
+ * way, a launch in front of the joint grid forms it: bwd_delta_kernel where dq of fa2_launch_info has at
+ * most 256 workgroups, else bwd_preprocess_kernel.  Touches no device.  No counterpart in the reference.
  */
 int fa2_joint_info_get(int batch, int nheads, int seqlen_q, int seqlen_k, int headdim, int config_id,
                        fa2_launch_part *out);

@@ -1,6 +1,6 @@
 // Host-side (run on the CPU by tests/test_joint_backward.py): reads "heads seqlen_q seqlen_k seqlen_q_rounded headdim" per line and
-// writes, for contiguous aligned tensors of one batch, the key groups of a dQ launch by itself, those of a joint grid (0: two
-// launches) and that grid's workgroups.
+// writes, for contiguous aligned tensors of one batch, the key groups of dQ in a call for it alone, those of a joint grid (0: two
+// launches), that grid's workgroups, and the key groups of dQ in front of a dK/dV kernel.
 #include <cstdio>
 
 #include "fa2_common.hpp"
@@ -17,7 +17,7 @@ int main() {
     const long long heads = p.nheads, rows = groups > 0 ? fa2::kDqBlockQ / groups : 1;
     const long long n_dq = (p.seqlen_q + rows - 1) / rows * heads;
     const long long n_dkdv = (p.seqlen_k + fa2::kDkvPairBlockKV - 1ll) / fa2::kDkvPairBlockKV * heads;
-    std::printf("%d %d %lld\n", fa2::dq_key_groups(dp, p), groups,
-                groups > 0 ? (long long)fa2::joint_workgroups(n_dq, n_dkdv, fa2::joint_period(groups)) : 0ll);
+    std::printf("%d %d %lld %d\n", fa2::dq_key_groups_of_call(dp, p), groups,
+                groups > 0 ? (long long)fa2::joint_workgroups(n_dq, n_dkdv, fa2::joint_period(groups)) : 0ll, fa2::dq_key_groups(dp, p));
   }
 }

@@ -460,8 +460,9 @@ def test_launch_info_knows_grids_of_two_kinds(capi):
     part = dict(form="joint", block_rows=64, key_groups=2, wg_per_cu=3, resident=1, workgroups=128)
     assert capi.joint_info(2, 4, 512, 512, 64) == part  # 64 workgroups of 64 rows and 64 of 64 keys
     assert capi.joint_info(1, 32, 2048, 2048, 64) == {**part, "block_rows": 128, "key_groups": 1, "resident": 0, "workgroups": 3 * 512}
-    assert capi.joint_info(1, 8, 4096, 4096, 128) == {**part, "wg_per_cu": 2, "resident": 0, "workgroups": 2 * 512}
-    for sizes in [(2, 32, 4096, 4096, 128), (2, 4, 512, 769, 64), (1, 8, 100, 100, 50)]:  # large; longer keys; no 16-byte rows
+    assert capi.joint_info(1, 8, 4096, 4096, 128) == {**part, "block_rows": 128, "key_groups": 1, "wg_per_cu": 2, "resident": 0, "workgroups": 768}
+    assert capi.launch_info(1, 8, 4096, 4096, 128)["dq"]["key_groups"] == 2  # in front of a dK/dV kernel; two launches are not what runs
+    for sizes in [(2, 32, 4096, 4096, 128), (2, 4, 512, 2049, 64), (1, 8, 100, 100, 50)]:  # large; longer keys; no 16-byte rows
         assert capi.joint_info(*sizes) is None
     for row in capi.config_table():
         if row["headdim_padded"] == 64 and (row["dq_atomic"] or row["fwd_exp_folded"]):

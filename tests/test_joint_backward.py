@@ -39,7 +39,8 @@ def test_every_workgroup_of_either_kind_once(tmp_path):
 
 @pytest.fixture(scope="module")
 def rule(tmp_path_factory):
-    """(heads, seqlen_q, seqlen_k, headdim[, seqlen_q_rounded]) ... -> (key groups of dQ by itself, of the joint grid, its workgroups) ..."""
+    """(heads, seqlen_q, seqlen_k, headdim[, seqlen_q_rounded]) ... -> (key groups of dQ in a call for it alone, of the joint grid, its
+    workgroups, key groups of dQ in front of dK/dV) ..."""
     program = _host_program("joint_rule.hip", tmp_path_factory.mktemp("rule"))
 
     def of(sizes):
@@ -53,40 +54,45 @@ def rule(tmp_path_factory):
 def test_a_grid_too_large_to_launch_is_two_launches(rule):
     """Sizes whose dQ and dK/dV grids can each be launched (16.7 million workgroups), but not the joint one; and rows of delta
     beyond what the launch in front of it takes, where dQ can form delta by itself."""
-    assert [groups for _, groups, _ in rule([
+    assert [groups for _, groups, _, _ in rule([
         (1, 100, 540_000_000, 8), (8_000_000, 128, 128, 128), (6_000_000, 128, 128, 256), (17, 1000, 1000, 64, 2**31 - 1)])] == [0] * 4
-    for _, groups, workgroups in rule([(h, n, nk, d) for h in (8, 1 << 16, 1 << 20, 3 << 20, 1 << 22, 8_000_000, 12_000_000)
-                                       for n in (96, 128, 700) for nk in (1, 128, 700, 100_000) for d in (64, 96, 128, 256)]):
+    for _, groups, workgroups, _ in rule([(h, n, nk, d) for h in (8, 1 << 16, 1 << 20, 3 << 20, 1 << 22, 8_000_000, 12_000_000)
+                                          for n in (96, 128, 700) for nk in (1, 128, 700, 100_000) for d in (64, 96, 128, 256)]):
         assert workgroups <= 0xFFFFFFFF // 256
 
 
-def test_dq_takes_the_key_groups_it_takes_by_itself(rule):
-    """The joint grid's dQ sums in the order of a dQ launch of its own: the same bits, whatever part of the gradient is asked for."""
+def test_a_call_for_dq_alone_takes_the_key_groups_of_the_whole_backward(rule):
+    """Sums in the same order, so the same bits, whatever part of the gradient is asked for."""
     sizes = [(h, n, n, d) for d in (32, 40, 48, 64, 72, 80, 96, 104, 128, 160, 176, 192, 224, 256)
              for n in (64, 100, 129, 256, 333, 512, 640, 1000, 1500, 2048, 3000, 4096, 5000, 8192) for h in (*range(1, 70), 80, 96, 128, 200, 512, 1024)]
     got = rule(sizes)
-    assert all(joint in (0, alone) for alone, joint, _ in got)
-    assert {joint for _, joint, _ in got} == {0, 1, 2}
+    assert all(alone == (joint or two_launches) for alone, joint, _, two_launches in got)
+    assert {(joint, two_launches) for _, joint, _, two_launches in got} == {(0, 1), (0, 2), (1, 1), (1, 2), (2, 2)}
 
 
-def test_unlike_lengths_are_two_launches(rule):
+def test_unlike_lengths(rule):
     """On both sides of each line of seqlen_k; what the sizes measured is at joint_key_groups."""
-    sizes = [(32, 512, 768, 192), (32, 512, 769, 192), (32, 512, 4096, 64), (32, 512, 1, 64),  # 128 workgroups of 128 rows
-             (24, 1024, 1536, 96), (24, 1024, 8192, 96), (256, 512, 512, 256), (256, 512, 511, 256), (256, 512, 640, 256), (256, 512, 641, 256)]
-    assert [groups for _, groups, _ in rule(sizes)] == [2, 0, 0, 2, 2, 0, 1, 0, 1, 0]
+    sizes = [(32, 512, 2048, 64), (32, 512, 2049, 64), (32, 512, 1, 64), (32, 512, 1024, 192), (32, 512, 1025, 192), (64, 256, 257, 160), (64, 256, 256, 160),
+             (48, 256, 512, 256), (48, 256, 513, 256), (3, 4096, 16384, 256),  # 128 workgroups of 128 rows
+             (16, 2048, 8192, 128), (16, 2048, 8193, 128), (64, 512, 102, 96), (64, 512, 103, 96), (8, 4096, 819, 192), (8, 4096, 820, 192), (128, 256, 25, 160),  # 512
+             (128, 1024, 2048, 128), (128, 1024, 300, 128), (128, 1024, 4097, 128), (256, 512, 2048, 256), (256, 1024, 4096, 256),  # 2000
+             (160, 1024, 512, 128), (160, 1024, 511, 128), (264, 1100, 1300, 128), (264, 1100, 1400, 128), (2048, 128, 160, 128), (2048, 128, 161, 128), (2048, 128, 127, 128)]
+    assert [groups for _, groups, _, _ in rule(sizes)] == [2, 0, 2, 2, 0, 0, 2, 2, 0, 2,
+                                                           1, 0, 1, 0, 1, 0, 0, 1, 1, 0, 1, 0, 1, 0, 1, 0, 1, 0, 0]
 
 
 @pytest.mark.parametrize("heads,n,d,groups", [
-    (96, 128, 64, 2), (97, 64, 64, 0), (64, 128, 256, 2), (65, 64, 192, 0), (48, 129, 160, 2), (64, 200, 224, 0), (64, 192, 256, 0), (42, 300, 192, 2),  # 128
-    (80, 192, 128, 1), (80, 192, 160, 0), (80, 256, 160, 1), (67, 300, 128, 1), (84, 256, 128, 0), (34, 768, 192, 1), (48, 512, 256, 0), (64, 512, 160, 0),  # 256
-    (80, 256, 64, 2), (56, 512, 64, 0), (32, 1024, 64, 0), (16, 2048, 64, 2), (64, 512, 128, 0), (8, 4096, 128, 2), (32, 1024, 128, 0),
-    (20, 1024, 96, 2), (24, 1024, 80, 2), (64, 333, 80, 0), (32, 1024, 96, 0), (17, 1024, 192, 2), (20, 1024, 160, 0),
-    (12, 3000, 32, 2), (16, 3000, 32, 0), (24, 2048, 64, 0), (32, 2048, 64, 1), (33, 2048, 64, 0), (24, 2048, 96, 0), (32, 2048, 80, 1),  # 512
-    (12, 4096, 128, 0), (112, 512, 128, 1), (128, 512, 128, 0), (96, 320, 112, 0), (32, 2048, 112, 1), (160, 192, 192, 0), (20, 2048, 192, 1),
-    (24, 2048, 192, 0), (12, 4096, 192, 1), (80, 512, 224, 0), (80, 512, 256, 1), (96, 512, 256, 0), (384, 64, 256, 0), (384, 128, 256, 1),
-    (256, 512, 224, 0), (640, 200, 224, 0), (1280, 192, 224, 0), (1280, 256, 160, 0), (1280, 256, 192, 0), (640, 160, 96, 0), (640, 161, 96, 0),  # beyond
-    (200, 512, 80, 1), (224, 512, 96, 0), (1024, 128, 128, 1), (1024, 256, 128, 0), (1024, 1024, 128, 0), (256, 1100, 128, 1), (4096, 512, 128, 0),
-    (520, 192, 256, 0), (520, 256, 256, 1), (1024, 512, 256, 1), (1024, 700, 256, 0), (1024, 1024, 64, 0), (4096, 512, 64, 0), (512, 2048, 32, 0)])
+    (96, 128, 64, 2), (97, 64, 64, 0), (64, 128, 256, 2), (65, 64, 192, 0), (48, 129, 160, 2), (64, 200, 224, 2), (42, 300, 192, 2),  # 128
+    (80, 192, 128, 1), (80, 192, 160, 0), (80, 256, 160, 1), (84, 256, 128, 0), (67, 300, 128, 1), (64, 512, 128, 1), (8, 4096, 128, 1),  # 256
+    (64, 512, 96, 0), (52, 512, 96, 1), (56, 513, 80, 0), (48, 640, 80, 1), (64, 500, 112, 0), (48, 640, 112, 1), (44, 500, 192, 1), (48, 512, 192, 0),
+    (40, 640, 192, 1), (8, 3100, 224, 1), (9, 3200, 224, 0), (52, 512, 256, 1), (56, 512, 256, 0), (48, 640, 256, 1), (16, 2048, 64, 1),
+    (14, 3000, 32, 1), (15, 3000, 32, 0), (24, 2048, 64, 1), (33, 2048, 64, 0), (32, 2048, 64, 1), (24, 2048, 96, 1), (48, 767, 96, 0), (48, 768, 96, 1),  # 512
+    (128, 512, 128, 1), (150, 256, 128, 0), (96, 320, 112, 1), (176, 192, 192, 1), (177, 192, 192, 0), (16, 3000, 160, 1), (17, 3000, 160, 0),
+    (12, 4096, 192, 1), (384, 96, 256, 1), (385, 96, 256, 0),
+    (576, 128, 224, 1), (600, 200, 224, 0), (72, 1000, 192, 1), (80, 1000, 192, 0), (288, 512, 224, 1), (256, 512, 224, 0), (1280, 192, 224, 0),  # beyond
+    (1280, 256, 160, 0), (400, 160, 96, 0), (400, 161, 96, 1), (200, 512, 80, 1), (224, 512, 96, 0), (4096, 128, 128, 1), (1496, 256, 128, 1),
+    (1504, 256, 128, 0), (256, 1024, 128, 0), (248, 1024, 128, 1), (256, 1100, 128, 1), (520, 192, 256, 0), (320, 192, 256, 1), (328, 192, 256, 0), (1024, 100, 256, 1),
+    (1024, 512, 256, 0), (1024, 1024, 64, 0), (512, 2048, 32, 0), (640, 512, 112, 0), (36, 2048, 64, 0), (32, 2300, 64, 1)])
 def test_joint_only_where_it_measured_faster(rule, heads, n, d, groups):
     """Both sides of the lines of joint_key_groups."""
     assert rule([(heads, n, n, d)])[0][1] == groups
