@@ -275,8 +275,9 @@ inline int joint_key_groups(int dp, const BwdParams &p) {
   return groups > 0 && joint_fits(p, groups) ? groups : 0;
 }
 // The key groups of dQ in a call of these sizes, whatever part of the gradient is asked for: so a call for a part gives the bits of a
-// call for all of it.  (dQ by itself would rather have two where the joint grid has one: 8 x 4096 D=128 58.5 us with two, 72.5 with
-// one; the whole backward 132 and, in the joint grid, 116.)
+// call for all of it.  (dQ by itself would rather have two where the joint grid has one: 8 x 4096 D=128 58.3 us with two, 74.2 with
+// one, 32 x 1024 D=256 41.3 and 42.6; the whole backward 132 in two launches and 116 in
+// the joint grid, 91.8 and 85.1.)
 inline int dq_key_groups_of_call(int dp, const BwdParams &p) {
   const int joint = joint_key_groups(dp, p);
   return joint > 0 ? joint : dq_key_groups(dp, p);

@@ -312,7 +312,8 @@ size_t fa2_bwd_workspace_bytes(int batch, int nheads, int seqlen_q, int seqlen_k
  * dK/dV and dQ are computed by two kernels launched back to back on `stream`, or by workgroups of both
  * kinds in one grid where that is faster (fa2_joint_info_get).  A caller that needs only part of the
  * gradient (or wants to time one kernel) may pass dq == NULL to skip dQ, or dk == dv == NULL to skip dK
- * and dV; what is left has the bits it has in a call for all of it.  dk and dv are given or omitted
+ * and dV; what is left has the bits it has in a call for all of it (for which dq alone sums in the joint
+ * grid's order, and may take up to 1.4 times what the order of two launches takes).  dk and dv are given or omitted
  * together, and at least one of the two groups must be present.
  */
 int fa2_bwd(const void *q, const void *k, const void *v, const void *d_o,
