@@ -154,7 +154,9 @@ def test_part_of_the_gradient_has_the_bits_of_all_of_it(capi, heads, n, d, dtype
     (41, 300, 333, 32, torch.bfloat16), (32, 1024, 1024, 64, torch.float16), (27, 1153, 1100, 72, torch.bfloat16),
     (11, 3000, 3000, 96, torch.bfloat16), (43, 500, 500, 256, torch.bfloat16), (60, 200, 200, 176, torch.bfloat16),
     (136, 520, 520, 128, torch.bfloat16), (136, 520, 520, 120, torch.bfloat16), (200, 512, 500, 80, torch.bfloat16), (200, 512, 520, 80, torch.float16),  # more than 512
-    (300, 100, 260, 160, torch.bfloat16), (520, 120, 120, 256, torch.bfloat16)], ids=lambda x: str(x).replace("torch.", ""))
+    (300, 100, 260, 160, torch.bfloat16), (520, 120, 120, 256, torch.bfloat16),
+    (33, 500, 2000, 64, torch.bfloat16), (64, 512, 60, 96, torch.float16), (17, 2048, 300, 128, torch.bfloat16), (33, 512, 1000, 192, torch.float16),  # unlike lengths
+    (176, 192, 192, 192, torch.bfloat16), (72, 1000, 1000, 192, torch.bfloat16), (576, 128, 128, 224, torch.float16)], ids=lambda x: str(x).replace("torch.", ""))
 def test_gradients_at_the_edges_of_the_rule(fa, heads, nq, nk, d, dtype):
     gen = torch.Generator(device="cuda").manual_seed(nq + heads)
     q, d_o = (torch.randn(1, heads, nq, d, generator=gen, device="cuda").to(dtype) for _ in range(2))
